@@ -19,6 +19,7 @@ HIP_SOURCES = [
     "kernels/gemv_generic.hip",
     "kernels/gemv_nbits.hip",
     "kernels/gemv_f32.hip",
+    "kernels/gemm_f32.hip",
     "kernels/decode_mfma.hip",
     "kernels/decode_packed.hip",
     "kernels/prefill_mfma.hip",

@@ -432,6 +432,9 @@ bool f32_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
     return true;
 }
 
+// Narrower f32 calls than this keep the streaming kernel and the catch-all; no projection of a model is that narrow.
+constexpr int64_t kGemmF32MinCols = 128;
+
 // The RMS-normalization prologue of a node on its way through the dispatch: the decode kernels over the repacked stream
 // apply it themselves (up to four rows); every other route first normalizes the rows into `owner`'s buffer with a
 // launch of its own.
@@ -734,6 +737,9 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         }
         rc = rocm_launch_prefill_mfma(&args, kn.ep->prefill_tile, scratch, scratch_bytes, stream);
         kn.variant = "prefill_mfma_lds";
+    } else if (args.n >= kGemmF32MinCols && rocm_gemm_f32_eligible(&args) && rocm_gemm_f32_pays(&args)) {
+        rc = rocm_launch_gemm_f32(&args, stream);
+        kn.variant = "gemm_f32_mfma";
     } else if (M <= 64 && f32_in_row_blocks(kn, args, rc)) {
         // done: f32 activations stay in f32 arithmetic end to end
     } else {

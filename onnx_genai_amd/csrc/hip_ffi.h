@@ -145,6 +145,11 @@ int rocm_launch_gemv_generic(const RocmMatMulNBitsArgs* args, rocm_stream_t stre
 /* f32 activations, M <= 4, block size >= 32, K % 4 == 0, A and B 16-byte aligned: f32 FMA streaming kernel */
 int rocm_gemv_f32_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_gemv_f32(const RocmMatMulNBitsArgs* args, rocm_stream_t stream);
+/* f32 activations, any M, block size >= 32, K % 4 == 0, A 16-byte and B 8-byte aligned: the activations cut into three bf16
+ * parts, the weights as bf16 integers, f32 sums on the matrix cores */
+int rocm_gemm_f32_eligible(const RocmMatMulNBitsArgs* args);
+int rocm_gemm_f32_pays(const RocmMatMulNBitsArgs* args);      /* 1: by its shape, ahead of passes of rocm_launch_gemv_f32 */
+int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* args, rocm_stream_t stream);
 
 /* Decode (M <= 16), f16/bf16 activations: split-K MFMA GEMV. Returns -1 when the shape is not eligible.
  * waves/col_groups = 0 lets the launcher choose. */

@@ -1,0 +1,294 @@
+// f32 activations at more than a few rows (block size >= 32, K % 4 == 0): the matrix cores with nothing rounded below f32.
+//
+// An f32 value is the exact sum of three bf16 values (its 24 significant bits cut in three runs of eight), and q - zp, an
+// integer of at most four bits and a sign, is a bf16 value as it stands. So
+//   y += scale * (sum a1*(q-zp) + sum a2*(q-zp) + sum a3*(q-zp))
+// over a run of 32 weights of one block, with products that are exact and sums in f32: the reference's fp32 route
+// (matmul_nbits.rs:7499-7566), three MFMAs where the f32 form of the instruction would take sixteen times the cycles of one.
+//
+// A wave works alone on its share of K out of registers, the next runs' loads in flight: no LDS and no barrier until the waves of
+// a workgroup, which split K between them, add up their sums in wave order at the end. Short grids get their parallelism from
+// that split.
+// Measured (block 32, f32 scales; the catch-all and, up to 64 rows, passes of the four-row streaming kernel before): 896 -> 4864
+// at 200 rows 1665 -> 23 us (75 TFLOP/s), 4864 -> 896 at 200 rows 2219 -> 33 us, 896 -> 9728
+// at 512 rows 8373 -> 69 us, 896 -> 896 at 64 rows 97 -> 5.8 us. What bounds it: a CU's vector memory path, which serves a load's 32 rows or columns
+// one cache line at a time (five to nine such loads per run of 32 k), then the vector ALU work of cutting activations and turning nibbles into
+// bf16 (about 120 instructions per lane, tile and run with two column tiles per wave, against 6 MFMAs of 32 cycles).
+#include "prefill_common.hiph"
+
+namespace mnb {
+
+struct GemmF32Params {
+    const float* a;
+    const uint8_t* b;
+    const void* scales;
+    const uint8_t* zp;
+    const void* bias;
+    void* y;
+    int64_t m, n, k, kb;
+    int64_t row_bytes, zp_row;
+    int bs_log2;
+    int scale_dtype, bias_dtype, y_dtype;
+    int units_per_wave;     // runs of 32 k a wave walks
+};
+
+// 8 * GROUPS f32 values as three bf16 operands each: plane[p][group].
+template <int GROUPS>
+__device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], uint4 (&plane)[3][GROUPS])
+{
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+        uint32_t out[3][4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t lo = v[8 * g + 2 * i], hi = v[8 * g + 2 * i + 1];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                out[p][i] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);      // the upper halves: both values cut to bf16
+                if (p < 2) {                                                // what the cut leaves, exactly
+                    lo = __float_as_uint(__uint_as_float(lo) - __uint_as_float(lo & 0xffff0000u));
+                    hi = __float_as_uint(__uint_as_float(hi) - __uint_as_float(hi & 0xffff0000u));
+                }
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p) plane[p][g] = make_uint4(out[p][0], out[p][1], out[p][2], out[p][3]);
+    }
+}
+
+// Eight nibbles of a packed dword as bf16 integers q - zp in element order; `shift` is 16 - zp in every byte.
+__device__ __forceinline__ uint4 nibbles_as_bf16(uint32_t w, uint32_t shift) { return dequant_dword_f32<true>(w, shift, 1.0f, -16.0f); }
+
+// The matrix-core step and the shape of its operands for tiles of 32 x 32 (16 k per MFMA, a run is two of them) and of
+// 16 x 16 (32 k per MFMA: a run is one). An operand lane holds 8 k of one row or column per MFMA.
+typedef __attribute__((ext_vector_type(4))) float f32x4_acc_t;
+template <int TILE> struct TileOps;
+template <> struct TileOps<32> {
+    using acc_t = float16_t;
+    static constexpr int kMfmas = 2, kAcc = 16;
+    static __device__ __forceinline__ acc_t mfma(const uint4& a, const uint4& b, acc_t c) { return mfma32<true>(a, b, c); }
+    static __device__ __forceinline__ int row_of(int e, int lane) { return (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3); }
+};
+template <> struct TileOps<16> {
+    using acc_t = f32x4_acc_t;
+    static constexpr int kMfmas = 1, kAcc = 4;
+    static __device__ __forceinline__ acc_t mfma(const uint4& a, const uint4& b, acc_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0); }
+    static __device__ __forceinline__ int row_of(int e, int lane) { return (lane >> 4) * 4 + e; }
+};
+
+// TILE: 16 or 32 rows and columns per matrix-core tile. CN: tiles along N per wave. DEPTH: runs in flight. WAVES: the most
+// waves a workgroup is launched with. ST: float, or uint16_t for f16 / bf16 scales.
+template <int TILE, int CN, int DEPTH, int WAVES, typename ST>
+__global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
+{
+    using Ops = TileOps<TILE>;
+    using acc_t = typename Ops::acc_t;
+    constexpr int G = Ops::kMfmas;                         // groups of 8 k a lane holds of a run
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int t = threadIdx.x;
+    const int lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int waves = static_cast<int>(blockDim.x >> 6);
+    const int r = lane & (TILE - 1), part = lane / TILE;   // operand row (A) or column (B), and which 8 G of a run's 32 k
+    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * TILE;
+    const int64_t n_base = static_cast<int64_t>(blockIdx.x) * (TILE * CN);
+    const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
+
+    const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.a + m_base * p.k, static_cast<uint64_t>(rows_left * p.k) * 4);
+    const __amdgpu_buffer_rsrc_t srd_b = make_srd(p.b + n_base * p.row_bytes, static_cast<uint64_t>(cols_left * p.row_bytes));
+    const __amdgpu_buffer_rsrc_t srd_s = make_srd(static_cast<const ST*>(p.scales) + n_base * p.kb, static_cast<uint64_t>(cols_left * p.kb) * sizeof(ST));
+    const __amdgpu_buffer_rsrc_t srd_z = make_srd(p.zp ? p.zp + n_base * p.zp_row : nullptr, p.zp ? static_cast<uint64_t>(cols_left * p.zp_row) : 0);
+    const uint32_t zp_mask = p.zp ? 0xfu : 0u, zp_default = p.zp ? 0u : 8u;
+    const bool scale_bf16 = p.scale_dtype == ROCM_DT_BF16;
+
+    const uint32_t a_off = static_cast<uint32_t>(r) * static_cast<uint32_t>(p.k) * 4u;
+    const bool row_live = r < rows_left;
+    uint32_t b_off[CN], s_off[CN], z_off[CN];
+#pragma unroll
+    for (int j = 0; j < CN; ++j) {                         // a column beyond N lies out of range by itself
+        b_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(part * 4 * G);
+        s_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.kb) * static_cast<uint32_t>(sizeof(ST));
+        z_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.zp_row);
+    }
+
+    struct Run {
+        u32x4_t a[2 * G];
+        uint32_t b[CN][G];
+        typename ScaleIo<ST>::raw_t s[CN];
+        uint32_t z[CN];
+        uint32_t zsh;
+    };
+    const int u0 = wave * p.units_per_wave;
+    const int u1 = min(u0 + p.units_per_wave, static_cast<int>((p.kb << p.bs_log2) >> 5));
+    // No branch: a run past the wave's share, a row beyond M and elements beyond K get offsets out of range, which read zeros.
+    auto request = [&](Run& x, int u) {
+        const bool live = u < u1;
+        const int k0 = u * 32 + part * 8 * G;
+#pragma unroll
+        for (int i = 0; i < 2 * G; ++i) {
+            const uint32_t off = live && row_live && k0 + i * 4 < p.k ? a_off + static_cast<uint32_t>(k0 + i * 4) * 4u : kOutOfRange;
+            x.a[i] = __builtin_amdgcn_raw_buffer_load_b128(srd_a, static_cast<int>(off), 0, 0);
+        }
+        const uint32_t oor = live ? 0u : kOutOfRange;
+        const uint32_t blk = static_cast<uint32_t>(u * 32) >> p.bs_log2;
+#pragma unroll
+        for (int j = 0; j < CN; ++j) {
+            const int off = static_cast<int>((b_off[j] + static_cast<uint32_t>(u) * 16u) | oor);
+            if constexpr (G == 2) {
+                const auto w = __builtin_amdgcn_raw_buffer_load_b64(srd_b, off, 0, 0);
+                x.b[j][0] = w[0];
+                x.b[j][1] = w[1];
+            } else {
+                x.b[j][0] = __builtin_amdgcn_raw_buffer_load_b32(srd_b, off, 0, 0);
+            }
+            x.s[j] = ScaleIo<ST>::load_raw(srd_s, (s_off[j] + blk * static_cast<uint32_t>(sizeof(ST))) | oor, 0);
+            x.z[j] = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(srd_z, static_cast<int>((z_off[j] + (blk >> 1)) | oor), 0, 0));
+        }
+        x.zsh = (blk & 1u) * 4u;
+    };
+
+    acc_t sum[CN], zero;
+#pragma unroll
+    for (int e = 0; e < Ops::kAcc; ++e) {
+        zero[e] = 0.f;
+#pragma unroll
+        for (int j = 0; j < CN; ++j) sum[j][e] = 0.f;
+    }
+
+    auto multiply = [&](const Run& x) {
+        uint32_t v[8 * G];
+#pragma unroll
+        for (int i = 0; i < 2 * G; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * i + e] = x.a[i][e];
+        uint4 plane[3][G];
+        cut_in_three<G>(v, plane);
+#pragma unroll
+        for (int j = 0; j < CN; ++j) {
+            const uint32_t zq = ((x.z[j] >> x.zsh) & zp_mask) | zp_default;
+            const uint32_t shift = (16u - zq) * 0x01010101u;
+            uint4 w[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) w[g] = nibbles_as_bf16(x.b[j][g], shift);
+            acc_t acc = zero;
+#pragma unroll
+            for (int q = 2; q >= 0; --q)                                      // smallest parts first
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc = Ops::mfma(plane[q][g], w[g], acc);
+            const float sc = ScaleIo<ST>::to_f32(x.s[j], scale_bf16);         // 0 for a column beyond N and past the end
+#pragma unroll
+            for (int e = 0; e < Ops::kAcc; ++e) sum[j][e] = fmaf(acc[e], sc, sum[j][e]);
+        }
+    };
+
+    Run x[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d) request(x[d], u0 + d);
+    for (int u = u0; u < u1; u += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            request(x[(d + DEPTH - 1) % DEPTH], u + d + DEPTH - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(x[d]);
+        }
+    }
+
+    // ---- the waves' sums through LDS, added in wave order: [wave][tile][accumulator][64] ----
+    constexpr int kOuts = CN * Ops::kAcc * 64;
+    float* parts = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int j = 0; j < CN; ++j)
+#pragma unroll
+        for (int e = 0; e < Ops::kAcc; ++e) parts[((wave * CN + j) * Ops::kAcc + e) * 64 + lane] = sum[j][e];
+    __syncthreads();
+    for (int i = t; i < kOuts; i += static_cast<int>(blockDim.x)) {
+        float v = 0.f;
+        for (int w = 0; w < waves; ++w) v += parts[w * kOuts + i];
+        const int l = i & 63;
+        const int64_t row = m_base + Ops::row_of((i >> 6) & (Ops::kAcc - 1), l);
+        const int64_t col = n_base + (i / (Ops::kAcc * 64)) * TILE + (l & (TILE - 1));
+        if (row < p.m && col < p.n) store_from_f32(p.y, p.y_dtype, row * p.n + col, with_bias(v, p.bias, p.bias_dtype, row, p.n, col, p.y_dtype));
+    }
+}
+
+template <int TILE, int CN, int DEPTH, int WAVES, typename ST>
+static int launch_gemm_f32(const GemmF32Params& p, int waves, hipStream_t stream)
+{
+    const dim3 grid(static_cast<unsigned>((p.n + TILE * CN - 1) / (TILE * CN)), static_cast<unsigned>((p.m + TILE - 1) / TILE));
+    const size_t lds = static_cast<size_t>(waves) * CN * TileOps<TILE>::kAcc * 256;               // at most 64 KiB
+    hipLaunchKernelGGL((gemm_f32_kernel<TILE, CN, DEPTH, WAVES, ST>), grid, dim3(static_cast<unsigned>(waves * 64)), lds, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
+}  // namespace mnb
+
+extern "C" int rocm_gemm_f32_eligible(const RocmMatMulNBitsArgs* a)
+{
+    if (a->a_dtype != ROCM_DT_F32 || a->m < 1 || a->n < 1 || a->k < 1 || a->block_size < 32 || a->k % 4 != 0) return 0;
+    const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
+    if (kb * a->block_size / 2 * 64 >= 0x7ffffff0 || a->k * 4 * 32 >= 0x7ffffff0 || (a->m + 31) / 32 > 65535) return 0;    // 32-bit offsets inside one tile
+    return (reinterpret_cast<uintptr_t>(a->a) & 15) == 0 && (reinterpret_cast<uintptr_t>(a->b) & 7) == 0;
+}
+
+namespace {
+
+// Tiles, and waves that share K, by the grid they make (f32 scales, block 32; us):
+//   * 16 x 16 tiles while they make at most one workgroup per CU: 896 -> 896 at 64 rows 5.8 against 7.8 with 32 x 32, 4864 -> 896
+//     at 64 rows 21 against 31; with more of them they lose (896 -> 896 at 200 rows 12.9 against 7.9).
+//   * 32 x 32 otherwise, two of them per wave once single ones make more than one workgroup per CU: the cut activations are used
+//     twice (4864 -> 896 at 512 rows 47.5 against 61.7; at 200 rows, 196 workgroups, 46 against 33).
+//   * eight waves share K up to one workgroup per CU, four beyond (896 -> 9728 at 512 rows 69 against 91 us), each with two runs or more.
+struct F32Plan { int tile, cn, waves; };
+F32Plan plan_gemm_f32(const RocmMatMulNBitsArgs* a, int units, int64_t cus)
+{
+    auto workgroups = [&](int rows, int cols) { return ((a->m + rows - 1) / rows) * ((a->n + cols - 1) / cols); };
+    F32Plan plan{32, 1, 8};
+    if (workgroups(16, 16) <= cus) plan.tile = 16;
+    else if (workgroups(32, 32) > cus) plan.cn = 2;
+    if (workgroups(plan.tile, plan.tile * plan.cn) > cus) plan.waves = 4;
+    while (plan.waves > 1 && units < 2 * plan.waves) plan.waves >>= 1;
+    return plan;
+}
+
+}  // namespace
+
+// From five rows; up to eight rows only on grids of at most two workgroups per CU (3584 -> 18944 at eight rows: two passes of the
+// streaming kernel 41 us, 47 here; 896 -> 9728 at five rows: 13.1 against 9.3 us).
+extern "C" int rocm_gemm_f32_pays(const RocmMatMulNBitsArgs* a)
+{
+    return a->m > 8 || (a->m > 4 && (a->n + 31) / 32 <= 2 * static_cast<int64_t>(rocm_ffi_compute_units()));
+}
+
+extern "C" int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* a, rocm_stream_t stream)
+{
+    if (!rocm_gemm_f32_eligible(a)) return -1;
+    mnb::GemmF32Params p;
+    p.a = static_cast<const float*>(a->a);
+    p.b = a->b;
+    p.scales = a->scales;
+    p.zp = a->zp;
+    p.bias = a->bias;
+    p.y = a->y;
+    p.m = a->m;
+    p.n = a->n;
+    p.k = a->k;
+    p.kb = (a->k + a->block_size - 1) / a->block_size;
+    p.row_bytes = p.kb * a->block_size / 2;
+    p.zp_row = (p.kb + 1) / 2;
+    p.bs_log2 = __builtin_ctz(static_cast<unsigned>(a->block_size));
+    p.scale_dtype = a->scale_dtype;
+    p.bias_dtype = a->bias_dtype;
+    p.y_dtype = a->y_dtype;
+    const int64_t cus = rocm_ffi_compute_units();
+    const int units = static_cast<int>(p.kb * a->block_size / 32);
+    const F32Plan plan = plan_gemm_f32(a, units, cus);
+    const int tile = plan.tile, cn = plan.cn, waves = plan.waves;
+    p.units_per_wave = (units + waves - 1) / waves;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    auto go = [&](auto st) {
+        using ST = decltype(st);
+        if (tile == 16) return mnb::launch_gemm_f32<16, 1, 4, 8, ST>(p, waves, s);
+        return cn == 2 ? mnb::launch_gemm_f32<32, 2, 2, 8, ST>(p, waves, s) : mnb::launch_gemm_f32<32, 1, 2, 8, ST>(p, waves, s);
+    };
+    return a->scale_dtype == ROCM_DT_F32 ? go(float{}) : go(uint16_t{});
+}

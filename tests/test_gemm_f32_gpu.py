@@ -1,0 +1,47 @@
+"""f32 activations on the matrix cores (csrc/kernels/gemm_f32.hip): edges of its tiles, its split of K and its dispatch, against the oracle in double precision."""
+import numpy as np
+import pytest
+
+from onnx_genai_amd import ep as E
+from onnx_genai_amd import synth
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+# Products are exact (three bf16 parts of an activation times an integer of four bits and a sign) and every sum is an f32 sum: at most
+# K + K / 32 roundings of 2^-24 on the way to an output. As independent errors they add up to sqrt(4864 * 33 / 32) * 2^-24 = 4.2e-6 of the
+# terms' norm, which for these zero-mean operands is the output's norm.
+TOL = 4.2e-6
+
+CASES = [
+    # s_dt, bs, zero points, m, n, k, bias, y type
+    (E.F32, 32, False, 5, 128, 32, "none", E.F32),          # one run of K, one wave
+    (E.F32, 32, True, 5, 129, 896, "column", E.F32),        # 16 x 16 tiles, a ragged last column tile
+    (E.F32, 64, True, 17, 130, 900, "none", E.F32),         # ... a ragged last row tile and a partial last block
+    (E.F16, 128, True, 63, 140, 4100, "row", E.F32),
+    (E.F32, 256, False, 64, 128, 4864, "column", E.F16),
+    (E.F32, 32, True, 65, 1100, 68, "none", E.F32),         # 32 x 32 tiles, fewer runs than waves
+    (E.BF16, 32, True, 200, 900, 896, "row", E.BF16),
+    (E.F32, 64, False, 300, 1000, 516, "column", E.F32),    # two column tiles per wave, the second one beyond N in the last workgroup
+    (E.F16, 32, True, 513, 2017, 160, "none", E.F32),       # more workgroups than CUs: four waves
+    (E.F32, 128, True, 8, 16416, 256, "none", E.F32),       # five to eight rows on a wide call: the streaming kernel keeps it
+]
+
+
+@pytest.mark.parametrize("s_dt,bs,zero_points,m,n,k,bias_kind,y_dt", CASES)
+def test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, bias_kind, y_dt):
+    b, s, zp = synth.make_weights(n, k, bs, n + k, zero_points=zero_points, scale_lo=0.002, scale_hi=0.01, scale_dtype=s_dt)
+    rng = np.random.default_rng(m)
+    # magnitudes over 24 binary orders: all three parts of a value matter
+    a = (synth.make_activation(m, k, n, E.F32).astype(np.float64) * np.exp2(rng.integers(-12, 12, (m, 1)))).astype(np.float32)
+    bias = None if bias_kind == "none" else rng.standard_normal((m, n) if bias_kind == "row" else n).astype(np.float32)
+    y, variant = E.matmul_nbits(ep, a, E.F32, b, s, s_dt, zp, n, k, bs, bias=bias, y_dtype=y_dt)
+    assert variant == ("gemv_f32_valu" if (m, n) == (8, 16416) else "gemm_f32_mfma")
+    want = port.matmul_f64(a, b, synth.to_f32(s, s_dt), zp, n, k, bs)
+    if bias is not None:
+        want = want + bias.astype(np.float64)
+    got = synth.to_f32(y, y_dt).astype(np.float64)
+    # a narrow result adds its own rounding, half a unit of 2^-10 (f16) or 2^-7 (bf16), to each value
+    tol = TOL + {E.F32: 0.0, E.F16: 2.0 ** -11, E.BF16: 2.0 ** -8}[y_dt]
+    for row in range(m):                                    # by row: the rows differ in magnitude
+        assert helpers.rel_l2(got[row], want[row]) <= tol, row
