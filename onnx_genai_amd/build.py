@@ -16,6 +16,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_SOURCES = [
     "hip_ffi.hip",
     "kernels/dequant.hip",
+    "kernels/regroup.hip",
     "kernels/gemv_generic.hip",
     "kernels/gemv_nbits.hip",
     "kernels/gemv_f32.hip",

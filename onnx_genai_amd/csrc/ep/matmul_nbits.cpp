@@ -156,6 +156,13 @@ struct NxrtRocmMatMulNBits {
     void* dense = nullptr;               // constant weights expanded to the activations' 16-bit type, [N, K] (dense_weights = resident)
     const void* dense_from[3] = {nullptr, nullptr, nullptr};
     int dense_dtype = 0, dense_scale_dtype = 0;
+    // constant act-order weights sorted by group: the order of K ([K] int32, first in the allocation) and B in that order; null where
+    // g_idx has another form (`regroup_failed`: asked once per pair of tensors)
+    void* regrouped = nullptr;
+    const void* regrouped_from[2] = {nullptr, nullptr};          // B, g_idx
+    bool regroup_failed = false;
+    void* gathered = nullptr;            // the call's activations in that order
+    size_t gathered_bytes = 0;
     std::mutex mu;                       // one execute at a time per kernel object: scratch, repacked copy and variant are per-object state
     bool no_alloc = false;               // the call in progress (under `mu`) may not allocate or free device memory
     NxrtKernelVtable vtable;
@@ -169,13 +176,15 @@ struct NxrtRocmMatMulNBits {
     {
         delete gate;
         delete up;
-        if ((scratch || packed || dense || norm || !retired.empty()) && ep->bind().code == NXRT_OK) {
+        if ((scratch || packed || dense || norm || regrouped || gathered || !retired.empty()) && ep->bind().code == NXRT_OK) {
             rocm_ffi_stream_sync(ep->stream);
             if (norm) rocm_ffi_free(norm);
             for (void* old : retired) rocm_ffi_free(old);
             if (scratch) rocm_ffi_free(scratch);
             if (packed) rocm_ffi_free(packed);
             if (dense) rocm_ffi_free(dense);
+            if (regrouped) rocm_ffi_free(regrouped);
+            if (gathered) rocm_ffi_free(gathered);
         }
         nxrt_rocm_ep_release(ep);
     }
@@ -235,6 +244,55 @@ void drop_weight_copy(NxrtRocmMatMulNBits& kn, void* old)
     }
     rocm_ffi_stream_sync(kn.ep->stream);
     rocm_ffi_free(old);
+}
+
+// Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on
+// first use, args.a the call's activations in the same order, args.g_idx null. Returns false with `args` untouched where the groups
+// are not whole blocks, or the copy or the gather's buffer cannot be made now (a capture is open, no memory): the kernels that look
+// groups up per element take the call then. `rc` receives a HIP error.
+bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, int& rc)
+{
+    rc = 0;
+    if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[4]) return false;
+    const size_t order_bytes = (static_cast<size_t>(args.k) * sizeof(int32_t) + 255) / 256 * 256;
+    if (kn.regrouped_from[0] != args.b || kn.regrouped_from[1] != args.g_idx) {
+        if (frozen(kn)) return false;
+        if (kn.regrouped) {
+            drop_weight_copy(kn, kn.regrouped);
+            kn.regrouped = nullptr;
+        }
+        kn.packed_from[0] = kn.dense_from[0] = nullptr;            // copies made from the old one: a new one may lie at its address
+        kn.regroup_failed = true;
+        const size_t b_bytes = static_cast<size_t>(args.n) * ((args.k + args.block_size - 1) / args.block_size) * static_cast<size_t>(args.block_size * kn.bits / 8);
+        int regular = 0;
+        if (args.block_size * kn.bits % 32 == 0 && rocm_ffi_malloc(&kn.regrouped, order_bytes + b_bytes) == 0) {
+            int32_t* const order = static_cast<int32_t*>(kn.regrouped);
+            rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, order, &regular, kn.ep->stream);
+            if (rc == 0 && regular)
+                rc = rocm_launch_regroup(args.b, order, args.n, args.k, args.block_size, static_cast<int>(kn.bits), static_cast<uint8_t*>(kn.regrouped) + order_bytes, kn.ep->stream);
+            if (rc != 0 || !regular) {
+                rocm_ffi_free(kn.regrouped);
+                kn.regrouped = nullptr;
+                if (rc != 0) return false;
+            } else {
+                kn.regroup_failed = false;
+            }
+        } else {
+            kn.regrouped = nullptr;
+        }
+        kn.regrouped_from[0] = args.b;
+        kn.regrouped_from[1] = args.g_idx;
+    }
+    if (kn.regroup_failed) return false;
+    const size_t need = static_cast<size_t>(args.m) * static_cast<size_t>(args.k) * (args.a_dtype == ROCM_DT_F32 ? 4 : 2);
+    if (kn.gathered_bytes < need && (frozen(kn) || grow_buffer(kn.gathered, kn.gathered_bytes, need, kn.retired) != 0)) return false;
+    const int32_t* const order = static_cast<const int32_t*>(kn.regrouped);
+    rc = rocm_launch_gather_columns(args.a, args.a_dtype, order, args.m, args.k, kn.gathered, kn.ep->stream);
+    kn.ep->launches.fetch_add(1);
+    args.a = kn.gathered;
+    args.b = static_cast<const uint8_t*>(kn.regrouped) + order_bytes;
+    args.g_idx = nullptr;
+    return true;
 }
 
 // True when the call can run on the repacked copy of constant weights; makes that copy on first use (never while a
@@ -647,13 +705,16 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         if (bad >= 0) return make_status(NXRT_INVALID_ARGUMENT, err("g_idx[" + std::to_string(bad) + "] is outside 0.." + std::to_string(kb)));
         kn.g_idx_checked = args.g_idx;
     }
-    if (kn.bits != 4 || G) {
-        // 2 and 8 bits, and act-order weights of any width: 16-bit calls from five rows expand the weights and run the tiled
+    const bool sorted = G && sort_by_group(kn, args, rc);
+    if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
+    if (kn.bits != 4 || args.g_idx) {
+        // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
         if (!dense_route(kn, args, rc)) {
             rc = rocm_launch_gemv_nbits(&args, static_cast<int>(kn.bits), stream);
             kn.variant = "gemv_nbits_f32";
         }
+        if (sorted) kn.variant = "act_order+" + kn.variant;
         kn.ep->launches.fetch_add(1);
         return hip_status(rc, "MatMulNBits: kernel launch");
     }
@@ -746,6 +807,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         rc = rocm_launch_gemv_generic(&args, stream);
         kn.variant = "gemv_generic_f32";
     }
+    if (sorted) kn.variant = "act_order+" + kn.variant;
     kn.ep->launches.fetch_add(1);
     return hip_status(rc, "MatMulNBits: kernel launch");
 }

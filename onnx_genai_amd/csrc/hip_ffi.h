@@ -140,6 +140,14 @@ int rocm_launch_dequant_gidx(const uint8_t* b, const void* scales, int scale_dty
 /* First index whose group lies outside 0..kb, or -1: synchronizes the stream and allocates (never inside a graph capture). */
 int rocm_g_idx_first_bad(const int32_t* g_idx, int64_t count, int64_t kb, int64_t* first_bad, rocm_stream_t stream);
 
+/* Act-order weights whose groups are whole blocks of K in another order (elements of group g: block_size, or what K leaves for the last):
+ * `order` (device, [K]) receives the elements of K group by group and *regular 1; *regular 0 and nothing written when the groups
+ * are not of that form. Synchronizes (never inside a graph capture). regroup: B'[n, j] = B[n, order[j]] in B's layout (row dwords
+ * of kb * block_size * bits / 32), for any of the widths; gather_columns: A'[m, j] = A[m, order[j]]. */
+int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, int* regular, rocm_stream_t stream);
+int rocm_launch_regroup(const uint8_t* b, const int32_t* order, int64_t n, int64_t k, int block_size, int bits, void* out, rocm_stream_t stream);
+int rocm_launch_gather_columns(const void* a, int a_dtype, const int32_t* order, int64_t m, int64_t k, void* out, rocm_stream_t stream);
+
 /* Any dtype mix, any K, any block size: f32 math, one wave per output column. */
 int rocm_launch_gemv_generic(const RocmMatMulNBitsArgs* args, rocm_stream_t stream);
 /* f32 activations, M <= 4, block size >= 32, K % 4 == 0, A and B 16-byte aligned: f32 FMA streaming kernel */

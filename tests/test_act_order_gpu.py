@@ -1,0 +1,105 @@
+"""Act-order weights whose groups are whole blocks in another order: sorted once, then served by the kernels for contiguous blocks."""
+import numpy as np
+import pytest
+
+from onnx_genai_amd import ep as E
+from onnx_genai_amd import synth
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+TOL = {E.F32: 1e-5, E.F16: 5e-3, E.BF16: 5e-3}      # the bars of the parity contract
+
+
+def weights(n, k, bs, bits, dt, seed):
+    if bits == 4:
+        return synth.make_weights(n, k, bs, seed, zero_points=True, scale_lo=0.005, scale_hi=0.02, scale_dtype=dt)
+    return synth.make_weights_bits(n, k, bs, bits, seed, zero_points=True, scale_lo=0.001, scale_hi=0.003, scale_dtype=dt)
+
+
+def shuffled_groups(k, bs, seed):
+    g = (np.arange(k) // bs).astype(np.int32)
+    np.random.default_rng(seed).shuffle(g)
+    return g
+
+
+def expected(port, a, a_dt, b, s, zp, g, n, k, bs, bits):
+    return synth.to_f32(a, a_dt).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, a_dt), zp, g, n, k, bs, bits).astype(np.float64).T
+
+
+@pytest.mark.parametrize("a_dt,bits,bs,m,n,k", [
+    (E.F16, 4, 128, 1, 300, 3584),
+    (E.BF16, 4, 32, 4, 129, 896),
+    (E.BF16, 4, 64, 16, 72, 1024),
+    (E.F16, 4, 128, 100, 264, 512),
+    (E.F32, 4, 32, 3, 64, 260),             # K % block_size != 0: the last group is the short one
+    (E.F32, 4, 32, 70, 160, 256),
+    (E.F16, 4, 16, 2, 40, 208),
+    (E.F16, 8, 32, 1, 100, 320),
+    (E.BF16, 8, 128, 9, 136, 512),
+    (E.F16, 2, 64, 3, 72, 512),
+])
+def test_matches_oracle(ep, port, a_dt, bits, bs, m, n, k):
+    b, s, zp = weights(n, k, bs, bits, a_dt, n)
+    g = shuffled_groups(k, bs, m)
+    a = synth.make_activation(m, k, 5, a_dt)
+    y, variant = E.matmul_nbits(ep, a, a_dt, b, s, a_dt, zp, n, k, bs, bits=bits, g_idx=g)
+    assert variant.startswith("act_order+")
+    assert helpers.rel_l2(synth.to_f32(y, a_dt), expected(port, a, a_dt, b, s, zp, g, n, k, bs, bits)) <= TOL[a_dt]
+
+
+def test_weights_that_change_and_groups_that_do_not_sort(ep, port):
+    """A node that moves to other tensors sorts those (a freed copy's address may come back), and one group longer than a block is served unsorted."""
+    a_dt, bs, bits, m, n, k = E.F16, 32, 4, 2, 64, 256
+    a = synth.make_activation(m, k, 5, a_dt)
+    ab, yb = ep.upload(a), ep.allocate(m * n * 2)
+    kernel = ep.get_kernel({"K": k, "N": n, "bits": bits, "block_size": bs})
+    kernel.set_constant_inputs([False, True, True, True, True])
+    out = [E.TensorView(yb.ptr, a_dt, (m, n))]
+    held = []
+    try:
+        for seed, regular in ((1, True), (2, True), (3, False), (4, True)):
+            b, s, zp = weights(n, k, bs, bits, a_dt, seed)
+            g = shuffled_groups(k, bs, seed)
+            if not regular:
+                g[g == 1] = 0
+            bufs = [ep.upload(x) for x in (b, s, zp, g)]
+            held += bufs
+            views = [E.TensorView(ab.ptr, a_dt, (m, k)), E.TensorView(bufs[0].ptr, E.U8, (n, k // bs, bs // 2)), E.TensorView(bufs[1].ptr, a_dt, (n, k // bs)),
+                     E.TensorView(bufs[2].ptr, E.U8, (n, k // bs // 2)), E.TensorView(bufs[3].ptr, E.I32, (k,))]
+            for _ in range(2):
+                kernel.execute(views, out)
+                assert kernel.last_variant().startswith("act_order+") == regular
+                got = ep.download(yb, (m, n), np.float16)
+                assert helpers.rel_l2(got.astype(np.float64), expected(port, a, a_dt, b, s, zp, g, n, k, bs, bits)) <= TOL[a_dt]
+    finally:
+        kernel.release()
+        for buf in held + [ab, yb]:
+            ep.deallocate(buf)
+
+
+def test_graph_replays_sort_the_rows_of_their_own_time(ep, port):
+    """A recorded call gathers the activations that lie in its input buffer when it is replayed."""
+    a_dt, bs, m, n, k = E.BF16, 64, 3, 96, 512
+    b, s, zp = weights(n, k, bs, 4, a_dt, 9)
+    g = shuffled_groups(k, bs, 9)
+    ops = E.DeviceOperands(ep, b, s, a_dt, zp, n, k, bs, g_idx=g)
+    ab, yb = ep.upload(synth.make_activation(m, k, 1, a_dt)), ep.allocate(m * n * 2)
+    try:
+        ops.run(ab, a_dt, m, yb)
+        ep.capture_begin()
+        ops.run(ab, a_dt, m, yb)
+        graph = ep.capture_end()
+        for seed in (2, 3, 4):
+            a = synth.make_activation(m, k, seed, a_dt)
+            ep.copy_from_host(ab, a)
+            graph.replay()
+            got = synth.to_f32(ep.download(yb, (m, n), np.uint16), a_dt)
+            assert helpers.rel_l2(got, expected(port, a, a_dt, b, s, zp, g, n, k, bs, 4)) <= TOL[a_dt]
+            ops.run(ab, a_dt, m, yb)
+            assert np.array_equal(got, synth.to_f32(ep.download(yb, (m, n), np.uint16), a_dt))
+        graph.release()
+    finally:
+        ep.deallocate(ab)
+        ep.deallocate(yb)
+        ops.free()
