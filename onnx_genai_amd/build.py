@@ -23,6 +23,7 @@ HIP_SOURCES = [
     "kernels/gemm_f32.hip",
     "kernels/decode_mfma.hip",
     "kernels/decode_packed.hip",
+    "kernels/decode_packed8.hip",
     "kernels/prefill_mfma.hip",
     "kernels/dense_gemm.hip",
     "kernels/swiglu.hip",

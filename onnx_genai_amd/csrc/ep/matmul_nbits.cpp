@@ -302,7 +302,8 @@ bool use_packed(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& r
 {
     rc = 0;
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[2] || (args.zp && !kn.constant_inputs[3])) return false;
-    if (!(kn.accuracy_level == 4 ? rocm_acc4_packed_eligible(&args) : rocm_decode_packed_eligible(&args))) return false;
+    const bool eight = kn.bits == 8;
+    if (!(eight ? rocm_decode_packed8_eligible(&args) : kn.accuracy_level == 4 ? rocm_acc4_packed_eligible(&args) : rocm_decode_packed_eligible(&args))) return false;
     const bool current = kn.packed && kn.packed_from[0] == args.b && kn.packed_from[1] == args.scales && kn.packed_from[2] == args.zp &&
                          kn.packed_scale_dtype == args.scale_dtype;
     if (current) return true;
@@ -311,11 +312,11 @@ bool use_packed(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& r
         drop_weight_copy(kn, kn.packed);
         kn.packed = nullptr;
     }
-    if (rocm_ffi_malloc(&kn.packed, rocm_decode_packed_bytes(&args)) != 0) {
+    if (rocm_ffi_malloc(&kn.packed, eight ? rocm_decode_packed8_bytes(&args) : rocm_decode_packed_bytes(&args)) != 0) {
         kn.packed = nullptr;
         return false;                       // no memory for a second copy: stream the caller's tensors instead
     }
-    rc = rocm_launch_pack_decode(&args, kn.packed, kn.ep->stream);
+    rc = eight ? rocm_launch_pack_decode8(&args, kn.packed, kn.ep->stream) : rocm_launch_pack_decode(&args, kn.packed, kn.ep->stream);
     if (rc != 0) {                          // a copy that was not made must not pass for current on the next call
         rocm_ffi_free(kn.packed);
         kn.packed = nullptr;
@@ -489,6 +490,10 @@ bool f32_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
     kn.variant = "gemv_f32_valu";
     return true;
 }
+
+// Elements of 8-bit weights from which a call streams a repacked copy: below, up to four rows, the plain kernel is level (bf16, block 128:
+// 3584 -> 1024 5.2 us, 3584 -> 1200 5.4 against 4.4), and a taller call that small is not worth a second copy of its weights.
+int64_t min_streamed_weights(int64_t rows) { return rows <= 4 ? int64_t{1} << 22 : int64_t{1} << 20; }
 
 // Narrower f32 calls than this keep the streaming kernel and the catch-all; no projection of a model is that narrow.
 constexpr int64_t kGemmF32MinCols = 128;
@@ -708,9 +713,15 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     const bool sorted = G && sort_by_group(kn, args, rc);
     if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
     if (kn.bits != 4 || args.g_idx) {
+        // Up to 64 rows of 8-bit weights stream the repacked copy; the accumulators' offset costs a 16-bit result nothing, so f32
+        // results stay on the routes below.
+        const bool streamed = kn.bits == 8 && !args.g_idx && M <= 64 && args.y_dtype != ROCM_DT_F32 && args.n * args.k >= min_streamed_weights(args.m) && use_packed(kn, args, rc);
         // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
-        if (!dense_route(kn, args, rc)) {
+        if (streamed) {
+            if (rc == 0) rc = rocm_launch_decode_packed8(&args, kn.packed, kn.ep->decode_waves, stream);
+            kn.variant = "decode_mfma_packed8";
+        } else if (!dense_route(kn, args, rc)) {
             rc = rocm_launch_gemv_nbits(&args, static_cast<int>(kn.bits), stream);
             kn.variant = "gemv_nbits_f32";
         }

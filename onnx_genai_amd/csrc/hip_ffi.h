@@ -199,6 +199,13 @@ int rocm_decode_packed_pair_fits(const RocmMatMulNBitsArgs* args, int waves);
 int rocm_launch_decode_packed_pair(const RocmMatMulNBitsArgs* args, const void* packed_gate, const void* packed_up, int decomposed, int waves,
                                    rocm_stream_t stream);
 
+/* The same for 8-bit weights (args->b [N, kb, bs], zp [N, kb] or NULL = 128; scales of the activations' type): the copy holds each
+ * tile as two planes of nibbles. */
+int rocm_decode_packed8_eligible(const RocmMatMulNBitsArgs* args);
+uint64_t rocm_decode_packed8_bytes(const RocmMatMulNBitsArgs* args);
+int rocm_launch_pack_decode8(const RocmMatMulNBitsArgs* args, void* packed, rocm_stream_t stream);
+int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* args, const void* packed, int waves, rocm_stream_t stream);
+
 /* Prefill (M > 16), f16/bf16 activations: B tiles dequantized into LDS, 32x32x16 MFMA.
  * tile_choice: 0 = by shape, 1 = 128 x 128, 2 = 256 x 128, 3 = 256 x 256, 4 = 128 x 64 tiles of Y per workgroup. */
 int rocm_prefill_mfma_eligible(const RocmMatMulNBitsArgs* args);

@@ -19,25 +19,10 @@
 // read instead of the caller's tensors, which are not touched again.
 #include <type_traits>
 
-#include "mfma_common.hiph"
-#include "swiglu.hiph"
+#include "decode_packed.hiph"
+#include "decode_packed8.hiph"
 
 namespace mnb {
-
-typedef __attribute__((ext_vector_type(8))) _Float16 half8p_t;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8p_t;
-typedef __attribute__((ext_vector_type(4))) float float4p_t;
-typedef __attribute__((ext_vector_type(2))) _Float16 half2p_t;
-
-constexpr int kGroupTiles = 4;
-constexpr int kChunkWeights = kGroupTiles * 1024;
-constexpr int kRowPitchP = 272;   // bytes between activation rows in LDS: 256 + 16
-
-__host__ __device__ constexpr int packed_record_bytes(int bs, int scale_bytes)
-{
-    const int nb = kGroupTiles * 128 / bs;
-    return (nb * scale_bytes + nb + 15) / 16 * 16;
-}
 
 struct PackParams {
     const uint8_t* b;
@@ -48,7 +33,11 @@ struct PackParams {
     int bs_log2, scale_bytes;
     int groups;             // tile groups per column group
     int chunk_bytes, record;
+    int bits;               // 4 or 8
 };
+
+// 8-bit weights travel as two planes of nibbles: (q - zp) * s = (q_low - zp_low) * s + (q_high - zp_high) * 16 s, so a tile of
+// 128 k becomes two tiles of the stream, the low nibbles and then the high ones, that meet the same activations.
 
 // grid (tile group, column group), 256 threads: four dwords of weights per thread, then one record per thread < 16.
 __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
@@ -63,9 +52,14 @@ __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
         const int x = it * 256 + t;              // dword of the weight part: u*256 + lane*4 + j
         const int u = x >> 8, lane = (x >> 2) & 63, j = x & 3;
         const int64_t col = cg * 16 + (lane & 15);
-        const int64_t k = (tg * kGroupTiles + u) * 128 + j * 32 + (lane >> 4) * 8;
+        const int64_t tile = tg * kGroupTiles + u;
+        const int64_t k = (p.bits == 8 ? tile >> 1 : tile) * 128 + j * 32 + (lane >> 4) * 8;
         uint32_t out = 0;
-        if (col < p.n && k < padded_k) {
+        if (p.bits == 8 && col < p.n && k < padded_k) {
+            const int plane_shift = static_cast<int>(tile & 1) * 4;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out |= ((static_cast<uint32_t>(p.b[col * p.row_bytes + k + e]) >> plane_shift) & 0xfu) << (4 * (e / 2) + 16 * (e % 2));
+        } else if (col < p.n && k < padded_k) {
             const uint32_t w = b32[(col * p.row_bytes + (k >> 1)) >> 2];   // eight weights, element e at bit 4e
             uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;    // even / odd elements, one per byte
             lo = (lo | (lo >> 4)) & 0x00ff00ffu;
@@ -82,926 +76,22 @@ __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
         const int64_t col = cg * 16 + t;
         for (int i = 0; i < p.record; ++i) rec[i] = 0;
         for (int bi = 0; bi < nb; ++bi) {
-            const int64_t blk = tg * nb + bi;
+            const int per_tile = nb / kGroupTiles;
+            const int64_t tile = tg * kGroupTiles + bi / per_tile;
+            const int64_t blk = p.bits == 8 ? (tile >> 1) * per_tile + bi % per_tile : tg * nb + bi;
             const bool live = col < p.n && blk < p.kb;
             if (p.scale_bytes == 4) {
                 reinterpret_cast<uint32_t*>(rec)[bi] = live ? static_cast<const uint32_t*>(p.scales)[col * p.kb + blk] : 0u;
             } else {
                 reinterpret_cast<uint16_t*>(rec)[bi] = live ? static_cast<const uint16_t*>(p.scales)[col * p.kb + blk] : static_cast<uint16_t>(0);
             }
-            rec[nb * p.scale_bytes + bi] = static_cast<uint8_t>(live ? zero_point_of(p.zp ? p.zp + col * p.zp_row : nullptr, blk) : 8);
-        }
-    }
-}
-
-struct PackedParams {
-    const uint16_t* a;
-    const uint8_t* packed;
-    const uint8_t* packed_up;   // paired launch only: the up projection's repacked copy (`packed` is the gate's)
-    int decomposed_silu;        // paired launch only
-    const void* bias;
-    void* y;
-    int64_t m, n, k;
-    int64_t cg_stride;      // bytes of one column group: groups * chunk_bytes
-    int groups;             // tile groups
-    int groups_per_wave;
-    int chunk_bytes;
-    int bias_dtype, y_dtype;
-    uint32_t nibble_mask;   // 0x000F000F
-    uint32_t magic;         // two 16-bit magic exponents; a kernel argument so that it stays in a scalar register
-    const void* gamma;      // NORM kernels: the RMS-normalization weight [k], f32 or the activations' type
-    int gamma_f32;
-    float norm_epsilon;
-};
-
-template <bool BF16>
-__device__ __forceinline__ float4p_t mfma16p(const uint4& act, const uint4& wgt, float4p_t acc)
-{
-    if constexpr (BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8p_t, act), __builtin_bit_cast(bf16x8p_t, wgt), acc, 0, 0, 0);
-    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8p_t, act), __builtin_bit_cast(half8p_t, wgt), acc, 0, 0, 0);
-}
-
-template <int NR, int NA, int NG>
-struct PackedGroup {
-    uint4 w[kGroupTiles];
-    uint4 r[NR];
-    uint4 a[NA];
-    uint4 gm[NG];     // NORM: the normalization weights of the activation pieces (two loads each: f32 weights are 32 bytes a piece)
-};
-
-// v + (v of the lane a DPP control selects): quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E, row_half_mirror = 0x141,
-// row_mirror = 0x140 - applied in that order they leave the sum over 4, 8, 16 lanes in every lane of the run.
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v)
-{
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_max(float v)
-{
-    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false)));
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp_addi(int v)
-{
-    return v + __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
-}
-
-// Sum of the 8 activations of one 16-byte piece, in f32.
-template <bool BF16>
-__device__ __forceinline__ float sum_piece(const uint4& v)
-{
-    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-    float s = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if constexpr (BF16) {
-            s += __uint_as_float(d[i] << 16);
-            s += __uint_as_float(d[i] & 0xffff0000u);
-        } else {
-            const half2p_t h = __builtin_bit_cast(half2p_t, d[i]);
-            s += static_cast<float>(h.x);
-            s += static_cast<float>(h.y);
-        }
-    }
-    return s;
-}
-
-// Sum over the BS / 8 consecutive lanes that hold one block's pieces; every lane of the run receives it.
-template <int BS>
-__device__ __forceinline__ float block_sum(float s)
-{
-    s = dpp_add<0xB1>(s);
-    s = dpp_add<0x4E>(s);
-    if constexpr (BS >= 64) s = dpp_add<0x141>(s);
-    if constexpr (BS >= 128) s = dpp_add<0x140>(s);
-    return s;
-}
-
-// BF16: activation element type. BS: block size. MR: rows staged (1, 4 or 16; M <= MR). ST: storage type of the scales.
-// SETS: register sets of one group each. 2: the next group's loads are in flight while this one is multiplied - for
-// launches with few waves, where each wave must cover memory latency by itself. 1: no prefetch, 62 registers, eight
-// waves per SIMD - for launches with thousands of waves, where the other resident waves cover it better (measured on
-// 3584 -> 37888: 15.6 us against 17.0 us). With two sets the one-row, block-128, 16-bit-scale variant fits 96
-// registers without spilling (a fifth wave per SIMD); the other variants keep the compiler's own choice.
-// PAIR: the fused gate/up node. The first half of the workgroup's waves runs the gate projection's column group, the
-// second half the up projection's - each half exactly as a launch of its own would (same split of K, same order of
-// summation, so the same f32 totals) - and the epilogue writes round16(silu(round16(gate)) * round16(up)).
-// NORM (up to 4 rows): the RMS-normalization prologue inside the kernel (the CUDA provider's form,
-// onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:3747-3783). Every wave first sums the squares of the call's rows in
-// the reference's order (32 lanes, four running sums over 4-element chunks, (s0 + s1) + (s2 + s3), a shuffle tree over
-// 32 lanes: half a wavefront plays one warp, so a wave covers two rows per pass), then replaces each activation piece it
-// loads by round16((a * inv_std) * gamma) before the piece is staged - the values a separate normalization launch
-// would have written, bit for bit.
-template <bool BF16, int BS, int MR, typename ST, int SETS, bool PAIR, bool NORM = false>
-__global__ __launch_bounds__((BS == 128 && sizeof(ST) == 2 && (MR != 16 || BF16)) ? 1024 : 512)   // block 128, 16-bit scales, up to 4 rows: up to 16 waves split a long K
-__attribute__((amdgpu_waves_per_eu((BS == 128 && MR == 1 && sizeof(ST) == 2 && !NORM) ? (SETS == 1 ? 8 : 5) : 1)))
-void decode_packed_kernel(PackedParams p)
-{
-    static_assert(!NORM || MR <= 4, "the fused normalization covers up to four rows");
-    constexpr int U = kGroupTiles;
-    constexpr int NBT = 128 / BS;
-    constexpr int NB = U * NBT;
-    constexpr int R = packed_record_bytes(BS, static_cast<int>(sizeof(ST)));
-    constexpr int NR = R / 16;
-    constexpr int RQ = MR == 1 ? 1 : MR / 4;       // loads per tile: each covers four rows (row g + 4 i, piece c)
-    constexpr int NA = MR == 1 ? 1 : U * RQ;
-    constexpr int NGP = MR == 1 ? 1 : U;           // activation pieces with distinct elements per group (rows share them)
-    constexpr int NG = NORM ? 2 * NGP : 1;
-    constexpr int kStageBytes = MR == 1 ? 1024 : MR * kRowPitchP;
-    constexpr float kMagicF = BF16 ? 128.0f : 1024.0f;
-    constexpr uint32_t kMagicNeg = BF16 ? 0xC300C300u : 0xE400E400u;
-    // How the magic offset and the zero point leave the accumulator. Launches of many short waves (one row, no
-    // prefetch) are bound by what a wave computes per byte: there they leave through the block's activation sum,
-    // y += scale * (acc - (magic + zp) * sum a), one FMA per block. Elsewhere a second MFMA per 32 elements against
-    // -(magic + zp) does it: more matrix-core work, but nothing between a wave's loads and its first MFMA, which is
-    // what the few-wave launches are sensitive to (measured: 3584 -> 37888 16.4 against 17.0 us and 3584 -> 152064 54.5
-    // against 59 us with the sums; 18944 -> 3584 12.2 against 11.4 us, so not there).
-    constexpr bool SUMS = MR == 1 && SETS == 1;
-    // With one row staged every accumulator row is a copy of row 0: only component 0 is scaled and reduced.
-    constexpr int kRowsKept = MR == 1 ? 1 : 4;
-    constexpr int kBlockLanes = BS / 8;         // lanes whose 16-byte pieces make up one block
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int waves = PAIR ? static_cast<int>(blockDim.x >> 7) : static_cast<int>(blockDim.x >> 6);      // per projection
-    const bool second = PAIR && wave >= waves;                                                           // wave-uniform
-    const int split = second ? wave - waves : wave;                                                      // this wave's share of K
-    const int c = lane & 15;
-    const int g = lane >> 4;
-    const int64_t n_base = static_cast<int64_t>(blockIdx.x) * 16;
-
-    const __amdgpu_buffer_rsrc_t srd_p = make_srd((second ? p.packed_up : p.packed) + static_cast<int64_t>(blockIdx.x) * p.cg_stride, static_cast<uint64_t>(p.cg_stride));
-    const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.a, static_cast<uint64_t>(p.m * p.k) * 2);
-    const __amdgpu_buffer_rsrc_t srd_g = make_srd(NORM ? p.gamma : p.a, NORM ? static_cast<uint64_t>(p.k) * (p.gamma_f32 ? 4 : 2) : 0);
-
-    const uint32_t w_off = static_cast<uint32_t>(lane * 16);
-    const uint32_t r_off = static_cast<uint32_t>(kChunkWeights + c * R);
-    // compact activation load. MR = 1: piece c of tile g of the group. MR = 4 / 16: row g (+ 4 i), piece c of one tile.
-    const uint32_t a_off = MR == 1 ? static_cast<uint32_t>(g * 256 + c * 16) : static_cast<uint32_t>(g) * static_cast<uint32_t>(p.k) * 2u + static_cast<uint32_t>(c * 16);
-    unsigned char* stage = smem + wave * (2 * kStageBytes);
-    const uint32_t st_write = MR == 1 ? static_cast<uint32_t>(lane * 16) : static_cast<uint32_t>(g * kRowPitchP + c * 16);
-    // operand of MFMA j: elements j*32 + g*8 .. +8 of the tile, of row c % MR
-    const uint32_t st_read = (MR == 1 ? 0u : static_cast<uint32_t>((c & (MR - 1)) * kRowPitchP)) + static_cast<uint32_t>(g * 16);
-    const uint32_t mask = __builtin_amdgcn_mov_dpp(p.nibble_mask, 0xE4, 0xf, 0xf, false), magic = p.magic;
-
-    float4p_t y = {0.f, 0.f, 0.f, 0.f};
-    float4p_t acc = {0.f, 0.f, 0.f, 0.f};
-
-    const int g_begin = split * p.groups_per_wave;
-    const int g_end = min(g_begin + p.groups_per_wave, p.groups);
-
-    using Grp = PackedGroup<NR, NA, NG>;
-    // No branch in here: a group past the wave's last one (the prefetch of the final iteration) gets every offset out of
-    // range, which fetches nothing and returns zeros - weights 0, scale 0, activations 0: a group that adds nothing.
-    // With a branch instead, the compiler waits for all loads in flight at the next use, the prefetch included.
-    auto fetch_group = [&](Grp& grp, int gi) {
-        const uint32_t oor = gi < g_end ? 0u : kOutOfRange;        // or-ed in: any offset with these bits is out of range
-        const uint32_t soff = static_cast<uint32_t>(gi) * static_cast<uint32_t>(p.chunk_bytes);
-        const int t0 = gi * U;
-        // every offset first, then the loads back to back: vector arithmetic between two loads can land in a register
-        // that an outstanding load still owns, and then waits for it
-        uint32_t a_voff[NA];
-#pragma unroll
-        for (int x = 0; x < NA; ++x) {
-            const int u = x / RQ, i = x % RQ;
-            const int tile = MR == 1 ? t0 + g : t0 + u;
-            const bool beyond = static_cast<int64_t>(tile) * 128 + c * 8 + 8 > p.k;        // K is a multiple of 8: a piece is all in or all out
-            // rows past M lie past the end of the activations' range and read as zeros
-            a_voff[x] = (beyond ? kOutOfRange : a_off + static_cast<uint32_t>(4 * i) * static_cast<uint32_t>(p.k) * 2u) | oor;
-        }
-        uint32_t g_voff[NG];
-        if constexpr (NORM) {
-#pragma unroll
-            for (int x = 0; x < NGP; ++x) {
-                const int tile = MR == 1 ? t0 + g : t0 + x;
-                const bool beyond = static_cast<int64_t>(tile) * 128 + c * 8 + 8 > p.k;
-                const uint32_t first = static_cast<uint32_t>(tile * 128 + c * 8) * (p.gamma_f32 ? 4u : 2u);
-                g_voff[2 * x] = (beyond ? kOutOfRange : first) | oor;
-                g_voff[2 * x + 1] = ((beyond || !p.gamma_f32) ? kOutOfRange : first + 16u) | oor;
-            }
-        }
-        const uint32_t w_voff = w_off | oor, r_voff = r_off | oor;
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < U; ++u) grp.w[u] = load16(srd_p, w_voff + static_cast<uint32_t>(u * 1024), soff);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) grp.r[i] = load16(srd_p, r_voff + static_cast<uint32_t>(i * 16), soff);
-#pragma unroll
-        for (int x = 0; x < NA; ++x) grp.a[x] = load16(srd_a, a_voff[x], static_cast<uint32_t>(MR == 1 ? t0 : t0 + x / RQ) * 256u);
-        if constexpr (NORM) {
-#pragma unroll
-            for (int x = 0; x < NG; ++x) grp.gm[x] = load16(srd_g, g_voff[x], 0u);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // ---- NORM: 1 / sqrt(mean(a^2) + eps) of this lane's row (row 0, or row g of up to four) ----
-    // With one row the wave's first group is requested before, so that its trip to memory overlaps the sums (with four
-    // rows the compiler would keep the group in scratch memory across the passes).
-    constexpr bool kEarly = NORM && MR == 1;
-    Grp ga;
-    if constexpr (kEarly || SETS == 2) fetch_group(ga, g_begin);
-    float inv_std = 1.0f;
-    if constexpr (NORM) {
-        // One wave per pair of rows does the sums (every wave doing them would re-read the rows once per wave: at 3584 ->
-        // 2 x 18944 three times the bytes of the weights) and leaves the results in LDS behind the staging buffers.
-        float* inv_shared = reinterpret_cast<float*>(smem + (blockDim.x >> 6) * (2 * kStageBytes));
-        const int all_waves = static_cast<int>(blockDim.x >> 6);
-        const int l32 = lane & 31;
-        const int items = static_cast<int>(p.k >> 7);
-#pragma unroll
-        for (int pass = 0; pass < (MR == 1 ? 1 : 2); ++pass) {
-            if (wave != pass % all_waves) continue;              // (wave-uniform)
-            const int row = 2 * pass + (lane >> 5);              // rows past M lie past the range and read as zeros
-            const uint32_t base = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.k) * 2u + static_cast<uint32_t>(l32 * 8);
-            float inv = 1.0f;
-            if (MR == 1 || 2 * pass < p.m) {                     // (wave-uniform) rows 2 and 3 only where the call has them
-                float ss0 = 0.f, ss1 = 0.f, ss2 = 0.f, ss3 = 0.f;
-                // sixteen loads in flight at a time: one after the other they would cost a trip to the cache each. A chunk past
-                // the row reads as zeros, and fma(0, 0, s) = s.
-                constexpr int kBatch = 16;
-                for (int first = 0; first < items; first += kBatch) {
-                    uint32_t d0[kBatch], d1[kBatch];
-#pragma unroll
-                    for (int i = 0; i < kBatch; ++i) {
-                        const auto raw = __builtin_amdgcn_raw_buffer_load_b64(srd_a, static_cast<int>(first + i < items ? base : kOutOfRange), (first + i) * 256, 0);
-                        d0[i] = raw[0];
-                        d1[i] = raw[1];
-                    }
-#pragma unroll
-                    for (int i = 0; i < kBatch; ++i) {
-                        const float v0 = BF16 ? __uint_as_float(d0[i] << 16) : f16_bits_to_f32(static_cast<uint16_t>(d0[i]));
-                        const float v1 = BF16 ? __uint_as_float(d0[i] & 0xffff0000u) : f16_bits_to_f32(static_cast<uint16_t>(d0[i] >> 16));
-                        const float v2 = BF16 ? __uint_as_float(d1[i] << 16) : f16_bits_to_f32(static_cast<uint16_t>(d1[i]));
-                        const float v3 = BF16 ? __uint_as_float(d1[i] & 0xffff0000u) : f16_bits_to_f32(static_cast<uint16_t>(d1[i] >> 16));
-                        ss0 = __fmaf_rn(v0, v0, ss0);
-                        ss1 = __fmaf_rn(v1, v1, ss1);
-                        ss2 = __fmaf_rn(v2, v2, ss2);
-                        ss3 = __fmaf_rn(v3, v3, ss3);
-                    }
-                }
-                float ss = __fadd_rn(__fadd_rn(ss0, ss1), __fadd_rn(ss2, ss3));
-#pragma unroll
-                for (int off = 16; off > 0; off >>= 1) ss = __fadd_rn(ss, __shfl_down(ss, off, 32));
-                // sqrtf and the divisions are correctly rounded (the compiler's default for f32)
-                inv = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, static_cast<float>(p.k)), p.norm_epsilon)));
-            }
-            if (l32 == 0) inv_shared[row] = inv;
-        }
-        __syncthreads();
-        inv_std = inv_shared[MR == 1 ? 0 : g];
-    }
-    // round16((a * inv_std) * gamma) of one 16-byte piece; g0 / g1: the piece's weights (16-bit: all eight in g0)
-    auto normalized = [&](const uint4& a, const uint4& g0, const uint4& g1) -> uint4 {
-        const uint32_t ad[4] = {a.x, a.y, a.z, a.w};
-        const uint32_t gd[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-        uint32_t out[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float v0 = BF16 ? __uint_as_float(ad[i] << 16) : f16_bits_to_f32(static_cast<uint16_t>(ad[i]));
-            const float v1 = BF16 ? __uint_as_float(ad[i] & 0xffff0000u) : f16_bits_to_f32(static_cast<uint16_t>(ad[i] >> 16));
-            float w0, w1;
-            if (p.gamma_f32) {
-                w0 = __uint_as_float(gd[2 * i]);
-                w1 = __uint_as_float(gd[2 * i + 1]);
+            if (p.bits == 8) {
+                const uint32_t z = live && p.zp ? p.zp[col * p.zp_row + blk] : 128u;
+                rec[nb * p.scale_bytes + bi] = static_cast<uint8_t>((z >> ((tile & 1) * 4)) & 0xfu);
             } else {
-                w0 = BF16 ? __uint_as_float(gd[i] << 16) : f16_bits_to_f32(static_cast<uint16_t>(gd[i]));
-                w1 = BF16 ? __uint_as_float(gd[i] & 0xffff0000u) : f16_bits_to_f32(static_cast<uint16_t>(gd[i] >> 16));
-            }
-            // (as_f32: the product is rounded to f32 before the 16-bit conversion sees it, never folded into one mixed-precision multiply)
-            const float y0 = as_f32(__fmul_rn(__fmul_rn(v0, inv_std), w0)), y1 = as_f32(__fmul_rn(__fmul_rn(v1, inv_std), w1));
-            const uint32_t lo = BF16 ? f32_to_bf16_bits(y0) : f32_to_f16_bits(y0);
-            const uint32_t hi = BF16 ? f32_to_bf16_bits(y1) : f32_to_f16_bits(y1);
-            out[i] = lo | (hi << 16);
-        }
-        return make_uint4(out[0], out[1], out[2], out[3]);
-    };
-    // `asum` (with SUMS): this lane's block sum of the group's tile lane / 16 (one load covers the group's four tiles).
-    auto compute_tile = [&](const Grp& grp, int u, int parity, float asum) {
-        unsigned char* st = stage + (MR == 1 ? parity : (u & 1)) * kStageBytes;
-        if constexpr (MR != 1) {
-#pragma unroll
-            for (int i = 0; i < RQ; ++i) {
-                if constexpr (NORM) *reinterpret_cast<uint4*>(st + st_write + i * 4 * kRowPitchP) = normalized(grp.a[u * RQ + i], grp.gm[2 * u], grp.gm[2 * u + 1]);
-                else *reinterpret_cast<uint4*>(st + st_write + i * 4 * kRowPitchP) = grp.a[u * RQ + i];
-            }
-            lds_order();
-        }
-        uint4 av[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) av[j] = *reinterpret_cast<const uint4*>(st + st_read + (MR == 1 ? u * 256 : 0) + j * 64);
-        const uint32_t wd[4] = {grp.w[u].x, grp.w[u].y, grp.w[u].z, grp.w[u].w};
-        uint32_t rr[NR * 4];
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            rr[4 * i] = grp.r[i].x;
-            rr[4 * i + 1] = grp.r[i].y;
-            rr[4 * i + 2] = grp.r[i].z;
-            rr[4 * i + 3] = grp.r[i].w;
-        }
-        // Every dword of the record counts as used here, also the padding at its end: a destination register of a load
-        // that the compiler knows to be dead is handed out again at once, and writing it waits for the load in flight.
-#pragma unroll
-        for (int i = 0; i < NR * 4; ++i) asm volatile("" : : "v"(rr[i]));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int bi = u * NBT + (j * 32) / BS;                          // block of the group (compile-time)
-            const int zbyte = NB * static_cast<int>(sizeof(ST)) + bi;
-            const uint32_t w = wd[j];
-            uint4 op;
-            op.x = (w & mask) | magic;
-            op.y = ((w >> 4) & mask) | magic;
-            op.z = ((w >> 8) & mask) | magic;
-            op.w = ((w >> 12) & mask) | magic;
-            acc = mfma16p<BF16>(av[j], op, acc);
-            const uint32_t z = (rr[zbyte / 4] >> ((zbyte % 4) * 8)) & 0xffu;
-            if constexpr (!SUMS) {
-                const uint32_t zpair = kMagicNeg | (z * 0x00010001u);
-                acc = mfma16p<BF16>(av[j], make_uint4(zpair, zpair, zpair, zpair), acc);
-            }
-            if (((j + 1) * 32) % BS == 0 || j == 3) {
-                float sf;
-                if constexpr (sizeof(ST) == 4) {
-                    sf = __uint_as_float(rr[bi]);
-                } else {
-                    const uint32_t raw = (rr[bi / 2] >> ((bi % 2) * 16)) & 0xffffu;
-                    sf = BF16 ? __uint_as_float(raw << 16) : f16_bits_to_f32(static_cast<uint16_t>(raw));
-                }
-                if constexpr (SUMS) {
-                    // the block's pieces sit in lanes first .. first + kBlockLanes - 1 of lane group u; any of them has the sum
-                    const int first = u * 16 + ((j * 32) / BS) % NBT * kBlockLanes;
-                    const float sa = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(asum), first));
-                    const float off = kMagicF + static_cast<float>(z);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        if (r < kRowsKept) y[r] = fmaf(sf, fmaf(-off, sa, acc[r]), y[r]);      // the product is not rounded on its own
-                        acc[r] = 0.f;
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        if (r < kRowsKept) y[r] = fmaf(sf, acc[r], y[r]);
-                        acc[r] = 0.f;
-                    }
-                }
+                rec[nb * p.scale_bytes + bi] = static_cast<uint8_t>(live ? zero_point_of(p.zp ? p.zp + col * p.zp_row : nullptr, blk) : 8);
             }
         }
-    };
-    auto run_group = [&](const Grp& cur, Grp& next, int gi, int parity, bool prefetch) {
-        // Nothing of this group moves up into the previous one: its activation piece is the newest load in flight
-        // there, and staging it early would wait for every load, the prefetch included.
-        __builtin_amdgcn_sched_barrier(0);
-        if (prefetch) fetch_group(next, gi + 1);
-        if constexpr (MR == 1) {
-            if constexpr (NORM) *reinterpret_cast<uint4*>(stage + parity * kStageBytes + st_write) = normalized(cur.a[0], cur.gm[0], cur.gm[1]);
-            else *reinterpret_cast<uint4*>(stage + parity * kStageBytes + st_write) = cur.a[0];
-            lds_order();
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) compute_tile(cur, u, parity, 0.f);
-    };
-
-    if constexpr (SETS == 2) {
-        Grp gb;
-        int gi = g_begin;
-        for (; gi + 1 < g_end; gi += 2) {                      // whole pairs, no branch inside: every wait counts loads exactly
-            run_group(ga, gb, gi, 0, true);
-            run_group(gb, ga, gi + 1, 1, true);                // past the end this prefetch fetches nothing
-        }
-        if (gi < g_end) run_group(ga, gb, gi, 0, false);       // an odd group out
-
-    } else {
-        auto multiply = [&]() {
-            float asum = 0.f;
-            if constexpr (MR == 1) {
-                uint4 piece = ga.a[0];
-                if constexpr (NORM) piece = normalized(ga.a[0], ga.gm[0], ga.gm[1]);
-                *reinterpret_cast<uint4*>(stage + st_write) = piece;
-                lds_order();
-                if constexpr (SUMS) asum = block_sum<BS>(sum_piece<BF16>(piece));
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) compute_tile(ga, u, 0, asum);
-        };
-        int gi = g_begin;
-        if constexpr (kEarly) {                                // the first group is already on its way
-            if (gi < g_end) multiply();
-            ++gi;
-        }
-        for (; gi < g_end; ++gi) {
-            fetch_group(ga, gi);
-            multiply();
-        }
-    }
-
-    // ---- split-K reduction across the waves of this workgroup, in wave order ----
-    __syncthreads();
-    float* red = reinterpret_cast<float*>(smem);       // [waves][4][64]
-#pragma unroll
-    for (int r = 0; r < kRowsKept; ++r) red[(wave * 4 + r) * 64 + lane] = y[r];
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < kRowsKept * 64; idx += blockDim.x) {
-        const int r = idx >> 6;
-        const int l = idx & 63;
-        const int row = 4 * (l >> 4) + r;
-        const int64_t col = n_base + (l & 15);
-        if (row < p.m && col < p.n) {
-            float total = 0.f;
-            for (int w = 0; w < waves; ++w) total += red[(w * 4 + r) * 64 + l];
-            if constexpr (PAIR) {
-                float total_up = 0.f;
-                for (int w = waves; w < 2 * waves; ++w) total_up += red[(w * 4 + r) * 64 + l];
-                const uint16_t gate16 = BF16 ? f32_to_bf16_bits(total) : f32_to_f16_bits(total);
-                const uint16_t up16 = BF16 ? f32_to_bf16_bits(total_up) : f32_to_f16_bits(total_up);
-                static_cast<uint16_t*>(p.y)[static_cast<int64_t>(row) * p.n + col] = swiglu16<BF16>(gate16, up16, p.decomposed_silu != 0);
-            } else {
-                total = with_bias(total, p.bias, p.bias_dtype, row, p.n, col, p.y_dtype);
-                store_from_f32(p.y, p.y_dtype, static_cast<int64_t>(row) * p.n + col, total);
-            }
-        }
-    }
-}
-
-// `waves` = waves per projection; a paired launch has twice as many in a workgroup.
-template <bool BF16, int BS, int MR, typename ST, int SETS>
-static int launch_packed_cfg(const PackedParams& p, int waves, hipStream_t stream)
-{
-    const unsigned grid = static_cast<unsigned>((p.n + 15) / 16);
-    const bool pair = p.packed_up != nullptr;
-    const int all = pair ? 2 * waves : waves;
-    const size_t stage = static_cast<size_t>(all) * 2 * (MR == 1 ? 1024 : MR * kRowPitchP);
-    const size_t red = static_cast<size_t>(all) * 1024;
-    const size_t lds = (stage > red ? stage : red) + (p.gamma ? 16 : 0);      // + the rows' 1 / rms of a launch with the normalization prologue
-    if constexpr (MR == 1 || (MR == 4 && SETS == 1)) {       // (four rows with a second register set and the weights of the prologue would spill)
-        if (p.gamma) {
-            if (pair) hipLaunchKernelGGL((decode_packed_kernel<BF16, BS, MR, ST, SETS, true, true>), dim3(grid), dim3(all * 64), lds, stream, p);
-            else hipLaunchKernelGGL((decode_packed_kernel<BF16, BS, MR, ST, SETS, false, true>), dim3(grid), dim3(all * 64), lds, stream, p);
-            return static_cast<int>(hipGetLastError());
-        }
-    }
-    if constexpr (MR >= 8) {
-        // sixteen staged rows of sixteen waves outgrow the 64 KiB a kernel gets without asking
-        if (lds > 65536) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(decode_packed_kernel<BF16, BS, MR, ST, SETS, false>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-            if (e != hipSuccess) return static_cast<int>(e);
-        }
-        hipLaunchKernelGGL((decode_packed_kernel<BF16, BS, MR, ST, SETS, false>), dim3(grid), dim3(all * 64), lds, stream, p);
-    } else {
-        if (pair) hipLaunchKernelGGL((decode_packed_kernel<BF16, BS, MR, ST, SETS, true>), dim3(grid), dim3(all * 64), lds, stream, p);
-        else hipLaunchKernelGGL((decode_packed_kernel<BF16, BS, MR, ST, SETS, false>), dim3(grid), dim3(all * 64), lds, stream, p);
-    }
-    return static_cast<int>(hipGetLastError());
-}
-
-template <bool BF16, int BS, typename ST>
-static int launch_packed_mr(const PackedParams& p, int waves, bool single_set, hipStream_t stream)
-{
-    if (p.m <= 1) return single_set ? launch_packed_cfg<BF16, BS, 1, ST, 1>(p, waves, stream) : launch_packed_cfg<BF16, BS, 1, ST, 2>(p, waves, stream);
-    if (p.m <= 4) return (single_set || p.gamma) ? launch_packed_cfg<BF16, BS, 4, ST, 1>(p, waves, stream) : launch_packed_cfg<BF16, BS, 4, ST, 2>(p, waves, stream);
-    // 5 .. 16 rows: one register set (64 registers of activations per group at 16 rows; a second set in flight measured
-    // slower). Up to 8 rows a build that stages eight: half the activation bytes per wave and group.
-    if (p.m <= 8) return launch_packed_cfg<BF16, BS, 8, ST, 1>(p, waves, stream);
-    return launch_packed_cfg<BF16, BS, 16, ST, 1>(p, waves, stream);
-}
-
-template <bool BF16, typename ST>
-static int launch_packed_bs(const PackedParams& p, int bs, int waves, bool single_set, hipStream_t stream)
-{
-    switch (bs) {
-        case 32: return launch_packed_mr<BF16, 32, ST>(p, waves, single_set, stream);
-        case 64: return launch_packed_mr<BF16, 64, ST>(p, waves, single_set, stream);
-        default: return launch_packed_mr<BF16, 128, ST>(p, waves, single_set, stream);
-    }
-}
-
-// ---------------------------------------------------------------------------------------------
-// The same stream for 5 <= M <= 64 and many columns: activations shared through LDS.
-// ---------------------------------------------------------------------------------------------
-//
-// With several rows the activations outweigh a column group's weights (16 rows x 128 k x 2 bytes against 16 columns
-// x 64 bytes per tile), and a kernel in which every wave fetches its own copy is bound by L2, not HBM. Here a
-// workgroup of eight waves owns eight column groups - one wave each, streaming the whole of K - and all eight read
-// the activations from one LDS copy, filled window by window (double buffered: the next window travels global ->
-// registers while the current one is multiplied, and moves registers -> LDS just before the barrier that ends the
-// window). No split-K, so no reduction: a wave stores its 16 columns itself. Weights are not prefetched: the kernel is
-// small enough for several workgroups per CU, and the other resident waves cover a wave's memory latency better than
-// a second register set does. Up to 64 rows ride on one pass over the weights: RB blocks of 16 rows, each with its own
-// accumulators, share every unpacked weight operand - up to that height the call still costs what streaming the
-// weights costs, which the tiled kernel cannot offer below a few hundred rows.
-
-constexpr int kWideWaves = 8;        // waves that fill the activation windows; a workgroup has 8 .. kWideWavesMax waves
-constexpr int kWideWavesMax = 12;    // (a launch picks the count that spreads its column groups evenly over the CUs)
-
-// RB: blocks of 16 rows (1, 2 or 4). A window is WT tiles of 128 k: a whole tile group for RB <= 2, half of one for
-// RB = 4, so that two buffers of RB * 16 rows stay within 66 KB.
-// SUMS: offset and zero point leave through the block activation sums (one FMA per accumulator and block) instead of a
-// second MFMA per 32 elements. Fewer matrix-core cycles, but 95 registers instead of 80 at 16 rows: launches with
-// several workgroups per CU run better with the sixth wave per SIMD (3584 -> 152064 at 16 rows: 59 against 64 us), the
-// others with the sums (3584 -> 37888: 22.9 against 24.5 us).
-// PF (with DEEP only): the next group's weights travel while the current one is multiplied (a second register set):
-// for grids with fewer workgroups than CUs, where no other workgroup covers a wave's memory latency.
-// DEEP: the activation windows travel two ahead instead of one (a second set of window registers; RB <= 2).
-// PAIR (RB = 1): the fused gate/up node at 5 .. 16 rows. Waves 0 .. 3 own four column groups of the gate projection,
-// waves 4 .. 7 the same four of the up projection - each wave exactly as in a launch of its projection alone (the whole
-// of K, the same order of summation) - and the epilogue writes round16(silu(round16(gate)) * round16(up)).
-// WMAX: the most waves a workgroup of this build may have (8, or 12 for the builds that balanced grids launch).
-template <bool BF16, int BS, typename ST, int RB, bool SUMS, bool PF, bool DEEP, bool PAIR = false, int WMAX = kWideWaves>
-__global__ __launch_bounds__(WMAX * 64)
-__attribute__((amdgpu_waves_per_eu((BS == 128 && sizeof(ST) == 2 && RB == 1) ? (PF ? (SUMS ? 3 : 4) : SUMS ? (DEEP || WMAX > kWideWaves ? 4 : 5) : (DEEP ? 5 : 6)) : (WMAX > kWideWaves ? 3 : 1))))
-void decode_wide_kernel(PackedParams p)
-{
-    static_assert(WMAX == kWideWaves || (WMAX == kWideWavesMax && RB == 1), "twelve waves: the one-block builds only");
-    static_assert(DEEP || !PF, "weights ahead only together with deep windows");
-    static_assert(!PAIR || RB == 1, "the paired form takes up to 16 rows");
-    // column groups per workgroup (and projection): one per wave. The first eight waves also fill the windows.
-    // (a build for eight waves knows both at compile time)
-    const int tile_waves = WMAX == kWideWaves ? (PAIR ? kWideWaves / 2 : kWideWaves) : (PAIR ? static_cast<int>(blockDim.x >> 7) : static_cast<int>(blockDim.x >> 6));
-    constexpr int U = kGroupTiles;
-    constexpr int NBT = 128 / BS;
-    constexpr int NB = U * NBT;
-    constexpr int R = packed_record_bytes(BS, static_cast<int>(sizeof(ST)));
-    constexpr int NR = R / 16;
-    constexpr int WT = RB == 4 ? 2 : 4;                 // tiles per window
-    constexpr int kWindowsPerGroup = U / WT;
-    constexpr int kPitch = WT * 256 + 16;               // bytes per LDS row: consecutive rows start in different bank quads
-    constexpr int kRows = RB * 16;
-    constexpr int kBufBytes = kRows * kPitch;
-    constexpr int kPieces = WT * 16;                    // 16-byte pieces per row of a window
-    constexpr int NW = kRows * kPieces / 512;           // pieces per thread per window (2 or 4)
-    constexpr float kMagicF = BF16 ? 128.0f : 1024.0f;
-    constexpr uint32_t kMagicNeg = BF16 ? 0xC300C300u : 0xE400E400u;
-    constexpr int kBlockLanes = BS / 8;                 // consecutive threads whose pieces make up one block of a row
-    constexpr int kWinBlocks = WT * NBT;                // blocks per window
-    constexpr int kSumBytes = kWinBlocks * kRows * 4;
-    // [2][kRows][kPitch] activations, then [2][kWinBlocks][kRows] f32 sums of each row over each block of the window:
-    // the magic offset and the zero point leave the accumulators through them, y += scale * (acc - (magic + zp) * sum a)
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    float* lds_sums = reinterpret_cast<float*>(smem + 2 * kBufBytes);
-
-    const int t = threadIdx.x;
-    const int lane = t & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int c = lane & 15;
-    const int g = lane >> 4;
-    const int64_t col_groups = (p.n + 15) / 16;
-    const bool filler = WMAX == kWideWaves || wave < kWideWaves;      // (wave-uniform)
-    const bool second = PAIR && wave >= tile_waves;       // (wave-uniform) the up projection's half
-    const int64_t cgi = static_cast<int64_t>(blockIdx.x) * tile_waves + (second ? wave - tile_waves : wave);
-    const bool active = cgi < col_groups;                 // a wave beyond the last column group still helps with the windows
-    const int64_t n_base = cgi * 16;
-
-    const __amdgpu_buffer_rsrc_t srd_p = make_srd((second ? p.packed_up : p.packed) + (active ? cgi : 0) * p.cg_stride, active ? static_cast<uint64_t>(p.cg_stride) : 0);
-    const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.a, static_cast<uint64_t>(p.m * p.k) * 2);
-
-    const uint32_t w_off = static_cast<uint32_t>(lane * 16);
-    const uint32_t r_off = static_cast<uint32_t>(kChunkWeights + c * R);
-    // operand of MFMA j of tile x of the window, row block rb: row rb*16 + c, elements x*128 + j*32 + g*8 .. +8
-    const uint32_t frag_off = static_cast<uint32_t>(c * kPitch + g * 16);
-    const uint32_t mask = __builtin_amdgcn_mov_dpp(p.nibble_mask, 0xE4, 0xf, 0xf, false), magic = p.magic;
-
-    float4p_t y[RB], acc[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-        y[rb] = float4p_t{0.f, 0.f, 0.f, 0.f};
-        acc[rb] = float4p_t{0.f, 0.f, 0.f, 0.f};
-    }
-
-    struct Grp {
-        uint4 w[kGroupTiles];
-        uint4 r[NR];
-    };
-    // a group past the last lies beyond the column group's range: the loads return zeros and touch no memory
-    auto fetch_group = [&](Grp& grp, int gi) {
-        const uint32_t soff = static_cast<uint32_t>(gi) * static_cast<uint32_t>(p.chunk_bytes);
-#pragma unroll
-        for (int u = 0; u < U; ++u) grp.w[u] = load16(srd_p, w_off + static_cast<uint32_t>(u * 1024), soff);
-#pragma unroll
-        for (int i = 0; i < NR; ++i) grp.r[i] = load16(srd_p, r_off + static_cast<uint32_t>(i * 16), soff);
-    };
-    // window fill: piece q = t + 512 i of the window's kRows * kPieces pieces -> (row q / kPieces, piece q % kPieces)
-    uint4 wa[NW];
-    uint4 wb[DEEP ? NW : 1];                               // DEEP: the second set of window registers
-    auto load_window_into = [&](uint4* dst, int win) {
-#pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            const int q = t + 512 * i;
-            const int row = q / kPieces, piece = q % kPieces;
-            const int64_t k0 = static_cast<int64_t>(win) * (WT * 128) + piece * 8;
-            uint32_t off = static_cast<uint32_t>(row) * static_cast<uint32_t>(p.k) * 2u + static_cast<uint32_t>(piece * 16);
-            if (row >= p.m || k0 >= p.k || !filler) off = kOutOfRange;       // K is a multiple of 8: a piece is all inside or all outside
-            dst[i] = load16(srd_a, off, static_cast<uint32_t>(win) * (WT * 256u));
-        }
-    };
-    auto load_window = [&](int win) { load_window_into(wa, win); };
-    auto store_window_from = [&](const uint4* src, int buf) {
-        if (!filler) return;
-#pragma unroll
-        for (int i = 0; i < NW; ++i) {
-            const int q = t + 512 * i;
-            const int row = q / kPieces, piece = q % kPieces;
-            *reinterpret_cast<uint4*>(smem + buf * kBufBytes + row * kPitch + piece * 16) = src[i];
-            if constexpr (SUMS) {
-                const float sum = block_sum<BS>(sum_piece<BF16>(src[i]));     // a block's pieces sit in consecutive lanes
-                if (piece % kBlockLanes == 0) lds_sums[(buf * kWinBlocks + piece / kBlockLanes) * kRows + row] = sum;
-            }
-        }
-    };
-    auto store_window = [&](int buf) { store_window_from(wa, buf); };
-    // tiles [first, first + WT) of the group against window buffer `buf`
-    auto compute_window = [&](const Grp& grp, int buf, int first) {
-        uint32_t rr[NR * 4];
-#pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            rr[4 * i] = grp.r[i].x;
-            rr[4 * i + 1] = grp.r[i].y;
-            rr[4 * i + 2] = grp.r[i].z;
-            rr[4 * i + 3] = grp.r[i].w;
-        }
-#pragma unroll
-        for (int x = 0; x < WT; ++x) {
-            const int u = first + x;                               // tile of the group (compile-time after unrolling)
-            const unsigned char* fa = smem + buf * kBufBytes + frag_off + x * 256;
-            const uint32_t wd[4] = {grp.w[u].x, grp.w[u].y, grp.w[u].z, grp.w[u].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int bi = u * NBT + (j * 32) / BS;
-                const int zbyte = NB * static_cast<int>(sizeof(ST)) + bi;
-                const uint32_t w = wd[j];
-                uint4 op;
-                op.x = (w & mask) | magic;
-                op.y = ((w >> 4) & mask) | magic;
-                op.z = ((w >> 8) & mask) | magic;
-                op.w = ((w >> 12) & mask) | magic;
-                const bool last = ((j + 1) * 32) % BS == 0 || j == 3;
-                float sf = 0.f, off = 0.f;
-                if (last) {
-                    if constexpr (sizeof(ST) == 4) {
-                        sf = __uint_as_float(rr[bi]);
-                    } else {
-                        const uint32_t raw = (rr[bi / 2] >> ((bi % 2) * 16)) & 0xffffu;
-                        sf = BF16 ? __uint_as_float(raw << 16) : f16_bits_to_f32(static_cast<uint16_t>(raw));
-                    }
-                    if constexpr (SUMS) off = kMagicF + static_cast<float>((rr[zbyte / 4] >> ((zbyte % 4) * 8)) & 0xffu);
-                }
-                const uint32_t zpair = kMagicNeg | (((rr[zbyte / 4] >> ((zbyte % 4) * 8)) & 0xffu) * 0x00010001u);
-                const uint4 zc = make_uint4(zpair, zpair, zpair, zpair);       // used without SUMS only
-                const int wb = x * NBT + (j * 32) / BS;                // block of the window
-#pragma unroll
-                for (int rb = 0; rb < RB; ++rb) {
-                    const uint4 av = *reinterpret_cast<const uint4*>(fa + rb * 16 * kPitch + j * 64);
-                    acc[rb] = mfma16p<BF16>(av, op, acc[rb]);
-                    if constexpr (!SUMS) acc[rb] = mfma16p<BF16>(av, zc, acc[rb]);
-                    if (last) {
-                        float sav[4] = {0.f, 0.f, 0.f, 0.f};
-                        if constexpr (SUMS) {
-                            // this lane's accumulator rows are rows rb * 16 + 4 g + r of the window
-                            const float4 sa = *reinterpret_cast<const float4*>(lds_sums + (buf * kWinBlocks + wb) * kRows + rb * 16 + 4 * g);
-                            sav[0] = sa.x;
-                            sav[1] = sa.y;
-                            sav[2] = sa.z;
-                            sav[3] = sa.w;
-                        }
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            y[rb][r] = fmaf(sf, SUMS ? fmaf(-off, sav[r], acc[rb][r]) : acc[rb][r], y[rb][r]);
-                            acc[rb][r] = 0.f;
-                        }
-                    }
-                }
-            }
-        }
-    };
-
-    const int windows = p.groups * kWindowsPerGroup;
-    Grp ga;
-    if constexpr (DEEP) {
-        // One window per group (RB <= 2). The next window's activations sit in one register set, the one after that is
-        // in flight into the other: a pass no longer lasts at least one L2 round trip. No branch inside a pass (a branch
-        // makes the compiler wait for every load in flight): a window or group past the end loads zeros, passes run in
-        // pairs so that the register sets alternate at compile time, an odd one is peeled.
-        static_assert(!DEEP || kWindowsPerGroup == 1, "deep windows: one window per group");
-        Grp gb;
-        load_window_into(wa, 0);
-        load_window_into(wb, 1);
-        if constexpr (PF) fetch_group(ga, 0);
-        store_window_from(wa, 0);
-        __syncthreads();
-        // `ready` holds window gi + 1, `idle` receives window gi + 2
-        auto pass = [&](Grp& cur, Grp& next, int gi, const uint4* ready, uint4* idle, bool prefetch) {
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (!PF) fetch_group(cur, gi);           // needed at once: issued first, so that the wait leaves the window in flight
-            load_window_into(idle, gi + 2);
-            if constexpr (PF) {
-                if (prefetch) fetch_group(next, gi + 1);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            compute_window(cur, gi & 1, 0);
-            store_window_from(ready, (gi & 1) ^ 1);
-            __syncthreads();
-        };
-        int gi = 0;
-        for (; gi + 1 < p.groups; gi += 2) {
-            pass(ga, gb, gi, wb, wa, true);
-            pass(PF ? gb : ga, ga, gi + 1, wa, wb, true);
-        }
-        if (gi < p.groups) pass(ga, gb, gi, wb, wa, false);
-    } else {
-        load_window(0);
-        store_window(0);
-        __syncthreads();
-        for (int gi = 0; gi < p.groups; ++gi) {
-            fetch_group(ga, gi);
-#pragma unroll
-            for (int h = 0; h < kWindowsPerGroup; ++h) {
-                const int win = gi * kWindowsPerGroup + h;
-                const int buf = win & 1;
-                if (win + 1 < windows) load_window(win + 1);
-                compute_window(ga, buf, h * WT);
-                if (win + 1 < windows) store_window(buf ^ 1);
-                __syncthreads();
-            }
-        }
-    }
-
-    if constexpr (PAIR) {
-        // every window has been read (the loop ends on a barrier): the up half leaves its totals where the windows were
-        float* up_totals = reinterpret_cast<float*>(smem);            // [tile_waves][4][64]
-        if (second) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) up_totals[((wave - tile_waves) * 4 + r) * 64 + lane] = y[0][r];
-        }
-        __syncthreads();
-        const int64_t col = n_base + c;
-        if (!second && active && col < p.n) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = 4 * g + r;
-                if (row < p.m) {
-                    const float up = up_totals[(wave * 4 + r) * 64 + lane];
-                    const uint16_t gate16 = BF16 ? f32_to_bf16_bits(y[0][r]) : f32_to_f16_bits(y[0][r]);
-                    const uint16_t up16 = BF16 ? f32_to_bf16_bits(up) : f32_to_f16_bits(up);
-                    static_cast<uint16_t*>(p.y)[static_cast<int64_t>(row) * p.n + col] = swiglu16<BF16>(gate16, up16, p.decomposed_silu != 0);
-                }
-            }
-        }
-    } else
-    if (active) {
-        const int64_t col = n_base + c;
-        if (col < p.n) {
-            const bool per_row = (p.bias_dtype & ROCM_BIAS_PER_ROW) != 0;
-            const BiasTerm bias = load_bias(p.bias, p.bias_dtype, 0, p.n, col);
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = rb * 16 + 4 * g + r;
-                    if (row < p.m) store_from_f32(p.y, p.y_dtype, static_cast<int64_t>(row) * p.n + col, add_bias(y[rb][r], per_row ? load_bias(p.bias, p.bias_dtype, row, p.n, col) : bias, p.y_dtype));
-                }
-            }
-        }
-    }
-}
-
-// What launch_wide_bs launches for a shape: the build (row blocks, sums or second MFMA, weights / windows ahead, the
-// workgroup's most waves), the waves per workgroup and the grid. No GPU work: a CPU test holds the answers for the model
-// shapes against a committed table, so that a change made for one shape cannot move another unnoticed.
-struct WidePlan {
-    int rb;            // blocks of 16 rows per wave: 1, 2 or 4
-    bool sums, pf, deep;
-    int wmax;          // kWideWaves or kWideWavesMax
-    int waves;         // per workgroup
-    unsigned grid;
-    bool ok;           // false: no build for this call (the dispatch does not send it here)
-};
-
-static WidePlan plan_wide(int64_t m, int64_t n, int bs, bool st16, bool pair, int64_t cus)
-{
-    WidePlan w{};
-    const int64_t col_groups = (n + 15) / 16;
-    const int64_t all_groups = pair ? 2 * col_groups : col_groups;
-    // A grid between one and one and a half workgroups of eight waves per CU (3584 -> 37888: 296 workgroups on 256 CUs)
-    // leaves some CUs with two workgroups while the others run one, and the launch lasts as long as the doubly loaded ones.
-    const bool in_between = all_groups > cus * kWideWaves && all_groups <= cus * kWideWavesMax;
-    const int64_t alone = (col_groups + kWideWaves - 1) / kWideWaves;
-    // How offset and zero point leave the accumulator (it shows in the last bits, so it is decided as for a launch of one
-    // projection alone, and a pair follows its projections). Through the block activation sums, except:
-    //  * grids of three or more workgroups per CU (3584 -> 152064 at 16 rows: 59 against 64 us);
-    //  * block size 32: the sums build takes 185-196 registers there, one workgroup per CU, and a grid above one workgroup
-    //    per CU runs in two rounds (3584 -> 37888 at 8 rows: 37.8 us; the second-MFMA build with the next group's
-    //    weights in flight 26.2, 4096 -> 14336 21.6 -> 17.2, 4096 -> 28672 24.0 -> 20.2);
-    //  * block size 64 where a launch of the projection gets a balanced grid (below): the sums build with weights ahead
-    //    takes 218 registers, too many for more than eight waves a workgroup.
-    w.sums = alone < 3 * cus && bs != 32 && !(bs == 64 && st16 && col_groups > cus * kWideWaves && col_groups <= cus * kWideWavesMax);
-    // Waves (= column groups) per workgroup: eight, unless the grid is in between and a build for more waves exists - then
-    // as many as spread the column groups over one workgroup per CU, up to twelve (3584 -> 37888 at block 128: ten waves,
-    // 237 workgroups, 22.6 -> 18.0 us at 8 rows; at block 64 23.7 -> 21.2). Larger workgroups lose where the grid is several
-    // times the CUs (3584 -> 152064 65 -> 80 us with ten). A paired launch holds half of its waves' column groups from each
-    // projection. The builds for twelve waves: block 128 with the sums, block 64 without (16-bit scales).
-    int ww = kWideWaves;
-    if (m <= 16 && st16 && in_between && ((bs == 128 && w.sums) || (bs == 64 && !w.sums && !pair))) {
-        ww = static_cast<int>((all_groups + cus - 1) / cus);
-        if (pair && (ww & 1)) ++ww;
-        if (ww > kWideWavesMax) ww = kWideWaves;
-    }
-    const int per_wg = pair ? ww / 2 : ww;
-    w.waves = ww;
-    w.grid = static_cast<unsigned>((col_groups + per_wg - 1) / per_wg);
-    w.wmax = ww > kWideWaves ? kWideWavesMax : kWideWaves;
-    w.rb = m <= 16 ? 1 : m <= 32 ? 2 : 4;
-    w.ok = true;
-    if (m <= 16) {
-        // The build by grid size. Measured at 8 / 16 rows (3584 -> 152064, 3584 -> 37888, 4096 -> 16384): three or more
-        // workgroups per CU run best with the windows two ahead (68 -> 64 us); fewer workgroups than CUs with weights and
-        // windows both ahead (17.2 -> 14.5 us); in between neither helps the sums build (20.6 us either way; with both ahead
-        // it spills at block size 32).
-        if (ww > kWideWaves) {
-            // a balanced grid has at most one workgroup per CU: the builds for few workgroups, compiled for twelve waves
-            if (bs == 128 && st16) {
-                w.pf = w.deep = w.grid < cus;
-            } else if (bs == 64 && st16 && !pair) {
-                w.pf = w.deep = true;              // (sums is false here)
-            } else {
-                w.ok = false;
-            }
-        } else if (!w.sums) {
-            w.deep = true;
-            w.pf = !(alone >= 3 * cus && bs != 32);
-        } else if (bs != 32) {
-            w.pf = w.deep = w.grid < cus;
-        } else {
-            w.ok = false;                          // (block size 32 never takes the sums)
-        }
-    } else {
-        // More row blocks per wave only where they fit the register file: two from block size 64, four at 128. The
-        // spilling forms ran several times slower than the routes that take those calls instead (3584 -> 37888: 153 us
-        // at block 32 and 32 rows against 2 x 37 us in blocks of 16 rows; 258 us at block 64 and 64 rows against 83 us
-        // in the tiled kernel). The paired form takes up to 16 rows.
-        w.sums = true;
-        w.pf = w.deep = false;
-        if (pair || bs == 32 || (m > 32 && bs == 64)) w.ok = false;
-    }
-    return w;
-}
-
-template <bool BF16, typename ST>
-static int launch_wide_bs(const PackedParams& p, int bs, int64_t cus, hipStream_t stream)
-{
-    const bool pair = p.packed_up != nullptr;
-    const WidePlan w = plan_wide(p.m, p.n, bs, sizeof(ST) == 2, pair, cus);
-    if (!w.ok) return -1;
-    const dim3 grid(w.grid);
-    auto go = [&](auto kernel, size_t lds) {
-        if (lds > 65536) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-            if (e != hipSuccess) return static_cast<int>(e);
-        }
-        hipLaunchKernelGGL(kernel, grid, dim3(w.waves * 64), lds, stream, p);
-        return static_cast<int>(hipGetLastError());
-    };
-    auto by_rows = [&](auto bs_tag) {
-        constexpr int BS = decltype(bs_tag)::value;
-        // two window buffers of rows x (tiles x 256 + 16) bytes, then two tables of (blocks per window) x rows f32 sums
-        constexpr int NBT = 128 / BS;
-        constexpr size_t lds16 = 2 * 16 * (4 * 256 + 16), sums16 = 2 * 4 * NBT * 16 * 4;
-        auto upto16 = [&](auto pair_tag) {
-            constexpr bool P = decltype(pair_tag)::value;
-            if (w.wmax > kWideWaves) {
-                if constexpr (BS == 128 && sizeof(ST) == 2) {
-                    if (w.pf) return go(decode_wide_kernel<BF16, BS, ST, 1, true, true, true, P, kWideWavesMax>, lds16 + sums16);
-                    return go(decode_wide_kernel<BF16, BS, ST, 1, true, false, false, P, kWideWavesMax>, lds16 + sums16);
-                } else if constexpr (BS == 64 && sizeof(ST) == 2 && !P) {
-                    return go(decode_wide_kernel<BF16, BS, ST, 1, false, true, true, false, kWideWavesMax>, lds16);
-                } else {
-                    return -1;
-                }
-            }
-            if (!w.sums) {
-                if (!w.pf) return go(decode_wide_kernel<BF16, BS, ST, 1, false, false, true, P>, lds16);
-                return go(decode_wide_kernel<BF16, BS, ST, 1, false, true, true, P>, lds16);
-            }
-            if constexpr (BS != 32) {
-                if (w.pf) return go(decode_wide_kernel<BF16, BS, ST, 1, true, true, true, P>, lds16 + sums16);
-                return go(decode_wide_kernel<BF16, BS, ST, 1, true, false, false, P>, lds16 + sums16);
-            } else {
-                return -1;
-            }
-        };
-        if (p.m <= 16) return pair ? upto16(std::true_type{}) : upto16(std::false_type{});
-        if constexpr (BS == 32) return -1;
-        else {
-            if (p.m <= 32) return go(decode_wide_kernel<BF16, BS, ST, 2, true, false, false>, 2 * 32 * (4 * 256 + 16) + 2 * 4 * NBT * 32 * 4);
-            if constexpr (BS == 64) return -1;
-            else return go(decode_wide_kernel<BF16, BS, ST, 4, true, false, false>, 2 * 64 * (2 * 256 + 16) + 2 * 2 * NBT * 64 * 4);
-        }
-    };
-    switch (bs) {
-        case 32: return by_rows(std::integral_constant<int, 32>{});
-        case 64: return by_rows(std::integral_constant<int, 64>{});
-        default: return by_rows(std::integral_constant<int, 128>{});
     }
 }
 
@@ -1484,25 +574,58 @@ extern "C" uint64_t rocm_decode_packed_bytes(const RocmMatMulNBitsArgs* a)
     return col_groups * static_cast<uint64_t>(mnb::packed_groups(a)) * static_cast<uint64_t>(mnb::packed_chunk_bytes(a));
 }
 
-extern "C" int rocm_launch_pack_decode(const RocmMatMulNBitsArgs* a, void* packed, rocm_stream_t stream)
+static int launch_pack_decode(const RocmMatMulNBitsArgs* a, int bits, int groups, void* packed, rocm_stream_t stream)
 {
     mnb::PackParams p;
+    p.bits = bits;
     p.b = a->b;
     p.scales = a->scales;
     p.zp = a->zp;
     p.out = static_cast<uint8_t*>(packed);
     p.n = a->n;
     p.kb = (a->k + a->block_size - 1) / a->block_size;
-    p.row_bytes = p.kb * a->block_size / 2;
-    p.zp_row = (p.kb + 1) / 2;
+    p.row_bytes = p.kb * a->block_size * bits / 8;
+    p.zp_row = (p.kb * bits + 7) / 8;
     p.bs_log2 = __builtin_ctz(static_cast<unsigned>(a->block_size));
     p.scale_bytes = a->scale_dtype == ROCM_DT_F32 ? 4 : 2;
-    p.groups = mnb::packed_groups(a);
+    p.groups = groups;
     p.chunk_bytes = mnb::packed_chunk_bytes(a);
     p.record = mnb::packed_record_bytes(a->block_size, p.scale_bytes);
     const dim3 grid(static_cast<unsigned>(p.groups), static_cast<unsigned>((a->n + 15) / 16));
     hipLaunchKernelGGL(mnb::pack_decode_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int rocm_launch_pack_decode(const RocmMatMulNBitsArgs* a, void* packed, rocm_stream_t stream)
+{
+    return launch_pack_decode(a, 4, mnb::packed_groups(a), packed, stream);
+}
+
+// The 4-bit call whose stream an 8-bit call's is, in everything that plans or sizes it: twice the tiles, the same activations.
+static RocmMatMulNBitsArgs as_planes(const RocmMatMulNBitsArgs* a)
+{
+    RocmMatMulNBitsArgs planes = *a;
+    const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
+    planes.k = (kb * a->block_size + 127) / 128 * 256;
+    return planes;
+}
+
+extern "C" int rocm_decode_packed8_eligible(const RocmMatMulNBitsArgs* a)
+{
+    const RocmMatMulNBitsArgs planes = as_planes(a);
+    return a->k % 8 == 0 && a->scale_dtype == a->a_dtype && !a->gamma && rocm_decode_packed_eligible(&planes);
+}
+
+extern "C" uint64_t rocm_decode_packed8_bytes(const RocmMatMulNBitsArgs* a)
+{
+    const RocmMatMulNBitsArgs planes = as_planes(a);
+    return rocm_decode_packed_bytes(&planes);
+}
+
+extern "C" int rocm_launch_pack_decode8(const RocmMatMulNBitsArgs* a, void* packed, rocm_stream_t stream)
+{
+    const RocmMatMulNBitsArgs planes = as_planes(a);
+    return launch_pack_decode(a, 8, mnb::packed_groups(&planes), packed, stream);
 }
 
 // The launch of rocm_launch_decode_packed; with `packed_up` the paired gate/up launch. `probe_only`: nothing is launched,
@@ -1686,17 +809,12 @@ extern "C" int rocm_decode_packed_plan(const RocmMatMulNBitsArgs* a, int waves, 
     return 0;
 }
 
-static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, const void* packed_up, int decomposed, int waves, bool probe_only,
-                                bool pair_member, rocm_stream_t stream)
+// Operands and stream geometry of a launch over `a`'s stream.
+static mnb::PackedParams packed_params(const RocmMatMulNBitsArgs* a, const void* packed)
 {
-    if (!rocm_decode_packed_eligible(a)) return probe_only ? 0 : -1;
-    const int64_t cus = rocm_ffi_compute_units();
-    const PackedPlan plan = plan_decode_packed(a, waves, pair_member, packed_up != nullptr, cus);
-    mnb::PackedParams p;
+    mnb::PackedParams p{};
     p.a = static_cast<const uint16_t*>(a->a);
     p.packed = static_cast<const uint8_t*>(packed);
-    p.packed_up = static_cast<const uint8_t*>(packed_up);
-    p.decomposed_silu = decomposed;
     p.bias = a->bias;
     p.y = a->y;
     p.m = a->m;
@@ -1708,11 +826,20 @@ static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed
     p.bias_dtype = a->bias_dtype;
     p.y_dtype = a->y_dtype;
     p.nibble_mask = 0x000F000Fu;
+    p.magic = a->a_dtype == ROCM_DT_BF16 ? 0x43004300u : 0x64006400u;
+    return p;
+}
+
+static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, const void* packed_up, int decomposed, int waves, bool probe_only,
+                                bool pair_member, rocm_stream_t stream)
+{
+    if (!rocm_decode_packed_eligible(a)) return probe_only ? 0 : -1;
+    const int64_t cus = rocm_ffi_compute_units();
+    const PackedPlan plan = plan_decode_packed(a, waves, pair_member, packed_up != nullptr, cus);
+    mnb::PackedParams p = packed_params(a, packed);
+    p.packed_up = static_cast<const uint8_t*>(packed_up);
+    p.decomposed_silu = decomposed;
     const bool bf16 = a->a_dtype == ROCM_DT_BF16;
-    p.magic = bf16 ? 0x43004300u : 0x64006400u;
-    p.gamma = nullptr;
-    p.gamma_f32 = 0;
-    p.norm_epsilon = 0.f;
     if (a->gamma) {
         if (!rocm_decode_packed_fuses_norm(a)) return probe_only ? 0 : -1;
         p.gamma = a->gamma;
@@ -1745,6 +872,25 @@ static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed
 extern "C" int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
 {
     return launch_decode_packed(a, packed, nullptr, 0, waves, false, false, stream);
+}
+
+extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+{
+    if (!rocm_decode_packed8_eligible(a)) return -1;
+    const RocmMatMulNBitsArgs planes = as_planes(a);
+    const int64_t cus = rocm_ffi_compute_units();
+    const PackedPlan plan = plan_decode_packed(&planes, waves, false, false, cus);
+    mnb::PackedParams p = packed_params(&planes, packed);
+    p.k = a->k;                              // what the activations have
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool bf16 = a->a_dtype == ROCM_DT_BF16;
+    if (plan.wide) {
+        p.groups_per_wave = p.groups;
+        const int64_t col_groups = (a->n + 15) / 16;
+        return mnb::launch_wide8(p, bf16, a->block_size, (col_groups + mnb::kWideWaves - 1) / mnb::kWideWaves < cus, s);
+    }
+    p.groups_per_wave = plan.groups_per_wave;
+    return mnb::launch_packed8(p, bf16, a->block_size, plan.waves, s);
 }
 
 extern "C" int rocm_launch_decode_packed_pair_member(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
