@@ -699,6 +699,21 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
             if (ns.code != NXRT_OK) return ns;
         }
     }
+    // The tiled kernel over packed weights. Small grids slice K and want scratch for the partial sums: the caller's workspace if it is
+    // large enough, else the kernel's own (grown outside a capture only; with too little the launcher slices less or not at all).
+    auto tiled = [&](auto launch) {
+        const uint64_t need = rocm_prefill_mfma_scratch_bytes(&args, kn.ep->prefill_tile);
+        void* scratch = workspace;
+        uint64_t scratch_bytes = workspace ? workspace_bytes : 0;
+        if (need > scratch_bytes) {
+            if (kn.scratch_bytes < need && !frozen(kn)) (void)grow_buffer(kn.scratch, kn.scratch_bytes, need, kn.retired);   // on failure: slice less
+            if (kn.scratch_bytes > scratch_bytes) {
+                scratch = kn.scratch;
+                scratch_bytes = kn.scratch_bytes;
+            }
+        }
+        return launch(&args, kn.ep->prefill_tile, scratch, scratch_bytes, stream);
+    };
     if (G && kn.g_idx_checked != args.g_idx) {
         // matmul_nbits.rs:3515-3521: every group must lie in 0..kb. Checked once per tensor (a device pass and a read-back).
         if (frozen(kn))
@@ -713,14 +728,18 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     const bool sorted = G && sort_by_group(kn, args, rc);
     if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
     if (kn.bits != 4 || args.g_idx) {
-        // Up to 64 rows of 8-bit weights stream the repacked copy; the accumulators' offset costs a 16-bit result nothing, so f32
-        // results stay on the routes below.
-        const bool streamed = kn.bits == 8 && !args.g_idx && M <= 64 && args.y_dtype != ROCM_DT_F32 && args.n * args.k >= min_streamed_weights(args.m) && use_packed(kn, args, rc);
+        // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
+        // row blocks over the stream took 97 / 101); the accumulators' offset costs a 16-bit result nothing, so f32 results stay on the routes below.
+        const bool streamed = kn.bits == 8 && !args.g_idx && M <= 32 && args.y_dtype != ROCM_DT_F32 && args.n * args.k >= min_streamed_weights(args.m) && use_packed(kn, args, rc);
         // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
         if (streamed) {
             if (rc == 0) rc = rocm_launch_decode_packed8(&args, kn.packed, kn.ep->decode_waves, stream);
             kn.variant = "decode_mfma_packed8";
+        } else if (kn.bits == 8 && !args.g_idx && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && args.n * args.k >= min_streamed_weights(args.m) &&
+                   rocm_prefill_mfma8_eligible(&args)) {
+            rc = tiled(rocm_launch_prefill_mfma8);
+            kn.variant = "prefill_mfma_lds8";
         } else if (!dense_route(kn, args, rc)) {
             rc = rocm_launch_gemv_nbits(&args, static_cast<int>(kn.bits), stream);
             kn.variant = "gemv_nbits_f32";
@@ -795,19 +814,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     } else if (dense_route(kn, args, rc)) {
         // done: weights expanded to 16 bits, then the library GEMM
     } else if (M > 16 && rocm_prefill_mfma_eligible(&args)) {
-        // Small grids slice K and want scratch for the partial sums: the caller's workspace if it is large enough, else
-        // the kernel's own (grown outside a capture only; with too little the launcher slices less or not at all).
-        const uint64_t need = rocm_prefill_mfma_scratch_bytes(&args, kn.ep->prefill_tile);
-        void* scratch = workspace;
-        uint64_t scratch_bytes = workspace ? workspace_bytes : 0;
-        if (need > scratch_bytes) {
-            if (kn.scratch_bytes < need && !frozen(kn)) (void)grow_buffer(kn.scratch, kn.scratch_bytes, need, kn.retired);   // on failure: slice less
-            if (kn.scratch_bytes > scratch_bytes) {
-                scratch = kn.scratch;
-                scratch_bytes = kn.scratch_bytes;
-            }
-        }
-        rc = rocm_launch_prefill_mfma(&args, kn.ep->prefill_tile, scratch, scratch_bytes, stream);
+        rc = tiled(rocm_launch_prefill_mfma);
         kn.variant = "prefill_mfma_lds";
     } else if (args.n >= kGemmF32MinCols && rocm_gemm_f32_eligible(&args) && rocm_gemm_f32_pays(&args)) {
         rc = rocm_launch_gemm_f32(&args, stream);

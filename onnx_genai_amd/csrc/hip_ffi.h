@@ -220,6 +220,10 @@ int rocm_prefill_mfma_plan(const RocmMatMulNBitsArgs* args, int tile_choice, uin
 int rocm_launch_slice_reduce(const float* partial, int slices, int64_t m, int64_t n, const void* bias, int bias_dtype, void* y, int y_dtype,
                              rocm_stream_t stream);
 int rocm_launch_prefill_mfma(const RocmMatMulNBitsArgs* args, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream);
+/* The same tiled kernel over packed 8-bit weights (args->b [N, kb, bs], zp [N, kb] or NULL = 128; scales of the activations' type), from
+ * one row; scratch as above (rocm_prefill_mfma_scratch_bytes: the plan does not depend on the width). */
+int rocm_prefill_mfma8_eligible(const RocmMatMulNBitsArgs* args);
+int rocm_launch_prefill_mfma8(const RocmMatMulNBitsArgs* args, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream);
 /* The same tiled kernel over weights that a launch of their own has expanded to a dense [N, K] matrix of the activations' 16-bit
  * type (w16_nk, 16-byte aligned; K % 64 == 0): the tall route of bits = 2 / 8 and of weights with g_idx, whose packed forms the
  * tile loader does not read. args->b / scales / zp are not read; tiles of 128 columns at most. */

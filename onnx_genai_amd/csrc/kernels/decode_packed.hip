@@ -613,7 +613,7 @@ static RocmMatMulNBitsArgs as_planes(const RocmMatMulNBitsArgs* a)
 extern "C" int rocm_decode_packed8_eligible(const RocmMatMulNBitsArgs* a)
 {
     const RocmMatMulNBitsArgs planes = as_planes(a);
-    return a->k % 8 == 0 && a->scale_dtype == a->a_dtype && !a->gamma && rocm_decode_packed_eligible(&planes);
+    return a->m <= 32 && a->k % 8 == 0 && a->scale_dtype == a->a_dtype && !a->gamma && rocm_decode_packed_eligible(&planes);
 }
 
 extern "C" uint64_t rocm_decode_packed8_bytes(const RocmMatMulNBitsArgs* a)

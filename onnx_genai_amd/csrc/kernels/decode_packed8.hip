@@ -46,7 +46,7 @@ int launch_packed8(const PackedParams& p, bool bf16, int block_size, int waves, 
 template <bool BF16, int BS, int RB, bool SUMS, bool PF, bool DEEP>
 static int launch_wide8_cfg(const PackedParams& p, hipStream_t stream)
 {
-    constexpr int AT = RB == 4 ? 1 : 2, NBT = 128 / BS, kRows = RB * 16;
+    constexpr int AT = 2, NBT = 128 / BS, kRows = RB * 16;
     const size_t lds = 2 * kRows * (AT * 256 + 16) + (SUMS ? 2 * AT * NBT * kRows * 4 : 0);
     const int64_t col_groups = (p.n + 15) / 16;
     hipLaunchKernelGGL((decode_wide8_kernel<BF16, BS, RB, SUMS, PF, DEEP>), dim3(static_cast<unsigned>((col_groups + kWideWaves - 1) / kWideWaves)), dim3(kWideWaves * 64), lds,
@@ -65,7 +65,6 @@ static int launch_wide8_bs(const PackedParams& p, bool few_workgroups, hipStream
     if constexpr (BS != 32) {
         if (p.m <= 32) return launch_wide8_cfg<BF16, BS, 2, true, false, false>(p, stream);
     }
-    if constexpr (BS == 128) return launch_wide8_cfg<BF16, BS, 4, true, false, false>(p, stream);
     return -1;
 }
 

@@ -25,9 +25,13 @@ namespace mnb {
 // everything else in f32.
 // DENSE: B is not packed 4-bit weights but a [N, K] matrix of the activations' 16-bit type (weights of another width or with
 // g_idx, expanded by a launch of their own): a lane copies its 16-byte pieces to LDS as they are; no scales, no zero points.
-template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false>
+// BITS: 4, or 8 (bytes of B are weights; zero points are bytes, 128 when absent): the bytes are dequantized on their way to LDS like
+// nibbles, instead of by a launch that writes all of B as 16 bits first (bf16, block 128, 500 rows: 3584 -> 37888 391 -> 208 us, 18944 -> 3584
+// 197 -> 103; 65 rows 262 -> 90 and 180 -> 50), and the 256 x 256 tile and slices of K are open to them.
+template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false, int BITS = 4>
 __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
 {
+    static_assert(BITS == 4 || (BITS == 8 && !DENSE && !SF32), "packed weights of 4 bits, or of 8 with 16-bit scales");
     static_assert(!DENSE || (BN <= 128 && !SF32), "dense weights: four times the bytes per column, so only the narrower tiles have the registers");
     constexpr bool F32MATH = BF16 || SF32;
     constexpr int WM = BM / 4;             // wave sub-tile rows
@@ -37,8 +41,8 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
     constexpr int A_LOADS = BM / 64;       // 16-byte pieces of A per lane per step
     constexpr int B_DW = BN / 64;          // packed dwords of B per lane per step (1, 2 or 4); dense: 16-byte pieces
     constexpr int B_PIECES = 8 / B_DW;     // lanes that share one column's 32 (dense: 128) bytes of a step
-    constexpr int B_REGS = DENSE ? 4 * B_DW : B_DW;
-    constexpr uint32_t kBStep = DENSE ? 128u : 32u;            // bytes of one column per step
+    constexpr int B_REGS = DENSE ? 4 * B_DW : BITS == 8 ? 2 * B_DW : B_DW;
+    constexpr uint32_t kBStep = DENSE ? 128u : BITS == 8 ? 64u : 32u;            // bytes of one column per step
     const uint32_t nib_mask = __builtin_amdgcn_mov_dpp(p.nibble_mask, 0xE4, 0xf, 0xf, false);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char* lds_a = smem;                                   // [2][BM][kPitch]
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
     const __amdgpu_buffer_rsrc_t srd_s = make_srd(static_cast<const unsigned char*>(p.scales) + n_base * p.kb * kScaleBytes,
                                                     static_cast<uint64_t>(cols_left * p.kb) * kScaleBytes);
     const bool has_zp = p.zp != nullptr;
-    const uint32_t zp_mask = has_zp ? 0xfu : 0u, zp_default = has_zp ? 0u : 8u;   // branch-free "8 when absent"
+    const uint32_t zp_mask = has_zp ? (1u << BITS) - 1u : 0u, zp_default = has_zp ? 0u : 1u << (BITS - 1);   // branch-free "8 (128) when absent"
     const __amdgpu_buffer_rsrc_t srd_z = make_srd(has_zp ? p.zp + n_base * p.zp_row : p.b, has_zp ? static_cast<uint64_t>(cols_left * p.zp_row) : 0);
 
     // A: lane -> (row t/8 + 64 i, piece t%8). B: lane -> (column t / B_PIECES, piece t % B_PIECES of the 64-element step).
@@ -68,7 +72,7 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
     const uint32_t a_gstep = 64u * static_cast<uint32_t>(p.k) * 2u;
     const uint32_t a_loff = static_cast<uint32_t>((t >> 3) * kPitch + (t & 7) * 16);
     const int bcol = t / B_PIECES, bpiece = t % B_PIECES;
-    const uint32_t b_goff = static_cast<uint32_t>(bcol) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(bpiece * B_DW * (DENSE ? 16 : 4));
+    const uint32_t b_goff = static_cast<uint32_t>(bcol) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(bpiece * B_DW * (DENSE ? 16 : BITS));
     const uint32_t b_loff = static_cast<uint32_t>(bcol * kPitch + bpiece * B_DW * 16);
     const uint32_t s_goff = static_cast<uint32_t>(bcol) * static_cast<uint32_t>(p.kb) * kScaleBytes;
     const uint32_t z_goff = static_cast<uint32_t>(bcol) * static_cast<uint32_t>(p.zp_row);
@@ -115,7 +119,23 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
             r.s = r.z = r.zsh = 0;
             return;
         }
-        if constexpr (B_DW == 1) {
+        if constexpr (BITS == 8) {
+            static_assert(B_REGS == 2 || B_REGS % 4 == 0, "8 or 16 bytes per load");
+            if constexpr (B_REGS == 2) {
+                const auto bw = __builtin_amdgcn_raw_buffer_load_b64(srd_b, static_cast<int>(b_goff), static_cast<int>(kt * kBStep), 0);
+                r.b[0] = bw[0];
+                r.b[1] = bw[1];
+            } else {
+#pragma unroll
+                for (int i = 0; i < B_REGS / 4; ++i) {
+                    const uint4 bw = load16(srd_b, b_goff + static_cast<uint32_t>(i) * 16u, static_cast<uint32_t>(kt) * kBStep);
+                    r.b[4 * i] = bw.x;
+                    r.b[4 * i + 1] = bw.y;
+                    r.b[4 * i + 2] = bw.z;
+                    r.b[4 * i + 3] = bw.w;
+                }
+            }
+        } else if constexpr (B_DW == 1) {
             r.b[0] = __builtin_amdgcn_raw_buffer_load_b32(srd_b, static_cast<int>(b_goff), static_cast<int>(kt * 32), 0);
         } else if constexpr (B_DW == 2) {
             const auto bw = __builtin_amdgcn_raw_buffer_load_b64(srd_b, static_cast<int>(b_goff), static_cast<int>(kt * 32), 0);
@@ -132,9 +152,9 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
         if constexpr (SF32) r.s = __builtin_amdgcn_raw_buffer_load_b32(srd_s, static_cast<int>(s_goff + blk * 4u), 0, 0);
         else r.s = __builtin_amdgcn_raw_buffer_load_b16(srd_s, static_cast<int>(s_goff + blk * 2u), 0, 0);
         // loaded even without zero points (the empty range then returns 0): a branch here would split the loop body
-        const uint32_t zraw = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(srd_z, static_cast<int>(z_goff + (blk >> 1)), 0, 0));
+        const uint32_t zraw = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(srd_z, static_cast<int>(z_goff + (BITS == 8 ? blk : blk >> 1)), 0, 0));
         r.z = zraw;                 // no arithmetic on a loaded value here: it would wait for the load at once
-        r.zsh = (blk & 1u) * 4u;
+        r.zsh = BITS == 8 ? 0u : (blk & 1u) * 4u;
     };
     // Quarter `part` (0..3) of one step's trip from registers to LDS: A pieces part, part+4, ... and one packed dword of
     // B, dequantized (with two dwords per lane: in quarters 0 and 2). Four quarters make a step; they are issued between
@@ -148,6 +168,14 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
         unsigned char* lb = lds_b + buf * (BN * kPitch) + b_loff;
         if constexpr (DENSE) {
             *reinterpret_cast<uint4*>(lb + dw * 16) = make_uint4(r.b[4 * dw], r.b[4 * dw + 1], r.b[4 * dw + 2], r.b[4 * dw + 3]);
+            return;
+        }
+        if constexpr (BITS == 8) {
+            const uint32_t zq = (r.z & zp_mask) | zp_default;
+            uint4 v;
+            if constexpr (BF16) v = dequant_bytes_bf16(r.b[2 * dw], r.b[2 * dw + 1], zq, __uint_as_float(r.s << 16));
+            else v = dequant_bytes_f16(r.b[2 * dw], r.b[2 * dw + 1], zq, r.s);
+            *reinterpret_cast<uint4*>(lb + dw * 16) = v;
             return;
         }
         const uint32_t w = r.b[dw];
@@ -244,12 +272,12 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
     }
 }
 
-template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false>
+template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false, int BITS = 4>
 static int launch_prefill(const PrefillParams& p, int splits, hipStream_t stream)
 {
     const dim3 grid(static_cast<unsigned>((p.n + BN - 1) / BN), static_cast<unsigned>((p.m + BM - 1) / BM), static_cast<unsigned>(splits));
     const size_t lds = 2 * static_cast<size_t>(BM + BN) * kPitch;
-    auto kernel = prefill_mfma_kernel<BF16, BM, BN, SF32, DENSE>;
+    auto kernel = prefill_mfma_kernel<BF16, BM, BN, SF32, DENSE, BITS>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return static_cast<int>(e);
@@ -387,7 +415,7 @@ extern "C" int rocm_prefill_mfma_plan(const RocmMatMulNBitsArgs* a, int tile_cho
 }
 
 // The launch of both entry points below. `dense`: a->b is a [N, K] matrix of the activations' 16-bit type instead of packed weights.
-static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
+static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int bits, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
 {
     mnb::PrefillParams p;
     p.a = static_cast<const uint16_t*>(a->a);
@@ -400,8 +428,8 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int tile_choic
     p.n = a->n;
     p.k = a->k;
     p.kb = (a->k + a->block_size - 1) / a->block_size;
-    p.row_bytes = dense ? a->k * 2 : p.kb * a->block_size / 2;
-    p.zp_row = (p.kb + 1) / 2;
+    p.row_bytes = dense ? a->k * 2 : p.kb * a->block_size * bits / 8;
+    p.zp_row = (p.kb * bits + 7) / 8;
     p.bs_log2 = __builtin_ctz(static_cast<unsigned>(a->block_size));
     p.scale_dtype = a->scale_dtype;
     p.bias_dtype = a->bias_dtype;
@@ -428,8 +456,16 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int tile_choic
         if (plan.tile == 3) return mnb::launch_prefill<B, 128, 64, false, true>(p, plan.splits, s);
         return mnb::launch_prefill<B, 128, 128, false, true>(p, plan.splits, s);
     };
+    auto go8 = [&](auto bf) {
+        constexpr bool B = decltype(bf)::value;
+        if (plan.tile == 2) return mnb::launch_prefill<B, 256, 256, false, false, 8>(p, plan.splits, s);
+        if (plan.tile == 1) return mnb::launch_prefill<B, 256, 128, false, false, 8>(p, plan.splits, s);
+        if (plan.tile == 3) return mnb::launch_prefill<B, 128, 64, false, false, 8>(p, plan.splits, s);
+        return mnb::launch_prefill<B, 128, 128, false, false, 8>(p, plan.splits, s);
+    };
     int rc;
-    if (dense) rc = bf16 ? go_dense(std::true_type{}) : go_dense(std::false_type{});
+    if (bits == 8) rc = bf16 ? go8(std::true_type{}) : go8(std::false_type{});
+    else if (dense) rc = bf16 ? go_dense(std::true_type{}) : go_dense(std::false_type{});
     else if (bf16 && sf32) rc = go(std::true_type{}, std::true_type{});
     else if (bf16) rc = go(std::true_type{}, std::false_type{});
     else if (sf32) rc = go(std::false_type{}, std::true_type{});
@@ -441,7 +477,21 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int tile_choic
 extern "C" int rocm_launch_prefill_mfma(const RocmMatMulNBitsArgs* a, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
 {
     if (!rocm_prefill_mfma_eligible(a)) return -1;
-    return launch_tiled(a, false, tile_choice, scratch, scratch_bytes, stream);
+    return launch_tiled(a, false, 4, tile_choice, scratch, scratch_bytes, stream);
+}
+
+extern "C" int rocm_prefill_mfma8_eligible(const RocmMatMulNBitsArgs* a)
+{
+    RocmMatMulNBitsArgs four = *a;
+    if (four.m < 17) four.m = 17;                          // (the kernel takes any height; what is below is the caller's choice)
+    const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
+    return a->m >= 1 && a->scale_dtype == a->a_dtype && kb * a->block_size * 256 < 0x7fffffff && rocm_prefill_mfma_eligible(&four);
+}
+
+extern "C" int rocm_launch_prefill_mfma8(const RocmMatMulNBitsArgs* a, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
+{
+    if (!rocm_prefill_mfma8_eligible(a)) return -1;
+    return launch_tiled(a, false, 8, tile_choice, scratch, scratch_bytes, stream);
 }
 
 extern "C" int rocm_prefill_dense16_eligible(const RocmMatMulNBitsArgs* a)
@@ -465,7 +515,7 @@ extern "C" int rocm_launch_prefill_dense16(const RocmMatMulNBitsArgs* a, const v
     d.zp = nullptr;
     d.scale_dtype = a->a_dtype;
     d.block_size = 64;                      // (the planner only reads it through the eligibility of the packed form)
-    return launch_tiled(&d, true, tile_choice, scratch, scratch_bytes, stream);
+    return launch_tiled(&d, true, 4, tile_choice, scratch, scratch_bytes, stream);
 }
 
 extern "C" int rocm_launch_slice_reduce(const float* partial, int slices, int64_t m, int64_t n, const void* bias, int bias_dtype, void* y, int y_dtype,

@@ -28,8 +28,7 @@ CASES = [
     (E.F16, 128, True, 5, 40000, 256),
     (E.BF16, 128, False, 12, 100000, 128),
     (E.BF16, 64, True, 31, 16400, 448),
-    (E.F16, 128, True, 33, 16385, 512),
-    (E.BF16, 128, True, 64, 16400, 648),
+    (E.F16, 128, True, 32, 16385, 512),
 ]
 
 
