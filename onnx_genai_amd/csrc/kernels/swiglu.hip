@@ -18,74 +18,111 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict_
 // RMS-normalization prologue (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4125-4205): out = round16((a * inv_std) *
 // gamma) per row, inv_std = 1 / sqrt(mean(a^2) + eps). The sum of squares follows the reference's order exactly - 32
 // lanes, each with four running sums over its 4-element chunks, (s0 + s1) + (s2 + s3), then the shuffle tree over 32
-// lanes - so half a wavefront plays one 32-lane warp. A workgroup of four waves normalizes two rows: its first wave
-// sums the squares of both (sixteen loads in flight at a time), all four then scale four elements per lane and step.
-template <bool BF16>
-__global__ __launch_bounds__(256) void rmsnorm16_kernel(const uint16_t* __restrict__ a, const void* __restrict__ gamma, int gamma_dtype, int64_t rows,
-                                                        int64_t k, float epsilon, uint16_t* __restrict__ out)
+// lanes. What bounds a call of few rows is the chain launch, trip to memory, sum, trip, store. So a workgroup of four waves takes
+// one row, requests all of it and gamma at once (16 bytes a load; the pieces stay in registers up to kHeld a thread), passes the
+// row through LDS, and every wave sums it from there - lanes 0..31 the running sums s0 and s1 of the reference's lanes, lanes 32..63
+// s2 and s3 - so that nothing but one barrier lies between the row's arrival and its results. K = 3584, one / 16 rows, as a node of a
+// recorded step: 6.2 / 8.0 us with one wave summing two rows straight from memory, 4.6 / 4.8 us so (3.0 with everything in a near cache).
+constexpr int kHeld = 2;                     // 16-byte pieces of the row a thread keeps: 4096 elements a row
+
+// x + (x of the lane `N` further on in its row of 16, cyclically)
+template <int N>
+__device__ __forceinline__ float add_rotated(float x)
 {
-    __shared__ float inv_shared[2];
-    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * 2;
+    return __fadd_rn(x, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false)));
+}
+
+// STAGED: the row passes through LDS (K * 2 bytes of it); otherwise (rows beyond LDS) the sums read memory.
+template <bool BF16, bool STAGED>
+__global__ __launch_bounds__(256) void rmsnorm16_kernel(const uint16_t* __restrict__ a, const void* __restrict__ gamma, int gamma_dtype, int64_t k, float epsilon,
+                                                        uint16_t* __restrict__ out)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int t = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const uint16_t* const x = a + row * k;
+    // eight elements of the row, from an 8-byte boundary
+    auto load_piece = [&](int piece) {
+        const uint2* const from = reinterpret_cast<const uint2*>(x) + 2 * piece;
+        const uint2 lo = from[0], hi = from[1];
+        return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
+    const int pieces = static_cast<int>(k >> 3);
+    const bool gf32 = gamma_dtype == ROCM_DT_F32;
     auto widen = [](uint32_t bits16) { return BF16 ? bf16_bits_to_f32(static_cast<uint16_t>(bits16)) : f16_bits_to_f32(static_cast<uint16_t>(bits16)); };
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x & 31;
-        const int64_t row = row0 + (threadIdx.x >> 5);
-        const bool live = row < rows;
-        const uint2* x = reinterpret_cast<const uint2*>(a + (live ? row : row0) * k);
-        const int items = static_cast<int>(k / 128);
-        float ss0 = 0.f, ss1 = 0.f, ss2 = 0.f, ss3 = 0.f;
-        constexpr int kBatch = 16;
-        for (int first = 0; first < items; first += kBatch) {
-            uint2 raw[kBatch];
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i) raw[i] = first + i < items ? x[lane + (first + i) * 32] : make_uint2(0u, 0u);      // fma(0, 0, s) = s
-#pragma unroll
-            for (int i = 0; i < kBatch; ++i) {
-                const float v0 = widen(raw[i].x & 0xffffu), v1 = widen(raw[i].x >> 16), v2 = widen(raw[i].y & 0xffffu), v3 = widen(raw[i].y >> 16);
-                ss0 = __fmaf_rn(v0, v0, ss0);
-                ss1 = __fmaf_rn(v1, v1, ss1);
-                ss2 = __fmaf_rn(v2, v2, ss2);
-                ss3 = __fmaf_rn(v3, v3, ss3);
-            }
+    struct Weights { uint4 lo, hi; };        // eight gamma values: 16-bit ones all in `lo`
+    auto load_gamma = [&](int piece) {
+        Weights w;
+        w.lo = w.hi = make_uint4(0u, 0u, 0u, 0u);
+        if (gf32) {
+            w.lo = static_cast<const uint4*>(gamma)[2 * piece];
+            w.hi = static_cast<const uint4*>(gamma)[2 * piece + 1];
+        } else {
+            const uint2* const g = static_cast<const uint2*>(gamma) + 2 * piece;               // (8-byte aligned only)
+            const uint2 g0 = g[0], g1 = g[1];
+            w.lo = make_uint4(g0.x, g0.y, g1.x, g1.y);
         }
-        float ss = __fadd_rn(__fadd_rn(ss0, ss1), __fadd_rn(ss2, ss3));
+        return w;
+    };
+
+    uint4 held[kHeld];
+    Weights weights[kHeld];
 #pragma unroll
-        for (int off = 16; off > 0; off >>= 1) ss = __fadd_rn(ss, __shfl_down(ss, off, 32));
+    for (int i = 0; i < kHeld; ++i)
+        if (t + i * 256 < pieces) held[i] = load_piece(t + i * 256);
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+        if (t + i * 256 < pieces) weights[i] = load_gamma(t + i * 256);
+    if constexpr (STAGED) {
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i)
+            if (t + i * 256 < pieces) reinterpret_cast<uint4*>(smem)[t + i * 256] = held[i];
+        for (int piece = t + kHeld * 256; piece < pieces; piece += 256) reinterpret_cast<uint4*>(smem)[piece] = load_piece(piece);
+        __syncthreads();
+    }
+    float inv_std;
+    {
+        const int lane = t & 63;
+        // elements 2 (lane / 32) and + 1 of chunk (lane % 32) + 32 i
+        const uint32_t* const pair = (STAGED ? reinterpret_cast<const uint32_t*>(smem) : reinterpret_cast<const uint32_t*>(x)) + (lane & 31) * 2 + (lane >> 5);
+        const int items = static_cast<int>(k >> 7);
+        float even = 0.f, odd = 0.f;
+#pragma unroll 8
+        for (int i = 0; i < items; ++i) {
+            const uint32_t raw = pair[i * 64];
+            const float v0 = widen(raw & 0xffffu), v1 = widen(raw >> 16);
+            even = __fmaf_rn(v0, v0, even);
+            odd = __fmaf_rn(v1, v1, odd);
+        }
+        float ss = __fadd_rn(even, odd);
+        ss = __fadd_rn(ss, __shfl_xor(ss, 32, 64));         // (s0 + s1) + (s2 + s3)
+        ss = __fadd_rn(ss, __shfl_xor(ss, 16, 64));         // the reference's tree: every lane ends with what its lane 0 has
+        ss = add_rotated<8>(ss);
+        ss = add_rotated<4>(ss);
+        ss = add_rotated<2>(ss);
+        ss = add_rotated<1>(ss);
         // sqrtf, not __fsqrt_rn: the latter is the hardware's approximate square root here; sqrtf and the division are
         // correctly rounded (the compiler's default for f32 divide and sqrt)
-        const float inv_std = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, static_cast<float>(k)), epsilon)));
-        if (lane == 0) inv_shared[threadIdx.x >> 5] = inv_std;
+        inv_std = __fdiv_rn(1.0f, sqrtf(__fadd_rn(__fdiv_rn(ss, static_cast<float>(k)), epsilon)));
     }
-    __syncthreads();
-    const int chunks = static_cast<int>(k / 4);
-    for (int r = 0; r < 2; ++r) {
-        const int64_t row = row0 + r;
-        if (row >= rows) break;
-        const float inv_std = inv_shared[r];
-        const uint2* x = reinterpret_cast<const uint2*>(a + row * k);
-        uint2* y = reinterpret_cast<uint2*>(out + row * k);
-        for (int chunk = threadIdx.x; chunk < chunks; chunk += 256) {
-            const uint2 raw = x[chunk];
-            float g[4];
-            if (gamma_dtype == ROCM_DT_F32) {
-                const float4 gv = static_cast<const float4*>(gamma)[chunk];
-                g[0] = gv.x, g[1] = gv.y, g[2] = gv.z, g[3] = gv.w;
-            } else {
-                const uint2 gv = static_cast<const uint2*>(gamma)[chunk];
-                const bool gbf = gamma_dtype == ROCM_DT_BF16;
-                auto gw = [gbf](uint32_t bits16) { return gbf ? bf16_bits_to_f32(static_cast<uint16_t>(bits16)) : f16_bits_to_f32(static_cast<uint16_t>(bits16)); };
-                g[0] = gw(gv.x & 0xffffu), g[1] = gw(gv.x >> 16), g[2] = gw(gv.y & 0xffffu), g[3] = gw(gv.y >> 16);
-            }
-            const float v[4] = {widen(raw.x & 0xffffu), widen(raw.x >> 16), widen(raw.y & 0xffffu), widen(raw.y >> 16)};
-            uint32_t o[4];
+    auto store = [&](int piece, const uint4& raw, const Weights& w) {
+        const uint32_t d[4] = {raw.x, raw.y, raw.z, raw.w};
+        const uint32_t g[8] = {w.lo.x, w.lo.y, w.lo.z, w.lo.w, w.hi.x, w.hi.y, w.hi.z, w.hi.w};
+        uint32_t o[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float scaled = as_f32(__fmul_rn(__fmul_rn(v[e], inv_std), g[e]));
-                o[e] = BF16 ? f32_to_bf16_bits(scaled) : f32_to_f16_bits(scaled);
-            }
-            y[chunk] = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+        for (int i = 0; i < 4; ++i) {
+            const float g0 = gf32 ? __uint_as_float(g[2 * i]) : widen(g[i] & 0xffffu), g1 = gf32 ? __uint_as_float(g[2 * i + 1]) : widen(g[i] >> 16);
+            const float y0 = as_f32(__fmul_rn(__fmul_rn(widen(d[i] & 0xffffu), inv_std), g0)), y1 = as_f32(__fmul_rn(__fmul_rn(widen(d[i] >> 16), inv_std), g1));
+            o[i] = BF16 ? f32_to_bf16_bits(y0) | (static_cast<uint32_t>(f32_to_bf16_bits(y1)) << 16) : f32_to_f16_bits(y0) | (static_cast<uint32_t>(f32_to_f16_bits(y1)) << 16);
         }
-    }
+        uint2* const y = reinterpret_cast<uint2*>(out + row * k) + 2 * piece;                  // (8-byte aligned only)
+        y[0] = make_uint2(o[0], o[1]);
+        y[1] = make_uint2(o[2], o[3]);
+    };
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i)
+        if (t + i * 256 < pieces) store(t + i * 256, held[i], weights[i]);
+    for (int piece = t + kHeld * 256; piece < pieces; piece += 256) store(piece, STAGED ? reinterpret_cast<const uint4*>(smem)[piece] : load_piece(piece), load_gamma(piece));
 }
 
 }  // namespace mnb
@@ -99,15 +136,15 @@ extern "C" int rocm_launch_rmsnorm16(const void* a, const void* gamma, int gamma
     const uintptr_t gamma_mask = gamma_dtype == ROCM_DT_F32 ? 15 : 7;
     if (((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(out)) & 7) != 0 || (reinterpret_cast<uintptr_t>(gamma) & gamma_mask) != 0)
         return static_cast<int>(hipErrorInvalidValue);
-    const unsigned blocks = static_cast<unsigned>((rows + 1) / 2);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == ROCM_DT_BF16)
-        hipLaunchKernelGGL(mnb::rmsnorm16_kernel<true>, dim3(blocks), dim3(256), 0, s, static_cast<const uint16_t*>(a), gamma, gamma_dtype, rows, k, epsilon,
-                           static_cast<uint16_t*>(out));
-    else
-        hipLaunchKernelGGL(mnb::rmsnorm16_kernel<false>, dim3(blocks), dim3(256), 0, s, static_cast<const uint16_t*>(a), gamma, gamma_dtype, rows, k, epsilon,
-                           static_cast<uint16_t*>(out));
-    return static_cast<int>(hipGetLastError());
+    const bool staged = k <= 32768;          // what fits the 64 KiB a kernel gets without asking
+    const size_t lds = staged ? static_cast<size_t>(k) * 2 : 0;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(rows)), dim3(256), lds, s, static_cast<const uint16_t*>(a), gamma, gamma_dtype, k, epsilon, static_cast<uint16_t*>(out));
+        return static_cast<int>(hipGetLastError());
+    };
+    if (dtype == ROCM_DT_BF16) return staged ? go(mnb::rmsnorm16_kernel<true, true>) : go(mnb::rmsnorm16_kernel<true, false>);
+    return staged ? go(mnb::rmsnorm16_kernel<false, true>) : go(mnb::rmsnorm16_kernel<false, false>);
 }
 
 extern "C" int rocm_launch_swiglu(const void* gate, const void* up, int64_t count, int dtype, int decomposed, void* y, rocm_stream_t stream)
