@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 from dataclasses import dataclass
 
 import numpy as np
@@ -114,9 +115,9 @@ def load_library() -> C.CDLL:
     L.nxrt_rocm_matmul_nbits_workspace_requirement.restype = S
     L.nxrt_rocm_matmul_nbits_workspace_requirement.argtypes = [v, C.POINTER(NxrtTensorDesc), u32, C.POINTER(WorkspaceRequirement)]
     L.nxrt_rocm_matmul_nbits_execute.restype = S
-    L.nxrt_rocm_matmul_nbits_execute.argtypes = [v, C.POINTER(CTensorView), u32, C.POINTER(CTensorView), u32, v, u64]
+    L.nxrt_rocm_matmul_nbits_execute.argtypes = [v, v, u32, v, u32, v, u64]          # (views as addresses: arrays of CTensorView)
     L.nxrt_rocm_matmul_nbits_execute_static.restype = S
-    L.nxrt_rocm_matmul_nbits_execute_static.argtypes = [v, C.POINTER(CTensorView), u32, C.POINTER(CTensorView), u32]
+    L.nxrt_rocm_matmul_nbits_execute_static.argtypes = [v, v, u32, v, u32]
     L.nxrt_rocm_device_allocation_count.restype = u64
     L.nxrt_rocm_device_allocation_count.argtypes = []
     L.nxrt_rocm_matmul_nbits_estimated_flops.restype = u64
@@ -218,24 +219,41 @@ class TensorView:
         return TensorView(None, dtype, ())
 
 
-def _c_views(views):
-    arr = (CTensorView * max(len(views), 1))()
-    keep = []
-    for i, t in enumerate(views):
-        shape = (C.c_uint64 * max(len(t.shape), 1))(*[int(d) for d in t.shape])
-        keep.append(shape)
-        arr[i].data = t.data
-        arr[i].dtype = t.dtype
-        arr[i].ndim = len(t.shape)
-        arr[i].shape = C.cast(shape, C.POINTER(C.c_uint64))
-        if t.strides is not None:
-            st = (C.c_int64 * max(len(t.strides), 1))(*[int(s) for s in t.strides])
-            keep.append(st)
-            arr[i].strides = C.cast(st, C.POINTER(C.c_int64))
-        arr[i].byte_offset = t.byte_offset
-        arr[i].device_type = t.device_type
-        arr[i].device_index = t.device_index
-    return arr, keep
+_VIEW_BYTES = C.sizeof(CTensorView)
+_layouts: dict = {}                # (dimensions, strides given) of every view of a call -> how its CTensorView array and dims are packed
+
+
+def _packed_views(views):
+    """One call's CTensorView array with the dims (and strides) it points to behind it, in a buffer of its own. One struct.pack for the
+    whole call: filling ctypes structures field by field cost three times as much, more than a short node takes on the GPU."""
+    key = tuple((len(t.shape), t.strides is not None) for t in views)
+    layout = _layouts.get(key)
+    if layout is None:
+        fmt, offsets, at = "=" + "QIIQQQII" * len(views), [], _VIEW_BYTES * len(views)
+        for ndim, strided in key:
+            offsets.append((at, at + 8 * ndim if strided else 0))
+            fmt += "Q" * ndim + ("q" * ndim if strided else "")
+            at += 8 * ndim * (2 if strided else 1)
+        if len(_layouts) >= 1024:  # (as many kinds of calls as a program has nodes; bounded all the same)
+            _layouts.clear()
+        layout = _layouts[key] = (struct.Struct(fmt), offsets)
+    packer, offsets = layout
+    buf = C.create_string_buffer(packer.size)
+    base = C.addressof(buf)
+    values, dims = [], []
+    for t, (shape_at, strides_at) in zip(views, offsets):
+        shape = t.shape
+        values += (t.data or 0, t.dtype, len(shape), base + shape_at, base + strides_at if strides_at else 0, t.byte_offset, t.device_type, t.device_index)
+        dims += shape
+        if strides_at:
+            dims += t.strides
+    try:
+        packer.pack_into(buf, 0, *values, *dims)
+    except struct.error:           # numbers that are not plain integers of their field: convert and wrap as ctypes does, the library judges them
+        widths = ["Q", "I", "I", "Q", "Q", "Q", "I", "I"] * len(views) + ["Q"] * len(dims)
+        wrapped = [int(x) & (0xFFFFFFFF if w == "I" else 0xFFFFFFFFFFFFFFFF) for w, x in zip(widths, values + dims)]
+        struct.pack_into("=" + "".join(widths), buf, 0, *wrapped)
+    return buf, base
 
 
 class RocmExecutionProvider:
@@ -448,16 +466,14 @@ class MatMulNBitsKernel:
         return out.bytes, out.alignment
 
     def execute(self, inputs, outputs, workspace: DeviceBuffer | None = None) -> None:
-        cin, k1 = _c_views(inputs)
-        cout, k2 = _c_views(outputs)
-        self.lib.nxrt_rocm_matmul_nbits_execute(self.handle, cin, len(inputs), cout, len(outputs),
+        buf, at = _packed_views((*inputs, *outputs))
+        self.lib.nxrt_rocm_matmul_nbits_execute(self.handle, at, len(inputs), at + _VIEW_BYTES * len(inputs), len(outputs),
                                                 workspace.ptr if workspace else None, workspace.nbytes if workspace else 0).check()
 
     def execute_static(self, inputs, outputs) -> None:
         """execute without any device allocation: scratch comes from the library's static per-GPU array."""
-        cin, k1 = _c_views(inputs)
-        cout, k2 = _c_views(outputs)
-        self.lib.nxrt_rocm_matmul_nbits_execute_static(self.handle, cin, len(inputs), cout, len(outputs)).check()
+        buf, at = _packed_views((*inputs, *outputs))
+        self.lib.nxrt_rocm_matmul_nbits_execute_static(self.handle, at, len(inputs), at + _VIEW_BYTES * len(inputs), len(outputs)).check()
 
     def estimated_flops(self) -> int:
         return self.lib.nxrt_rocm_matmul_nbits_estimated_flops(self.handle)
