@@ -7,12 +7,24 @@
 
 namespace mnb {
 
+// Eight elements a lane (16-byte loads and stores) where all three matrices are 16-byte aligned; the remainder, and other alignments, one by
+// one. Bound by vector instructions and memory about equally: 8192 x 14336 elements, f16, about 365 -> 189 us (3.7 TB/s), 777 rows 43 -> 24.
 template <bool BF16>
-__global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up, int64_t count, int decomposed,
+__global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict__ gate, const uint16_t* __restrict__ up, int64_t count, int64_t pieces, int decomposed,
                                                      uint16_t* __restrict__ y)
 {
-    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < count; i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        y[i] = swiglu16<BF16>(gate[i], up[i], decomposed != 0);
+    const int64_t first = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x, step = static_cast<int64_t>(gridDim.x) * blockDim.x;
+    const bool dec = decomposed != 0;
+    for (int64_t i = first; i < pieces; i += step) {
+        const uint4 g = reinterpret_cast<const uint4*>(gate)[i], u = reinterpret_cast<const uint4*>(up)[i];
+        const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
+        uint32_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            o[j] = swiglu16<BF16>(gw[j] & 0xffffu, uw[j] & 0xffffu, dec) | (static_cast<uint32_t>(swiglu16<BF16>(gw[j] >> 16, uw[j] >> 16, dec)) << 16);
+        reinterpret_cast<uint4*>(y)[i] = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    for (int64_t i = pieces * 8 + first; i < count; i += step) y[i] = swiglu16<BF16>(gate[i], up[i], dec);
 }
 
 // RMS-normalization prologue (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4125-4205): out = round16((a * inv_std) *
@@ -151,13 +163,16 @@ extern "C" int rocm_launch_swiglu(const void* gate, const void* up, int64_t coun
 {
     if (count <= 0) return 0;
     if (dtype != ROCM_DT_F16 && dtype != ROCM_DT_BF16) return static_cast<int>(hipErrorInvalidValue);
-    int64_t blocks = (count + 255) / 256;
+    const bool wide = ((reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+    const int64_t pieces = wide ? count / 8 : 0;
+    const int64_t items = wide && pieces > 0 ? pieces : count;
+    int64_t blocks = (items + 255) / 256;
     if (blocks > 65536) blocks = 65536;
     const uint16_t* g = static_cast<const uint16_t*>(gate);
     const uint16_t* u = static_cast<const uint16_t*>(up);
     uint16_t* out = static_cast<uint16_t*>(y);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == ROCM_DT_BF16) hipLaunchKernelGGL(mnb::swiglu_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g, u, count, decomposed, out);
-    else hipLaunchKernelGGL(mnb::swiglu_kernel<false>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g, u, count, decomposed, out);
+    if (dtype == ROCM_DT_BF16) hipLaunchKernelGGL(mnb::swiglu_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g, u, count, pieces, decomposed, out);
+    else hipLaunchKernelGGL(mnb::swiglu_kernel<false>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, g, u, count, pieces, decomposed, out);
     return static_cast<int>(hipGetLastError());
 }
