@@ -14,6 +14,8 @@
 // at 512 rows 8373 -> 69 us, 896 -> 896 at 64 rows 97 -> 5.8 us. What bounds it: a CU's vector memory path, which serves a load's 32 rows or columns
 // one cache line at a time (five to nine such loads per run of 32 k), then the vector ALU work of cutting activations and turning nibbles into
 // bf16 (about 120 instructions per lane, tile and run with two column tiles per wave, against 6 MFMAs of 32 cycles).
+#include <type_traits>
+
 #include "prefill_common.hiph"
 
 namespace mnb {
@@ -32,8 +34,8 @@ struct GemmF32Params {
     int units_per_wave;     // runs of 32 k a wave walks
 };
 
-// 8 * GROUPS f32 values as three bf16 operands each: plane[p][group].
-template <int GROUPS>
+// 8 * GROUPS f32 values as three bf16 operands each: plane[p][group]. What a cut leaves of an infinity is NaN; with WIDE it is 0.
+template <int GROUPS, bool WIDE>
 __device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], uint4 (&plane)[3][GROUPS])
 {
 #pragma unroll
@@ -46,8 +48,9 @@ __device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], ui
             for (int p = 0; p < 3; ++p) {
                 out[p][i] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);      // the upper halves: both values cut to bf16
                 if (p < 2) {                                                // what the cut leaves, exactly
-                    lo = __float_as_uint(__uint_as_float(lo) - __uint_as_float(lo & 0xffff0000u));
-                    hi = __float_as_uint(__uint_as_float(hi) - __uint_as_float(hi & 0xffff0000u));
+                    const bool lo_inf = WIDE && (lo & 0x7fffffffu) == 0x7f800000u, hi_inf = WIDE && (hi & 0x7fffffffu) == 0x7f800000u;
+                    lo = lo_inf ? 0u : __float_as_uint(__uint_as_float(lo) - __uint_as_float(lo & 0xffff0000u));
+                    hi = hi_inf ? 0u : __float_as_uint(__uint_as_float(hi) - __uint_as_float(hi & 0xffff0000u));
                 }
             }
         }
@@ -155,14 +158,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
         for (int j = 0; j < CN; ++j) sum[j][e] = 0.f;
     }
 
-    auto multiply = [&](const Run& x) {
+    auto multiply = [&](const Run& x, auto wide) {
+        constexpr bool kWide = decltype(wide)::value;
         uint32_t v[8 * G];
 #pragma unroll
         for (int i = 0; i < 2 * G; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * i + e] = x.a[i][e];
+            for (int e = 0; e < 4; ++e) v[4 * i + e] = kWide ? __float_as_uint(__uint_as_float(x.a[i][e]) * 0x1p-16f) : x.a[i][e];
         uint4 plane[3][G];
-        cut_in_three<G>(v, plane);
+        cut_in_three<G, kWide>(v, plane);
 #pragma unroll
         for (int j = 0; j < CN; ++j) {
             const uint32_t zq = ((x.z[j] >> x.zsh) & zp_mask) | zp_default;
@@ -175,7 +179,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
             for (int q = 2; q >= 0; --q)                                      // smallest parts first
 #pragma unroll
                 for (int g = 0; g < G; ++g) acc = Ops::mfma(plane[q][g], w[g], acc);
-            const float sc = ScaleIo<ST>::to_f32(x.s[j], scale_bf16);         // 0 for a column beyond N and past the end
+            const float sc = ScaleIo<ST>::to_f32(x.s[j], scale_bf16) * (kWide ? 0x1p16f : 1.f);         // 0 for a column beyond N and past the end
 #pragma unroll
             for (int e = 0; e < Ops::kAcc; ++e) sum[j][e] = fmaf(acc[e], sc, sum[j][e]);
         }
@@ -189,7 +193,25 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
         for (int d = 0; d < DEPTH; ++d) {
             request(x[(d + DEPTH - 1) % DEPTH], u + d + DEPTH - 1);
             __builtin_amdgcn_sched_barrier(0);
-            multiply(x[d]);
+            multiply(x[d], std::false_type{});
+        }
+    }
+
+    // A sum that is not finite: an activation was infinite (NaN came of it above), or so large that the unscaled sum of a run overflowed,
+    // or the result is what it is. The wave walks its share once more with the activations scaled by 2^-16, so that a run's 32
+    // products of up to 15 fit, and infinities kept whole in their first part. Asked once per wave, not per run: no cost otherwise.
+    bool finite = true;
+#pragma unroll
+    for (int j = 0; j < CN; ++j)
+#pragma unroll
+        for (int e = 0; e < Ops::kAcc; ++e) finite = finite && __builtin_isfinite(sum[j][e]);
+    if (__builtin_expect(__any(!finite), 0)) {
+#pragma unroll
+        for (int j = 0; j < CN; ++j) sum[j] = zero;
+#pragma unroll 1
+        for (int u = u0; u < u1; ++u) {
+            request(x[0], u);
+            multiply(x[0], std::true_type{});
         }
     }
 

@@ -45,3 +45,26 @@ def test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, bias
     tol = TOL + {E.F32: 0.0, E.F16: 2.0 ** -11, E.BF16: 2.0 ** -8}[y_dt]
     for row in range(m):                                    # by row: the rows differ in magnitude
         assert helpers.rel_l2(got[row], want[row]) <= tol, row
+
+
+@pytest.mark.parametrize("m,n,k", [(20, 128, 96), (70, 1100, 96), (600, 1100, 96)])      # the three tile shapes
+def test_infinities_nan_and_the_largest_values(ep, port, m, n, k):
+    """An infinite activation gives what its products give (NaN only over a weight of zero or against the other infinity), one near the
+    end of the range a finite result, and no other row notices."""
+    b, s, zp = synth.make_weights(n, k, 32, n, zero_points=True, scale_lo=0.002, scale_hi=0.01, scale_dtype=E.F32)
+    a = synth.make_activation(m, k, n, E.F32)
+    a[1, 5], a[2, 40], a[3, 70], a[4, 3], a[4, 64] = np.inf, -np.inf, np.nan, np.inf, -np.inf
+    a[5, 32:64] = np.finfo(np.float32).max * np.where(np.arange(32) % 3 == 0, -1, 1)
+    y, variant = E.matmul_nbits(ep, a, E.F32, b, s, E.F32, zp, n, k, 32, y_dtype=E.F32)
+    assert variant == "gemm_f32_mfma"
+    w = port.dequantize_nk_bits(b, s, zp, n, k, 32, 4).astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = np.stack([(a[r].astype(np.float64) * w).sum(axis=1) for r in range(m)])
+    for row in range(m):
+        if row in (1, 2, 3, 4):
+            assert np.array_equal(y[row].astype(np.float64), want[row], equal_nan=True), row
+        elif row == 5:                                      # outputs beyond the range of f32 are infinities
+            inside = np.abs(want[row]) < 0.99 * np.finfo(np.float32).max
+            assert inside.any() and helpers.rel_l2(y[row][inside].astype(np.float64) * 2.0 ** -100, want[row][inside] * 2.0 ** -100) <= TOL
+        else:
+            assert helpers.rel_l2(y[row].astype(np.float64), want[row]) <= TOL, row
