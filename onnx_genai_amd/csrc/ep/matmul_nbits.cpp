@@ -246,6 +246,13 @@ void drop_weight_copy(NxrtRocmMatMulNBits& kn, void* old)
     rocm_ffi_free(old);
 }
 
+// Taller calls on weights that are neither 4 bits nor contiguous may round them to 16 bits - the 16-bit copy that the dense route makes and
+// the tiled kernels' own tiles alike - from five rows up and while that copy is within its limit; everything else keeps its weights in 32 bits.
+bool weights_in_16_bits(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args)
+{
+    return static_cast<uint64_t>(args.n) * static_cast<uint64_t>(args.k) * 2 <= kn.ep->dense_gemm_max_bytes && rocm_prefill_dense16_eligible(&args);
+}
+
 // Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on
 // first use, args.a the call's activations in the same order, args.g_idx null. Returns false with `args` untouched where the groups
 // are not whole blocks, or the copy or the gather's buffer cannot be made now (a capture is open, no memory): the kernels that look
@@ -254,6 +261,8 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, int& rc)
 {
     rc = 0;
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[4]) return false;
+    // f32 results of 16-bit rows that the f32 GEMV has: the offset in the 4-bit streams' accumulators would show in their last bits
+    if (args.a_dtype != ROCM_DT_F32 && args.y_dtype == ROCM_DT_F32 && !weights_in_16_bits(kn, args)) return false;
     const size_t order_bytes = (static_cast<size_t>(args.k) * sizeof(int32_t) + 255) / 256 * 256;
     if (kn.regrouped_from[0] != args.b || kn.regrouped_from[1] != args.g_idx) {
         if (frozen(kn)) return false;
@@ -495,6 +504,30 @@ bool f32_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
 // 3584 -> 1024 5.2 us, 3584 -> 1200 5.4 against 4.4), and a taller call that small is not worth a second copy of its weights.
 int64_t min_streamed_weights(int64_t rows) { return rows <= 4 ? int64_t{1} << 22 : int64_t{1} << 20; }
 
+// 8-bit weights through the repacked stream, in blocks of the 32 (or 16) rows that its kernels take. Returns false (nothing launched)
+// when the shape is not theirs or there is no copy.
+bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& rc)
+{
+    rc = 0;
+    RocmMatMulNBitsArgs part = args;
+    int64_t rows = args.m < 32 ? args.m : 32;
+    part.m = rows;
+    if (!rocm_decode_packed8_eligible(&part)) {
+        part.m = rows = args.m < 16 ? args.m : 16;
+        if (args.m <= 32 || !rocm_decode_packed8_eligible(&part)) return false;      // (17..32 rows: one pass or the other routes)
+    }
+    if (!use_packed(kn, part, rc)) return false;
+    for (int64_t row0 = 0; row0 < args.m && rc == 0; row0 += rows) {
+        part.m = args.m - row0 < rows ? args.m - row0 : rows;
+        part.a = static_cast<const uint8_t*>(args.a) + static_cast<size_t>(row0) * static_cast<size_t>(args.k) * 2;      // 16-bit activations and results
+        part.y = static_cast<uint8_t*>(args.y) + static_cast<size_t>(row0) * static_cast<size_t>(args.n) * 2;
+        part.bias = rows_of_bias(args, row0);
+        rc = rocm_launch_decode_packed8(&part, kn.packed, kn.ep->decode_waves, kn.ep->stream);
+    }
+    kn.variant = "decode_mfma_packed8";
+    return true;
+}
+
 // Narrower f32 calls than this keep the streaming kernel and the catch-all; no projection of a model is that narrow.
 constexpr int64_t kGemmF32MinCols = 128;
 
@@ -730,14 +763,14 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     if (kn.bits != 4 || args.g_idx) {
         // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
         // row blocks over the stream took 97 / 101); the accumulators' offset costs a 16-bit result nothing, so f32 results stay on the routes below.
-        const bool streamed = kn.bits == 8 && !args.g_idx && M <= 32 && args.y_dtype != ROCM_DT_F32 && args.n * args.k >= min_streamed_weights(args.m) && use_packed(kn, args, rc);
+        // Weights that stay in 32 bits come in blocks of 32 rows at any height.
+        const bool eight = kn.bits == 8 && !args.g_idx && args.n * args.k >= min_streamed_weights(args.m);
+        const bool in_tiles = eight && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && weights_in_16_bits(kn, args) && rocm_prefill_mfma8_eligible(&args);
         // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
-        if (streamed) {
-            if (rc == 0) rc = rocm_launch_decode_packed8(&args, kn.packed, kn.ep->decode_waves, stream);
-            kn.variant = "decode_mfma_packed8";
-        } else if (kn.bits == 8 && !args.g_idx && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && args.n * args.k >= min_streamed_weights(args.m) &&
-                   rocm_prefill_mfma8_eligible(&args)) {
+        if (eight && args.y_dtype != ROCM_DT_F32 && (M <= 32 || !weights_in_16_bits(kn, args)) && stream_eight_bits(kn, args, rc)) {
+            // done
+        } else if (in_tiles) {
             rc = tiled(rocm_launch_prefill_mfma8);
             kn.variant = "prefill_mfma_lds8";
         } else if (!dense_route(kn, args, rc)) {
@@ -809,7 +842,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     } else if (M <= 16 && rocm_decode_mfma_eligible(&args)) {
         rc = rocm_launch_decode_mfma(&args, kn.ep->decode_waves, kn.ep->decode_col_groups, stream);
         kn.variant = "decode_mfma_splitk";
-    } else if (M <= 32 && decode_in_row_blocks(kn, args, rc)) {
+    } else if ((M <= 32 || (sorted && !weights_in_16_bits(kn, args))) && decode_in_row_blocks(kn, args, rc)) {
         // done: a few passes of the streaming kernels beat one pass of the tiled kernel at these heights
     } else if (dense_route(kn, args, rc)) {
         // done: weights expanded to 16 bits, then the library GEMM

@@ -1,0 +1,45 @@
+"""Weights that a route may not round to 16 bits: beyond the 16-bit copy's size limit, and under f32 results of the f32 GEMV."""
+import numpy as np
+import pytest
+
+from onnx_genai_amd import ep as E
+from onnx_genai_amd import synth
+from tests import helpers
+
+pytestmark = pytest.mark.gpu
+
+# One rounding of the result, 2^-11 over sqrt(3) in the 2-norm; a rounding of the weights would add as much again (factor 1.41)
+TOL_F16 = 2.0 ** -11 / 3 ** 0.5 * 1.1
+
+
+@pytest.mark.parametrize("m", [33, 70, 100])
+def test_eight_bit_weights_beyond_the_limit_stream_in_row_blocks(port, m):
+    ep = E.RocmExecutionProvider(0, {"dense_gemm_max_mb": "1"})
+    n, k, bs = 2100, 1024, 64
+    b, s, zp = synth.make_weights_bits(n, k, bs, 8, m, zero_points=True, scale_lo=0.002, scale_hi=0.004, scale_dtype=E.F16)
+    a = synth.make_activation(m, k, m, E.F16)
+    bias = np.random.default_rng(m).standard_normal((m, n)).astype(np.float16)
+    want = port.matmul_f64_bits(synth.to_f32(a, E.F16), b, synth.to_f32(s, E.F16), zp, n, k, bs, 8)
+    y, variant = E.matmul_nbits(ep, a, E.F16, b, s, E.F16, zp, n, k, bs, bias=bias, bias_dtype=E.F16, bits=8)
+    assert variant == "decode_mfma_packed8"
+    assert helpers.rel_l2(synth.to_f32(y, E.F16), want + bias.astype(np.float64)) <= TOL_F16
+    y, variant = E.matmul_nbits(ep, a, E.F16, b, s, E.F16, zp, n, k, bs, bits=8, y_dtype=E.F32)
+    assert variant == "gemv_nbits_f32" and helpers.rel_l2(y, want) <= 2e-6
+    ep.shutdown()
+
+
+@pytest.mark.parametrize("limit_mb,m,y_dt,expect", [
+    ("1024", 2, E.F32, "gemv_nbits_f32"), ("1", 40, E.F32, "gemv_nbits_f32"), ("1", 100, E.F16, "act_order+decode_mfma_packed"), ("1024", 100, E.F16, "act_order+prefill_mfma_lds")])
+def test_act_order(port, limit_mb, m, y_dt, expect):
+    ep = E.RocmExecutionProvider(0, {"dense_gemm_max_mb": limit_mb})
+    n, k, bs = 1100, 1024, 128
+    b, s, zp = synth.make_weights(n, k, bs, m, zero_points=True, scale_lo=0.005, scale_hi=0.02, scale_dtype=E.F16)
+    g = (np.arange(k) // bs).astype(np.int32)
+    np.random.default_rng(m).shuffle(g)
+    a = synth.make_activation(m, k, m, E.F16)
+    y, variant = E.matmul_nbits(ep, a, E.F16, b, s, E.F16, zp, n, k, bs, g_idx=g, y_dtype=y_dt)
+    assert variant == expect
+    want = synth.to_f32(a, E.F16).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, E.F16), zp, g, n, k, bs, 4).astype(np.float64).T
+    tol = 2e-6 if y_dt == E.F32 else TOL_F16 if limit_mb == "1" else TOL_F16 * 2 ** 0.5
+    assert helpers.rel_l2(synth.to_f32(y, y_dt), want) <= tol
+    ep.shutdown()
