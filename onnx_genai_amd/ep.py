@@ -251,6 +251,7 @@ def _packed_views(views):
         packer.pack_into(buf, 0, *values, *dims)
     except struct.error:           # numbers that are not plain integers of their field: convert and wrap as ctypes does, the library judges them
         widths = ["Q", "I", "I", "Q", "Q", "Q", "I", "I"] * len(views) + ["Q"] * len(dims)
+        values = [x.value or 0 if isinstance(x, C.c_void_p) else x for x in values]
         wrapped = [int(x) & (0xFFFFFFFF if w == "I" else 0xFFFFFFFFFFFFFFFF) for w, x in zip(widths, values + dims)]
         struct.pack_into("=" + "".join(widths), buf, 0, *wrapped)
     return buf, base

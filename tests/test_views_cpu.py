@@ -1,4 +1,6 @@
 """The packed view arrays that execute hands to the C ABI: field for field what a CTensorView array holds."""
+import ctypes as C
+
 import numpy as np
 
 from onnx_genai_amd import ep as E
@@ -16,3 +18,10 @@ def test_packed_views_read_back_as_ctensorviews():
             assert bool(g.strides) == (v.strides is not None)
             if v.strides is not None:
                 assert [g.strides[i] for i in range(g.ndim)] == list(v.strides)
+
+
+def test_addresses_as_ctypes_pointers():
+    """What a ctypes field takes as an address is an address here too."""
+    for given, address in ((C.c_void_p(0x6000), 0x6000), (C.c_void_p(), 0)):
+        buf, at = E._packed_views((E.TensorView(given, E.F32, (4,)),))
+        assert (E.CTensorView.from_address(at).data or 0) == address
