@@ -336,15 +336,22 @@ constexpr int kPitch8 = 80;          // bytes per LDS row: 64 codes + 16 of padd
 
 // NBS: blocks per step - 2 (block size 32), 1 (block size 64) or 0 (block size >= 128: a block spans several steps).
 // SF32: scales stored as f32 (else 16 bits, f16 or bf16 by a run-time flag).
-// Eight waves, 4 (rows) x 2 (columns); each owns a 32 x 64 sub-tile: two MFMA tiles, 32 f32 results per lane. The
+// Eight waves, 4 (rows) x 2 (columns). TM = 1: each owns a 32 x 64 sub-tile: two MFMA tiles, 32 f32 results per lane. The
 // small per-wave state leaves room for four waves per SIMD, which is what overlaps one wave's flush arithmetic
 // with another's MFMAs.
+// TM = 2: 64 x 64 per wave, 256 x 128 per workgroup, two waves per SIMD of up to 256 registers: a weight is unpacked and an operand of B read
+// from LDS for twice the rows, one tile's MFMAs run under the other's flush inside a wave, and the registers hold three steps of
+// loads in flight (the two-set form of TM = 1 waits for memory: with two sets TM = 2 was level with it, 4970 us against 4266 with four on 8192 -> 57344 at
+// 4096 rows, block 64; 128 x 128 tiles 5494). Same sums in the same order, bit for bit. 8192 -> 57344 at 4096 rows: 0.70 -> 0.90 POP/s.
 // PROBE: every int32 tile that is flushed is also stored to p.acc_probe ([M, N, kb]); the same code otherwise.
-template <int NBS, bool SF32, int D, bool PROBE>
+template <int NBS, bool SF32, int TM, int D, bool PROBE>
 __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
 {
+    static_assert(TM == 1 || (TM == 2 && !PROBE && NBS != 2));
+    constexpr int kRows = TM * kTile;                          // rows of the workgroup
     constexpr int kSlots = NBS == 2 ? 2 : 1;                   // scale slots per step
-    constexpr int kBufBytes = 2 * kTile * kPitch8 + 2 * kSlots * kTile * 4;
+    constexpr int kSaSlots = TM == 1 ? kSlots : 2;             // (two row tiles: room for one from every thread)
+    constexpr int kBufBytes = (kRows + kTile) * kPitch8 + (kSaSlots * kRows + kSlots * kTile) * 4;
     constexpr int TN = 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -352,7 +359,7 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * kTile;
+    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * kRows;
     const int64_t n_base = static_cast<int64_t>(blockIdx.x) * kTile;
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
     const bool has_zp = p.zp != nullptr;
@@ -367,19 +374,19 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     const __amdgpu_buffer_rsrc_t srd_z = make_srd(has_zp ? p.zp + n_base * p.zp_row : p.b, has_zp ? static_cast<uint64_t>(cols_left * p.zp_row) : 0);
     const __amdgpu_buffer_rsrc_t srd_sa = make_srd(p.sa_t, static_cast<uint64_t>(p.kb * p.m) * 4);
 
-    // codes: thread -> (row t/4, 16-byte piece t%4). weights: thread -> (column t/4, 8-byte quarter t%4 of the step).
+    // codes: thread -> (row t/4 of every 128, 16-byte piece t%4). weights: thread -> (column t/4, 8-byte quarter t%4 of the step).
     const int prow = t >> 2, quarter = t & 3;
     const uint32_t a_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.padded_k) + static_cast<uint32_t>(quarter * 16);
     const uint32_t a_loff = static_cast<uint32_t>(prow * kPitch8 + quarter * 16);
     const uint32_t b_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(quarter * 8);
-    const uint32_t b_loff = static_cast<uint32_t>(kTile * kPitch8 + prow * kPitch8 + quarter * 16);
+    const uint32_t b_loff = static_cast<uint32_t>(kRows * kPitch8 + prow * kPitch8 + quarter * 16);
     const uint32_t s_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.kb) * kScaleBytes;
     const uint32_t z_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.zp_row);
-    // activation scales: thread -> (slot t/128, row t%128)
-    const int sa_slot = t >> 7, sa_row = t & 127;
+    // activation scales: thread -> (slot t/rows, row t%rows)
+    const int sa_slot = TM == 1 ? t >> 7 : wave >> 2, sa_row = t & (kRows - 1);
     const uint32_t sa_goff = (sa_slot < kSlots && m_base + sa_row < p.m) ? static_cast<uint32_t>(m_base + sa_row) * 4u : kOutOfRange;
-    constexpr int kSaOff = 2 * kTile * kPitch8;                 // [kSlots][128] f32 activation scales of the step
-    constexpr int kSbOff = kSaOff + kSlots * kTile * 4;         // [kSlots][128] f32 weight scales of the step
+    constexpr int kSaOff = (kRows + kTile) * kPitch8;           // [kSaSlots][rows] f32 activation scales of the step
+    constexpr int kSbOff = kSaOff + kSaSlots * kRows * 4;       // [kSlots][128] f32 weight scales of the step
 
     // PROBE: this lane's first accumulator element, (row m_base + wm * 32 + 4 (lane / 32), column n_base + wn * 64 + lane % 32),
     // as a byte offset into the [M, N, kb] probe (the launcher refuses probes of 2^31 bytes or more)
@@ -390,12 +397,14 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     // MFMA operand reads: lane (r = lane % 32, h = lane / 32) reads 16 consecutive codes of row r.
     const uint32_t frag_off = static_cast<uint32_t>((lane & 31) * kPitch8 + (lane >> 5) * 16);
 
-    int16_t_v acc[NBS == 0 ? TN : 1];   // integer accumulators that outlive a step (block size >= 128 only)
-    float y[TN][16];
+    int16_t_v acc[TM][NBS == 0 ? TN : 1];   // integer accumulators that outlive a step (block size >= 128 only)
+    float y[TM][TN][16];
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+    for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) y[j][r] = 0.f;
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) y[m][j][r] = 0.f;
 
     // K range of this workgroup: all of K, or one of grid.z slices whose f32 partial sums a second kernel adds in slice
     // order (small grids: few tiles of Y, long K). `kt` below counts steps from the slice's first.
@@ -406,18 +415,22 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     // over (measured +2 to +8 %). A grid with at most one workgroup per CU gains nothing from that and runs its lone
     // workgroup 30 % faster with four sets in flight; so does block size 32, whose steps hold two flushes.
     struct Regs {
-        uint4 a;
+        uint4 a[TM];
         uint2 b;
         uint32_t s, z, zsh, sa;
     };
     Regs regs[D];
 
-    auto block_of = [&](int kt, int offset) -> uint32_t { return static_cast<uint32_t>((kt * kStep + offset) >> p.bs_log2); };
+    const int bs_log2 = TM > 1 && NBS == 1 ? 6 : p.bs_log2;
+    auto block_of = [&](int kt, int offset) -> uint32_t { return static_cast<uint32_t>((kt * kStep + offset) >> bs_log2); };
     auto load_global = [&](Regs& r, int kt_in_slice) {
         const int kt = kt_base + kt_in_slice;
-        uint32_t off = a_goff;
-        if (ragged_k && static_cast<int64_t>(kt) * kStep + quarter * 16 >= p.padded_k) off = kOutOfRange;   // else the next row's codes
-        r.a = load16(srd_a, off, static_cast<uint32_t>(kt) * 64u);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+            uint32_t off = a_goff + static_cast<uint32_t>(m * kTile) * static_cast<uint32_t>(p.padded_k);
+            if (ragged_k && static_cast<int64_t>(kt) * kStep + quarter * 16 >= p.padded_k) off = kOutOfRange;   // else the next row's codes
+            r.a[m] = load16(srd_a, off, static_cast<uint32_t>(kt) * 64u);
+        }
         const auto w = __builtin_amdgcn_raw_buffer_load_b64(srd_b, static_cast<int>(b_goff), static_cast<int>(kt * 32), 0);
         r.b = make_uint2(w[0], w[1]);
         const uint32_t blk = block_of(kt, quarter * 16);
@@ -446,8 +459,18 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
         const uint32_t hi = (((w >> 4) & 0x0f0f0f0fu) + c4) ^ 0x80808080u;     // elements 1,3,5,7
         *reinterpret_cast<uint2*>(base + b_loff + part * 8) = make_uint2(lo, hi);
         if (part == 0) {
-            *reinterpret_cast<uint4*>(base + a_loff) = r.a;
+#pragma unroll
+            for (int m = 0; m < TM; ++m) *reinterpret_cast<uint4*>(base + a_loff + m * kTile * kPitch8) = r.a[m];
         } else {
+            if constexpr (TM > 1) {
+                // No branch here: around one the compiler moves whole row tiles of the arithmetic, and spills. Threads of one column and
+                // block store the same scale; the activation scales have room for every thread.
+                float f16_scale = f16_bits_to_f32(static_cast<uint16_t>(r.s)), bf16_scale = __uint_as_float(r.s << 16);
+                asm("" : "+v"(f16_scale), "+v"(bf16_scale));
+                *reinterpret_cast<float*>(base + kSbOff + prow * 4) = SF32 ? __uint_as_float(r.s) : p.scales_bf16 ? bf16_scale : f16_scale;
+                *reinterpret_cast<uint32_t*>(base + kSaOff + t * 4) = r.sa;
+                return;
+            }
             if ((quarter & 1) == 0 && (quarter >> 1) < kSlots) {
                 const float sc = SF32 ? __uint_as_float(r.s) : (p.scales_bf16 ? __uint_as_float(r.s << 16) : f16_bits_to_f32(static_cast<uint16_t>(r.s)));
                 *reinterpret_cast<float*>(base + kSbOff + ((quarter >> 1) * kTile + prow) * 4) = sc;
@@ -460,17 +483,17 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     // halves carry the wave's 32 rows). Its result has the accumulators' layout, tile j in components 16 j .. 16 j + 15.
     // The matrix cores are mostly idle in this kernel and the vector ALUs are not: this takes one multiply per
     // accumulator and block off them.
-    auto scale_tiles = [&](int buf, int slot) -> float32_v {
+    auto scale_tiles = [&](int buf, int slot, int m) -> float32_v {
         const unsigned char* base = smem + buf * kBufBytes;
-        const float sa = *reinterpret_cast<const float*>(base + kSaOff + (slot * kTile + wm * 32 + (lane & 31)) * 4);
+        const float sa = *reinterpret_cast<const float*>(base + kSaOff + (slot * kRows + (wm * TM + m) * 32 + (lane & 31)) * 4);
         const float sb = *reinterpret_cast<const float*>(base + kSbOff + (slot * kTile + wn * 64 + lane) * 4);
         const float32_v zero = {};
         return __builtin_amdgcn_mfma_f32_32x32x1f32(sa, sb, zero, 0, 0, 0);
     };
-    // y[j] += f32(tile) * (scale_a[row] * scale_b[column]) for 32x32 tile j.
-    auto flush_tile = [&](const int16_t_v& tile, const float32_v& sc, int j) {
+    // y[m][j] += f32(tile) * (scale_a[row] * scale_b[column]) for 32x32 tile j of row tile m.
+    auto flush_tile = [&](const int16_t_v& tile, const float32_v& sc, int m, int j) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) y[j][i] = fmaf(static_cast<float>(tile[i]), sc[j * 16 + i], y[j][i]);
+        for (int i = 0; i < 16; ++i) y[m][j][i] = fmaf(static_cast<float>(tile[i]), sc[j * 16 + i], y[m][j][i]);
     };
     // PROBE: the finished int32 tile j of block `blk`, stored before its scale products are formed (fewer registers live
     // than at the flush itself; the integers are final once the block's last MFMA has written them).
@@ -494,66 +517,74 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     };
     auto compute = [&](int buf, int kt_in_slice, const Regs& next, bool store_next) {
         const int kt = kt_base + kt_in_slice;
-        const unsigned char* la = smem + buf * kBufBytes + wm * (32 * kPitch8) + frag_off;
-        const unsigned char* lb = smem + buf * kBufBytes + kTile * kPitch8 + wn * (64 * kPitch8) + frag_off;
+        const unsigned char* la = smem + buf * kBufBytes + wm * (TM * 32 * kPitch8) + frag_off;
+        const unsigned char* lb = smem + buf * kBufBytes + kRows * kPitch8 + wn * (64 * kPitch8) + frag_off;
         u32x4_t fa[2], fb[2][TN];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            fa[kk] = *reinterpret_cast<const u32x4_t*>(la + kk * 32);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) fb[kk][j] = *reinterpret_cast<const u32x4_t*>(lb + j * 32 * kPitch8 + kk * 32);
-        }
         const int16_t_v zero = {};
-        if constexpr (NBS == 1) {
-            // One block per step: the integer accumulators live only from the MFMAs to the flush.
-            int16_t_v t0 = mfma(fa[0], fb[0][0], zero);
-            int16_t_v t1 = mfma(fa[0], fb[0][1], zero);
-            t0 = mfma(fa[1], fb[1][0], t0);
-            t1 = mfma(fa[1], fb[1][1], t1);
-            probe_tile(t0, 0, kt);
-            probe_tile(t1, 1, kt);
-            const float32_v sc = scale_tiles(buf, 0);
-            if (store_next) store_part(next, buf ^ 1, 0);
-            flush_tile(t0, sc, 0);
-            if (store_next) store_part(next, buf ^ 1, 1);
-            flush_tile(t1, sc, 1);
-        } else if constexpr (NBS == 2) {
-            const bool second = static_cast<int64_t>(kt) * 2 + 1 < p.kb;   // the step's second block exists
-            const int16_t_v t0 = mfma(fa[0], fb[0][0], zero);
-            const int16_t_v t1 = mfma(fa[0], fb[0][1], zero);
-            const int16_t_v u0 = mfma(fa[1], fb[1][0], zero);
-            const int16_t_v u1 = mfma(fa[1], fb[1][1], zero);
-            probe_tile(t0, 0, 2 * static_cast<int64_t>(kt));
-            probe_tile(t1, 1, 2 * static_cast<int64_t>(kt));
-            probe_tile(u0, 0, 2 * static_cast<int64_t>(kt) + 1);           // (a second block past K is not stored: blk < kb)
-            probe_tile(u1, 1, 2 * static_cast<int64_t>(kt) + 1);
-            const float32_v sc0 = scale_tiles(buf, 0);
-            const float32_v sc1 = scale_tiles(buf, 1);
-            if (store_next) store_part(next, buf ^ 1, 0);
-            flush_tile(t0, sc0, 0);
-            flush_tile(t1, sc0, 1);
-            if (store_next) store_part(next, buf ^ 1, 1);
-            if (second) {
-                flush_tile(u0, sc1, 0);
-                flush_tile(u1, sc1, 1);
+        // what of the next step's bytes goes to LDS between the pieces of arithmetic: halves, behind the first row tile's
+        auto store_next_part = [&](int m, int part) {
+            if (m == 0 && store_next) store_part(next, buf ^ 1, part);
+        };
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk) {
+                fa[kk] = *reinterpret_cast<const u32x4_t*>(la + m * 32 * kPitch8 + kk * 32);
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    if (m == 0) fb[kk][j] = *reinterpret_cast<const u32x4_t*>(lb + j * 32 * kPitch8 + kk * 32);
             }
-        } else {
-            // Block size >= 128: the step opens and / or closes a block (wave-uniform).
-            const bool opens = ((kt * kStep) & ((1 << p.bs_log2) - 1)) == 0;
-            const bool closes = (((kt + 1) * kStep) & ((1 << p.bs_log2) - 1)) == 0;
+            if constexpr (NBS == 1) {
+                // One block per step: the integer accumulators live only from the MFMAs to the flush.
+                int16_t_v t0 = mfma(fa[0], fb[0][0], zero);
+                int16_t_v t1 = mfma(fa[0], fb[0][1], zero);
+                t0 = mfma(fa[1], fb[1][0], t0);
+                t1 = mfma(fa[1], fb[1][1], t1);
+                probe_tile(t0, 0, kt);
+                probe_tile(t1, 1, kt);
+                const float32_v sc = scale_tiles(buf, 0, m);
+                store_next_part(m, 0);
+                flush_tile(t0, sc, m, 0);
+                store_next_part(m, 1);
+                flush_tile(t1, sc, m, 1);
+            } else if constexpr (NBS == 2) {
+                const bool second = static_cast<int64_t>(kt) * 2 + 1 < p.kb;   // the step's second block exists
+                const int16_t_v t0 = mfma(fa[0], fb[0][0], zero);
+                const int16_t_v t1 = mfma(fa[0], fb[0][1], zero);
+                const int16_t_v u0 = mfma(fa[1], fb[1][0], zero);
+                const int16_t_v u1 = mfma(fa[1], fb[1][1], zero);
+                probe_tile(t0, 0, 2 * static_cast<int64_t>(kt));
+                probe_tile(t1, 1, 2 * static_cast<int64_t>(kt));
+                probe_tile(u0, 0, 2 * static_cast<int64_t>(kt) + 1);           // (a second block past K is not stored: blk < kb)
+                probe_tile(u1, 1, 2 * static_cast<int64_t>(kt) + 1);
+                const float32_v sc0 = scale_tiles(buf, 0, m);
+                const float32_v sc1 = scale_tiles(buf, 1, m);
+                store_next_part(m, 0);
+                flush_tile(t0, sc0, m, 0);
+                flush_tile(t1, sc0, m, 1);
+                store_next_part(m, 1);
+                if (second) {
+                    flush_tile(u0, sc1, m, 0);
+                    flush_tile(u1, sc1, m, 1);
+                }
+            } else {
+                // Block size >= 128: the step opens and / or closes a block (wave-uniform).
+                const bool opens = ((kt * kStep) & ((1 << p.bs_log2) - 1)) == 0;
+                const bool closes = (((kt + 1) * kStep) & ((1 << p.bs_log2) - 1)) == 0;
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                if (opens) acc[j] = mfma(fa[0], fb[0][j], zero);
-                else acc[j] = mfma(fa[0], fb[0][j], acc[j]);
-                acc[j] = mfma(fa[1], fb[1][j], acc[j]);
-                if (store_next) store_part(next, buf ^ 1, j);
-            }
-            if (closes) {
+                for (int j = 0; j < TN; ++j) {
+                    if (opens) acc[m][j] = mfma(fa[0], fb[0][j], zero);
+                    else acc[m][j] = mfma(fa[0], fb[0][j], acc[m][j]);
+                    acc[m][j] = mfma(fa[1], fb[1][j], acc[m][j]);
+                    store_next_part(m, j);
+                }
+                if (closes) {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) probe_tile(acc[j], j, (static_cast<int64_t>(kt) * kStep) >> p.bs_log2);
-                const float32_v sc = scale_tiles(buf, 0);
+                    for (int j = 0; j < TN; ++j) probe_tile(acc[m][j], j, (static_cast<int64_t>(kt) * kStep) >> p.bs_log2);
+                    const float32_v sc = scale_tiles(buf, 0, m);
 #pragma unroll
-                for (int j = 0; j < TN; ++j) flush_tile(acc[j], sc, j);
+                    for (int j = 0; j < TN; ++j) flush_tile(acc[m][j], sc, m, j);
+                }
             }
         }
     };
@@ -598,13 +629,13 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
         const BiasTerm bias = load_bias(bias_ptr, p.bias_dtype, 0, p.n, col);
         float* part = p.partial ? p.partial + static_cast<int64_t>(blockIdx.z) * p.m * p.n : nullptr;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 4 * TM; ++q) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int64_t row = m_base + wm * 32 + q * 8 + row_group + r;
+                const int64_t row = m_base + wm * (32 * TM) + (q >> 2) * 32 + (q & 3) * 8 + row_group + r;
                 if (row >= p.m) continue;
-                if (part) part[row * p.n + col] = y[j][q * 4 + r];
-                else store_from_f32(p.y, p.y_dtype, row * p.n + col, add_bias(y[j][q * 4 + r], per_row ? load_bias(bias_ptr, p.bias_dtype, row, p.n, col) : bias, p.y_dtype));
+                if (part) part[row * p.n + col] = y[q >> 2][j][(q & 3) * 4 + r];
+                else store_from_f32(p.y, p.y_dtype, row * p.n + col, add_bias(y[q >> 2][j][(q & 3) * 4 + r], per_row ? load_bias(bias_ptr, p.bias_dtype, row, p.n, col) : bias, p.y_dtype));
             }
         }
     }
@@ -637,24 +668,56 @@ static int acc4_steps_per_slice(int64_t padded_k, int block_size, int slices)
     return static_cast<int>(per);
 }
 
+// Two row tiles per wave (256 x 128 tiles of Y, one workgroup per CU) where that grid fills the rounds it takes: the share of the 128 x 128
+// tiles wanted in what the rounds could hold, which a row tile half empty and a last round half empty both lower. Against 128 x 128
+// tiles, f16, zero points, 12 heights of 200 - 4096 rows on six shapes (us, before and after):
+//   block 64, K >= 8192, 78 % or more full: 8192 -> 57344 at 512 / 4096 rows 717 -> 582, 5476 -> 4252; 28672 -> 8192 at 1000 / 4096 624 -> 504,
+//     2559 -> 2113; 8192 -> 10240 at 2048 (83 % full) 452 -> 436. At 66 - 73 % (300, 600 rows) 529 -> 548, 859 -> 838.
+//   block 64, a shorter K: the tiles' ends weigh more. 4096 -> 28672 at 512 / 4096 rows (87, 100 %) 172 -> 158, 1219 -> 1097; 3584 -> 37888 at 1000
+//     (92 %) 369 -> 348, but at 768 and 1600 rows (87, 83 %) 274 -> 279, 583 -> 616.
+//   block 128: one flush for two steps is less work to overlap. 8192 -> 57344 at 512 / 4096 606 -> 546, 4700 -> 3937; 8192 -> 10240 at 2048
+//     (83 %) 411 -> 417; 3584 -> 37888 at 4096 rows (100 %) 1211 -> 1249: only from K = 8192.
+//   block 32 (two flushes a step) does not fit 256 registers with the loads this far ahead.
+static bool acc4_tall_tiles(const Acc4PrefillParams& p, int slices, int blocks_per_step)
+{
+    const int64_t cus = rocm_ffi_compute_units(), columns = (p.n + kTile - 1) / kTile, tiles = columns * ((p.m + 2 * kTile - 1) / (2 * kTile));
+    if (slices != 1 || p.acc_probe || tiles < cus || p.padded_k * 2 * kTile >= 0x7fffffff) return false;
+    const int64_t full = 100 * columns * ((p.m + kTile - 1) / kTile) / (2 * cus * ((tiles + cus - 1) / cus));
+    if (blocks_per_step == 0) return p.padded_k >= 8192 && full >= 86;
+    return full >= (p.padded_k >= 8192 ? 78 : 87);
+}
+
+template <int NBS, bool SF32, int TM, int D, bool PROBE>
+static int launch_acc4_prefill_cfg(const Acc4PrefillParams& p, int slices, hipStream_t stream)
+{
+    const dim3 grid(static_cast<unsigned>((p.n + kTile - 1) / kTile), static_cast<unsigned>((p.m + TM * kTile - 1) / (TM * kTile)), static_cast<unsigned>(slices));
+    constexpr int kSlots = NBS == 2 ? 2 : 1;
+    const size_t lds = 2 * ((TM + 1) * kTile * kPitch8 + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
+    auto kernel = acc4_prefill_kernel<NBS, SF32, TM, D, PROBE>;
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        if (e != hipSuccess) return static_cast<int>(e);
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, p);
+    return static_cast<int>(hipGetLastError());
+}
+
 template <int NBS, bool SF32>
 static int launch_acc4_prefill(const Acc4PrefillParams& p, int slices, hipStream_t stream)
 {
-    const dim3 grid(static_cast<unsigned>((p.n + kTile - 1) / kTile), static_cast<unsigned>((p.m + kTile - 1) / kTile), static_cast<unsigned>(slices));
-    const size_t lds = 2 * (2 * kTile * kPitch8 + 2 * (NBS == 2 ? 2 : 1) * kTile * 4);
-    const bool deep = NBS == 2 || static_cast<uint64_t>(grid.x) * grid.y * grid.z <= static_cast<uint64_t>(rocm_ffi_compute_units());    // at most one workgroup per CU anyway
+    const uint64_t workgroups = static_cast<uint64_t>((p.n + kTile - 1) / kTile) * static_cast<uint64_t>((p.m + kTile - 1) / kTile) * static_cast<uint64_t>(slices);
+    const bool deep = workgroups <= static_cast<uint64_t>(rocm_ffi_compute_units());    // at most one workgroup per CU anyway
+    // (block size 32 with four register sets in flight has no room left for the probe's stores: its probe build keeps two -
+    // the depth of the load pipeline changes when a step's operands arrive, not what is computed from them)
     if (p.acc_probe) {
-        // (block size 32 with four register sets in flight has no room left for the probe's stores: its probe build keeps two -
-        // the depth of the load pipeline changes when a step's operands arrive, not what is computed from them)
-        if constexpr (NBS == 2) {
-            hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, 2, true>), grid, dim3(512), lds, stream, p);
-        } else {
-            if (deep) hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, 4, true>), grid, dim3(512), lds, stream, p);
-            else hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, 2, true>), grid, dim3(512), lds, stream, p);
-        }
-    } else if (deep) hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, 4, false>), grid, dim3(512), lds, stream, p);
-    else hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, NBS == 2 ? 4 : 2, false>), grid, dim3(512), lds, stream, p);
-    return static_cast<int>(hipGetLastError());
+        if (NBS != 2 && deep) return launch_acc4_prefill_cfg<NBS, SF32, 1, NBS == 2 ? 2 : 4, true>(p, slices, stream);
+        return launch_acc4_prefill_cfg<NBS, SF32, 1, 2, true>(p, slices, stream);
+    }
+    if constexpr (NBS != 2) {
+        if (acc4_tall_tiles(p, slices, NBS)) return launch_acc4_prefill_cfg<NBS, SF32, 2, 4, false>(p, slices, stream);
+    }
+    if (NBS == 2 || deep) return launch_acc4_prefill_cfg<NBS, SF32, 1, 4, false>(p, slices, stream);
+    return launch_acc4_prefill_cfg<NBS, SF32, 1, NBS == 2 ? 4 : 2, false>(p, slices, stream);
 }
 
 }  // namespace mnb
