@@ -913,9 +913,10 @@ NxrtStatus execute_swiglu(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in,
     // kernel): one launch over both repacked copies. The copies are made (and every weight tensor validated) by the
     // projections' own first call below, so this path serves the calls after the first with the same weight tensors; it
     // sums each projection exactly as that first call did.
-    // (accuracy_level 4 stays on its own int8 kernels for every call: the paired launch is the float path)
+    // (accuracy_level 4 stays on its own int8 kernels for every call, and 8-bit weights on theirs: the paired launch is the float path, and
+    // the copies it reads are those of 4-bit weights)
     const void* normalized = nullptr;                    // the rows after a normalization launch of their own, once made
-    if (M <= 16 && kn.accuracy_level != 4 && kn.gate->packed && kn.up->packed) {
+    if (M <= 16 && kn.bits == 4 && kn.accuracy_level != 4 && kn.gate->packed && kn.up->packed) {
         auto current = [&](const NxrtRocmMatMulNBits& child, const NxrtRocmTensorView& w, const NxrtRocmTensorView& s, const NxrtRocmTensorView* zp) {
             auto at = [](const NxrtRocmTensorView& v) { return static_cast<const void*>(static_cast<const uint8_t*>(v.data) + v.byte_offset); };
             return child.packed_from[0] == at(w) && child.packed_from[1] == at(s) && child.packed_from[2] == (zp ? at(*zp) : nullptr) &&
