@@ -24,6 +24,7 @@ HIP_SOURCES = [
     "kernels/decode_mfma.hip",
     "kernels/decode_packed.hip",
     "kernels/decode_packed8.hip",
+    "kernels/decode_plain.hip",
     "kernels/prefill_mfma.hip",
     "kernels/dense_gemm.hip",
     "kernels/swiglu.hip",

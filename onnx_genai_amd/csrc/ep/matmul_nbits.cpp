@@ -255,14 +255,25 @@ bool weights_in_16_bits(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs
 
 // Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on
 // first use, args.a the call's activations in the same order, args.g_idx null. Returns false with `args` untouched where the groups
-// are not whole blocks, or the copy or the gather's buffer cannot be made now (a capture is open, no memory): the kernels that look
-// groups up per element take the call then. `rc` receives a HIP error.
+// are not whole blocks, where no kernel for contiguous blocks is the better one, or the copy or the gather's buffer cannot be made now (a
+// capture is open, no memory): the kernels that look groups up per element take the call then. `rc` receives a HIP error.
 bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, int& rc)
 {
     rc = 0;
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[4]) return false;
-    // f32 results of 16-bit rows that the f32 GEMV has: the offset in the 4-bit streams' accumulators would show in their last bits
-    if (args.a_dtype != ROCM_DT_F32 && args.y_dtype == ROCM_DT_F32 && !weights_in_16_bits(kn, args)) return false;
+    if (args.a_dtype != ROCM_DT_F32) {
+        const bool in_16_bits = weights_in_16_bits(kn, args);
+        if (args.y_dtype == ROCM_DT_F32 && !in_16_bits) return false;      // (f32 results of 16-bit rows keep the f32 GEMV)
+        // five rows or more of 4-bit weights that neither the stream with plain sums nor the tiled kernel takes: the 16-bit copy serves them unsorted
+        if (kn.bits == 4 && in_16_bits) {
+            RocmMatMulNBitsArgs probe = args;
+            probe.a = nullptr;                                             // (the gathered rows and the sorted copy are aligned)
+            probe.b = nullptr;
+            const bool tiled = args.m > 16 && rocm_prefill_mfma_eligible(&probe);
+            if (probe.m > 16) probe.m = 16;
+            if (!tiled && !(args.m <= 32 && rocm_decode_plain_eligible(&probe))) return false;
+        }
+    }
     const size_t order_bytes = (static_cast<size_t>(args.k) * sizeof(int32_t) + 255) / 256 * 256;
     if (kn.regrouped_from[0] != args.b || kn.regrouped_from[1] != args.g_idx) {
         if (frozen(kn)) return false;
@@ -525,6 +536,35 @@ bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
         rc = rocm_launch_decode_packed8(&part, kn.packed, kn.ep->decode_waves, kn.ep->stream);
     }
     kn.variant = "decode_mfma_packed8";
+    return true;
+}
+
+// Sorted act-order weights through the repacked 4-bit stream with plain sums: one pass of up to 32 rows where the shared-activation kernel takes
+// them, else passes of 16. Returns false (nothing launched) when the shape is not theirs, there is no copy, or the tiled kernel is the better
+// route (block size 32 below 16384 columns, as in decode_in_row_blocks).
+bool stream_sorted(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& rc)
+{
+    rc = 0;
+    const bool in_16_bits = weights_in_16_bits(kn, args);
+    if (args.m > 32 && in_16_bits) return false;
+    RocmMatMulNBitsArgs part = args;
+    int64_t rows = args.m < 32 ? args.m : 32;
+    part.m = rows;
+    if (!rocm_decode_plain_eligible(&part)) {
+        part.m = rows = args.m < 16 ? args.m : 16;
+        if (!rocm_decode_plain_eligible(&part)) return false;
+        if (args.m > 16 && in_16_bits && args.block_size == 32 && args.n < 16384 && rocm_prefill_mfma_eligible(&args)) return false;
+    }
+    if (!use_packed(kn, part, rc)) return false;
+    const size_t y_elem = args.y_dtype == ROCM_DT_F32 ? 4 : 2;
+    for (int64_t row0 = 0; row0 < args.m && rc == 0; row0 += rows) {
+        part.m = args.m - row0 < rows ? args.m - row0 : rows;
+        part.a = static_cast<const uint8_t*>(args.a) + static_cast<size_t>(row0) * static_cast<size_t>(args.k) * 2;      // eligibility means f16 / bf16 activations
+        part.y = static_cast<uint8_t*>(args.y) + static_cast<size_t>(row0) * static_cast<size_t>(args.n) * y_elem;
+        part.bias = rows_of_bias(args, row0);
+        rc = rocm_launch_decode_plain(&part, kn.packed, kn.ep->decode_waves, kn.ep->stream);
+    }
+    kn.variant = "decode_mfma_packed";
     return true;
 }
 
@@ -835,6 +875,19 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
                 kn.variant = "acc4_gemv_dot4";
             }
         }
+    } else if (sorted && args.a_dtype != ROCM_DT_F32) {
+        // (the kernels over the 4-bit stream whose accumulators carry an offset are not for these: see decode_packed.hiph)
+        if (stream_sorted(kn, args, rc)) {
+            // done
+        } else if (dense_route(kn, args, rc)) {
+            // done: weights expanded to 16 bits, then the library GEMM
+        } else if (M > 16 && rocm_prefill_mfma_eligible(&args)) {
+            rc = tiled(rocm_launch_prefill_mfma);
+            kn.variant = "prefill_mfma_lds";
+        } else {
+            rc = rocm_launch_gemv_generic(&args, stream);
+            kn.variant = "gemv_generic_f32";
+        }
     } else if (M <= 64 && use_packed(kn, args, rc)) {
         if (rc == 0) rc = (kn.pair_member && M <= 16) ? rocm_launch_decode_packed_pair_member(&args, kn.packed, kn.ep->decode_waves, stream)
                                                       : rocm_launch_decode_packed(&args, kn.packed, kn.ep->decode_waves, stream);
@@ -842,7 +895,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     } else if (M <= 16 && rocm_decode_mfma_eligible(&args)) {
         rc = rocm_launch_decode_mfma(&args, kn.ep->decode_waves, kn.ep->decode_col_groups, stream);
         kn.variant = "decode_mfma_splitk";
-    } else if ((M <= 32 || (sorted && !weights_in_16_bits(kn, args))) && decode_in_row_blocks(kn, args, rc)) {
+    } else if (M <= 32 && decode_in_row_blocks(kn, args, rc)) {
         // done: a few passes of the streaming kernels beat one pass of the tiled kernel at these heights
     } else if (dense_route(kn, args, rc)) {
         // done: weights expanded to 16 bits, then the library GEMM

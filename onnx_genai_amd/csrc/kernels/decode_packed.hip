@@ -21,6 +21,7 @@
 
 #include "decode_packed.hiph"
 #include "decode_packed8.hiph"
+#include "decode_plain.hiph"
 
 namespace mnb {
 
@@ -891,6 +892,27 @@ extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const vo
     }
     p.groups_per_wave = plan.groups_per_wave;
     return mnb::launch_packed8(p, bf16, a->block_size, plan.waves, s);
+}
+
+extern "C" int rocm_decode_plain_eligible(const RocmMatMulNBitsArgs* a)
+{
+    return a->m <= 32 && !a->gamma && rocm_decode_packed_eligible(a);
+}
+
+extern "C" int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+{
+    if (!rocm_decode_plain_eligible(a)) return -1;
+    const int64_t cus = rocm_ffi_compute_units();
+    const PackedPlan plan = plan_decode_packed(a, waves, false, false, cus);
+    mnb::PackedParams p = packed_params(a, packed);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const bool bf16 = a->a_dtype == ROCM_DT_BF16, f32_scales = a->scale_dtype == ROCM_DT_F32;
+    if (plan.wide) {
+        const int64_t col_groups = (a->n + 15) / 16;
+        return mnb::launch_plain_wide(p, bf16, f32_scales, a->block_size, (col_groups + mnb::kWideWaves - 1) / mnb::kWideWaves < cus, s);
+    }
+    p.groups_per_wave = plan.groups_per_wave;
+    return mnb::launch_plain(p, bf16, f32_scales, a->block_size, plan.waves, s);
 }
 
 extern "C" int rocm_launch_decode_packed_pair_member(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
