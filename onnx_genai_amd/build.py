@@ -23,7 +23,6 @@ HIP_SOURCES = [
     "kernels/gemm_f32.hip",
     "kernels/decode_mfma.hip",
     "kernels/decode_packed.hip",
-    "kernels/decode_packed8.hip",
     "kernels/decode_plain.hip",
     "kernels/prefill_mfma.hip",
     "kernels/dense_gemm.hip",

@@ -802,7 +802,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
     if (kn.bits != 4 || args.g_idx) {
         // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
-        // row blocks over the stream took 97 / 101); the accumulators' offset costs a 16-bit result nothing, so f32 results stay on the routes below.
+        // row blocks over the stream took 97 / 101). f32 results of 16-bit rows keep the routes below.
         // Weights that stay in 32 bits come in blocks of 32 rows at any height.
         const bool eight = kn.bits == 8 && !args.g_idx && args.n * args.k >= min_streamed_weights(args.m);
         const bool in_tiles = eight && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && weights_in_16_bits(kn, args) && rocm_prefill_mfma8_eligible(&args);

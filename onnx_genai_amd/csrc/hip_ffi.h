@@ -199,13 +199,13 @@ int rocm_decode_packed_pair_fits(const RocmMatMulNBitsArgs* args, int waves);
 int rocm_launch_decode_packed_pair(const RocmMatMulNBitsArgs* args, const void* packed_gate, const void* packed_up, int decomposed, int waves,
                                    rocm_stream_t stream);
 
-/* The same over the same copy with plain sums: f32 sums of activation times (q - zp), nothing else in the accumulators - for weights
- * whose other kernels have those, up to 32 rows. */
+/* The same over the same copy with plain sums: f32 sums of activation times (q - zp), nothing else in the accumulators - for act-order
+ * weights sorted by group, whose other kernels have those; up to 32 rows. */
 int rocm_decode_plain_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* args, const void* packed, int waves, rocm_stream_t stream);
 
-/* The same for 8-bit weights (args->b [N, kb, bs], zp [N, kb] or NULL = 128; scales of the activations' type): the copy holds each
- * tile as two planes of nibbles. */
+/* Plain sums for 8-bit weights (args->b [N, kb, bs], zp [N, kb] or NULL = 128; scales of the activations' type): a copy of the same form with
+ * two tiles for 128 k. */
 int rocm_decode_packed8_eligible(const RocmMatMulNBitsArgs* args);
 uint64_t rocm_decode_packed8_bytes(const RocmMatMulNBitsArgs* args);
 int rocm_launch_pack_decode8(const RocmMatMulNBitsArgs* args, void* packed, rocm_stream_t stream);

@@ -20,7 +20,6 @@
 #include <type_traits>
 
 #include "decode_packed.hiph"
-#include "decode_packed8.hiph"
 #include "decode_plain.hiph"
 
 namespace mnb {
@@ -37,8 +36,8 @@ struct PackParams {
     int bits;               // 4 or 8
 };
 
-// 8-bit weights travel as two planes of nibbles: (q - zp) * s = (q_low - zp_low) * s + (q_high - zp_high) * 16 s, so a tile of
-// 128 k becomes two tiles of the stream, the low nibbles and then the high ones, that meet the same activations.
+// 8-bit weights: a tile of 128 k becomes two tiles of the stream, the first with bytes 0..3 and the second with bytes 4..7 of each lane's eight
+// weights. Their zero points fill the record's bytes, and both tiles' entries are alike.
 
 // grid (tile group, column group), 256 threads: four dwords of weights per thread, then one record per thread < 16.
 __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
@@ -54,12 +53,10 @@ __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
         const int u = x >> 8, lane = (x >> 2) & 63, j = x & 3;
         const int64_t col = cg * 16 + (lane & 15);
         const int64_t tile = tg * kGroupTiles + u;
-        const int64_t k = (p.bits == 8 ? tile >> 1 : tile) * 128 + j * 32 + (lane >> 4) * 8;
+        const int64_t k = (p.bits == 8 ? tile >> 1 : tile) * 128 + j * 32 + (lane >> 4) * 8 + (p.bits == 8 ? (tile & 1) * 4 : 0);
         uint32_t out = 0;
         if (p.bits == 8 && col < p.n && k < padded_k) {
-            const int plane_shift = static_cast<int>(tile & 1) * 4;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) out |= ((static_cast<uint32_t>(p.b[col * p.row_bytes + k + e]) >> plane_shift) & 0xfu) << (4 * (e / 2) + 16 * (e % 2));
+            out = b32[(col * p.row_bytes + k) >> 2];
         } else if (col < p.n && k < padded_k) {
             const uint32_t w = b32[(col * p.row_bytes + (k >> 1)) >> 2];   // eight weights, element e at bit 4e
             uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;    // even / odd elements, one per byte
@@ -87,8 +84,7 @@ __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
                 reinterpret_cast<uint16_t*>(rec)[bi] = live ? static_cast<const uint16_t*>(p.scales)[col * p.kb + blk] : static_cast<uint16_t>(0);
             }
             if (p.bits == 8) {
-                const uint32_t z = live && p.zp ? p.zp[col * p.zp_row + blk] : 128u;
-                rec[nb * p.scale_bytes + bi] = static_cast<uint8_t>((z >> ((tile & 1) * 4)) & 0xfu);
+                rec[nb * p.scale_bytes + bi] = live && p.zp ? p.zp[col * p.zp_row + blk] : 128;
             } else {
                 rec[nb * p.scale_bytes + bi] = static_cast<uint8_t>(live ? zero_point_of(p.zp ? p.zp + col * p.zp_row : nullptr, blk) : 8);
             }
@@ -603,30 +599,30 @@ extern "C" int rocm_launch_pack_decode(const RocmMatMulNBitsArgs* a, void* packe
 }
 
 // The 4-bit call whose stream an 8-bit call's is, in everything that plans or sizes it: twice the tiles, the same activations.
-static RocmMatMulNBitsArgs as_planes(const RocmMatMulNBitsArgs* a)
+static RocmMatMulNBitsArgs as_four_bits(const RocmMatMulNBitsArgs* a)
 {
-    RocmMatMulNBitsArgs planes = *a;
+    RocmMatMulNBitsArgs four = *a;
     const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
-    planes.k = (kb * a->block_size + 127) / 128 * 256;
-    return planes;
+    four.k = (kb * a->block_size + 127) / 128 * 256;
+    return four;
 }
 
 extern "C" int rocm_decode_packed8_eligible(const RocmMatMulNBitsArgs* a)
 {
-    const RocmMatMulNBitsArgs planes = as_planes(a);
-    return a->m <= 32 && a->k % 8 == 0 && a->scale_dtype == a->a_dtype && !a->gamma && rocm_decode_packed_eligible(&planes);
+    const RocmMatMulNBitsArgs four = as_four_bits(a);
+    return a->m <= 32 && a->k % 8 == 0 && a->scale_dtype == a->a_dtype && !a->gamma && rocm_decode_packed_eligible(&four);
 }
 
 extern "C" uint64_t rocm_decode_packed8_bytes(const RocmMatMulNBitsArgs* a)
 {
-    const RocmMatMulNBitsArgs planes = as_planes(a);
-    return rocm_decode_packed_bytes(&planes);
+    const RocmMatMulNBitsArgs four = as_four_bits(a);
+    return rocm_decode_packed_bytes(&four);
 }
 
 extern "C" int rocm_launch_pack_decode8(const RocmMatMulNBitsArgs* a, void* packed, rocm_stream_t stream)
 {
-    const RocmMatMulNBitsArgs planes = as_planes(a);
-    return launch_pack_decode(a, 8, mnb::packed_groups(&planes), packed, stream);
+    const RocmMatMulNBitsArgs four = as_four_bits(a);
+    return launch_pack_decode(a, 8, mnb::packed_groups(&four), packed, stream);
 }
 
 // The launch of rocm_launch_decode_packed; with `packed_up` the paired gate/up launch. `probe_only`: nothing is launched,
@@ -875,44 +871,42 @@ extern "C" int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* a, const voi
     return launch_decode_packed(a, packed, nullptr, 0, waves, false, false, stream);
 }
 
-extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
-{
-    if (!rocm_decode_packed8_eligible(a)) return -1;
-    const RocmMatMulNBitsArgs planes = as_planes(a);
-    const int64_t cus = rocm_ffi_compute_units();
-    const PackedPlan plan = plan_decode_packed(&planes, waves, false, false, cus);
-    mnb::PackedParams p = packed_params(&planes, packed);
-    p.k = a->k;                              // what the activations have
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool bf16 = a->a_dtype == ROCM_DT_BF16;
-    if (plan.wide) {
-        p.groups_per_wave = p.groups;
-        const int64_t col_groups = (a->n + 15) / 16;
-        return mnb::launch_wide8(p, bf16, a->block_size, (col_groups + mnb::kWideWaves - 1) / mnb::kWideWaves < cus, s);
-    }
-    p.groups_per_wave = plan.groups_per_wave;
-    return mnb::launch_packed8(p, bf16, a->block_size, plan.waves, s);
-}
-
 extern "C" int rocm_decode_plain_eligible(const RocmMatMulNBitsArgs* a)
 {
     return a->m <= 32 && !a->gamma && rocm_decode_packed_eligible(a);
 }
 
-extern "C" int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+// `a`'s call over its stream, planned as `four`'s.
+static int launch_decode_plain(const RocmMatMulNBitsArgs* a, const RocmMatMulNBitsArgs* four, int bits, const void* packed, int waves, rocm_stream_t stream)
 {
-    if (!rocm_decode_plain_eligible(a)) return -1;
     const int64_t cus = rocm_ffi_compute_units();
-    const PackedPlan plan = plan_decode_packed(a, waves, false, false, cus);
-    mnb::PackedParams p = packed_params(a, packed);
+    const PackedPlan plan = plan_decode_packed(four, waves, false, false, cus);
+    mnb::PackedParams p = packed_params(four, packed);
+    p.k = a->k;                              // what the activations have
+    p.magic = 0x64006400u;                   // both types' operands are made from f16 ones
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16 = a->a_dtype == ROCM_DT_BF16, f32_scales = a->scale_dtype == ROCM_DT_F32;
     if (plan.wide) {
+        // a grid between one and one and a half workgroups of eight waves per CU: as many waves as spread it over one a CU, as in plan_wide
+        // (3584 -> 37888, block 128, 16 rows: 8 bits, bf16 38.3 -> 31.6 us, act-order 4 bits, f16 26.7 -> 20.9)
         const int64_t col_groups = (a->n + 15) / 16;
-        return mnb::launch_plain_wide(p, bf16, f32_scales, a->block_size, (col_groups + mnb::kWideWaves - 1) / mnb::kWideWaves < cus, s);
+        const bool in_between = a->m <= 16 && (bits == 8 || a->block_size != 32) && col_groups > cus * mnb::kWideWaves && col_groups <= cus * mnb::kWideWavesMax;
+        return mnb::launch_plain_wide(p, bits, bf16, f32_scales, a->block_size, in_between ? static_cast<int>((col_groups + cus - 1) / cus) : mnb::kWideWaves, s);
     }
     p.groups_per_wave = plan.groups_per_wave;
-    return mnb::launch_plain(p, bf16, f32_scales, a->block_size, plan.waves, s);
+    return mnb::launch_plain(p, bits, bf16, f32_scales, a->block_size, plan.waves, s);
+}
+
+extern "C" int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+{
+    return rocm_decode_plain_eligible(a) ? launch_decode_plain(a, a, 4, packed, waves, stream) : -1;
+}
+
+extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+{
+    if (!rocm_decode_packed8_eligible(a)) return -1;
+    const RocmMatMulNBitsArgs four = as_four_bits(a);
+    return launch_decode_plain(a, &four, 8, packed, waves, stream);
 }
 
 extern "C" int rocm_launch_decode_packed_pair_member(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)

@@ -1,31 +1,40 @@
-// The decode kernels over the repacked 4-bit stream with plain sums (decode_packed.hiph says which weights they serve and why; decode_packed.hip
-// plans the launches as those of the builds that carry the offset).
+// The decode kernels over the repacked stream with plain sums (decode_packed.hiph says which weights they serve and why; decode_packed.hip
+// plans the launches as those of the builds that carry the offset, an 8-bit one's as those of the 4-bit call with twice the tiles).
+//
+// 8 bits: what is streamed is 1.01 bytes per weight and the bound is HBM. bf16, block 128, 1 / 4 / 16 rows, against a GEMV of one wave per column up to four
+// rows and weights expanded to 16 bits on every call from five: 3584 -> 152064 144 / 344 / 5535 -> 106 / 103 / 113 us, 3584 -> 37888 39.6 / 90 / 255
+// -> 28.7 / 31.4 / 31.6, 18944 -> 3584 29 / 47 / 180 -> 16.8 / 18.3 / 24.2. (As two planes of nibbles whose accumulators carried the offset: 106 / 108 / 115,
+// 29.3 / 39.1 / 39.6, 17.1 / 18.6 / 24.4 - twice the matrix instructions.)
+// 4 bits, act-order, gather included: HBM in f16 (3584 -> 37888, block 128, 1 / 16 rows 18.3 / 20.9 us, 18.0 / 20.1 with the offset), the vector ALU work of
+// turning nibbles into bf16 integers otherwise (20.6 / 24.5 against 17.9 / 20.7).
 #include "decode_plain.hiph"
 
 namespace mnb {
 
-template <bool BF16, int BS, int MR, typename ST>
+template <bool BF16, int BS, int MR, typename ST, int BITS>
 __global__ __launch_bounds__((BS == 128 && sizeof(ST) == 2 && (MR != 16 || BF16)) ? 1024 : 512)
 void decode_plain_kernel(PackedParams p)
 {
-    decode_packed_body<BF16, BS, MR, ST, 1, false, false, 4, true>(p);
+    decode_packed_body<BF16, BS, MR, ST, 1, false, false, BITS, true>(p);
 }
 
-template <bool BF16, int BS, typename ST, int RB, bool PF, bool DEEP>
-__global__ __launch_bounds__(kWideWaves * 64)
+// One block of rows: weights and windows both ahead (8 bits, block 128, 16 rows, 3584 -> 152064: 112 us, windows alone 120, neither 114; act-order
+// 4 bits 83 / 85 / 89); two: neither (registers).
+template <bool BF16, int BS, typename ST, int RB, int WMAX, int BITS>
+__global__ __launch_bounds__(WMAX * 64)
 void decode_plain_wide_kernel(PackedParams p)
 {
-    decode_wide_body<BF16, BS, ST, RB, false, PF, DEEP, false, kWideWaves, 4, true>(p);
+    decode_wide_body<BF16, BS, ST, RB, false, RB == 1, RB == 1, false, WMAX, BITS, true>(p);
 }
 
-template <bool BF16, int BS, int MR, typename ST>
+template <bool BF16, int BS, int MR, typename ST, int BITS>
 static int launch_plain_mr(const PackedParams& p, int waves, hipStream_t stream)
 {
     const unsigned grid = static_cast<unsigned>((p.n + 15) / 16);
     const size_t stage = static_cast<size_t>(waves) * 2 * (MR == 1 ? 1024 : MR * kRowPitchP);
     const size_t red = static_cast<size_t>(waves) * 1024;
     const size_t lds = stage > red ? stage : red;
-    auto kernel = decode_plain_kernel<BF16, BS, MR, ST>;
+    auto kernel = decode_plain_kernel<BF16, BS, MR, ST, BITS>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return static_cast<int>(e);
@@ -34,63 +43,74 @@ static int launch_plain_mr(const PackedParams& p, int waves, hipStream_t stream)
     return static_cast<int>(hipGetLastError());
 }
 
-template <bool BF16, int BS, typename ST>
+template <bool BF16, int BS, typename ST, int BITS>
 static int launch_plain_bs(const PackedParams& p, int waves, hipStream_t stream)
 {
-    if (p.m <= 1) return launch_plain_mr<BF16, BS, 1, ST>(p, waves, stream);
-    if (p.m <= 4) return launch_plain_mr<BF16, BS, 4, ST>(p, waves, stream);
-    if (p.m <= 8) return launch_plain_mr<BF16, BS, 8, ST>(p, waves, stream);
-    return launch_plain_mr<BF16, BS, 16, ST>(p, waves, stream);
+    if (p.m <= 1) return launch_plain_mr<BF16, BS, 1, ST, BITS>(p, waves, stream);
+    if (p.m <= 4) return launch_plain_mr<BF16, BS, 4, ST, BITS>(p, waves, stream);
+    if (p.m <= 8) return launch_plain_mr<BF16, BS, 8, ST, BITS>(p, waves, stream);
+    return launch_plain_mr<BF16, BS, 16, ST, BITS>(p, waves, stream);
 }
 
-template <bool BF16, int BS, typename ST, int RB, bool PF, bool DEEP>
-static int launch_plain_wide_cfg(const PackedParams& p, hipStream_t stream)
+template <bool BF16, int BS, typename ST, int RB, int WMAX, int BITS>
+static int launch_plain_wide_cfg(const PackedParams& p, int waves, hipStream_t stream)
 {
-    constexpr size_t lds = 2 * RB * 16 * (4 * 256 + 16);           // two windows of four tiles
+    constexpr size_t lds = 2 * RB * 16 * (4 / (BITS / 4) * 256 + 16);      // two windows of the activations that four tiles of the stream meet
     const int64_t col_groups = (p.n + 15) / 16;
-    auto kernel = decode_plain_wide_kernel<BF16, BS, ST, RB, PF, DEEP>;
+    auto kernel = decode_plain_wide_kernel<BF16, BS, ST, RB, WMAX, BITS>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         if (e != hipSuccess) return static_cast<int>(e);
     }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((col_groups + kWideWaves - 1) / kWideWaves)), dim3(kWideWaves * 64), lds, stream, p);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((col_groups + waves - 1) / waves)), dim3(waves * 64), lds, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
-template <bool BF16, int BS, typename ST>
-static int launch_plain_wide_bs(const PackedParams& p, bool few_workgroups, hipStream_t stream)
+template <bool BF16, int BS, typename ST, int BITS>
+static int launch_plain_wide_bs(const PackedParams& p, int waves, hipStream_t stream)
 {
-    if (p.m <= 16) return few_workgroups ? launch_plain_wide_cfg<BF16, BS, ST, 1, true, true>(p, stream) : launch_plain_wide_cfg<BF16, BS, ST, 1, false, true>(p, stream);
+    if (p.m <= 16) {
+        if constexpr (BITS == 8 || BS != 32) {             // (sixteen scales a group: 4 bits at block 32 take more registers than twelve waves leave)
+            if (waves > kWideWaves) return launch_plain_wide_cfg<BF16, BS, ST, 1, kWideWavesMax, BITS>(p, waves, stream);
+        }
+        return launch_plain_wide_cfg<BF16, BS, ST, 1, kWideWaves, BITS>(p, kWideWaves, stream);
+    }
     if constexpr (BS != 32) {
-        if (p.m <= 32) return launch_plain_wide_cfg<BF16, BS, ST, 2, false, false>(p, stream);
+        if (p.m <= 32) return launch_plain_wide_cfg<BF16, BS, ST, 2, kWideWaves, BITS>(p, kWideWaves, stream);
     }
     return -1;
 }
 
-// `go`: called with the element type, the block size and the scales' storage type as compile-time values
+// `go`: called with the element type, the block size, the scales' storage type and the bits as compile-time values
 template <typename Go>
-static int by_build(bool bf16, bool f32_scales, int block_size, Go go)
+static int by_build(int bits, bool bf16, bool f32_scales, int block_size, Go go)
 {
-    auto by_block = [&](auto bf, auto st) {
+    auto by_block = [&](auto bf, auto st, auto bi) {
         switch (block_size) {
-            case 32: return go(bf, std::integral_constant<int, 32>{}, st);
-            case 64: return go(bf, std::integral_constant<int, 64>{}, st);
-            default: return go(bf, std::integral_constant<int, 128>{}, st);
+            case 32: return go(bf, std::integral_constant<int, 32>{}, st, bi);
+            case 64: return go(bf, std::integral_constant<int, 64>{}, st, bi);
+            default: return go(bf, std::integral_constant<int, 128>{}, st, bi);
         }
     };
-    if (bf16) return f32_scales ? by_block(std::true_type{}, float{}) : by_block(std::true_type{}, uint16_t{});
-    return f32_scales ? by_block(std::false_type{}, float{}) : by_block(std::false_type{}, uint16_t{});
+    auto by_scales = [&](auto bf) {
+        if (bits == 8) return f32_scales ? -1 : by_block(bf, uint16_t{}, std::integral_constant<int, 8>{});
+        return f32_scales ? by_block(bf, float{}, std::integral_constant<int, 4>{}) : by_block(bf, uint16_t{}, std::integral_constant<int, 4>{});
+    };
+    return bf16 ? by_scales(std::true_type{}) : by_scales(std::false_type{});
 }
 
-int launch_plain(const PackedParams& p, bool bf16, bool f32_scales, int block_size, int waves, hipStream_t stream)
+int launch_plain(const PackedParams& p, int bits, bool bf16, bool f32_scales, int block_size, int waves, hipStream_t stream)
 {
-    return by_build(bf16, f32_scales, block_size, [&](auto bf, auto bs, auto st) { return launch_plain_bs<decltype(bf)::value, decltype(bs)::value, decltype(st)>(p, waves, stream); });
+    return by_build(bits, bf16, f32_scales, block_size, [&](auto bf, auto bs, auto st, auto bi) {
+        return launch_plain_bs<decltype(bf)::value, decltype(bs)::value, decltype(st), decltype(bi)::value>(p, waves, stream);
+    });
 }
 
-int launch_plain_wide(const PackedParams& p, bool bf16, bool f32_scales, int block_size, bool few_workgroups, hipStream_t stream)
+int launch_plain_wide(const PackedParams& p, int bits, bool bf16, bool f32_scales, int block_size, int waves, hipStream_t stream)
 {
-    return by_build(bf16, f32_scales, block_size,
-                    [&](auto bf, auto bs, auto st) { return launch_plain_wide_bs<decltype(bf)::value, decltype(bs)::value, decltype(st)>(p, few_workgroups, stream); });
+    return by_build(bits, bf16, f32_scales, block_size, [&](auto bf, auto bs, auto st, auto bi) {
+        return launch_plain_wide_bs<decltype(bf)::value, decltype(bs)::value, decltype(st), decltype(bi)::value>(p, waves, stream);
+    });
 }
 
 }  // namespace mnb

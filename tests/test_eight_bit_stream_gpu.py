@@ -1,4 +1,4 @@
-"""8-bit weights over the repacked stream of nibble planes: row counts of every build, ragged edges, block sizes, against the oracle."""
+"""8-bit weights over the repacked stream: row counts of every build, ragged edges, block sizes, against the oracle."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from tests import helpers
 pytestmark = pytest.mark.gpu
 
 # The result's own rounding: half a unit of 2^-10 (f16) or 2^-7 (bf16), relative to a value at least half the unit's binade, uniform in it:
-# 2^-11 / sqrt(3) and 2^-8 / sqrt(3) in the 2-norm. The f32 accumulator carries the weights with an offset of 2^10 (2^7): below 1e-4.
+# 2^-11 / sqrt(3) and 2^-8 / sqrt(3) in the 2-norm, and 1e-4 of room (test_plain_sums_gpu.py holds the sums to less).
 TOL = {E.F16: 2.0 ** -11 / 3 ** 0.5 + 1e-4, E.BF16: 2.0 ** -8 / 3 ** 0.5 + 1e-4}
 
 CASES = [
@@ -47,7 +47,7 @@ def test_matches_oracle(ep, port, dt, bs, zero_points, m, n, k):
 
 
 def test_f32_results_keep_their_route(ep, port):
-    """An f32 result of a 16-bit row would show the accumulator's offset: it stays on the kernel with plain f32 sums."""
+    """An f32 result of a 16-bit row stays on the plain GEMV."""
     m, n, k, bs = 2, 4100, 1024, 128
     b, s, zp = synth.make_weights_bits(n, k, bs, 8, 3, zero_points=True, scale_lo=0.002, scale_hi=0.004, scale_dtype=E.F16)
     a = synth.make_activation(m, k, 3, E.F16)

@@ -1,4 +1,4 @@
-"""Act-order weights with 16-bit activations: sums as good as plain f32 sums of activation times (q - zp), and infinities, NaN and values
+"""8-bit and act-order weights with 16-bit activations: sums as good as plain f32 sums of activation times (q - zp), and infinities, NaN and values
 near the end of the range that come out as those sums give them."""
 import numpy as np
 import pytest
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 ONE_ROUNDING = {E.F16: 2.0 ** -11 / 3 ** 0.5 * 1.1, E.BF16: 2.0 ** -8 / 3 ** 0.5 * 1.1}      # of the result, in the 2-norm
 
-# bits, type, block size, m, n, k - the row counts of every build, then the wide ones
+# bits, type, block size, m, n, k - the row counts of every build, then the wide ones; n * k at least what streams a repacked copy
 CASES = [
     (4, E.F16, 128, 1, 1200, 3584),
     (4, E.BF16, 32, 1, 700, 904),
@@ -21,6 +21,14 @@ CASES = [
     (4, E.F16, 32, 16, 23000, 256),
     (4, E.BF16, 128, 12, 18448, 640),
     (4, E.F16, 64, 29, 14400, 448),
+    (8, E.F16, 128, 1, 1200, 3584),
+    (8, E.BF16, 32, 1, 4700, 904),
+    (8, E.BF16, 128, 4, 1200, 3584),
+    (8, E.F16, 64, 7, 640, 2048),
+    (8, E.BF16, 128, 16, 1200, 3584),
+    (8, E.F16, 32, 16, 23000, 256),
+    (8, E.BF16, 128, 12, 18448, 640),
+    (8, E.F16, 64, 29, 14400, 448),
 ]
 
 
