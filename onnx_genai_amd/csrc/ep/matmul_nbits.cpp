@@ -881,7 +881,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
             // done
         } else if (dense_route(kn, args, rc)) {
             // done: weights expanded to 16 bits, then the library GEMM
-        } else if (M > 16 && rocm_prefill_mfma_eligible(&args)) {
+        } else if (M > 16 && weights_in_16_bits(kn, args) && rocm_prefill_mfma_eligible(&args)) {
             rc = tiled(rocm_launch_prefill_mfma);
             kn.variant = "prefill_mfma_lds";
         } else {

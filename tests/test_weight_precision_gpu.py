@@ -43,3 +43,19 @@ def test_act_order(port, limit_mb, m, y_dt, expect):
     tol = 2e-6 if y_dt == E.F32 else TOL_F16 if limit_mb == "1" else TOL_F16 * 2 ** 0.5
     assert helpers.rel_l2(synth.to_f32(y, y_dt), want) <= tol
     ep.shutdown()
+
+
+@pytest.mark.parametrize("bs,m", [(32, 40), (32, 100), (256, 40), (256, 100), (128, 24)])
+def test_act_order_beyond_the_limit_keeps_its_weights(port, bs, m):
+    """Whatever the block size: no route that rounds the weights takes the call."""
+    ep = E.RocmExecutionProvider(0, {"dense_gemm_max_mb": "1"})
+    n, k = 1100, 1024
+    b, s, zp = synth.make_weights(n, k, bs, m, zero_points=True, scale_lo=0.005, scale_hi=0.02, scale_dtype=E.F16)
+    g = (np.arange(k) // bs).astype(np.int32)
+    np.random.default_rng(m).shuffle(g)
+    a = synth.make_activation(m, k, m, E.F16)
+    y, variant = E.matmul_nbits(ep, a, E.F16, b, s, E.F16, zp, n, k, bs, g_idx=g)
+    want = synth.to_f32(a, E.F16).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, E.F16), zp, g, n, k, bs, 4).astype(np.float64).T
+    # f32 sums round to another f16 value than the 64-bit ones only where these lie next to a boundary, weights rounded to f16 move every second result
+    assert (np.asarray(y) != want.astype(np.float16)).mean() <= 0.02, variant
+    ep.shutdown()
