@@ -256,13 +256,13 @@ bool weights_in_16_bits(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs
 // Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on
 // first use, args.a the call's activations in the same order, args.g_idx null. Returns false with `args` untouched where the groups
 // are not whole blocks, where no kernel for contiguous blocks is the better one, or the copy or the gather's buffer cannot be made now (a
-// capture is open, no memory): the kernels that look groups up per element take the call then. `rc` receives a HIP error.
-bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, int& rc)
+// capture is open, no memory): the kernels that look groups up per element take the call then. `in_16_bits`: weights_in_16_bits of the call as it
+// came. `rc` receives a HIP error.
+bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_16_bits, int& rc)
 {
     rc = 0;
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[4]) return false;
     if (args.a_dtype != ROCM_DT_F32) {
-        const bool in_16_bits = weights_in_16_bits(kn, args);
         if (args.y_dtype == ROCM_DT_F32 && !in_16_bits) return false;      // (f32 results of 16-bit rows keep the f32 GEMV)
         // five rows or more of 4-bit weights that neither the stream with plain sums nor the tiled kernel takes: the 16-bit copy serves them unsorted
         if (kn.bits == 4 && in_16_bits) {
@@ -542,10 +542,9 @@ bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
 // Sorted act-order weights through the repacked 4-bit stream with plain sums: one pass of up to 32 rows where the shared-activation kernel takes
 // them, else passes of 16. Returns false (nothing launched) when the shape is not theirs, there is no copy, or the tiled kernel is the better
 // route (block size 32 below 16384 columns, as in decode_in_row_blocks).
-bool stream_sorted(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& rc)
+bool stream_sorted(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, bool in_16_bits, int& rc)
 {
     rc = 0;
-    const bool in_16_bits = weights_in_16_bits(kn, args);
     if (args.m > 32 && in_16_bits) return false;
     RocmMatMulNBitsArgs part = args;
     int64_t rows = args.m < 32 ? args.m : 32;
@@ -798,22 +797,25 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         if (bad >= 0) return make_status(NXRT_INVALID_ARGUMENT, err("g_idx[" + std::to_string(bad) + "] is outside 0.." + std::to_string(kb)));
         kn.g_idx_checked = args.g_idx;
     }
-    const bool sorted = G && sort_by_group(kn, args, rc);
+    // Asked before the rows are gathered: what keeps its weights in 32 bits for an A off a 16-byte boundary keeps them behind the gather, too.
+    const bool in_16_bits = weights_in_16_bits(kn, args);
+    const bool dense_off = args.g_idx && args.a_dtype != ROCM_DT_F32 && (reinterpret_cast<uintptr_t>(args.a) & 15) != 0;
+    const bool sorted = G && sort_by_group(kn, args, in_16_bits, rc);
     if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
     if (kn.bits != 4 || args.g_idx) {
         // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
         // row blocks over the stream took 97 / 101). f32 results of 16-bit rows keep the routes below.
         // Weights that stay in 32 bits come in blocks of 32 rows at any height.
         const bool eight = kn.bits == 8 && !args.g_idx && args.n * args.k >= min_streamed_weights(args.m);
-        const bool in_tiles = eight && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && weights_in_16_bits(kn, args) && rocm_prefill_mfma8_eligible(&args);
+        const bool in_tiles = eight && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && in_16_bits && rocm_prefill_mfma8_eligible(&args);
         // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
-        if (eight && args.y_dtype != ROCM_DT_F32 && (M <= 32 || !weights_in_16_bits(kn, args)) && stream_eight_bits(kn, args, rc)) {
+        if (eight && args.y_dtype != ROCM_DT_F32 && (M <= 32 || !in_16_bits) && stream_eight_bits(kn, args, rc)) {
             // done
         } else if (in_tiles) {
             rc = tiled(rocm_launch_prefill_mfma8);
             kn.variant = "prefill_mfma_lds8";
-        } else if (!dense_route(kn, args, rc)) {
+        } else if (dense_off || !dense_route(kn, args, rc)) {
             rc = rocm_launch_gemv_nbits(&args, static_cast<int>(kn.bits), stream);
             kn.variant = "gemv_nbits_f32";
         }
@@ -877,11 +879,11 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         }
     } else if (sorted && args.a_dtype != ROCM_DT_F32) {
         // (the kernels over the 4-bit stream whose accumulators carry an offset are not for these: see decode_packed.hiph)
-        if (stream_sorted(kn, args, rc)) {
+        if (stream_sorted(kn, args, in_16_bits, rc)) {
             // done
-        } else if (dense_route(kn, args, rc)) {
+        } else if (!dense_off && dense_route(kn, args, rc)) {
             // done: weights expanded to 16 bits, then the library GEMM
-        } else if (M > 16 && weights_in_16_bits(kn, args) && rocm_prefill_mfma_eligible(&args)) {
+        } else if (M > 16 && in_16_bits && rocm_prefill_mfma_eligible(&args)) {
             rc = tiled(rocm_launch_prefill_mfma);
             kn.variant = "prefill_mfma_lds";
         } else {

@@ -59,3 +59,27 @@ def test_act_order_beyond_the_limit_keeps_its_weights(port, bs, m):
     # f32 sums round to another f16 value than the 64-bit ones only where these lie next to a boundary, weights rounded to f16 move every second result
     assert (np.asarray(y) != want.astype(np.float16)).mean() <= 0.02, variant
     ep.shutdown()
+
+
+@pytest.mark.parametrize("bits,bs,m", [(4, 128, 24), (4, 128, 100), (4, 256, 40), (8, 64, 24), (8, 64, 100), (2, 64, 40)])
+def test_act_order_with_unaligned_activations_keeps_its_weights(ep, port, bits, bs, m):
+    """The 16-bit copy's kernel wants A on 16 bytes: calls whose A is not, which keep their weights, keep them sorted too (the gathered rows are aligned)."""
+    n, k, dt = 1100, 1024, E.F16
+    make = synth.make_weights if bits == 4 else lambda *args, **kw: synth.make_weights_bits(args[0], args[1], args[2], bits, args[3], **kw)
+    b, s, zp = make(n, k, bs, m, zero_points=True, scale_lo=0.002, scale_hi=0.004, scale_dtype=dt)
+    g = (np.arange(k) // bs).astype(np.int32)
+    np.random.default_rng(m).shuffle(g)
+    a = synth.make_activation(m, k, m, dt)
+    ops = E.DeviceOperands(ep, b, s, dt, zp, n, k, bs, bits=bits, g_idx=g)
+    ab, yb = ep.upload(np.concatenate([np.zeros(1, np.float16), a.ravel()])), ep.allocate(m * n * 2)
+    try:
+        views = ops.views(ab, dt, m)
+        views[0] = E.TensorView(ab.ptr, dt, (m, k), byte_offset=2)
+        ops.kernel.execute(views, [E.TensorView(yb.ptr, dt, (m, n))])
+        got, variant = ep.download(yb, (m, n), np.float16), ops.kernel.last_variant()
+    finally:
+        ep.deallocate(ab)
+        ep.deallocate(yb)
+        ops.free()
+    want = synth.to_f32(a, dt).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, dt), zp, g, n, k, bs, bits).astype(np.float64).T
+    assert (got != want.astype(np.float16)).mean() <= 0.02, variant
