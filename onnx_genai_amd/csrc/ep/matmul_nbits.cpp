@@ -247,10 +247,11 @@ void drop_weight_copy(NxrtRocmMatMulNBits& kn, void* old)
 }
 
 // Taller calls on weights that are neither 4 bits nor contiguous may round them to 16 bits - the 16-bit copy that the dense route makes and
-// the tiled kernels' own tiles alike - from five rows up and while that copy is within its limit; everything else keeps its weights in 32 bits.
+// the tiled kernels' own tiles alike - from five rows up and while that copy is within its limit; everything else keeps its weights in 32 bits,
+// a call that may not allocate (and so has no such copy) among it.
 bool weights_in_16_bits(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args)
 {
-    return static_cast<uint64_t>(args.n) * static_cast<uint64_t>(args.k) * 2 <= kn.ep->dense_gemm_max_bytes && rocm_prefill_dense16_eligible(&args);
+    return !kn.no_alloc && static_cast<uint64_t>(args.n) * static_cast<uint64_t>(args.k) * 2 <= kn.ep->dense_gemm_max_bytes && rocm_prefill_dense16_eligible(&args);
 }
 
 // Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on

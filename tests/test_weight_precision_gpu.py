@@ -83,3 +83,29 @@ def test_act_order_with_unaligned_activations_keeps_its_weights(ep, port, bits, 
         ops.free()
     want = synth.to_f32(a, dt).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, dt), zp, g, n, k, bs, bits).astype(np.float64).T
     assert (got != want.astype(np.float16)).mean() <= 0.02, variant
+
+
+@pytest.mark.parametrize("bits,m,first", [(8, 40, False), (8, 100, True), (4, 100, True), (4, 100, False)])
+def test_calls_that_may_not_allocate_keep_their_weights(ep, port, bits, m, first):
+    """execute_static has no 16-bit copy of 8-bit or act-order weights to multiply by: they stay in 32 bits there, also behind an execute of the node."""
+    n, k, bs, dt = 1100, 1024, 128, E.F16
+    make = synth.make_weights if bits == 4 else lambda *args, **kw: synth.make_weights_bits(args[0], args[1], args[2], 8, args[3], **kw)
+    b, s, zp = make(n, k, bs, m, zero_points=True, scale_lo=0.002, scale_hi=0.004, scale_dtype=dt)
+    g = (np.arange(k) // bs).astype(np.int32)
+    if bits == 4:
+        np.random.default_rng(m).shuffle(g)
+    a = synth.make_activation(m, k, m, dt)
+    ops = E.DeviceOperands(ep, b, s, dt, zp, n, k, bs, bits=bits, g_idx=g if bits == 4 else None)
+    ab, yb = ep.upload(a), ep.allocate(m * n * 4)
+    try:
+        # (g_idx is range-checked once, by an execute)
+        if first or bits == 4:
+            ops.kernel.execute(ops.views(ab, dt, m if first else 1), [E.TensorView(yb.ptr, dt, (m if first else 1, n))])
+        ops.kernel.execute_static(ops.views(ab, dt, m), [E.TensorView(yb.ptr, E.F32, (m, n))])
+        got, variant = ep.download(yb, (m, n), np.float32), ops.kernel.last_variant()
+    finally:
+        ep.deallocate(ab)
+        ep.deallocate(yb)
+        ops.free()
+    want = synth.to_f32(a, dt).astype(np.float64) @ port.dequantize_nk_gidx(b, synth.to_f32(s, dt), zp, g, n, k, bs, bits).astype(np.float64).T
+    assert helpers.rel_l2(got, want) <= 2e-6, variant
