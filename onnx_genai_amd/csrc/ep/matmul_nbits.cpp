@@ -517,8 +517,8 @@ bool f32_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
 int64_t min_streamed_weights(int64_t rows) { return rows <= 4 ? int64_t{1} << 22 : int64_t{1} << 20; }
 
 // 8-bit weights through the repacked stream, in blocks of the 32 (or 16) rows that its kernels take. Returns false (nothing launched)
-// when the shape is not theirs or there is no copy.
-bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& rc)
+// when the shape is not theirs or there is no copy, and at 17..32 rows in two passes where the weights may be rounded (the tiled kernel's then).
+bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, bool in_16_bits, int& rc)
 {
     rc = 0;
     RocmMatMulNBitsArgs part = args;
@@ -526,7 +526,7 @@ bool stream_eight_bits(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
     part.m = rows;
     if (!rocm_decode_packed8_eligible(&part)) {
         part.m = rows = args.m < 16 ? args.m : 16;
-        if (args.m <= 32 || !rocm_decode_packed8_eligible(&part)) return false;      // (17..32 rows: one pass or the other routes)
+        if ((in_16_bits && args.m <= 32) || !rocm_decode_packed8_eligible(&part)) return false;
     }
     if (!use_packed(kn, part, rc)) return false;
     for (int64_t row0 = 0; row0 < args.m && rc == 0; row0 += rows) {
@@ -806,12 +806,12 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     if (kn.bits != 4 || args.g_idx) {
         // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
         // row blocks over the stream took 97 / 101). f32 results of 16-bit rows keep the routes below.
-        // Weights that stay in 32 bits come in blocks of 32 rows at any height.
+        // Weights that stay in 32 bits come in blocks of 32 rows, or of 16 where one pass takes no more, at any height.
         const bool eight = kn.bits == 8 && !args.g_idx && args.n * args.k >= min_streamed_weights(args.m);
         const bool in_tiles = eight && M > 4 && kn.ep->dense_gemm_min_rows <= 0 && !kn.ep->dense_resident && in_16_bits && rocm_prefill_mfma8_eligible(&args);
         // 2 and 8 bits, and act-order weights of any width that are not sorted by group: 16-bit calls from five rows expand the weights and run the tiled
         // kernel over the dense copy (or, opt-in, the library GEMM), everything else the plain f32 GEMV
-        if (eight && args.y_dtype != ROCM_DT_F32 && (M <= 32 || !in_16_bits) && stream_eight_bits(kn, args, rc)) {
+        if (eight && args.y_dtype != ROCM_DT_F32 && (M <= 32 || !in_16_bits) && stream_eight_bits(kn, args, in_16_bits, rc)) {
             // done
         } else if (in_tiles) {
             rc = tiled(rocm_launch_prefill_mfma8);

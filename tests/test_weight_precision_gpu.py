@@ -12,10 +12,10 @@ pytestmark = pytest.mark.gpu
 TOL_F16 = 2.0 ** -11 / 3 ** 0.5 * 1.1
 
 
-@pytest.mark.parametrize("m", [33, 70, 100])
-def test_eight_bit_weights_beyond_the_limit_stream_in_row_blocks(port, m):
+@pytest.mark.parametrize("m,n,bs", [(33, 2100, 64), (70, 2100, 64), (100, 2100, 64), (17, 2100, 32), (24, 2100, 128), (32, 2100, 64), (24, 15000, 32), (100, 15000, 32)])
+def test_eight_bit_weights_beyond_the_limit_stream_in_row_blocks(port, m, n, bs):
     ep = E.RocmExecutionProvider(0, {"dense_gemm_max_mb": "1"})
-    n, k, bs = 2100, 1024, 64
+    k = 1024
     b, s, zp = synth.make_weights_bits(n, k, bs, 8, m, zero_points=True, scale_lo=0.002, scale_hi=0.004, scale_dtype=E.F16)
     a = synth.make_activation(m, k, m, E.F16)
     bias = np.random.default_rng(m).standard_normal((m, n)).astype(np.float16)
