@@ -389,7 +389,7 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     constexpr int kSbOff = kSaOff + kSaSlots * kRows * 4;       // [kSlots][128] f32 weight scales of the step
 
     // PROBE: this lane's first accumulator element, (row m_base + wm * 32 + 4 (lane / 32), column n_base + wn * 64 + lane % 32),
-    // as a byte offset into the [M, N, kb] probe (the launcher refuses probes of 2^31 bytes or more)
+    // as a byte offset into the [M, N, kb] probe (the launcher refuses probes of 2^31 - 16 bytes or more)
     const int64_t probe_row = m_base + wm * 32 + (lane >> 5) * 4;
     const uint32_t probe_voff = PROBE ? static_cast<uint32_t>((probe_row * p.n + n_base + wn * 64 + (lane & 31)) * p.kb) * 4u : 0u;
     const __amdgpu_buffer_rsrc_t srd_probe = make_srd(PROBE ? p.acc_probe : nullptr, PROBE ? static_cast<uint64_t>(p.m * p.n * p.kb) * 4 : 0);
@@ -733,7 +733,7 @@ extern "C" int rocm_acc4_mfma_eligible(const RocmMatMulNBitsArgs* a)
         return bs_ok && padded_k / 2 * 16 < 0x7fffffff && a->m * padded_k < 0x7ffffff0;
     }
     // prefill: 32-bit offsets inside one 128-row / 128-column window and inside the block-major scales
-    return padded_k / 2 * 128 < 0x7fffffff && padded_k * 128 < 0x7fffffff && kb * a->m * 4 < 0x7fffffff;
+    return padded_k / 2 * 128 < 0x7fffffff && padded_k * 128 < 0x7fffffff && kb * a->m * 4 < 0x7ffffff0;
 }
 
 extern "C" uint64_t rocm_acc4_mfma_scratch_bytes(const RocmMatMulNBitsArgs* a)
@@ -768,7 +768,7 @@ extern "C" int rocm_launch_acc4_mfma(const RocmMatMulNBitsArgs* a, const RocmAcc
         q.bias_dtype = a->bias_dtype;
         q.y_dtype = a->y_dtype;
         q.acc_probe = a->acc_probe;
-        if (q.acc_probe && q.m * q.n * q.kb * 4 >= 0x7fffffff) return -1;            // the probe is addressed with 32-bit offsets
+        if (q.acc_probe && q.m * q.n * q.kb * 4 >= 0x7ffffff0) return -1;            // the probe is addressed with 32-bit offsets
         const bool sf32 = a->scale_dtype == ROCM_DT_F32;
         // slices of K when the grid is small and the workspace has room for their partial sums
         int slices = mnb::acc4_prefill_slices(a->m, a->n, q.padded_k, a->block_size);

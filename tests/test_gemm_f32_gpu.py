@@ -68,3 +68,15 @@ def test_infinities_nan_and_the_largest_values(ep, port, m, n, k):
             assert inside.any() and helpers.rel_l2(y[row][inside].astype(np.float64) * 2.0 ** -100, want[row][inside] * 2.0 ** -100) <= TOL
         else:
             assert helpers.rel_l2(y[row].astype(np.float64), want[row]) <= TOL, row
+
+
+def test_activations_of_more_than_two_gib(ep, port):
+    """Elements beyond K read as zeros wherever the row lies: weights in the padding of a last, partial block meet nothing."""
+    m, n, k, bs, rows = 140000, 128, 4100, 32, 1000
+    b, s, zp = synth.make_weights(n, k, bs, 1, zero_points=True, scale_lo=0.002, scale_hi=0.01, scale_dtype=E.F32)
+    a = synth.make_activation(rows, k, 1, E.F32)
+    y, variant = E.matmul_nbits(ep, np.tile(a, (m // rows, 1)), E.F32, b, s, E.F32, zp, n, k, bs)
+    assert variant == "gemm_f32_mfma"
+    blocks = y.reshape(m // rows, rows, n)
+    assert helpers.rel_l2(blocks[0], port.matmul_f64(a, b, s, zp, n, k, bs)) <= TOL
+    assert all(np.array_equal(block, blocks[0]) for block in blocks[1:])
