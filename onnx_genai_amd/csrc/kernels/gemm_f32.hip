@@ -1,6 +1,7 @@
 // f32 activations at more than a few rows (block size >= 32, K % 4 == 0): the matrix cores with nothing rounded below f32.
 //
-// An f32 value is the exact sum of three bf16 values (its 24 significant bits cut in three runs of eight), and q - zp, an
+// An f32 value is the exact sum of three bf16 values (its 24 significant bits cut in three runs of eight) down to 2^-110, and beside values of 2^-95 and more
+// what is lost below that is none of an f32 sum's bits; rows of smaller values only are scaled up first (at the second walk below). q - zp, an
 // integer of at most four bits and a sign, is a bf16 value as it stands. So
 //   y += scale * (sum a1*(q-zp) + sum a2*(q-zp) + sum a3*(q-zp))
 // over a run of 32 weights of one block, with products that are exact and sums in f32: the reference's fp32 route
@@ -158,13 +159,18 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
         for (int j = 0; j < CN; ++j) sum[j][e] = 0.f;
     }
 
+    uint32_t seen = 0;                                     // the bits of all this lane's activations or-ed together
+    float scale_up = 1.f, scale_down[Ops::kAcc];           // of the second walk: this lane's operand row, its accumulators' rows
     auto multiply = [&](const Run& x, auto wide) {
         constexpr bool kWide = decltype(wide)::value;
         uint32_t v[8 * G];
 #pragma unroll
         for (int i = 0; i < 2 * G; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[4 * i + e] = kWide ? __float_as_uint(__uint_as_float(x.a[i][e]) * 0x1p-16f) : x.a[i][e];
+            for (int e = 0; e < 4; ++e) {
+                v[4 * i + e] = kWide ? __float_as_uint(__uint_as_float(x.a[i][e]) * scale_up) : x.a[i][e];
+                if (!kWide) seen |= x.a[i][e];
+            }
         uint4 plane[3][G];
         cut_in_three<G, kWide>(v, plane);
 #pragma unroll
@@ -179,9 +185,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
             for (int q = 2; q >= 0; --q)                                      // smallest parts first
 #pragma unroll
                 for (int g = 0; g < G; ++g) acc = Ops::mfma(plane[q][g], w[g], acc);
-            const float sc = ScaleIo<ST>::to_f32(x.s[j], scale_bf16) * (kWide ? 0x1p16f : 1.f);         // 0 for a column beyond N and past the end
+            const float sc = ScaleIo<ST>::to_f32(x.s[j], scale_bf16);         // 0 for a column beyond N and past the end
 #pragma unroll
-            for (int e = 0; e < Ops::kAcc; ++e) sum[j][e] = fmaf(acc[e], sc, sum[j][e]);
+            for (int e = 0; e < Ops::kAcc; ++e) sum[j][e] = fmaf(acc[e], kWide ? sc * scale_down[e] : sc, sum[j][e]);
         }
     };
 
@@ -198,14 +204,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     }
 
     // A sum that is not finite: an activation was infinite (NaN came of it above), or so large that the unscaled sum of a run overflowed,
-    // or the result is what it is. The wave walks its share once more with the activations scaled by 2^-16, so that a run's 32
-    // products of up to 15 fit, and infinities kept whole in their first part. Asked once per wave, not per run: no cost otherwise.
+    // or the result is what it is. Or a row whose values in the wave's share, not all of them zero, are all below 2^-95 (the or-ed exponents tell): their parts fall
+    // under bf16's smallest value. The wave then walks its share once more with infinities kept whole in their first part and each row scaled
+    // for itself: one with a value of 2 or more by 2^-16, so that a run's 32 products of up to 15 fit, one of tiny values by 2^64. Asked
+    // once per wave, not per run; or-ing the values costs one instruction for two of them.
+#pragma unroll
+    for (int off = TILE; off < 64; off <<= 1) seen |= __shfl_xor(seen, off, 64);
+    const bool tiny = (seen & 0x7fffffffu) != 0 && (seen & 0x70000000u) == 0;
     bool finite = true;
 #pragma unroll
     for (int j = 0; j < CN; ++j)
 #pragma unroll
         for (int e = 0; e < Ops::kAcc; ++e) finite = finite && __builtin_isfinite(sum[j][e]);
-    if (__builtin_expect(__any(!finite), 0)) {
+    if (__builtin_expect(__any(!finite || tiny), 0)) {
+        scale_up = tiny ? 0x1p64f : (seen & 0x40000000u) != 0 ? 0x1p-16f : 1.f;
+        const float inverse = tiny ? 0x1p-64f : (seen & 0x40000000u) != 0 ? 0x1p16f : 1.f;
+#pragma unroll
+        for (int e = 0; e < Ops::kAcc; ++e) scale_down[e] = __shfl(inverse, Ops::row_of(e, lane), 64);
 #pragma unroll
         for (int j = 0; j < CN; ++j) sum[j] = zero;
 #pragma unroll 1

@@ -80,3 +80,24 @@ def test_activations_of_more_than_two_gib(ep, port):
     blocks = y.reshape(m // rows, rows, n)
     assert helpers.rel_l2(blocks[0], port.matmul_f64(a, b, s, zp, n, k, bs)) <= TOL
     assert all(np.array_equal(block, blocks[0]) for block in blocks[1:])
+
+
+@pytest.mark.parametrize("m,n,k", [(20, 128, 96), (70, 1100, 96), (600, 1100, 96)])
+def test_the_smallest_values(ep, port, m, n, k):
+    """Rows of tiny activations, down to subnormal ones, keep their 24 bits - alone, and beside rows whose infinities or largest values send a wave round again."""
+    b, s, zp = synth.make_weights(n, k, 32, n, zero_points=True, scale_lo=8.0, scale_hi=16.0, scale_dtype=E.F32)
+    a = synth.make_activation(m, k, n, E.F32)
+    tiny = {1: -112, 3: -118, 5: -126, 7: -130, 9: -100, 19: -122}
+    for row, e in tiny.items():
+        a[row] = (a[row].astype(np.float64) * 2.0 ** e).astype(np.float32)
+    w = port.dequantize_nk_bits(b, s, zp, n, k, 32, 4).astype(np.float64)
+    for beside in ("ordinary", "infinite", "largest"):
+        if beside == "infinite":
+            a[0, 5], a[4, 40] = np.inf, -np.inf
+        elif beside == "largest":
+            a[0, 5], a[4, 40] = 1.0, 1.0
+            a[2, 0:32] = np.finfo(np.float32).max * np.where(np.arange(32) % 3 == 0, -1, 1)
+        y, variant = E.matmul_nbits(ep, a, E.F32, b, s, E.F32, zp, n, k, 32, y_dtype=E.F32)
+        assert variant == "gemm_f32_mfma"
+        for row in [*tiny, 6, m - 1]:
+            assert helpers.rel_l2(y[row].astype(np.float64) * 2.0 ** 120, (a[row].astype(np.float64) * w).sum(axis=1) * 2.0 ** 120) <= TOL, (beside, row)
