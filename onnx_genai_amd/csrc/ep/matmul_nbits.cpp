@@ -157,7 +157,7 @@ struct NxrtRocmMatMulNBits {
     const void* dense_from[3] = {nullptr, nullptr, nullptr};
     int dense_dtype = 0, dense_scale_dtype = 0;
     // constant act-order weights sorted by group: the order of K ([K] int32, first in the allocation) and B in that order; null where
-    // g_idx has another form (`regroup_failed`: asked once per pair of tensors)
+    // g_idx has another form (`regroup_failed`: found once per pair of tensors)
     void* regrouped = nullptr;
     const void* regrouped_from[2] = {nullptr, nullptr};          // B, g_idx
     bool regroup_failed = false;
@@ -283,10 +283,14 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
             kn.regrouped = nullptr;
         }
         kn.packed_from[0] = kn.dense_from[0] = nullptr;            // copies made from the old one: a new one may lie at its address
-        kn.regroup_failed = true;
-        const size_t b_bytes = static_cast<size_t>(args.n) * ((args.k + args.block_size - 1) / args.block_size) * static_cast<size_t>(args.block_size * kn.bits / 8);
+        kn.regrouped_from[0] = nullptr;                            // (no memory now, or an error: the next call asks again)
         int regular = 0;
-        if (args.block_size * kn.bits % 32 == 0 && rocm_ffi_malloc(&kn.regrouped, order_bytes + b_bytes) == 0) {
+        if (args.block_size * kn.bits % 32 == 0) {
+            const size_t b_bytes = static_cast<size_t>(args.n) * ((args.k + args.block_size - 1) / args.block_size) * static_cast<size_t>(args.block_size * kn.bits / 8);
+            if (rocm_ffi_malloc(&kn.regrouped, order_bytes + b_bytes) != 0) {
+                kn.regrouped = nullptr;
+                return false;
+            }
             int32_t* const order = static_cast<int32_t*>(kn.regrouped);
             rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, order, &regular, kn.ep->stream);
             if (rc == 0 && regular)
@@ -295,12 +299,9 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
                 rocm_ffi_free(kn.regrouped);
                 kn.regrouped = nullptr;
                 if (rc != 0) return false;
-            } else {
-                kn.regroup_failed = false;
             }
-        } else {
-            kn.regrouped = nullptr;
         }
+        kn.regroup_failed = !regular;
         kn.regrouped_from[0] = args.b;
         kn.regrouped_from[1] = args.g_idx;
     }
