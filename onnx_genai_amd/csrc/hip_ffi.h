@@ -230,8 +230,8 @@ int rocm_launch_prefill_mfma(const RocmMatMulNBitsArgs* args, int tile_choice, v
 int rocm_prefill_mfma8_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_prefill_mfma8(const RocmMatMulNBitsArgs* args, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream);
 /* The same tiled kernel over weights that a launch of their own has expanded to a dense [N, K] matrix of the activations' 16-bit
- * type (w16_nk, 16-byte aligned; K % 64 == 0): the tall route of bits = 2 / 8 and of weights with g_idx, whose packed forms the
- * tile loader does not read. args->b / scales / zp are not read; tiles of 128 columns at most. */
+ * type (w16_nk, 16-byte aligned; K % 64 == 0): the tall route of bits = 2, of unsorted g_idx and of the 8-bit calls that
+ * rocm_launch_prefill_mfma8 does not get. args->b / scales / zp are not read; tiles of 128 columns at most. */
 int rocm_prefill_dense16_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_prefill_dense16(const RocmMatMulNBitsArgs* args, const void* w16_nk, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream);
 
@@ -265,6 +265,9 @@ int rocm_acc4_mfma_eligible(const RocmMatMulNBitsArgs* args);
 /* Bytes of partial sums the tiled kernel wants when it cuts K into slices (small grids); 0 when it does not. With less
  * it uses fewer slices or none. */
 uint64_t rocm_acc4_mfma_scratch_bytes(const RocmMatMulNBitsArgs* args);
+/* What a call of more than 16 rows runs on a chip of `compute_units` CUs with that scratch: rows of its tiles (128 or 256, by 128 columns), slices
+ * of K. -1: not its shape. No GPU work. */
+int rocm_acc4_mfma_plan(const RocmMatMulNBitsArgs* args, int compute_units, int* tile_rows, int* slices);
 int rocm_launch_acc4_mfma(const RocmMatMulNBitsArgs* args, const RocmAcc4Workspace* ws, int waves, rocm_stream_t stream);
 /* One row over the repacked copy of constant weights (the copy rocm_launch_pack_decode makes); code_order 2. */
 int rocm_acc4_packed_eligible(const RocmMatMulNBitsArgs* args);

@@ -673,18 +673,19 @@ static int acc4_steps_per_slice(int64_t padded_k, int block_size, int slices)
 // tiles, f16, zero points, 12 heights of 200 - 4096 rows on six shapes (us, before and after):
 //   block 64, K >= 8192, 78 % or more full: 8192 -> 57344 at 512 / 4096 rows 717 -> 582, 5476 -> 4252; 28672 -> 8192 at 1000 / 4096 624 -> 504,
 //     2559 -> 2113; 8192 -> 10240 at 2048 (83 % full) 452 -> 436. At 66 - 73 % (300, 600 rows) 529 -> 548, 859 -> 838.
-//   block 64, a shorter K: the tiles' ends weigh more. 4096 -> 28672 at 512 / 4096 rows (87, 100 %) 172 -> 158, 1219 -> 1097; 3584 -> 37888 at 1000
-//     (92 %) 369 -> 348, but at 768 and 1600 rows (87, 83 %) 274 -> 279, 583 -> 616.
+//   block 64, a shorter K: the tiles' ends weigh more. 4096 -> 28672 at 512 / 4096 rows (87.5, 100 %) 172 -> 158, 1219 -> 1097; 3584 -> 37888 at 1000
+//     (92 %) 369 -> 348; left out, at 768 and 1600 rows (86.7, 83 %) 274 -> 279, 583 -> 616. Between the two, 5120 -> 27648, 6144 -> 24576 and 7168 -> 20480 at 12
+//     heights of 200 - 3000 rows gain 6 - 14 % wherever the rule takes them (6144 -> 24576 at 900 / 1000 rows 396 -> 344, 403 -> 351).
 //   block 128: one flush for two steps is less work to overlap. 8192 -> 57344 at 512 / 4096 606 -> 546, 4700 -> 3937; 8192 -> 10240 at 2048
 //     (83 %) 411 -> 417; 3584 -> 37888 at 4096 rows (100 %) 1211 -> 1249: only from K = 8192.
 //   block 32 (two flushes a step) does not fit 256 registers with the loads this far ahead.
-static bool acc4_tall_tiles(const Acc4PrefillParams& p, int slices, int blocks_per_step)
+static bool acc4_tall_tiles(int64_t m, int64_t n, int64_t padded_k, int block_size, int slices, int64_t cus)
 {
-    const int64_t cus = rocm_ffi_compute_units(), columns = (p.n + kTile - 1) / kTile, tiles = columns * ((p.m + 2 * kTile - 1) / (2 * kTile));
-    if (slices != 1 || p.acc_probe || tiles < cus || p.padded_k * 2 * kTile >= 0x7fffffff) return false;
-    const int64_t full = 100 * columns * ((p.m + kTile - 1) / kTile) / (2 * cus * ((tiles + cus - 1) / cus));
-    if (blocks_per_step == 0) return p.padded_k >= 8192 && full >= 86;
-    return full >= (p.padded_k >= 8192 ? 78 : 87);
+    const int64_t columns = (n + kTile - 1) / kTile, tiles = columns * ((m + 2 * kTile - 1) / (2 * kTile));
+    if (block_size == 32 || slices != 1 || tiles < cus || padded_k * 2 * kTile >= 0x7fffffff) return false;
+    const int64_t full = 100 * columns * ((m + kTile - 1) / kTile) / (2 * cus * ((tiles + cus - 1) / cus));
+    if (block_size > kStep) return padded_k >= 8192 && full >= 86;
+    return full >= (padded_k >= 8192 ? 78 : 87);
 }
 
 template <int NBS, bool SF32, int TM, int D, bool PROBE>
@@ -714,7 +715,7 @@ static int launch_acc4_prefill(const Acc4PrefillParams& p, int slices, hipStream
         return launch_acc4_prefill_cfg<NBS, SF32, 1, 2, true>(p, slices, stream);
     }
     if constexpr (NBS != 2) {
-        if (acc4_tall_tiles(p, slices, NBS)) return launch_acc4_prefill_cfg<NBS, SF32, 2, 4, false>(p, slices, stream);
+        if (acc4_tall_tiles(p.m, p.n, p.padded_k, 1 << p.bs_log2, slices, rocm_ffi_compute_units())) return launch_acc4_prefill_cfg<NBS, SF32, 2, 4, false>(p, slices, stream);
     }
     if (NBS == 2 || deep) return launch_acc4_prefill_cfg<NBS, SF32, 1, 4, false>(p, slices, stream);
     return launch_acc4_prefill_cfg<NBS, SF32, 1, NBS == 2 ? 4 : 2, false>(p, slices, stream);
@@ -742,6 +743,16 @@ extern "C" uint64_t rocm_acc4_mfma_scratch_bytes(const RocmMatMulNBitsArgs* a)
     const int64_t padded_k = (a->k + a->block_size - 1) / a->block_size * a->block_size;
     const int slices = mnb::acc4_prefill_slices(a->m, a->n, padded_k, a->block_size);
     return slices > 1 ? static_cast<uint64_t>(slices) * static_cast<uint64_t>(a->m) * static_cast<uint64_t>(a->n) * 4 : 0;
+}
+
+extern "C" int rocm_acc4_mfma_plan(const RocmMatMulNBitsArgs* a, int compute_units, int* tile_rows, int* slices)
+{
+    if (a->m <= 16 || compute_units <= 0 || !rocm_acc4_mfma_eligible(a)) return -1;
+    const int64_t padded_k = (a->k + a->block_size - 1) / a->block_size * a->block_size;
+    const int s = mnb::acc4_prefill_slices(a->m, a->n, padded_k, a->block_size);
+    if (tile_rows) *tile_rows = !a->acc_probe && mnb::acc4_tall_tiles(a->m, a->n, padded_k, a->block_size, s, compute_units) ? 2 * mnb::kTile : mnb::kTile;
+    if (slices) *slices = s;
+    return 0;
 }
 
 extern "C" int rocm_launch_acc4_mfma(const RocmMatMulNBitsArgs* a, const RocmAcc4Workspace* ws, int waves, rocm_stream_t stream)

@@ -62,3 +62,14 @@ def test_plans_follow_the_compute_unit_count(lib):
     assert lib.rocm_decode_packed_plan(C.byref(b), 0, 0, 256, C.byref(q256)) == 0
     assert q128.waves <= q256.waves and q128.waves * q128.groups_per_wave >= 10 and q256.waves * q256.groups_per_wave >= 10
     assert lib.rocm_decode_packed_plan(C.byref(a), 0, 0, 0, C.byref(p256)) == -1
+
+
+def test_acc4_calls_that_take_the_taller_tiles(lib):
+    """accuracy_level 4: 256 x 128 tiles where their grid fills its rounds, from K = 8192 at block 128 and never at block 32; the same shares of a smaller chip."""
+    def rows(m, n, k, bs, cus=256):
+        out = C.c_int()
+        assert lib.rocm_acc4_mfma_plan(C.byref(T.ffi_args(T.F16, bs, True, m, n, k)), cus, C.byref(out), None) == 0
+        return out.value
+    assert rows(4096, 57344, 8192, 64) == rows(2048, 10240, 8192, 64) == rows(512, 28672, 4096, 64) == rows(512, 57344, 8192, 128) == 256
+    assert rows(768, 37888, 3584, 64) == rows(600, 57344, 8192, 64) == rows(2048, 10240, 8192, 128) == rows(4096, 37888, 3584, 128) == rows(4096, 57344, 8192, 32) == 128
+    assert rows(512, 14336, 4096, 64, cus=128) == 256 and rows(512, 14336, 4096, 64) == 128
