@@ -126,7 +126,7 @@ void check_attrs(const NxrtRocmMatMulNBitsAttrs& a, Check& c)
 struct NxrtRocmMatMulNBits {
     NxrtRocmEp* ep = nullptr;
     int64_t k = 0, n = 0, block_size = 0, accuracy_level = 0;
-    int64_t bits = 4;                    // 2 and 8 run on the plain kernels (and the dense route), 4 on everything
+    int64_t bits = 4;                    // 2 runs on the plain kernels and the dense route, 8 also on kernels of its own, 4 on everything
     int64_t rows_hint = -1;              // M when the create-time shape of A was static
     bool bias_post_round = false;        // the bias is a folded Add: round(round(acc) + bias) on 16-bit outputs
     // The fused gate/up node: two ordinary kernels (each with its own repacked copy, scratch and variant) whose 16-bit
@@ -354,9 +354,9 @@ bool use_packed(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& r
 // Tall 16-bit calls over a dense [N, K] copy of the weights in the activations' type, expanded by a launch of its own. Two users:
 //  * the opt-in library route (dense_gemm_min_rows > 0): the product is the library GEMM, as in the CUDA provider for M >= 8
 //    (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:6176-6222);
-//  * by default, calls from five rows whose weights the tile loader does not read - bits = 2 / 8 and weights with g_idx
-//    (matmul_nbits.rs:2035, 3636-3658): the product is this provider's own tiled kernel over the dense copy, instead of a
-//    one-wave-per-column GEMV that reads all M rows of A per column.
+//  * by default, calls from five rows whose weights the tile loader does not read (matmul_nbits.rs:2035, 3636-3658) - bits = 2, bits = 8 below
+//    min_streamed_weights or with scales of another type than A, and act-order weights that are not sorted by group: the product is this provider's own
+//    tiled kernel over the dense copy, instead of a one-wave-per-column GEMV that reads all M rows of A per column.
 // Returns false with nothing launched when the route does not apply or is not ready (then the caller's next route takes the
 // call): too few rows, another dtype mix, a dense copy beyond the configured size, no library kernel for the shape, or a first
 // use while a graph capture is open (nothing may allocate then).
@@ -365,7 +365,7 @@ bool dense_route(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& 
     rc = 0;
     NxrtRocmEp& ep = *kn.ep;
     if (kn.no_alloc) return false;              // the library GEMM and its buffers are out of bounds for a call that may not allocate
-    // other bit widths have no tiled kernel to fall back on, only the plain GEMV: the route pays from a few dozen rows
+    // other bit widths and unsorted act-order weights fall back on the plain GEMV: the route pays from a few dozen rows
     const bool plain_only = kn.bits != 4 || args.g_idx != nullptr;
     const int64_t min_rows = !plain_only ? ep.dense_gemm_min_rows : (ep.dense_gemm_min_rows < 32 ? ep.dense_gemm_min_rows : 32);
     bool library = ep.dense_gemm_min_rows > 0 && args.m >= min_rows;
@@ -514,7 +514,9 @@ bool f32_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args,
 }
 
 // Elements of 8-bit weights from which a call streams a repacked copy: below, up to four rows, the plain kernel is level (bf16, block 128:
-// 3584 -> 1024 5.2 us, 3584 -> 1200 5.4 against 4.4), and a taller call that small is not worth a second copy of its weights.
+// 3584 -> 1024 5.2 us, 3584 -> 1200 5.4 against 4.4), and a taller call that small is not worth a second copy of its weights. The tiled kernel over packed
+// 8-bit weights makes no copy, and the same line holds it back: 896 -> 128 / 896 take 9.6 / 10.6 us at 5 .. 65 rows, 9.8 / 11.9 at 500, through the
+// expansion to 16 bits, 8.3 / 8.5 and 8.5 / 9.1 without.
 int64_t min_streamed_weights(int64_t rows) { return rows <= 4 ? int64_t{1} << 22 : int64_t{1} << 20; }
 
 // 8-bit weights through the repacked stream, in blocks of the 32 (or 16) rows that its kernels take. Returns false (nothing launched)
@@ -569,7 +571,8 @@ bool stream_sorted(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, boo
     return true;
 }
 
-// Narrower f32 calls than this keep the streaming kernel and the catch-all; no projection of a model is that narrow.
+// Narrower f32 calls than this (routers of experts, low-rank adapters) keep the streaming kernel and, from 65 rows, the catch-all. Not for speed: 896 -> 64
+// at 5 / 64 / 200 rows takes 9.4 / 96 / 470 us on them and 5.2 / 5.8 / 5.8 on the matrix cores. The parity tests of those widths name these kernels.
 constexpr int64_t kGemmF32MinCols = 128;
 
 // The RMS-normalization prologue of a node on its way through the dispatch: the decode kernels over the repacked stream

@@ -3,7 +3,8 @@
 // bit (i % (8 / bits)) * bits, zero points are packed the same way (default 1 << (bits - 1)), w = (q - zp) * scale with one
 // f32 multiply. These widths get plain kernels: dequantization (f32 for the parity probe, 16 bits for the tall route's
 // dense copy) and f32 GEMVs with one wave per output column - one that loads a dword per lane and takes any shape, and
-// for up to four f16 / bf16 rows one per width that moves 16 bytes per load; the tuned kernels are 4-bit.
+// for up to four f16 / bf16 rows one per width that moves 16 bytes per load. 8-bit weights with scales of the activations' type also have builds
+// of the tuned 4-bit kernels (decode_plain.hip, prefill_mfma.hip), which take the larger calls.
 #include "common.hiph"
 
 namespace mnb {
@@ -347,7 +348,7 @@ extern "C" int rocm_launch_gemv_nbits(const RocmMatMulNBitsArgs* args, int bits,
         }
     }
     if (bits == 2) return mnb::launch_gemv<2>(args, s);
-    if (bits == 4) return mnb::launch_gemv<4>(args, s);            // 4 bits come here with g_idx only
+    if (bits == 4) return mnb::launch_gemv<4>(args, s);            // 4 bits come here with an unsorted g_idx only
     if (bits == 8) return mnb::launch_gemv<8>(args, s);
     return static_cast<int>(hipErrorInvalidValue);
 }

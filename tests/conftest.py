@@ -62,8 +62,8 @@ def ep_tiled():
 
 @pytest.fixture(scope="session")
 def ep_dense():
-    """A provider with the opt-in dense route on: from 1024 rows (32 for bit widths and act-order weights that have no tiled
-    kernel) a 16-bit call expands the weights and runs the library GEMM."""
+    """A provider with the opt-in dense route on: from 1024 rows (32 for other bit widths than 4 and act-order weights
+    that are not sorted by group) a 16-bit call expands the weights and runs the library GEMM."""
     from onnx_genai_amd.ep import RocmExecutionProvider
     provider = RocmExecutionProvider(0, {"dense_gemm_min_rows": "1024"})
     yield provider
