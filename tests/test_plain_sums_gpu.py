@@ -21,6 +21,12 @@ CASES = [
     (4, E.F16, 32, 16, 23000, 256),
     (4, E.BF16, 128, 12, 18448, 640),
     (4, E.F16, 64, 29, 14400, 448),
+    (4, E.F16, 128, 16, 36890, 256),                    # grids that workgroups of more than eight waves spread over the CUs
+    (4, E.BF16, 64, 5, 40010, 192),
+    (4, E.BF16, 32, 9, 40010, 128),
+    (8, E.BF16, 128, 4, 36890, 256),
+    (8, E.F16, 32, 16, 40010, 128),
+    (8, E.BF16, 64, 12, 60010, 192),                    # more columns than that
     (8, E.F16, 128, 1, 1200, 3584),
     (8, E.BF16, 32, 1, 4700, 904),
     (8, E.BF16, 128, 4, 1200, 3584),
@@ -32,14 +38,14 @@ CASES = [
 ]
 
 
-def node(bits, dt, bs, m, n, k, scale):
-    """(b, scales, zp, g_idx or None, the weights in 64 bits for a sample of columns, the sample)"""
+def node(bits, dt, bs, m, n, k, scale, s_dt=None):
+    """(b, scales, zp, g_idx or None, the groups in any case, a sample of the columns)"""
     make = synth.make_weights if bits == 4 else lambda *args, **kw: synth.make_weights_bits(args[0], args[1], args[2], 8, args[3], **kw)
-    b, s, zp = make(n, k, bs, n + m, zero_points=True, scale_lo=scale, scale_hi=2 * scale, scale_dtype=dt)
+    b, s, zp = make(n, k, bs, n + m, zero_points=True, scale_lo=scale, scale_hi=2 * scale, scale_dtype=s_dt or dt)
     g = (np.arange(k) // bs).astype(np.int32)
     if bits == 4:                                        # act-order: the groups' elements scattered over K
         np.random.default_rng(m).shuffle(g)
-    cols = np.arange(n) if n <= 1200 else np.unique(np.random.default_rng(n).integers(0, n, 1200))
+    cols = np.arange(n) if n <= 1200 else np.unique(np.concatenate([np.random.default_rng(n).integers(0, n, 1200), np.arange(n - 40, n)]))
     return b, s, zp, g if bits == 4 else None, g, cols
 
 
@@ -81,7 +87,7 @@ def test_infinities_nan_and_the_largest_values(ep, port, bits, dt, bs, m, n, k):
             elif kind == "nan":
                 a[row, 70] = np.nan
             elif kind == "both":
-                a[row, 3], a[row, 200] = np.inf, -np.inf
+                a[row, 3], a[row, k - 60] = np.inf, -np.inf
             else:
                 a[row, 64:68] = top * np.array([1, -1, 1, 1])
         y, variant = E.matmul_nbits(ep, synth.to_dtype(a, dt), dt, b, s, dt, zp, n, k, bs, bits=bits, g_idx=g)
@@ -95,3 +101,23 @@ def test_infinities_nan_and_the_largest_values(ep, port, bits, dt, bs, m, n, k):
                     assert fits.any() and helpers.rel_l2(got[row][fits] / (top if kind else 1.0), want[fits] / (top if kind else 1.0)) <= ONE_ROUNDING[dt], (row, kind, variant)
                 else:
                     assert np.array_equal(got[row], want, equal_nan=True), (row, kind, variant)
+
+
+@pytest.mark.parametrize("dt,bs,m,n,k", [(E.F16, 32, 1, 300, 904), (E.BF16, 128, 4, 300, 1024), (E.F16, 64, 16, 300, 1024), (E.BF16, 64, 8, 23000, 256), (E.BF16, 128, 31, 14400, 256)])
+def test_act_order_with_f32_scales(ep, port, dt, bs, m, n, k):
+    b, s, zp, g, order, cols = node(4, dt, bs, m, n, k, 0.004, E.F32)
+    a = synth.to_f32(synth.make_activation(m, k, m, dt), dt)
+    a[0, 5] = np.inf
+    if m > 1 and dt == E.BF16:
+        a[1, 64:68] = 3.3895313892515355e38 * np.array([1, -1, 1, 1])
+    y, variant = E.matmul_nbits(ep, synth.to_dtype(a, dt), dt, b, s, E.F32, zp, n, k, bs, g_idx=g)
+    assert variant == "act_order+decode_mfma_packed"
+    got = synth.to_f32(y, dt).reshape(m, n)[:, cols].astype(np.float64)
+    w = weights64(port, b, s, zp, order, cols, k, bs, 4, E.F32)
+    for row in range(m):
+        with np.errstate(invalid="ignore"):
+            want = (a[row].astype(np.float64) * w).sum(axis=1)
+        if row == 0:
+            assert np.array_equal(got[row], want, equal_nan=True)
+        else:
+            assert helpers.rel_l2(got[row] / np.abs(a[row]).max(), want / np.abs(a[row]).max()) <= ONE_ROUNDING[dt], row
