@@ -2,17 +2,20 @@
 // plans the launches as those of the builds that carry the offset, an 8-bit one's as those of the 4-bit call with twice the tiles).
 //
 // 8 bits: what is streamed is 1.01 bytes per weight and the bound is HBM. bf16, block 128, 1 / 4 / 16 rows, against a GEMV of one wave per column up to four
-// rows and weights expanded to 16 bits on every call from five: 3584 -> 152064 144 / 344 / 5535 -> 106 / 103 / 113 us, 3584 -> 37888 39.6 / 90 / 255
-// -> 28.7 / 31.4 / 31.6, 18944 -> 3584 29 / 47 / 180 -> 16.8 / 18.3 / 24.2. (As two planes of nibbles whose accumulators carried the offset: 106 / 108 / 115,
+// rows and weights expanded to 16 bits on every call from five: 3584 -> 152064 144 / 344 / 5535 -> 104 / 102 / 113 us, 3584 -> 37888 39.6 / 90 / 255
+// -> 28.4 / 31.4 / 31.5, 18944 -> 3584 29 / 47 / 180 -> 16.9 / 18.0 / 23.8. (As two planes of nibbles whose accumulators carried the offset: 106 / 108 / 115,
 // 29.3 / 39.1 / 39.6, 17.1 / 18.6 / 24.4 - twice the matrix instructions.)
-// 4 bits, act-order, gather included: HBM in f16 (3584 -> 37888, block 128, 1 / 16 rows 18.3 / 20.9 us, 18.0 / 20.1 with the offset), the vector ALU work of
-// turning nibbles into bf16 integers otherwise (20.6 / 24.5 against 17.9 / 20.7).
+// 4 bits, act-order, gather included: HBM in f16 (3584 -> 37888, block 128, 1 / 16 rows 18.1 / 20.9 us, 17.8 / 20.1 with the offset), the vector ALU work of
+// turning nibbles into bf16 integers otherwise (19.0 / 24.4 against 17.8 / 20.5).
 #include "decode_plain.hiph"
 
 namespace mnb {
 
+// At most 80 scalar registers: with more, which only the rare second summation asks for, seven waves fit a SIMD instead of eight, and one workgroup of
+// fourteen a CU instead of two (8 bits, bf16, one row, 3584 -> 37888: 28.6 -> 32.7 us).
 template <bool BF16, int BS, int MR, typename ST, int BITS>
 __global__ __launch_bounds__((BS == 128 && sizeof(ST) == 2 && (MR != 16 || BF16)) ? 1024 : 512)
+__attribute__((amdgpu_num_sgpr(80)))
 void decode_plain_kernel(PackedParams p)
 {
     decode_packed_body<BF16, BS, MR, ST, 1, false, false, BITS, true>(p);

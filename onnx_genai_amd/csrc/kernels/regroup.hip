@@ -3,7 +3,7 @@
 //   B'[n, j] = B[n, order[j]],  A'[m, j] = A[m, order[j]],  order = the elements of K, group by group,
 // with the scales and zero points as they are, so that the kernels for contiguous blocks serve it - of those over the repacked stream the ones with plain
 // sums, which the per-element kernels have too. B' is made once for constant weights and the stream once more from it: two copies of the weights beside the caller's; A' costs one gather per call (7 KB of a 3584-element row: 2 us) where the kernels that look a group up per element
-// paid for it on every weight: 3584 -> 37888, one f16 row, block 128: 501 us, against 18.3 us for gather and repacked-stream kernel together.
+// paid for it on every weight: 3584 -> 37888, one f16 row, block 128: 501 us, against 18.1 us for gather and repacked-stream kernel together.
 #include <vector>
 
 #include "common.hiph"

@@ -75,12 +75,12 @@ def test_infinities_nan_and_the_largest_values(ep, port, bits, dt, bs, m, n, k):
     b, s, zp, g, order, cols = node(bits, dt, bs, m, n, k, 0.004 if bits == 4 else 0.0004)
     top = 65504.0 if dt == E.F16 else 3.3895313892515355e38
     w = weights64(port, b, s, zp, order, cols, k, bs, bits, dt)
-    kinds = ["plus", "minus", "nan", "both", "top"]
+    kinds = ["plus", "minus", "nan", "both", "top", "plus and top"]
     for first in range(0, len(kinds), m):                  # a kind a row, over as many calls as that takes
         a = synth.to_f32(synth.make_activation(m, k, first, dt), dt)
         row_kind = dict(enumerate(kinds[first:first + m]))
         for row, kind in row_kind.items():
-            if kind == "plus":
+            if kind.startswith("plus"):
                 a[row, 5] = np.inf
             elif kind == "minus":
                 a[row, k - 1] = -np.inf
@@ -88,7 +88,7 @@ def test_infinities_nan_and_the_largest_values(ep, port, bits, dt, bs, m, n, k):
                 a[row, 70] = np.nan
             elif kind == "both":
                 a[row, 3], a[row, k - 60] = np.inf, -np.inf
-            else:
+            if kind.endswith("top"):
                 a[row, 64:68] = top * np.array([1, -1, 1, 1])
         y, variant = E.matmul_nbits(ep, synth.to_dtype(a, dt), dt, b, s, dt, zp, n, k, bs, bits=bits, g_idx=g)
         got = synth.to_f32(y, dt).reshape(m, n)[:, cols].astype(np.float64)
