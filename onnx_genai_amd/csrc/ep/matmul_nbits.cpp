@@ -270,7 +270,7 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
             RocmMatMulNBitsArgs probe = args;
             probe.a = nullptr;                                             // (the gathered rows and the sorted copy are aligned)
             probe.b = nullptr;
-            const bool tiled = args.m > 16 && rocm_prefill_mfma_eligible(&probe);
+            const bool tiled = rocm_prefill_mfma_any_rows_eligible(&probe);
             if (probe.m > 16) probe.m = 16;
             if (!tiled && !(args.m <= 32 && rocm_decode_plain_eligible(&probe))) return false;
         }
@@ -888,7 +888,8 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
             // done
         } else if (!dense_off && dense_route(kn, args, rc)) {
             // done: weights expanded to 16 bits, then the library GEMM
-        } else if (M > 16 && in_16_bits && rocm_prefill_mfma_eligible(&args)) {
+        } else if (in_16_bits && rocm_prefill_mfma_any_rows_eligible(&args)) {
+            // more than 32 rows; fewer where the stream does not take the block size, or its copy cannot be made now
             rc = tiled(rocm_launch_prefill_mfma);
             kn.variant = "prefill_mfma_lds";
         } else {

@@ -214,6 +214,8 @@ int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* args, const void* pack
 /* Prefill (M > 16), f16/bf16 activations: B tiles dequantized into LDS, 32x32x16 MFMA.
  * tile_choice: 0 = by shape, 1 = 128 x 128, 2 = 256 x 128, 3 = 256 x 256, 4 = 128 x 64 tiles of Y per workgroup. */
 int rocm_prefill_mfma_eligible(const RocmMatMulNBitsArgs* args);
+/* The same from one row: the kernel takes any height, and the heights above are those at which it is the first choice. */
+int rocm_prefill_mfma_any_rows_eligible(const RocmMatMulNBitsArgs* args);
 /* Small grids with long K are cut into slices of K whose f32 partial sums land in `scratch` ([slices][M][N]) and are added up
  * by a second kernel; rocm_prefill_mfma_scratch_bytes says how much the preferred plan wants (0 = no slicing). With less
  * scratch the launcher uses fewer slices, with none it does not slice. */

@@ -474,18 +474,23 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int bits, int 
     return rocm_launch_slice_reduce(static_cast<const float*>(scratch), plan.splits, a->m, a->n, a->bias, a->bias_dtype, a->y, a->y_dtype, stream);
 }
 
+extern "C" int rocm_prefill_mfma_any_rows_eligible(const RocmMatMulNBitsArgs* a)
+{
+    RocmMatMulNBitsArgs tall = *a;
+    if (tall.m < 17) tall.m = 17;
+    return a->m >= 1 && rocm_prefill_mfma_eligible(&tall);
+}
+
 extern "C" int rocm_launch_prefill_mfma(const RocmMatMulNBitsArgs* a, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
 {
-    if (!rocm_prefill_mfma_eligible(a)) return -1;
+    if (!rocm_prefill_mfma_any_rows_eligible(a)) return -1;
     return launch_tiled(a, false, 4, tile_choice, scratch, scratch_bytes, stream);
 }
 
 extern "C" int rocm_prefill_mfma8_eligible(const RocmMatMulNBitsArgs* a)
 {
-    RocmMatMulNBitsArgs four = *a;
-    if (four.m < 17) four.m = 17;                          // (the kernel takes any height; what is below is the caller's choice)
     const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
-    return a->m >= 1 && a->scale_dtype == a->a_dtype && kb * a->block_size * 256 < 0x7fffffff && rocm_prefill_mfma_eligible(&four);
+    return a->scale_dtype == a->a_dtype && kb * a->block_size * 256 < 0x7fffffff && rocm_prefill_mfma_any_rows_eligible(a);
 }
 
 extern "C" int rocm_launch_prefill_mfma8(const RocmMatMulNBitsArgs* a, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)

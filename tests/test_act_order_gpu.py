@@ -103,3 +103,33 @@ def test_graph_replays_sort_the_rows_of_their_own_time(ep, port):
         ep.deallocate(ab)
         ep.deallocate(yb)
         ops.free()
+
+
+@pytest.mark.parametrize("bs,m", [(128, 8), (128, 1), (256, 5)])
+def test_a_height_recorded_without_a_repacked_copy(ep, port, bs, m):
+    """A prompt sorts the weights but makes no repacked copy; a few rows first seen inside a capture take the tiled kernel from five rows, and the
+    f32 GEMV below."""
+    a_dt, n, k, tall = E.F16, 300, 512, 40
+    b, s, zp = weights(n, k, bs, 4, a_dt, 9)
+    g = shuffled_groups(k, bs, 9)
+    ops = E.DeviceOperands(ep, b, s, a_dt, zp, n, k, bs, g_idx=g)
+    ab, yb = ep.upload(synth.make_activation(tall, k, 1, a_dt)), ep.allocate(tall * n * 2)
+    try:
+        ops.run(ab, a_dt, tall, yb)
+        assert ops.kernel.last_variant() == "act_order+prefill_mfma_lds"
+        ep.capture_begin()
+        ops.run(ab, a_dt, m, yb)
+        variant = ops.kernel.last_variant()
+        graph = ep.capture_end()
+        assert variant == ("act_order+prefill_mfma_lds" if m >= 5 else "act_order+gemv_generic_f32")
+        for seed in (2, 3, 4):
+            a = synth.make_activation(m, k, seed, a_dt)
+            ep.copy_from_host(ab, a)
+            graph.replay()
+            got = synth.to_f32(ep.download(yb, (m, n), np.float16), a_dt)
+            assert helpers.rel_l2(got, expected(port, a, a_dt, b, s, zp, g, n, k, bs, 4)) <= TOL[a_dt]
+        graph.release()
+    finally:
+        ep.deallocate(ab)
+        ep.deallocate(yb)
+        ops.free()
