@@ -334,6 +334,24 @@ constexpr int kTile = 128;           // rows and columns of Y per workgroup
 constexpr int kStep = 64;            // codes of K per step
 constexpr int kPitch8 = 80;          // bytes per LDS row: 64 codes + 16 of padding (16 rows then cover all 64 banks)
 
+// The tile of Y that this workgroup of a (columns x rows x slices) grid takes. Workgroups go to the eight XCDs in turn, and each XCD has an L2 of
+// its own: with tiles handed out in launch order it holds every eighth column block and shares a row block of codes among few of them.
+// So an XCD takes one run of tiles, and the run goes down kTileRows row blocks before it moves on to the next column block: what its 32 CUs work
+// on at a time is a patch of 4 x 8 tiles, which asks the memory behind the L2 for about 100 KB a step instead of 150 (256 x 128 tiles).
+// 8192 -> 57344 and 28672 -> 8192 at 4096 rows, block 64, with their quantizers: 6482 -> 6194 us. (The f16 / bf16 tiles of prefill_mfma.hip, whose
+// step takes twice as long for the same bytes of weights, ran level with it and keep launch order.)
+struct TileAt { uint32_t row, col; };
+constexpr uint32_t kXcds = 8, kTileRows = 4;
+__device__ __forceinline__ TileAt tile_of_workgroup()
+{
+    const uint32_t columns = gridDim.x, rows = gridDim.y, tiles = columns * rows;
+    const uint32_t id = blockIdx.y * columns + blockIdx.x, xcd = id % kXcds;
+    const uint32_t tile = xcd * (tiles / kXcds) + min(xcd, tiles % kXcds) + id / kXcds;       // one-to-one: the first tiles % 8 XCDs have one more
+    const uint32_t band = tile / (kTileRows * columns), within = tile - band * (kTileRows * columns);
+    const uint32_t high = min(kTileRows, rows - band * kTileRows);
+    return {band * kTileRows + within % high, within / high};
+}
+
 // NBS: blocks per step - 2 (block size 32), 1 (block size 64) or 0 (block size >= 128: a block spans several steps).
 // SF32: scales stored as f32 (else 16 bits, f16 or bf16 by a run-time flag).
 // Eight waves, 4 (rows) x 2 (columns). TM = 1: each owns a 32 x 64 sub-tile: two MFMA tiles, 32 f32 results per lane. The
@@ -359,8 +377,9 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * kRows;
-    const int64_t n_base = static_cast<int64_t>(blockIdx.x) * kTile;
+    const TileAt at = tile_of_workgroup();
+    const int64_t m_base = static_cast<int64_t>(at.row) * kRows;
+    const int64_t n_base = static_cast<int64_t>(at.col) * kTile;
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
     const bool has_zp = p.zp != nullptr;
     const bool ragged_k = (p.padded_k & 63) != 0;
