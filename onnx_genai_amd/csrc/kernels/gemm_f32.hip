@@ -7,14 +7,15 @@
 // over a run of 32 weights of one block, with products that are exact and sums in f32: the reference's fp32 route
 // (matmul_nbits.rs:7499-7566), three MFMAs where the f32 form of the instruction would take sixteen times the cycles of one.
 //
-// A wave works alone on its share of K out of registers, the next runs' loads in flight: no LDS and no barrier until the waves of
-// a workgroup, which split K between them, add up their sums in wave order at the end. Short grids get their parallelism from
-// that split.
-// Measured (block 32, f32 scales; the catch-all and, up to 64 rows, passes of the four-row streaming kernel before): 896 -> 4864
-// at 200 rows 1665 -> 23 us (75 TFLOP/s), 4864 -> 896 at 200 rows 2219 -> 33 us, 896 -> 9728
-// at 512 rows 8373 -> 69 us, 896 -> 896 at 64 rows 97 -> 5.8 us. What bounds it: a CU's vector memory path, which serves a load's 32 rows or columns
-// one cache line at a time (five to nine such loads per run of 32 k), then the vector ALU work of cutting activations and turning nibbles into
-// bf16 (about 120 instructions per lane, tile and run with two column tiles per wave, against 6 MFMAs of 32 cycles).
+// A wave works alone on its share of K, the next run's loads in flight, and no barrier until the waves of a workgroup, which split K
+// between them, add up their sums in wave order at the end. Short grids get their parallelism from that split.
+// What bounds it is a CU's vector memory path, which serves a load one cache line at a time: an operand lane that loads its own row's
+// activations asks for 32 lines with every load, 128 times a run. So where K is a whole number of blocks (WHOLE) eight lanes load one row's 128
+// bytes of a run, eight lines a load, and the wave turns them round through LDS of its own (no bank conflicts). The weights' loads (16 bytes of 32
+// columns) are left as they are.
+// Measured, whole calls in a row, block 32, f32 scales, lanes loading rows of their own before: 896 -> 4864 at 200 rows 27.5 -> 23.8 us,
+// 4864 -> 896 at 200 rows 35.2 -> 24.7; a 0.5B layer at 100 / 200 / 512 rows 101 -> 83, 115 -> 96, 164 -> 142. (Offsets and nibbles worked out in a
+// quarter fewer instructions gave 1 % of that; a third or fourth run in flight costs registers and 8 - 12 %.) The catch-all took 1665 and 2219 us for the first two.
 #include <type_traits>
 
 #include "prefill_common.hiph"
@@ -33,9 +34,10 @@ struct GemmF32Params {
     int bs_log2;
     int scale_dtype, bias_dtype, y_dtype;
     int units_per_wave;     // runs of 32 k a wave walks
+    uint32_t nibble_mask, magic;    // 0x000F000F, 0x64006400 (see plain_nibbles)
 };
 
-// 8 * GROUPS f32 values as three bf16 operands each: plane[p][group]. What a cut leaves of an infinity is NaN; with WIDE it is 0.
+// 8 * GROUPS f32 values as three bf16 operands each: plane[p][group], in plain_nibbles' order. What a cut leaves of an infinity is NaN; with WIDE it is 0.
 template <int GROUPS, bool WIDE>
 __device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], uint4 (&plane)[3][GROUPS])
 {
@@ -44,7 +46,7 @@ __device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], ui
         uint32_t out[3][4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            uint32_t lo = v[8 * g + 2 * i], hi = v[8 * g + 2 * i + 1];
+            uint32_t lo = v[8 * g + i], hi = v[8 * g + i + 4];
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
                 out[p][i] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);      // the upper halves: both values cut to bf16
@@ -59,9 +61,6 @@ __device__ __forceinline__ void cut_in_three(const uint32_t (&v)[8 * GROUPS], ui
         for (int p = 0; p < 3; ++p) plane[p][g] = make_uint4(out[p][0], out[p][1], out[p][2], out[p][3]);
     }
 }
-
-// Eight nibbles of a packed dword as bf16 integers q - zp in element order; `shift` is 16 - zp in every byte.
-__device__ __forceinline__ uint4 nibbles_as_bf16(uint32_t w, uint32_t shift) { return dequant_dword_f32<true>(w, shift, 1.0f, -16.0f); }
 
 // The matrix-core step and the shape of its operands for tiles of 32 x 32 (16 k per MFMA, a run is two of them) and of
 // 16 x 16 (32 k per MFMA: a run is one). An operand lane holds 8 k of one row or column per MFMA.
@@ -82,7 +81,9 @@ template <> struct TileOps<16> {
 
 // TILE: 16 or 32 rows and columns per matrix-core tile. CN: tiles along N per wave. DEPTH: runs in flight. WAVES: the most
 // waves a workgroup is launched with. ST: float, or uint16_t for f16 / bf16 scales.
-template <int TILE, int CN, int DEPTH, int WAVES, typename ST>
+// WHOLE: K is a whole number of blocks, so that no run is cut short: activations go through LDS, and the offsets of a wave's loads do not change from
+// run to run (the run goes into the scalar offset). The other build works out per run and load whether elements lie within K.
+template <int TILE, int CN, int DEPTH, int WAVES, typename ST, bool WHOLE>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
 {
     using Ops = TileOps<TILE>;
@@ -104,9 +105,21 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     const __amdgpu_buffer_rsrc_t srd_z = make_srd(p.zp ? p.zp + n_base * p.zp_row : nullptr, p.zp ? static_cast<uint64_t>(cols_left * p.zp_row) : 0);
     const uint32_t zp_mask = p.zp ? 0xfu : 0u, zp_default = p.zp ? 0u : 8u;
     const bool scale_bf16 = p.scale_dtype == ROCM_DT_BF16;
+    const uint32_t mask = __builtin_amdgcn_mov_dpp(p.nibble_mask, 0xE4, 0xf, 0xf, false);
 
     const uint32_t a_off = static_cast<uint32_t>(r) * static_cast<uint32_t>(p.k) * 4u;
     const bool row_live = r < rows_left;
+    // WHOLE: eight lanes load one row's 128 bytes of a run; lane -> (row lane / 8 + 8 i, piece lane % 8). Rows beyond M lie out of range by themselves.
+    // The 16-byte piece c of row x lies at c ^ (x / 2 % 8) in the wave's 128-byte rows of LDS: writes, and reads by rows, cover all banks.
+    unsigned char* const a_stage = smem + wave * (TILE * 128);
+    uint32_t a_piece[2 * G], a_write[2 * G];
+#pragma unroll
+    for (int i = 0; i < 2 * G; ++i) {
+        const uint32_t x = static_cast<uint32_t>(8 * i + (lane >> 3)), c = static_cast<uint32_t>(lane & 7);
+        a_piece[i] = x * static_cast<uint32_t>(p.k) * 4u + c * 16u;
+        a_write[i] = x * 128u + ((c ^ ((x >> 1) & 7u)) * 16u);
+    }
+    const uint32_t a_read = static_cast<uint32_t>(r) * 128u + ((static_cast<uint32_t>(part * 2 * G) ^ ((static_cast<uint32_t>(r) >> 1) & 7u)) * 16u);
     uint32_t b_off[CN], s_off[CN], z_off[CN];
 #pragma unroll
     for (int j = 0; j < CN; ++j) {                         // a column beyond N lies out of range by itself
@@ -127,6 +140,27 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     // No branch: a run past the wave's share, a row beyond M and elements beyond K get offsets out of range, which read zeros.
     auto request = [&](Run& x, int u) {
         const bool live = u < u1;
+        if constexpr (WHOLE) {
+            // (a run past the wave's share: its last one again, with scales of zero)
+            const int at = min(u, u1 - 1);
+            const uint32_t blk = static_cast<uint32_t>(at * 32) >> p.bs_log2, oor = live ? 0u : kOutOfRange;
+#pragma unroll
+            for (int i = 0; i < 2 * G; ++i) x.a[i] = __builtin_amdgcn_raw_buffer_load_b128(srd_a, static_cast<int>(a_piece[i]), at * 128, 0);
+#pragma unroll
+            for (int j = 0; j < CN; ++j) {
+                if constexpr (G == 2) {
+                    const auto w = __builtin_amdgcn_raw_buffer_load_b64(srd_b, static_cast<int>(b_off[j]), at * 16, 0);
+                    x.b[j][0] = w[0];
+                    x.b[j][1] = w[1];
+                } else {
+                    x.b[j][0] = __builtin_amdgcn_raw_buffer_load_b32(srd_b, static_cast<int>(b_off[j]), at * 16, 0);
+                }
+                x.s[j] = ScaleIo<ST>::load_raw(srd_s, s_off[j] | oor, blk * static_cast<uint32_t>(sizeof(ST)));
+                x.z[j] = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b8(srd_z, static_cast<int>(z_off[j]), static_cast<int>(blk >> 1), 0));
+            }
+            x.zsh = (blk & 1u) * 4u;
+            return;
+        }
         const int k0 = u * 32 + part * 8 * G;
 #pragma unroll
         for (int i = 0; i < 2 * G; ++i) {
@@ -163,23 +197,34 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     float scale_up = 1.f, scale_down[Ops::kAcc];           // of the second walk: this lane's operand row, its accumulators' rows
     auto multiply = [&](const Run& x, auto wide) {
         constexpr bool kWide = decltype(wide)::value;
+        u32x4_t a[2 * G];
+        if constexpr (WHOLE) {
+#pragma unroll
+            for (int i = 0; i < 2 * G; ++i) *reinterpret_cast<u32x4_t*>(a_stage + a_write[i]) = x.a[i];
+            lds_order();
+#pragma unroll
+            for (int i = 0; i < 2 * G; ++i) a[i] = *reinterpret_cast<const u32x4_t*>(a_stage + (a_read ^ static_cast<uint32_t>(i * 16)));
+            lds_order();
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2 * G; ++i) a[i] = x.a[i];
+        }
         uint32_t v[8 * G];
 #pragma unroll
         for (int i = 0; i < 2 * G; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[4 * i + e] = kWide ? __float_as_uint(__uint_as_float(x.a[i][e]) * scale_up) : x.a[i][e];
-                if (!kWide) seen |= x.a[i][e];
+                v[4 * i + e] = kWide ? __float_as_uint(__uint_as_float(a[i][e]) * scale_up) : a[i][e];
+                if (!kWide) seen |= a[i][e];
             }
         uint4 plane[3][G];
         cut_in_three<G, kWide>(v, plane);
 #pragma unroll
         for (int j = 0; j < CN; ++j) {
             const uint32_t zq = ((x.z[j] >> x.zsh) & zp_mask) | zp_default;
-            const uint32_t shift = (16u - zq) * 0x01010101u;
             uint4 w[G];
 #pragma unroll
-            for (int g = 0; g < G; ++g) w[g] = nibbles_as_bf16(x.b[j][g], shift);
+            for (int g = 0; g < G; ++g) w[g] = plain_nibbles<true>(x.b[j][g], zq, mask, p.magic);
             acc_t acc = zero;
 #pragma unroll
             for (int q = 2; q >= 0; --q)                                      // smallest parts first
@@ -233,6 +278,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     // ---- the waves' sums through LDS, added in wave order: [wave][tile][accumulator][64] ----
     constexpr int kOuts = CN * Ops::kAcc * 64;
     float* parts = reinterpret_cast<float*>(smem);
+    if constexpr (WHOLE) __syncthreads();                  // (the waves' activations lay there)
 #pragma unroll
     for (int j = 0; j < CN; ++j)
 #pragma unroll
@@ -248,12 +294,13 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     }
 }
 
-template <int TILE, int CN, int DEPTH, int WAVES, typename ST>
+template <int TILE, int CN, int DEPTH, int WAVES, typename ST, bool WHOLE>
 static int launch_gemm_f32(const GemmF32Params& p, int waves, hipStream_t stream)
 {
     const dim3 grid(static_cast<unsigned>((p.n + TILE * CN - 1) / (TILE * CN)), static_cast<unsigned>((p.m + TILE - 1) / TILE));
-    const size_t lds = static_cast<size_t>(waves) * CN * TileOps<TILE>::kAcc * 256;               // at most 64 KiB
-    hipLaunchKernelGGL((gemm_f32_kernel<TILE, CN, DEPTH, WAVES, ST>), grid, dim3(static_cast<unsigned>(waves * 64)), lds, stream, p);
+    constexpr int kWaveLds = CN * TileOps<TILE>::kAcc * 256, kStageLds = WHOLE ? TILE * 128 : 0;
+    const size_t lds = static_cast<size_t>(waves) * (kWaveLds > kStageLds ? kWaveLds : kStageLds);        // at most 64 KiB
+    hipLaunchKernelGGL((gemm_f32_kernel<TILE, CN, DEPTH, WAVES, ST, WHOLE>), grid, dim3(static_cast<unsigned>(waves * 64)), lds, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -314,6 +361,8 @@ extern "C" int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* a, rocm_stream_t 
     p.zp_row = (p.kb + 1) / 2;
     p.bs_log2 = __builtin_ctz(static_cast<unsigned>(a->block_size));
     p.scale_dtype = a->scale_dtype;
+    p.nibble_mask = 0x000F000Fu;
+    p.magic = 0x64006400u;
     p.bias_dtype = a->bias_dtype;
     p.y_dtype = a->y_dtype;
     const int64_t cus = rocm_ffi_compute_units();
@@ -322,10 +371,12 @@ extern "C" int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* a, rocm_stream_t 
     const int tile = plan.tile, cn = plan.cn, waves = plan.waves;
     p.units_per_wave = (units + waves - 1) / waves;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    auto go = [&](auto st) {
+    auto go = [&](auto st, auto whole) {
         using ST = decltype(st);
-        if (tile == 16) return mnb::launch_gemm_f32<16, 1, 4, 8, ST>(p, waves, s);
-        return cn == 2 ? mnb::launch_gemm_f32<32, 2, 2, 8, ST>(p, waves, s) : mnb::launch_gemm_f32<32, 1, 2, 8, ST>(p, waves, s);
+        constexpr bool W = decltype(whole)::value;
+        if (tile == 16) return mnb::launch_gemm_f32<16, 1, 4, 8, ST, W>(p, waves, s);
+        return cn == 2 ? mnb::launch_gemm_f32<32, 2, 2, 8, ST, W>(p, waves, s) : mnb::launch_gemm_f32<32, 1, 2, 8, ST, W>(p, waves, s);
     };
-    return a->scale_dtype == ROCM_DT_F32 ? go(float{}) : go(uint16_t{});
+    if (a->k % a->block_size != 0) return a->scale_dtype == ROCM_DT_F32 ? go(float{}, std::false_type{}) : go(uint16_t{}, std::false_type{});
+    return a->scale_dtype == ROCM_DT_F32 ? go(float{}, std::true_type{}) : go(uint16_t{}, std::true_type{});
 }

@@ -101,3 +101,16 @@ def test_the_smallest_values(ep, port, m, n, k):
         assert variant == "gemm_f32_mfma"
         for row in [*tiny, 6, m - 1]:
             assert helpers.rel_l2(y[row].astype(np.float64) * 2.0 ** 120, (a[row].astype(np.float64) * w).sum(axis=1) * 2.0 ** 120) <= TOL, (beside, row)
+
+
+@pytest.mark.parametrize("s_dt,bs,zero_points,m,n,k", [
+    (E.F16, 64, True, 15, 130, 896),       # 16 x 16 tiles: a row short of one, and one row more
+    (E.F32, 32, False, 17, 128, 96),       # ... fewer runs than waves
+    (E.F32, 256, True, 33, 1100, 4864),
+    (E.F32, 32, True, 95, 1100, 704),      # 32 x 32 tiles: 22 runs over eight waves, the last one has one
+    (E.BF16, 32, False, 97, 1100, 800),    # ... 25 runs: four a wave, the last wave has none
+    (E.F32, 32, True, 545, 1100, 288),     # two column tiles a wave, nine runs
+])
+def test_whole_blocks(ep, port, s_dt, bs, zero_points, m, n, k):
+    """K a whole number of blocks: rows pass through LDS. Rows and shares of K at the edges of tiles."""
+    test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, "none", E.F32)
