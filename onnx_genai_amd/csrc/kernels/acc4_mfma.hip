@@ -342,8 +342,8 @@ __device__ __forceinline__ uint32_t swizzled(uint32_t row, uint32_t piece) { ret
 // its own: with tiles handed out in launch order it holds every eighth column block and shares a row block of codes among few of them.
 // So an XCD takes one run of tiles, and the run goes down kTileRows row blocks before it moves on to the next column block: what its 32 CUs work
 // on at a time is a patch of 4 x 8 tiles, which asks the memory behind the L2 for about 100 KB a step instead of 150 (256 x 128 tiles).
-// 8192 -> 57344 and 28672 -> 8192 at 4096 rows, block 64, with their quantizers: 6482 -> 6194 us. (The f16 / bf16 tiles of prefill_mfma.hip, whose
-// step takes twice as long for the same bytes of weights, ran level with it and keep launch order.)
+// 8192 -> 57344 and 28672 -> 8192 at 4096 rows, block 64, with their quantizers: 6482 -> 6194 us. (The f16 / bf16
+// tiles of prefill_mfma.hip ran level with it, 0.994 - 1.001 of the time, and keep launch order.)
 struct TileAt { uint32_t row, col; };
 constexpr uint32_t kXcds = 8, kTileRows = 4;
 __device__ __forceinline__ TileAt tile_of_workgroup()
@@ -364,7 +364,8 @@ __device__ __forceinline__ TileAt tile_of_workgroup()
 // TM = 2: 64 x 64 per wave, 256 x 128 per workgroup, two waves per SIMD of up to 256 registers: a weight is unpacked and an operand of B read
 // from LDS for twice the rows, one tile's MFMAs run under the other's flush inside a wave, and the registers hold three steps of
 // loads in flight (the two-set form of TM = 1 waits for memory: with two sets TM = 2 was level with it, 4970 us against 4266 with four on 8192 -> 57344 at
-// 4096 rows, block 64; 128 x 128 tiles 5494). Same sums in the same order, bit for bit. 8192 -> 57344 at 4096 rows: 0.70 -> 0.90 POP/s.
+// 4096 rows, block 64; 128 x 128 tiles 5494). Same sums in the same order, bit for bit. 8192 -> 57344 at 4096 rows: 0.70 -> 0.90 POP/s (0.96 with the
+// order of tiles above and LDS rows without padding).
 // PROBE: every int32 tile that is flushed is also stored to p.acc_probe ([M, N, kb]); the same code otherwise.
 template <int NBS, bool SF32, int TM, int D, bool PROBE>
 __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
