@@ -270,6 +270,8 @@ uint64_t rocm_acc4_mfma_scratch_bytes(const RocmMatMulNBitsArgs* args);
 /* What a call of more than 16 rows runs on a chip of `compute_units` CUs with that scratch: rows of its tiles (128 or 256, by 128 columns), slices
  * of K. -1: not its shape. No GPU work. */
 int rocm_acc4_mfma_plan(const RocmMatMulNBitsArgs* args, int compute_units, int* tile_rows, int* slices);
+/* M > 16: the tile of Y, in row and column blocks, that workgroup `workgroup` of a slice's grid works on (columns counted first). */
+int rocm_acc4_mfma_tile(const RocmMatMulNBitsArgs* args, int compute_units, int64_t workgroup, int64_t* row, int64_t* col);
 int rocm_launch_acc4_mfma(const RocmMatMulNBitsArgs* args, const RocmAcc4Workspace* ws, int waves, rocm_stream_t stream);
 /* One row over the repacked copy of constant weights (the copy rocm_launch_pack_decode makes); code_order 2. */
 int rocm_acc4_packed_eligible(const RocmMatMulNBitsArgs* args);

@@ -328,6 +328,7 @@ struct Acc4PrefillParams {
     int steps_per_slice;    // K steps per grid.z slice (a whole number of blocks); all steps when there is one slice
     float* partial;         // [slices, M, N] f32 partial sums when K is cut into slices, else NULL
     int32_t* acc_probe;     // PROBE builds: int32 [M, N, kb] block accumulators, as flushed
+    int full_rows;          // see acc4_tile
 };
 
 constexpr int kTile = 128;           // rows and columns of Y per workgroup
@@ -338,21 +339,24 @@ constexpr int kPitch8 = 64;          // bytes per LDS row: 64 codes, no padding
 // itself 27 % of the kernel's. 4096 rows, block 64, 8192 -> 57344 and 28672 -> 8192: 6194 -> 6030 us; 13 heights and shapes of block 32 - 128 +0.3 to +2.5 %.
 __device__ __forceinline__ uint32_t swizzled(uint32_t row, uint32_t piece) { return row * kPitch8 + ((piece ^ ((row >> 2) & 3u)) * 16u); }
 
-// The tile of Y that this workgroup of a (columns x rows x slices) grid takes. Workgroups go to the eight XCDs in turn, and each XCD has an L2 of
-// its own: with tiles handed out in launch order it holds every eighth column block and shares a row block of codes among few of them.
-// So an XCD takes one run of tiles, and the run goes down kTileRows row blocks before it moves on to the next column block: what its 32 CUs work
-// on at a time is a patch of 4 x 8 tiles, which asks the memory behind the L2 for about 100 KB a step instead of 150 (256 x 128 tiles).
-// 8192 -> 57344 and 28672 -> 8192 at 4096 rows, block 64, with their quantizers: 6482 -> 6194 us. (The f16 / bf16
-// tiles of prefill_mfma.hip ran level with it, 0.994 - 1.001 of the time, and keep launch order.)
+// The tile of Y that workgroup (x, y) of a (columns x rows x slices) grid takes. Workgroups go to the eight XCDs in turn, and each XCD has an L2 of
+// its own. In launch order (full = 0) an XCD has every eighth column block; otherwise it takes one run of tiles, which goes down kTileRows row blocks before
+// it moves on to the next column block. `full` counts the row blocks handed out that way. A last row block that is not whole follows behind them, in
+// runs of columns: its tiles take the least time, and a grid should end with those. (Among the others they cost calls of 777 rows 3 - 13 %: 896 -> 4864
+// at block 64 26.3 -> 30.2 us.) acc4_full_rows() says which calls take runs, and what it gives them.
 struct TileAt { uint32_t row, col; };
 constexpr uint32_t kXcds = 8, kTileRows = 4;
-__device__ __forceinline__ TileAt tile_of_workgroup()
+__host__ __device__ __forceinline__ TileAt acc4_tile(uint32_t x, uint32_t y, uint32_t columns, uint32_t full)
 {
-    const uint32_t columns = gridDim.x, rows = gridDim.y, tiles = columns * rows;
-    const uint32_t id = blockIdx.y * columns + blockIdx.x, xcd = id % kXcds;
-    const uint32_t tile = xcd * (tiles / kXcds) + min(xcd, tiles % kXcds) + id / kXcds;       // one-to-one: the first tiles % 8 XCDs have one more
-    const uint32_t band = tile / (kTileRows * columns), within = tile - band * (kTileRows * columns);
-    const uint32_t high = min(kTileRows, rows - band * kTileRows);
+    // one-to-one over 0 .. count - 1: the first count % 8 XCDs have one more
+    auto in_runs = [](uint32_t id, uint32_t count) {
+        const uint32_t xcd = id % kXcds, more = count % kXcds;
+        return xcd * (count / kXcds) + (xcd < more ? xcd : more) + id / kXcds;
+    };
+    if (full == 0) return {y, x};
+    if (y >= full) return {y, in_runs(x, columns)};
+    const uint32_t tile = in_runs(y * columns + x, columns * full), band = tile / (kTileRows * columns), within = tile - band * (kTileRows * columns);
+    const uint32_t left = full - band * kTileRows, high = left < kTileRows ? left : kTileRows;
     return {band * kTileRows + within % high, within / high};
 }
 
@@ -382,7 +386,7 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const TileAt at = tile_of_workgroup();
+    const TileAt at = acc4_tile(blockIdx.x, blockIdx.y, gridDim.x, static_cast<uint32_t>(p.full_rows));
     const int64_t m_base = static_cast<int64_t>(at.row) * kRows;
     const int64_t n_base = static_cast<int64_t>(at.col) * kTile;
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
@@ -713,9 +717,31 @@ static bool acc4_tall_tiles(int64_t m, int64_t n, int64_t padded_k, int block_si
     return full >= (padded_k >= 8192 ? 78 : 87);
 }
 
-template <int NBS, bool SF32, int TM, int D, bool PROBE>
-static int launch_acc4_prefill_cfg(const Acc4PrefillParams& p, int slices, hipStream_t stream)
+// acc4_tile's `full` of a call, 0 for launch order. Runs of tiles pay (us, launch order and runs; f16, zero points):
+//   * where a CU holds one workgroup and the grid takes more than a round (256 x 128 tiles, `tall`, and block size 32). 32 CUs then work on a patch of 4 x 8
+//     tiles, which at 256 x 128 asks the memory behind their L2 for 96 KB a step, against 96 - 160 for every eighth of a row of column blocks: at 4096
+//     rows, block 64, 8192 -> 57344 misses L2 75 M and 24 M times (4275 and 4057 us), 28672 -> 8192 12 M times either way (2088 and 2058). Block 32, 8192 -> 57344,
+//     4096 rows 7059 and 6629. Over 400 shapes and heights of these two kinds 0 to + 9 % but for 1 % here and there.
+//   * on wide grids whose rows of B lie a multiple of 4096 bytes apart, at any height. Block 64, 8192 -> 57344 at 17 / 300 / 600 rows 176 and 153, 551 and 491, 916 and 791;
+//     -> 32768 at 300 rows 341 and 279; -> 16384 at 17 and 300 rows 54.8 and 49.8, 169 and 161; -> 10240 at 600 rows 168 and 170, so from 128 column
+//     blocks. It is the distance: K = 8448 instead of 8192 takes 289 and 284 us at 300 rows -> 32768. Half of it, on grids wider still: 4096 -> 65536 at 64 / 300 rows
+//     95 and 87, 275 and 258; -> 32768 at 300 rows 146 and 148.
+// Two workgroups share a CU in the other calls, and which two, and which come last, matters more than what they share: runs are level with launch order to 4 % slower
+// there (4096 -> 6144, block 64, 1300 rows 144 and 146; 3584 -> 4608, block 128, 385 rows 4 %). (The f16 / bf16 tiles of prefill_mfma.hip
+// ran level with runs, 0.994 - 1.001 of the time, and keep launch order.)
+static int acc4_full_rows(int64_t m, int64_t n, int64_t row_bytes, int block_size, bool tall, int64_t cus)
 {
+    const int64_t height = tall ? 2 * kTile : kTile, columns = (n + kTile - 1) / kTile, rows = (m + height - 1) / height;
+    const bool alone = tall || (block_size == 32 && rows * columns >= cus);
+    const bool apart = row_bytes % 4096 == 0 ? columns >= 128 : row_bytes % 2048 == 0 && columns >= 352;
+    if (!alone && !apart) return 0;
+    return static_cast<int>(rows == 1 ? 1 : m / height);
+}
+
+template <int NBS, bool SF32, int TM, int D, bool PROBE>
+static int launch_acc4_prefill_cfg(Acc4PrefillParams p, int slices, hipStream_t stream)
+{
+    p.full_rows = acc4_full_rows(p.m, p.n, p.row_bytes, 1 << p.bs_log2, TM == 2, rocm_ffi_compute_units());
     const dim3 grid(static_cast<unsigned>((p.n + kTile - 1) / kTile), static_cast<unsigned>((p.m + TM * kTile - 1) / (TM * kTile)), static_cast<unsigned>(slices));
     constexpr int kSlots = NBS == 2 ? 2 : 1;
     const size_t lds = 2 * ((TM + 1) * kTile * kPitch8 + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
@@ -777,6 +803,20 @@ extern "C" int rocm_acc4_mfma_plan(const RocmMatMulNBitsArgs* a, int compute_uni
     const int s = mnb::acc4_prefill_slices(a->m, a->n, padded_k, a->block_size);
     if (tile_rows) *tile_rows = !a->acc_probe && mnb::acc4_tall_tiles(a->m, a->n, padded_k, a->block_size, s, compute_units) ? 2 * mnb::kTile : mnb::kTile;
     if (slices) *slices = s;
+    return 0;
+}
+
+extern "C" int rocm_acc4_mfma_tile(const RocmMatMulNBitsArgs* a, int compute_units, int64_t workgroup, int64_t* row, int64_t* col)
+{
+    int height = 0;
+    if (rocm_acc4_mfma_plan(a, compute_units, &height, nullptr) != 0) return -1;
+    const int64_t columns = (a->n + mnb::kTile - 1) / mnb::kTile, rows = (a->m + height - 1) / height;
+    if (workgroup < 0 || workgroup >= columns * rows) return -1;
+    const int64_t row_bytes = (a->k + a->block_size - 1) / a->block_size * a->block_size / 2;
+    const int full = mnb::acc4_full_rows(a->m, a->n, row_bytes, a->block_size, height > mnb::kTile, compute_units);
+    const mnb::TileAt at = mnb::acc4_tile(static_cast<uint32_t>(workgroup % columns), static_cast<uint32_t>(workgroup / columns), static_cast<uint32_t>(columns), static_cast<uint32_t>(full));
+    *row = at.row;
+    *col = at.col;
     return 0;
 }
 

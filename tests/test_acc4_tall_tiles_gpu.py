@@ -23,6 +23,8 @@ def tile_rows(ep, m, n, k, bs):
     (E.F16, 64, True, 500, 16370, 192, "column"),      # ragged last tiles both ways, an odd count of steps
     (E.F32, 64, False, 385, 16384, 64, "none"),        # one step; one row in the last 32 x 32 tiles
     (E.BF16, 64, True, 512, 16257, 576, "row"),        # nine steps: whole rounds of loads and a rest
+    (E.F16, 64, True, 1200, 12763, 192, "column"),     # 5 x 100 tiles: a band of four whole row blocks, and one of 176 rows
+    (E.BF16, 64, True, 2304, 7040, 192, "none"),       # 9 x 55: bands of four, four and one row block, a count that eight XCDs do not divide
     (E.F16, 128, True, 500, 16370, 8192, "row"),       # a block over two steps
     (E.F32, 256, False, 511, 16300, 8448, "column"),   # ... over four
 ])

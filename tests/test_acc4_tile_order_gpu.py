@@ -34,3 +34,27 @@ def test_every_tile_once(ep, port, m, n, k, bs, slices):
     assert helpers.rel_l2(y, want) <= 1e-5        # the bar of the parity contract
     worst = np.abs(y - want).max()
     assert worst <= 1e-4 * np.sqrt(np.mean(np.square(want.astype(np.float64)))), worst      # no tile stands out
+
+
+@pytest.mark.parametrize("s_dt,m,n,k,bs", [
+    (E.F16, 777, 4864, 96, 32),          # block size 32: 7 x 38, nine rows in the last row block
+    (E.F32, 1153, 3500, 160, 32),        # ... 10 x 28: bands of four, four and one whole row block, and one of one row
+    (E.BF16, 60, 33000, 64, 32),         # ... one row block, not whole
+    (E.F16, 300, 16300, 8192, 64),       # rows of B 4096 bytes apart: 3 x 128, over no slices
+    (E.F16, 17, 16384, 8192, 128),       # ... 1 x 128 over slices of K
+])
+def test_runs_of_tiles(ep, port, s_dt, m, n, k, bs):
+    """Grids whose tiles go out in runs instead of launch order: a column of every column block, over all rows."""
+    a_dt = E.BF16 if s_dt == E.BF16 else E.F16
+    args, tile = ffi_args(E.F16, bs, True, m, n, k), [C.c_int64(), C.c_int64()]
+    assert ep.lib.rocm_acc4_mfma_tile(C.byref(args), ep.device_info()["compute_units"], C.c_int64(8), C.byref(tile[0]), C.byref(tile[1])) == 0
+    assert (tile[0].value, tile[1].value) != (0, 8)
+    b, s, zp = synth.make_weights(n, k, bs, n + k, zero_points=True, scale_lo=0.002, scale_hi=0.01, scale_dtype=s_dt)
+    a = synth.make_activation(m, k, m, a_dt)
+    y, variant = E.matmul_nbits(ep, a, a_dt, b, s, s_dt, zp, n, k, bs, accuracy_level=4, y_dtype=E.F32)
+    assert variant == "acc4_mfma_i8"
+    cols = np.append(np.arange(0, n, 128) + np.arange(-(-n // 128)) * 37 % (n - (n - 1) // 128 * 128), n - 1)
+    want = port.matmul_acc4_f32(synth.to_f32(a, a_dt), b[cols], synth.to_f32(s, s_dt)[cols], zp[cols], cols.size, k, bs, oracle.ROUND_HALF_EVEN)
+    assert helpers.rel_l2(y[:, cols], want) <= 1e-5        # the bar of the parity contract
+    worst = np.abs(y[:, cols] - want).max()
+    assert worst <= 1e-4 * np.sqrt(np.mean(np.square(want.astype(np.float64)))), worst
