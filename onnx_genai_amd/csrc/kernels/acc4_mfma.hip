@@ -333,11 +333,13 @@ struct Acc4PrefillParams {
 
 constexpr int kTile = 128;           // rows and columns of Y per workgroup
 constexpr int kStep = 64;            // codes of K per step
-constexpr int kPitch8 = 64;          // bytes per LDS row: 64 codes, no padding
-// The 16-byte piece `piece` of row `row` lies at piece ^ (row / 4 % 4): 16 rows' pieces of one place and four rows' whole pieces (a read of an MFMA
-// operand, and a write) then both cover all 64 banks. With rows of 80 bytes instead the writes met in a bank - a quarter of the cycles that LDS was busy,
-// itself 27 % of the kernel's. 4096 rows, block 64, 8192 -> 57344 and 28672 -> 8192: 6194 -> 6030 us; 13 heights and shapes of block 32 - 128 +0.3 to +2.5 %.
-__device__ __forceinline__ uint32_t swizzled(uint32_t row, uint32_t piece) { return row * kPitch8 + ((piece ^ ((row >> 2) & 3u)) * 16u); }
+// LDS rows of 64 codes are 64 bytes apart: the 16-byte piece `piece` of row `row` lies at piece ^ (row / 4 % 4), so that 16 rows' pieces of one place and
+// four rows' whole pieces (a read of an MFMA operand, and a write) both cover all 64 banks. With rows of 80 bytes instead the writes met in a bank - a quarter of the
+// cycles that LDS was busy, itself 27 % of the kernel's (22 % now). 4096 rows, block 64, 8192 -> 57344 and 28672 -> 8192, in launch order: 4362 -> 4275, 2139 -> 2088 us;
+// 648 shapes and heights + 0.8 % in the mean. Not the 128 x 128 build of block size 64 with two register sets, which keeps 80 bytes: 64 cost it 2 % up to 128 rows
+// (3584 -> 37888 at 40 rows 73.9 and 75.5 us), 0.4 % in the mean of 377 shapes and heights.
+template <int NBS, int TM, int D> constexpr int kPitch8 = NBS == 1 && TM == 1 && D == 2 ? 80 : 64;
+template <int PITCH> __device__ __forceinline__ uint32_t piece_at(uint32_t row, uint32_t piece) { return row * PITCH + (PITCH == 64 ? piece ^ ((row >> 2) & 3u) : piece) * 16u; }
 
 // The tile of Y that workgroup (x, y) of a (columns x rows x slices) grid takes. Workgroups go to the eight XCDs in turn, and each XCD has an L2 of
 // its own. In launch order (full = 0) an XCD has every eighth column block; otherwise it takes one run of tiles, which goes down kTileRows row blocks before
@@ -376,9 +378,10 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
 {
     static_assert(TM == 1 || (TM == 2 && !PROBE && NBS != 2));
     constexpr int kRows = TM * kTile;                          // rows of the workgroup
+    constexpr int kPitch = kPitch8<NBS, TM, D>;
     constexpr int kSlots = NBS == 2 ? 2 : 1;                   // scale slots per step
     constexpr int kSaSlots = TM == 1 ? kSlots : 2;             // (two row tiles: room for one from every thread)
-    constexpr int kBufBytes = (kRows + kTile) * kPitch8 + (kSaSlots * kRows + kSlots * kTile) * 4;
+    constexpr int kBufBytes = (kRows + kTile) * kPitch + (kSaSlots * kRows + kSlots * kTile) * 4;
     constexpr int TN = 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
@@ -405,15 +408,15 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     // codes: thread -> (row t/4 of every 128, 16-byte piece t%4). weights: thread -> (column t/4, 8-byte quarter t%4 of the step).
     const int prow = t >> 2, quarter = t & 3;
     const uint32_t a_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.padded_k) + static_cast<uint32_t>(quarter * 16);
-    const uint32_t a_loff = swizzled(static_cast<uint32_t>(prow), static_cast<uint32_t>(quarter));
+    const uint32_t a_loff = piece_at<kPitch>(static_cast<uint32_t>(prow), static_cast<uint32_t>(quarter));
     const uint32_t b_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(quarter * 8);
-    const uint32_t b_loff = kRows * kPitch8 + a_loff;
+    const uint32_t b_loff = kRows * kPitch + a_loff;
     const uint32_t s_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.kb) * kScaleBytes;
     const uint32_t z_goff = static_cast<uint32_t>(prow) * static_cast<uint32_t>(p.zp_row);
     // activation scales: thread -> (slot t/rows, row t%rows)
     const int sa_slot = TM == 1 ? t >> 7 : wave >> 2, sa_row = t & (kRows - 1);
     const uint32_t sa_goff = (sa_slot < kSlots && m_base + sa_row < p.m) ? static_cast<uint32_t>(m_base + sa_row) * 4u : kOutOfRange;
-    constexpr int kSaOff = (kRows + kTile) * kPitch8;           // [kSaSlots][rows] f32 activation scales of the step
+    constexpr int kSaOff = (kRows + kTile) * kPitch;           // [kSaSlots][rows] f32 activation scales of the step
     constexpr int kSbOff = kSaOff + kSaSlots * kRows * 4;       // [kSlots][128] f32 weight scales of the step
 
     // PROBE: this lane's first accumulator element, (row m_base + wm * 32 + 4 (lane / 32), column n_base + wn * 64 + lane % 32),
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     const __amdgpu_buffer_rsrc_t srd_probe = make_srd(PROBE ? p.acc_probe : nullptr, PROBE ? static_cast<uint64_t>(p.m * p.n * p.kb) * 4 : 0);
 
     // MFMA operand reads: lane (r = lane % 32, h = lane / 32) reads 16 consecutive codes of row r.
-    const uint32_t frag_off[2] = {swizzled(lane & 31, lane >> 5), swizzled(lane & 31, 2 + (lane >> 5))};
+    const uint32_t frag_off[2] = {piece_at<kPitch>(lane & 31, lane >> 5), piece_at<kPitch>(lane & 31, 2 + (lane >> 5))};
 
     int16_t_v acc[TM][NBS == 0 ? TN : 1];   // integer accumulators that outlive a step (block size >= 128 only)
     float y[TM][TN][16];
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
         *reinterpret_cast<uint2*>(base + b_loff + part * 8) = make_uint2(lo, hi);
         if (part == 0) {
 #pragma unroll
-            for (int m = 0; m < TM; ++m) *reinterpret_cast<uint4*>(base + a_loff + m * kTile * kPitch8) = r.a[m];
+            for (int m = 0; m < TM; ++m) *reinterpret_cast<uint4*>(base + a_loff + m * kTile * kPitch) = r.a[m];
         } else {
             if constexpr (TM > 1) {
                 // No branch here: around one the compiler moves whole row tiles of the arithmetic, and spills. Threads of one column and
@@ -545,8 +548,8 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
     };
     auto compute = [&](int buf, int kt_in_slice, const Regs& next, bool store_next) {
         const int kt = kt_base + kt_in_slice;
-        const unsigned char* la = smem + buf * kBufBytes + wm * (TM * 32 * kPitch8);
-        const unsigned char* lb = smem + buf * kBufBytes + kRows * kPitch8 + wn * (64 * kPitch8);
+        const unsigned char* la = smem + buf * kBufBytes + wm * (TM * 32 * kPitch);
+        const unsigned char* lb = smem + buf * kBufBytes + kRows * kPitch + wn * (64 * kPitch);
         u32x4_t fa[2], fb[2][TN];
         const int16_t_v zero = {};
         // what of the next step's bytes goes to LDS between the pieces of arithmetic: halves, behind the first row tile's
@@ -558,10 +561,10 @@ __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
             if (TM > 1 && m > 0) __builtin_amdgcn_sched_barrier(0);      // mixed with the row tile before, the operands do not fit 256 registers
 #pragma unroll
             for (int kk = 0; kk < 2; ++kk) {
-                fa[kk] = *reinterpret_cast<const u32x4_t*>(la + m * 32 * kPitch8 + frag_off[kk]);
+                fa[kk] = *reinterpret_cast<const u32x4_t*>(la + m * 32 * kPitch + frag_off[kk]);
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    if (m == 0) fb[kk][j] = *reinterpret_cast<const u32x4_t*>(lb + j * 32 * kPitch8 + frag_off[kk]);
+                    if (m == 0) fb[kk][j] = *reinterpret_cast<const u32x4_t*>(lb + j * 32 * kPitch + frag_off[kk]);
             }
             if constexpr (NBS == 1) {
                 // One block per step: the integer accumulators live only from the MFMAs to the flush.
@@ -744,7 +747,7 @@ static int launch_acc4_prefill_cfg(Acc4PrefillParams p, int slices, hipStream_t 
     p.full_rows = acc4_full_rows(p.m, p.n, p.row_bytes, 1 << p.bs_log2, TM == 2, rocm_ffi_compute_units());
     const dim3 grid(static_cast<unsigned>((p.n + kTile - 1) / kTile), static_cast<unsigned>((p.m + TM * kTile - 1) / (TM * kTile)), static_cast<unsigned>(slices));
     constexpr int kSlots = NBS == 2 ? 2 : 1;
-    const size_t lds = 2 * ((TM + 1) * kTile * kPitch8 + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
+    const size_t lds = 2 * ((TM + 1) * kTile * kPitch8<NBS, TM, D> + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
     auto kernel = acc4_prefill_kernel<NBS, SF32, TM, D, PROBE>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));

@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (130, 1920, 128, 128, 1),       # 15 x 2
     (100, 1200, 2048, 64, 4),       # 10 x 1 over slices of K
     (400, 700, 4096, 128, 8),       # 6 x 4
+    (520, 8200, 192, 64, 1),        # 65 x 5: two workgroups on a CU, padded rows in LDS
 ])
 def test_every_tile_once(ep, port, m, n, k, bs, slices):
     got = C.c_int()
