@@ -747,13 +747,9 @@ static int launch_acc4_prefill_cfg(Acc4PrefillParams p, int slices, hipStream_t 
     p.full_rows = acc4_full_rows(p.m, p.n, p.row_bytes, 1 << p.bs_log2, TM == 2, rocm_ffi_compute_units());
     const dim3 grid(static_cast<unsigned>((p.n + kTile - 1) / kTile), static_cast<unsigned>((p.m + TM * kTile - 1) / (TM * kTile)), static_cast<unsigned>(slices));
     constexpr int kSlots = NBS == 2 ? 2 : 1;
-    const size_t lds = 2 * ((TM + 1) * kTile * kPitch8<NBS, TM, D> + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
-    auto kernel = acc4_prefill_kernel<NBS, SF32, TM, D, PROBE>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return static_cast<int>(e);
-    }
-    hipLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, p);
+    constexpr int kLds = 2 * ((TM + 1) * kTile * kPitch8<NBS, TM, D> + ((TM == 1 ? kSlots : 2) * TM + kSlots) * kTile * 4);
+    static_assert(kLds <= 65536);            // what a launch may ask for without an attribute of the kernel
+    hipLaunchKernelGGL((acc4_prefill_kernel<NBS, SF32, TM, D, PROBE>), grid, dim3(512), kLds, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
