@@ -47,7 +47,11 @@ def test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, bias
         assert helpers.rel_l2(got[row], want[row]) <= tol, row
 
 
-@pytest.mark.parametrize("m,n,k", [(20, 128, 96), (70, 1100, 96), (600, 1100, 96)])      # the three tile shapes
+# the three tile shapes; K a whole number of blocks in one wave, K that ends inside a block, and both split over the waves of a workgroup
+SPECIAL = [(20, 128, 96), (70, 1100, 96), (600, 1100, 96), (20, 128, 100), (70, 1100, 100), (600, 1100, 100), (20, 128, 896), (70, 1100, 896), (600, 1100, 900)]
+
+
+@pytest.mark.parametrize("m,n,k", SPECIAL)
 def test_infinities_nan_and_the_largest_values(ep, port, m, n, k):
     """An infinite activation gives what its products give (NaN only over a weight of zero or against the other infinity), one near the
     end of the range a finite result, and no other row notices."""
@@ -82,7 +86,7 @@ def test_activations_of_more_than_two_gib(ep, port):
     assert all(np.array_equal(block, blocks[0]) for block in blocks[1:])
 
 
-@pytest.mark.parametrize("m,n,k", [(20, 128, 96), (70, 1100, 96), (600, 1100, 96)])
+@pytest.mark.parametrize("m,n,k", SPECIAL)
 def test_the_smallest_values(ep, port, m, n, k):
     """Rows of tiny activations, down to subnormal ones, keep their 24 bits - alone, and beside rows whose infinities or largest values send a wave round again."""
     b, s, zp = synth.make_weights(n, k, 32, n, zero_points=True, scale_lo=8.0, scale_hi=16.0, scale_dtype=E.F32)
@@ -114,3 +118,36 @@ def test_the_smallest_values(ep, port, m, n, k):
 def test_whole_blocks(ep, port, s_dt, bs, zero_points, m, n, k):
     """K a whole number of blocks: rows pass through LDS. Rows and shares of K at the edges of tiles."""
     test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, "none", E.F32)
+
+
+@pytest.mark.parametrize("s_dt,bs,zero_points,m,n,k", [
+    (E.BF16, 32, True, 200, 900, 900),     # 32 x 32 tiles
+    (E.F16, 64, False, 100, 1100, 836),    # ... fewer runs in the last block than in the others
+    (E.F16, 32, True, 513, 2017, 164),     # two column tiles a wave
+    (E.BF16, 128, False, 545, 1100, 1028),
+])
+def test_partial_last_blocks_under_16_bit_scales(ep, port, s_dt, bs, zero_points, m, n, k):
+    test_matches_double_precision(ep, port, s_dt, bs, zero_points, m, n, k, "none", E.F32)
+
+
+@pytest.mark.parametrize("k", [896, 900])
+@pytest.mark.parametrize("m,n", [(20, 128), (70, 1100), (600, 1100)])
+def test_one_waves_share_is_walked_again(ep, port, m, n, k):
+    """Infinities and tiny rows in one wave's share of K: that wave goes round again while the others wait for its sums."""
+    b, s, zp = synth.make_weights(n, k, 32, n, zero_points=True, scale_lo=8.0, scale_hi=16.0, scale_dtype=E.F32)
+    a = synth.make_activation(m, k, n, E.F32)
+    w = port.dequantize_nk_bits(b, s, zp, n, k, 32, 4).astype(np.float64)
+    for start in (0, 448, k - 36):                          # the first wave's share, one in the middle, the last one's
+        x = a.copy()
+        x[1] = x[3] = 0.0
+        x[1, start:start + 32] = (a[1, :32].astype(np.float64) * 2.0 ** -118).astype(np.float32)
+        x[3, start + 4:start + 36] = (a[3, :32].astype(np.float64) * 2.0 ** -126).astype(np.float32)
+        for infinite in (False, True):
+            if infinite:
+                x[2, start + 9] = np.inf
+            y, variant = E.matmul_nbits(ep, x, E.F32, b, s, E.F32, zp, n, k, 32, y_dtype=E.F32)
+            assert variant == "gemm_f32_mfma"
+            for row in (0, 1, 3, 4, m - 1):
+                assert helpers.rel_l2(y[row].astype(np.float64) * 2.0 ** 120, (x[row].astype(np.float64) * w).sum(axis=1) * 2.0 ** 120) <= TOL, (start, infinite, row)
+        with np.errstate(invalid="ignore"):
+            assert np.array_equal(y[2].astype(np.float64), (x[2].astype(np.float64) * w).sum(axis=1), equal_nan=True), start
