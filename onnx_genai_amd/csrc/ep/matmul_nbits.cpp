@@ -572,7 +572,7 @@ bool stream_sorted(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, boo
 }
 
 // Narrower f32 calls than this (routers of experts, low-rank adapters) keep the streaming kernel and, from 65 rows, the catch-all. Not for speed: 896 -> 64
-// at 5 / 64 / 200 rows takes 9.4 / 96 / 470 us on them and 5.2 / 5.8 / 5.8 on the matrix cores. The parity tests of those widths name these kernels.
+// at 5 / 64 / 200 rows takes 10 / 96 / 467 us on them and 5.7 / 5.9 / 6.0 on the matrix cores. The parity tests of those widths name these kernels.
 constexpr int64_t kGemmF32MinCols = 128;
 
 // The RMS-normalization prologue of a node on its way through the dispatch: the decode kernels over the repacked stream

@@ -334,12 +334,16 @@ struct Acc4PrefillParams {
 constexpr int kTile = 128;           // rows and columns of Y per workgroup
 constexpr int kStep = 64;            // codes of K per step
 // LDS rows of 64 codes are 64 bytes apart: the 16-byte piece `piece` of row `row` lies at piece ^ (row / 4 % 4), so that 16 rows' pieces of one place and
-// four rows' whole pieces (a read of an MFMA operand, and a write) both cover all 64 banks. With rows of 80 bytes instead the writes met in a bank - a quarter of the
-// cycles that LDS was busy, itself 27 % of the kernel's (22 % now). 4096 rows, block 64, 8192 -> 57344 and 28672 -> 8192, in launch order: 4362 -> 4275, 2139 -> 2088 us;
-// 648 shapes and heights + 0.8 % in the mean. Not the 128 x 128 build of block size 64 with two register sets, which keeps 80 bytes: 64 cost it 2 % up to 128 rows
-// (3584 -> 37888 at 40 rows 73.9 and 75.5 us), 0.4 % in the mean of 377 shapes and heights.
+// four rows' whole pieces (a read of an MFMA operand, and a write) both cover all 64 banks. With rows of 80 bytes instead the writes met in a bank - a
+// quarter of the cycles that LDS was busy, itself 27 % of the kernel's (22 % now). 4096 rows, block 64, 8192 -> 57344 and 28672 -> 8192, in launch order:
+// 4362 -> 4275, 2139 -> 2088 us; 648 shapes and heights + 0.8 % in the mean. Not the 128 x 128 build of block size 64 with two register sets, which keeps
+// 80 bytes: 64 cost it 2 % up to 128 rows (3584 -> 37888 at 40 rows 73.9 and 75.5 us), 0.4 % in the mean of 377 shapes and heights.
 template <int NBS, int TM, int D> constexpr int kPitch8 = NBS == 1 && TM == 1 && D == 2 ? 80 : 64;
-template <int PITCH> __device__ __forceinline__ uint32_t piece_at(uint32_t row, uint32_t piece) { return row * PITCH + (PITCH == 64 ? piece ^ ((row >> 2) & 3u) : piece) * 16u; }
+template <int PITCH>
+__device__ __forceinline__ uint32_t piece_at(uint32_t row, uint32_t piece)
+{
+    return row * PITCH + (PITCH == 64 ? piece ^ ((row >> 2) & 3u) : piece) * 16u;
+}
 
 // The tile of Y that workgroup (x, y) of a (columns x rows x slices) grid takes. Workgroups go to the eight XCDs in turn, and each XCD has an L2 of
 // its own. In launch order (full = 0) an XCD has every eighth column block; otherwise it takes one run of tiles, which goes down kTileRows row blocks before
@@ -370,8 +374,8 @@ __host__ __device__ __forceinline__ TileAt acc4_tile(uint32_t x, uint32_t y, uin
 // TM = 2: 64 x 64 per wave, 256 x 128 per workgroup, two waves per SIMD of up to 256 registers: a weight is unpacked and an operand of B read
 // from LDS for twice the rows, one tile's MFMAs run under the other's flush inside a wave, and the registers hold three steps of
 // loads in flight (the two-set form of TM = 1 waits for memory: with two sets TM = 2 was level with it, 4970 us against 4266 with four on 8192 -> 57344 at
-// 4096 rows, block 64; 128 x 128 tiles 5494). Same sums in the same order, bit for bit. 8192 -> 57344 at 4096 rows: 0.70 -> 0.90 POP/s (0.96 with the
-// order of tiles above and LDS rows without padding).
+// 4096 rows, block 64; 128 x 128 tiles 5494). Same sums in the same order, bit for bit. 8192 -> 57344 at 4096 rows: 0.70 -> 0.90 POP/s (0.95, the
+// quantizer's time included, with the order of tiles above and LDS rows without padding).
 // PROBE: every int32 tile that is flushed is also stored to p.acc_probe ([M, N, kb]); the same code otherwise.
 template <int NBS, bool SF32, int TM, int D, bool PROBE>
 __global__ __launch_bounds__(512) void acc4_prefill_kernel(Acc4PrefillParams p)
@@ -721,16 +725,17 @@ static bool acc4_tall_tiles(int64_t m, int64_t n, int64_t padded_k, int block_si
 }
 
 // acc4_tile's `full` of a call, 0 for launch order. Runs of tiles pay (us, launch order and runs; f16, zero points):
-//   * where a CU holds one workgroup and the grid takes more than a round (256 x 128 tiles, `tall`, and block size 32). 32 CUs then work on a patch of 4 x 8
-//     tiles, which at 256 x 128 asks the memory behind their L2 for 96 KB a step, against 96 - 160 for every eighth of a row of column blocks: at 4096
-//     rows, block 64, 8192 -> 57344 misses L2 75 M and 24 M times (4275 and 4057 us), 28672 -> 8192 12 M times either way (2088 and 2058). Block 32, 8192 -> 57344,
-//     4096 rows 7059 and 6629. Over 400 shapes and heights of these two kinds 0 to + 9 % but for 1 % here and there.
-//   * on wide grids whose rows of B lie a multiple of 4096 bytes apart, at any height. Block 64, 8192 -> 57344 at 17 / 300 / 600 rows 176 and 153, 551 and 491, 916 and 791;
-//     -> 32768 at 300 rows 341 and 279; -> 16384 at 17 and 300 rows 54.8 and 49.8, 169 and 161; -> 10240 at 600 rows 168 and 170, so from 128 column
-//     blocks. It is the distance: K = 8448 instead of 8192 takes 289 and 284 us at 300 rows -> 32768. Half of it, on grids wider still: 4096 -> 65536 at 64 / 300 rows
-//     95 and 87, 275 and 258; -> 32768 at 300 rows 146 and 148.
-// Two workgroups share a CU in the other calls, and which two, and which come last, matters more than what they share: runs are level with launch order to 4 % slower
-// there (4096 -> 6144, block 64, 1300 rows 144 and 146; 3584 -> 4608, block 128, 385 rows 4 %). (The f16 / bf16 tiles of prefill_mfma.hip
+//   * where a CU holds one workgroup and the grid takes more than a round (256 x 128 tiles, `tall`, and block size 32). 32 CUs then work on a patch of
+//     4 x 8 tiles, which at 256 x 128 asks the memory behind their L2 for 96 KB a step, against 96 - 160 for every eighth of a row of column blocks: at
+//     4096 rows, block 64, 8192 -> 57344 misses L2 75 M and 24 M times (4275 and 4057 us), 28672 -> 8192 12 M times either way (2088 and 2058). Block 32,
+//     8192 -> 57344, 4096 rows 7059 and 6629. Of 949 shapes and heights of these two kinds
+//     (+ 0.9 % in the mean, up to 9) 18 are 1 - 3 % worse.
+//   * on wide grids whose rows of B lie a multiple of 4096 bytes apart, at any height. Block 64, 8192 -> 57344 at 17 / 300 / 600 rows 176 and 153, 551 and
+//     491, 916 and 791; -> 32768 at 300 rows 341 and 279; -> 16384 at 17 and 300 rows 54.8 and 49.8, 169 and 161; -> 10240 at 600 rows 168 and 170, so from
+//     128 column blocks. It is the distance: K = 8448 instead of 8192 takes 289 and 284 us at 300 rows -> 32768. Half of it, on grids wider still: 4096 -> 65536
+//     at 64 / 300 rows 95 and 87, 275 and 258; -> 32768 at 300 rows 146 and 148.
+// Two workgroups share a CU in the other calls, and which two, and which come last, matters more than what they share: runs are level with launch order to
+// 4 % slower there (4096 -> 6144, block 64, 1300 rows 144 and 146; 3584 -> 4608, block 128, 385 rows 4 %). (The f16 / bf16 tiles of prefill_mfma.hip
 // ran level with runs, 0.994 - 1.001 of the time, and keep launch order.)
 static int acc4_full_rows(int64_t m, int64_t n, int64_t row_bytes, int block_size, bool tall, int64_t cus)
 {
@@ -813,7 +818,8 @@ extern "C" int rocm_acc4_mfma_tile(const RocmMatMulNBitsArgs* a, int compute_uni
     if (workgroup < 0 || workgroup >= columns * rows) return -1;
     const int64_t row_bytes = (a->k + a->block_size - 1) / a->block_size * a->block_size / 2;
     const int full = mnb::acc4_full_rows(a->m, a->n, row_bytes, a->block_size, height > mnb::kTile, compute_units);
-    const mnb::TileAt at = mnb::acc4_tile(static_cast<uint32_t>(workgroup % columns), static_cast<uint32_t>(workgroup / columns), static_cast<uint32_t>(columns), static_cast<uint32_t>(full));
+    const mnb::TileAt at = mnb::acc4_tile(static_cast<uint32_t>(workgroup % columns), static_cast<uint32_t>(workgroup / columns), static_cast<uint32_t>(columns),
+                                          static_cast<uint32_t>(full));
     *row = at.row;
     *col = at.col;
     return 0;

@@ -7,15 +7,16 @@
 // over a run of 32 weights of one block, with products that are exact and sums in f32: the reference's fp32 route
 // (matmul_nbits.rs:7499-7566), three MFMAs where the f32 form of the instruction would take sixteen times the cycles of one.
 //
-// A wave works alone on its share of K, the next run's loads in flight, and no barrier until the waves of a workgroup, which split K
-// between them, add up their sums in wave order at the end. Short grids get their parallelism from that split.
-// What bounds it is a CU's vector memory path, which serves a load one cache line at a time: an operand lane that loads its own row's
-// activations asks for 32 lines with every load, 128 times a run. So where K is a whole number of blocks (WHOLE) eight lanes load one row's 128
+// A wave works alone on its share of K, the next loads in flight (one run ahead on 32 x 32 tiles, three on 16 x 16), and no barrier until the waves of a
+// workgroup, which split K between them, add up their sums in wave order at the end. Short grids get their parallelism from that split.
+// What bounds it is a CU's vector memory path, which serves a load one cache line at a time: on 32 x 32 tiles, operand lanes that load their own rows'
+// activations ask for 32 lines with each of a run's four loads. So where K is a whole number of blocks (WHOLE) eight lanes load one row's 128
 // bytes of a run, eight lines a load, and the wave turns them round through LDS of its own (no bank conflicts). The weights' loads (16 bytes of 32
 // columns) are left as they are.
-// Measured, whole calls in a row, block 32, f32 scales, lanes loading rows of their own before: 896 -> 4864 at 200 rows 27.5 -> 23.8 us,
-// 4864 -> 896 at 200 rows 35.2 -> 24.7; a 0.5B layer at 100 / 200 / 512 rows 101 -> 83, 115 -> 96, 164 -> 142. (Offsets and nibbles worked out in a
-// quarter fewer instructions gave 1 % of that; a third or fourth run in flight costs registers and 8 - 12 %.) The catch-all took 1665 and 2219 us for the first two.
+// Measured, block 32, f32 scales, lanes loading rows of their own before: as nodes of a recorded graph, 896 -> 4864 at 200 rows 24.4 -> 21.1 us,
+// 4864 -> 896 at 200 rows 33.2 -> 22.6; a 0.5B layer's nodes called in a row at 100 / 200 / 512 rows 98 -> 80, 111 -> 90, 164 -> 136. (Offsets and nibbles worked
+// out in a quarter fewer instructions gave 1 % of that; a third or fourth run in flight costs registers and 8 - 12 %.) The catch-all took 1665 and 2219 us for
+// the first two. Where K ends inside a block the other build gains 1 % in the mean by the nibbles, and loses up to 3 % where K is a few runs.
 #include <type_traits>
 
 #include "prefill_common.hiph"
@@ -141,7 +142,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     auto request = [&](Run& x, int u) {
         const bool live = u < u1;
         if constexpr (WHOLE) {
-            // (a run past the wave's share: its last one again, with scales of zero)
+            // (A run past the wave's share: its last one again, with scales of zero. Offsets out of range for all its loads, as below, take 2 - 5 % off 16 x 16
+            // tiles (3584 -> 3584 at 16 rows 13.9 and 13.4 us) and add up to 3 % to 32 x 32 ones (4864 -> 896, block 128, 200 rows 20.3 and 20.8).)
             const int at = min(u, u1 - 1);
             const uint32_t blk = static_cast<uint32_t>(at * 32) >> p.bs_log2, oor = live ? 0u : kOutOfRange;
 #pragma unroll
@@ -316,12 +318,14 @@ extern "C" int rocm_gemm_f32_eligible(const RocmMatMulNBitsArgs* a)
 
 namespace {
 
-// Tiles, and waves that share K, by the grid they make (f32 scales, block 32; us):
-//   * 16 x 16 tiles while they make at most one workgroup per CU: 896 -> 896 at 64 rows 5.8 against 7.8 with 32 x 32, 4864 -> 896
-//     at 64 rows 21 against 31; with more of them they lose (896 -> 896 at 200 rows 12.9 against 7.9).
+// Tiles, and waves that share K, by the grid they make (f32 scales, block 32; us, nodes of a recorded graph):
+//   * 16 x 16 tiles while they make at most one workgroup per CU: 896 -> 896 at 64 rows 6.3 against 7.0 with 32 x 32, 4864 -> 896
+//     at 64 rows 17.4 against 19.3; with more of them they lose (896 -> 896 at 200 rows 12.1 against 7.3).
 //   * 32 x 32 otherwise, two of them per wave once single ones make more than one workgroup per CU: the cut activations are used
-//     twice (4864 -> 896 at 512 rows 47.5 against 61.7; at 200 rows, 196 workgroups, 46 against 33).
-//   * eight waves share K up to one workgroup per CU, four beyond (896 -> 9728 at 512 rows 69 against 91 us), each with two runs or more.
+//     twice (4864 -> 896 at 512 rows 39.5 against 44.3; at 200 rows, 196 workgroups, 35.3 against 23.4).
+//   * eight waves share K up to one workgroup per CU, four beyond (896 -> 9728 at 512 rows 62.5 against 80.5 us), each with two runs or more.
+// The lines were drawn before activations went through LDS and hold at these shapes; between them single tiles of eight waves can be the better ones
+// (896 -> 4864 at 200 rows, 1064 of them, 19.6 against 21.1).
 struct F32Plan { int tile, cn, waves; };
 F32Plan plan_gemm_f32(const RocmMatMulNBitsArgs* a, int units, int64_t cus)
 {
@@ -336,8 +340,9 @@ F32Plan plan_gemm_f32(const RocmMatMulNBitsArgs* a, int units, int64_t cus)
 
 }  // namespace
 
-// From five rows; up to eight rows only on grids of at most two workgroups per CU (3584 -> 18944 at eight rows: two passes of the
-// streaming kernel 41 us, 47 here; 896 -> 9728 at five rows: 13.1 against 9.3 us).
+// From five rows; up to eight rows only on grids of at most two workgroups per CU (896 -> 9728 at five rows: 9.1 against 12.9 us in two passes of the
+// streaming kernel). Beyond that, five rows of a long K are the streaming kernel's (3584 -> 18944 43.6 against 45.3 us). Six to eight are not since activations go
+// through LDS (eight rows 56 against 44), nor is a K of 896 (-> 151936 at five rows 95 against 53): the line is older.
 extern "C" int rocm_gemm_f32_pays(const RocmMatMulNBitsArgs* a)
 {
     return a->m > 8 || (a->m > 4 && (a->n + 31) / 32 <= 2 * static_cast<int64_t>(rocm_ffi_compute_units()));
