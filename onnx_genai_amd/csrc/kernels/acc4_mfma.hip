@@ -727,9 +727,10 @@ static bool acc4_tall_tiles(int64_t m, int64_t n, int64_t padded_k, int block_si
 // acc4_tile's `full` of a call, 0 for launch order. Runs of tiles pay (us, launch order and runs; f16, zero points):
 //   * where a CU holds one workgroup and the grid takes more than a round (256 x 128 tiles, `tall`, and block size 32). 32 CUs then work on a patch of
 //     4 x 8 tiles, which at 256 x 128 asks the memory behind their L2 for 96 KB a step, against 96 - 160 for every eighth of a row of column blocks: at
-//     4096 rows, block 64, 8192 -> 57344 misses L2 75 M and 24 M times (4275 and 4057 us), 28672 -> 8192 12 M times either way (2088 and 2058). Block 32,
-//     8192 -> 57344, 4096 rows 7059 and 6629. Of 949 shapes and heights of these two kinds
-//     (+ 0.9 % in the mean, up to 9) 18 are 1 - 3 % worse.
+//     4096 rows, block 64, 8192 -> 57344 misses L2 75 M and 24 - 28 M times (4275 and 4057 us), 28672 -> 8192 12 M times either way (2088 and 2058). Block 32,
+//     8192 -> 57344, 4096 rows 7059 and 6629. Of 949 shapes and heights of these two kinds (+ 0.9 % in the mean, up to 9) 18 are 1 - 3 % worse.
+//     Bands of 2 / 4 / 8 row blocks (kTileRows): 28672 -> 8192 2027 / 2011 / 2051, 8192 -> 57344 4014 / 4008 / 4048, block 32 6636 / 6612 / 6631; eight
+//     shapes of 300 to 4096 rows within 0.5 % at two, up to 2 % slower at eight.
 //   * on wide grids whose rows of B lie a multiple of 4096 bytes apart, at any height. Block 64, 8192 -> 57344 at 17 / 300 / 600 rows 176 and 153, 551 and
 //     491, 916 and 791; -> 32768 at 300 rows 341 and 279; -> 16384 at 17 and 300 rows 54.8 and 49.8, 169 and 161; -> 10240 at 600 rows 168 and 170, so from
 //     128 column blocks. It is the distance: K = 8448 instead of 8192 takes 289 and 284 us at 300 rows -> 32768. Half of it, on grids wider still: 4096 -> 65536

@@ -79,14 +79,15 @@ def test_acc4_calls_that_take_the_taller_tiles(lib):
     # block size 32 and 256 x 128 tiles: runs of tiles
     (777, 4864, 896, 32, 128, True),             # 266 tiles of 128 x 128, nine rows in the last row block
     (130, 37888, 3584, 32, 128, True),           # two rows in the last of two row blocks
-    (1200, 12763, 4096, 64, 256, True),     # 5 x 100: a band of four whole row blocks, and one of 176 rows
-    (2304, 7040, 4096, 64, 256, True),      # 9 x 55: bands of four, four and one row block
-    (385, 16384, 64, 64, 256, True),        # one whole row block and one of 129 rows
+    (1200, 12763, 4096, 64, 256, True),          # 5 x 100: a band of four whole row blocks, and one of 176 rows
+    (2304, 7040, 4096, 64, 256, True),           # 9 x 55: bands of four, four and one row block
+    (385, 16384, 64, 64, 256, True),             # one whole row block and one of 129 rows
     (60, 37888, 3584, 32, 128, True),            # one row block, not whole
     # wide grids whose rows of B are a multiple of 4096 (2048) bytes apart
     (300, 57300, 8192, 64, 128, True), (17, 16384, 16384, 128, 128, True), (100, 45056, 4096, 64, 128, True),
     # the others keep launch order
-    (777, 4864, 896, 64, 128, False), (1300, 6144, 4096, 64, 128, False), (600, 10240, 8192, 64, 128, False), (300, 32768, 4096, 64, 128, False), (300, 32768, 8448, 64, 128, False), (130, 4608, 3584, 128, 128, False),
+    (777, 4864, 896, 64, 128, False), (1300, 6144, 4096, 64, 128, False), (600, 10240, 8192, 64, 128, False), (300, 32768, 4096, 64, 128, False),
+    (300, 32768, 8448, 64, 128, False), (130, 4608, 3584, 128, 128, False),
 ])
 def test_acc4_tiles_are_handed_out_once_and_partial_rows_last(lib, m, n, k, bs, height, runs):
     """accuracy_level 4, tall calls: workgroups to tiles is one-to-one, and the tiles of a last row block that is not whole come behind all others."""
