@@ -103,25 +103,27 @@ __global__ __launch_bounds__(256) void pack_decode_kernel(PackParams p)
 
 typedef __attribute__((ext_vector_type(4))) int int4p_t;
 
-struct Acc4PackedParams {
-    const int8_t* qa;       // [m, padded_k] codes, packed order
-    const float* aq;        // one row: [kb, 2] = scale_a, f32(sum of codes)
-    const float* aux16;     // 2 .. 16 rows: [kb, 16, 2], the same pairs block-major
-    int64_t m;
-    const void* a;          // FUSE: the one row itself, f16 or bf16 [k]; every wave quantizes the groups it multiplies
-    int64_t k;
-    int rounding;           // FUSE: 0 = ties to even, 1 = ties away from zero
-    const uint8_t* packed;
+// Arguments that the kernel needs only behind its first loads.
+struct Acc4PackedRest {
     const void* bias;
     void* y;
-    int64_t n, kb;
-    int64_t padded_k;
-    int64_t cg_stride;
-    int groups, groups_per_wave, chunk_bytes;
     int bias_dtype, y_dtype;
+    int rounding;           // FUSE: 0 = ties to even, 1 = ties away from zero
     int scales_bf16;
     int32_t* acc_probe;     // PROBE builds: int32 [M, N, kb] block accumulators, as flushed
 };
+// (fourteen dwords of plain arguments in front, as in PackedParams)
+struct Acc4PackedParams {
+    const void* rows;       // [m, padded_k] codes, packed order; FUSE: the rows themselves, f16 or bf16 [m, k], which every wave quantizes for the groups it multiplies
+    const float* pairs;     // one row: [kb, 2] = scale_a, f32(sum of codes); 2 .. 16 rows: [kb, 16, 2], the same pairs block-major; FUSE: not read
+    const uint8_t* packed;
+    int m, n, k, kb;
+    int padded_k;
+    int groups, groups_per_wave, waves;
+    Acc4PackedRest rest;
+};
+#define MNB_ACC4_ARGS const void *rows, const float *pairs, const uint8_t *packed, int m, int n, int k, int kb, int padded_k, int groups, int groups_per_wave, int waves_, Acc4PackedRest rest
+#define MNB_ACC4_PARAMS Acc4PackedParams{rows, pairs, packed, m, n, k, kb, padded_k, groups, groups_per_wave, waves_, rest}
 
 constexpr int kCodePitchP = 144;   // bytes between the rows of one tile of codes in LDS: 128 + 16
 
@@ -152,9 +154,13 @@ struct Bf16Scale {
     uint16_t bits;
 };
 
+// (waves_per_eu: builds that the compiler, left alone, gives a few registers more than fit that many waves)
 template <int BS, typename ST, int SETS, int FUSE, bool PROBE, int MR = 1>
-__global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
+__global__ __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(PROBE ? 1 : MR == 8 && BS == (sizeof(ST) == 4 ? 128 : 64) ? 8 : BS == 128 && sizeof(ST) == 2 && MR == 16 ? 7 : BS == 128 && sizeof(ST) == 2 && MR == 4 && FUSE != 0 ? 6 : 1)))
+void acc4_packed_kernel(MNB_ACC4_ARGS)
 {
+    const Acc4PackedParams p = MNB_ACC4_PARAMS;
     static_assert(MR == 1 || ((MR == 4 || MR == 8 || MR == 16) && (FUSE == 0 || MR == 4) && SETS == 1),
                   "several rows: one register set; codes from the workspace, or up to four rows quantized here");
     constexpr int U = kGroupTiles;
@@ -172,15 +178,17 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int waves = blockDim.x >> 6;
+    const int waves = p.waves;
     const int c = lane & 15;
     const int g = lane >> 4;
     const int64_t n_base = static_cast<int64_t>(blockIdx.x) * 16;
-    const bool bf16_scales = std::is_same<ST, Bf16Scale>::value || (MR == 1 && p.scales_bf16 != 0);
+    const bool bf16_scales = std::is_same<ST, Bf16Scale>::value || (MR == 1 && p.rest.scales_bf16 != 0);
 
-    const __amdgpu_buffer_rsrc_t srd_p = make_srd(p.packed + static_cast<int64_t>(blockIdx.x) * p.cg_stride, static_cast<uint64_t>(p.cg_stride));
-    const __amdgpu_buffer_rsrc_t srd_a = FUSE ? make_srd(p.a, static_cast<uint64_t>(p.m * p.k) * 2) : make_srd(p.qa, static_cast<uint64_t>(p.m * p.padded_k));
-    const __amdgpu_buffer_rsrc_t srd_x = MR == 1 ? make_srd(p.aq, FUSE ? 0 : static_cast<uint64_t>(p.kb) * 8) : make_srd(p.aux16, static_cast<uint64_t>(p.kb) * 128);
+    constexpr int kChunkBytes = kChunkWeights + 16 * R;
+    const uint32_t cg_stride = static_cast<uint32_t>(p.groups) * static_cast<uint32_t>(kChunkBytes);      // bytes of one column group
+    const __amdgpu_buffer_rsrc_t srd_p = make_srd(p.packed + static_cast<uint64_t>(blockIdx.x) * cg_stride, cg_stride);
+    const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.rows, static_cast<uint64_t>(p.m) * static_cast<uint64_t>(FUSE ? 2 * static_cast<int64_t>(p.k) : p.padded_k));
+    const __amdgpu_buffer_rsrc_t srd_x = make_srd(p.pairs, MR == 1 && FUSE ? 0 : static_cast<uint64_t>(p.kb) * (MR == 1 ? 8 : 128));
     constexpr int kBlockLanes = BS / 8;
 
     const uint32_t w_off = static_cast<uint32_t>(lane * 16);
@@ -211,7 +219,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
     // past the wave's last one gets every offset out of range, fetches nothing and reads as zeros - it adds nothing.
     auto fetch_group = [&](Grp& grp, int gi) {
         const uint32_t oor = gi < g_end ? 0u : kOutOfRange;        // or-ed in: any offset with these bits is out of range
-        const uint32_t soff = static_cast<uint32_t>(gi) * static_cast<uint32_t>(p.chunk_bytes);
+        const uint32_t soff = static_cast<uint32_t>(gi) * static_cast<uint32_t>(kChunkBytes);
 #pragma unroll
         for (int u = 0; u < U; ++u) grp.w[u] = load16(srd_p, (w_off + static_cast<uint32_t>(u * 1024)) | oor, soff);
 #pragma unroll
@@ -245,6 +253,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
             grp.x[0].x = v[0];
             grp.x[0].y = v[1];
         }
+        asm volatile("" : : "s"(p.rest.bias), "s"(p.rest.y), "s"(p.rest.bias_dtype), "s"(p.rest.y_dtype));      // there from here on, not read behind the last barrier
     };
     auto compute_group = [&](const Grp& grp, int gi, int slot) {
         unsigned char* st = stage + slot * 512;
@@ -286,7 +295,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
                     sum += q[i];
                 }
             };
-            if (p.rounding == 1) round_all(std::true_type{});      // wave-uniform: one branch per group, not one select per element
+            if (p.rest.rounding == 1) round_all(std::true_type{});      // wave-uniform: one branch per group, not one select per element
             else round_all(std::false_type{});
             sum = dpp_addi<0xB1>(sum);
             sum = dpp_addi<0x4E>(sum);
@@ -382,7 +391,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
                             if constexpr (PROBE) {
                                 const int64_t blk = static_cast<int64_t>(gi) * NB + bi;
                                 const int64_t row = g * kRowsKept + r;
-                                if (row < p.m && n_base + c < p.n && blk < p.kb) p.acc_probe[(row * p.n + n_base + c) * p.kb + blk] = static_cast<int>(f);
+                                if (row < p.m && n_base + c < p.n && blk < p.kb) p.rest.acc_probe[(row * p.n + n_base + c) * p.kb + blk] = static_cast<int>(f);
                             }
                         }
                     } else {
@@ -393,7 +402,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
                         y[0] = fmaf(f, __fmul_rn(sa, sb), y[0]);
                         if constexpr (PROBE) {                                       // row 0 sits in lanes 0..15
                             const int64_t blk = static_cast<int64_t>(gi) * NB + bi;
-                            if (lane < 16 && n_base + lane < p.n && blk < p.kb) p.acc_probe[(n_base + lane) * p.kb + blk] = static_cast<int>(f);
+                            if (lane < 16 && n_base + lane < p.n && blk < p.kb) p.rest.acc_probe[(n_base + lane) * p.kb + blk] = static_cast<int>(f);
                         }
                     }
                 }
@@ -432,7 +441,7 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
 #pragma unroll
         for (int r = 0; r < kRowsKept; ++r) red[(wave * kRowsKept + r) * 64 + lane] = y[r];
         __syncthreads();
-        for (int idx = threadIdx.x; idx < kRowsKept * 64; idx += blockDim.x) {
+        for (int idx = threadIdx.x; idx < kRowsKept * 64; idx += waves * 64) {
             const int r = idx >> 6;
             const int l = idx & 63;
             const int row = (l >> 4) * kRowsKept + r;
@@ -440,8 +449,8 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
             if (row < p.m && col < p.n) {
                 float total = 0.f;
                 for (int w = 0; w < waves; ++w) total += red[(w * kRowsKept + r) * 64 + l];
-                total = with_bias(total, p.bias, p.bias_dtype, row, p.n, col, p.y_dtype);
-                store_from_f32(p.y, p.y_dtype, static_cast<int64_t>(row) * p.n + col, total);
+                total = with_bias(total, p.rest.bias, p.rest.bias_dtype, row, p.n, col, p.rest.y_dtype);
+                store_from_f32(p.rest.y, p.rest.y_dtype, static_cast<int64_t>(row) * p.n + col, total);
             }
         }
     } else {                                           // [waves][16]: row 0 lives in lanes 0..15
@@ -452,38 +461,39 @@ __global__ __launch_bounds__(512) void acc4_packed_kernel(Acc4PackedParams p)
             if (col < p.n) {
                 float total = 0.f;
                 for (int w = 0; w < waves; ++w) total += red[w * 16 + threadIdx.x];
-                total = with_bias(total, p.bias, p.bias_dtype, 0, p.n, col, p.y_dtype);       // one row
-                store_from_f32(p.y, p.y_dtype, col, total);
+                total = with_bias(total, p.rest.bias, p.rest.bias_dtype, 0, p.n, col, p.rest.y_dtype);       // one row
+                store_from_f32(p.rest.y, p.rest.y_dtype, col, total);
             }
         }
     }
 }
 
 template <int BS, typename ST>
-static int launch_acc4_packed(const Acc4PackedParams& p, int waves, bool single_set, int fuse, hipStream_t stream)
+static int launch_acc4_packed(Acc4PackedParams p, int waves, bool single_set, int fuse, hipStream_t stream)
 {
-    const unsigned grid = static_cast<unsigned>((p.n + 15) / 16);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.n) + 15) / 16);
+    p.waves = waves;
     if (p.m > 1) {
         if constexpr (std::is_same<ST, uint16_t>::value) {
-            if (p.scales_bf16) return launch_acc4_packed<BS, Bf16Scale>(p, waves, single_set, fuse, stream);
+            if (p.rest.scales_bf16) return launch_acc4_packed<BS, Bf16Scale>(p, waves, single_set, fuse, stream);
         }
         // two tiles of codes in turn + the group's pairs per wave; the reduction reuses the space (1 KiB per wave)
         const size_t lds16 = static_cast<size_t>(waves) * (2 * 16 * kCodePitchP + kGroupTiles * (128 / BS) * 128);
         if (fuse != 0) {
             // up to four f16 / bf16 rows: the kernel quantizes them itself (no codes, no pairs, no launch before this one)
-            if (p.m > 4 || p.acc_probe) return -1;
-            if (fuse == 2) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 2, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p);
-            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 1, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p);
+            if (p.m > 4 || p.rest.acc_probe) return -1;
+            if (fuse == 2) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 2, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 1, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
             return static_cast<int>(hipGetLastError());
         }
         if (p.m <= 4) {
-            if (p.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p);
-            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p);
+            if (p.rest.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 4>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
         } else if (p.m <= 8) {
-            if (p.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 8>), dim3(grid), dim3(waves * 64), lds16, stream, p);
-            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 8>), dim3(grid), dim3(waves * 64), lds16, stream, p);
-        } else if (p.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 16>), dim3(grid), dim3(waves * 64), lds16, stream, p);
-        else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 16>), dim3(grid), dim3(waves * 64), lds16, stream, p);
+            if (p.rest.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 8>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 8>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+        } else if (p.rest.acc_probe) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, true, 16>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+        else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, 0, false, 16>), dim3(grid), dim3(waves * 64), lds16, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
         return static_cast<int>(hipGetLastError());
     }
     if constexpr (std::is_same<ST, Bf16Scale>::value) {
@@ -492,11 +502,11 @@ static int launch_acc4_packed(const Acc4PackedParams& p, int waves, bool single_
     const size_t lds = static_cast<size_t>(waves) * 1024;
     auto go = [&](auto fuse) {
         constexpr int F = decltype(fuse)::value;
-        if (p.acc_probe) {
-            if (single_set) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, F, true>), dim3(grid), dim3(waves * 64), lds, stream, p);
-            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 2, F, true>), dim3(grid), dim3(waves * 64), lds, stream, p);
-        } else if (single_set) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, F, false>), dim3(grid), dim3(waves * 64), lds, stream, p);
-        else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 2, F, false>), dim3(grid), dim3(waves * 64), lds, stream, p);
+        if (p.rest.acc_probe) {
+            if (single_set) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, F, true>), dim3(grid), dim3(waves * 64), lds, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+            else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 2, F, true>), dim3(grid), dim3(waves * 64), lds, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+        } else if (single_set) hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 1, F, false>), dim3(grid), dim3(waves * 64), lds, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
+        else hipLaunchKernelGGL((acc4_packed_kernel<BS, ST, 2, F, false>), dim3(grid), dim3(waves * 64), lds, stream, p.rows, p.pairs, p.packed, p.m, p.n, p.k, p.kb, p.padded_k, p.groups, p.groups_per_wave, p.waves, p.rest);
     };
     if (fuse == 1) go(std::integral_constant<int, 1>{});
     else if (fuse == 2) go(std::integral_constant<int, 2>{});
@@ -560,7 +570,7 @@ extern "C" int rocm_decode_packed_eligible(const RocmMatMulNBitsArgs* a)
     RocmMatMulNBitsArgs base = *a;
     if (base.m > 16) base.m = 16;                         // the shared-activation kernel takes up to 64 rows
     if (!rocm_decode_mfma_eligible(&base)) return 0;
-    if (a->m * a->k * 2 >= 0x7ffffff0) return 0;
+    if (a->m * a->k * 2 >= 0x7ffffff0 || a->n > 0x7fffffff) return 0;      // (sizes are 32-bit arguments)
     if (a->m > 16 && !wide_shape(a, false)) return 0;    // up to 16 rows the split-K kernel stages the rows per wave
     return static_cast<int64_t>(mnb::packed_groups(a)) * mnb::packed_chunk_bytes(a) < 0x7fffffff;
 }
@@ -646,7 +656,7 @@ static int waves_per_simd(const RocmMatMulNBitsArgs* a, bool f32_scales)
 {
     // [f16 / bf16][rows: 1, 2-4, 5-8, 9-16][block 32, 64, 128][16-bit / f32 scales]
     static const unsigned char table[2][4][3][2] = {
-        {{{5, 6}, {7, 7}, {8, 8}}, {{5, 4}, {5, 6}, {6, 6}}, {{4, 4}, {5, 5}, {5, 5}}, {{4, 3}, {4, 4}, {3, 4}}},
+        {{{5, 6}, {8, 7}, {8, 8}}, {{5, 4}, {5, 6}, {6, 6}}, {{4, 4}, {5, 5}, {5, 5}}, {{4, 3}, {4, 4}, {3, 4}}},
         {{{7, 6}, {8, 7}, {8, 8}}, {{5, 4}, {6, 6}, {7, 6}}, {{4, 4}, {5, 5}, {5, 5}}, {{4, 3}, {4, 4}, {4, 4}}},
     };
     const int rows = a->m <= 1 ? 0 : a->m <= 4 ? 1 : a->m <= 8 ? 2 : 3;
@@ -812,18 +822,14 @@ static mnb::PackedParams packed_params(const RocmMatMulNBitsArgs* a, const void*
     mnb::PackedParams p{};
     p.a = static_cast<const uint16_t*>(a->a);
     p.packed = static_cast<const uint8_t*>(packed);
-    p.bias = a->bias;
-    p.y = a->y;
-    p.m = a->m;
-    p.n = a->n;
-    p.k = a->k;
+    p.m = static_cast<int>(a->m);
+    p.k = static_cast<int>(a->k);
+    p.n = static_cast<int>(a->n);
     p.groups = mnb::packed_groups(a);
-    p.chunk_bytes = mnb::packed_chunk_bytes(a);
-    p.cg_stride = static_cast<int64_t>(p.groups) * p.chunk_bytes;
-    p.bias_dtype = a->bias_dtype;
-    p.y_dtype = a->y_dtype;
-    p.nibble_mask = 0x000F000Fu;
-    p.magic = a->a_dtype == ROCM_DT_BF16 ? 0x43004300u : 0x64006400u;
+    p.rest.bias = a->bias;
+    p.rest.y = a->y;
+    p.rest.bias_dtype = a->bias_dtype;
+    p.rest.y_dtype = a->y_dtype;
     return p;
 }
 
@@ -835,13 +841,13 @@ static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed
     const PackedPlan plan = plan_decode_packed(a, waves, pair_member, packed_up != nullptr, cus);
     mnb::PackedParams p = packed_params(a, packed);
     p.packed_up = static_cast<const uint8_t*>(packed_up);
-    p.decomposed_silu = decomposed;
+    p.rest.decomposed_silu = decomposed;
     const bool bf16 = a->a_dtype == ROCM_DT_BF16;
     if (a->gamma) {
         if (!rocm_decode_packed_fuses_norm(a)) return probe_only ? 0 : -1;
         p.gamma = a->gamma;
-        p.gamma_f32 = a->gamma_dtype == ROCM_DT_F32;
-        p.norm_epsilon = a->norm_epsilon;
+        p.rest.gamma_f32 = a->gamma_dtype == ROCM_DT_F32;
+        p.rest.norm_epsilon = a->norm_epsilon;
     }
 
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -882,8 +888,7 @@ static int launch_decode_plain(const RocmMatMulNBitsArgs* a, const RocmMatMulNBi
     const int64_t cus = rocm_ffi_compute_units();
     const PackedPlan plan = plan_decode_packed(four, waves, false, false, cus);
     mnb::PackedParams p = packed_params(four, packed);
-    p.k = a->k;                              // what the activations have
-    p.magic = 0x64006400u;                   // both types' operands are made from f16 ones
+    p.k = static_cast<int>(a->k);            // what the activations have
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16 = a->a_dtype == ROCM_DT_BF16, f32_scales = a->scale_dtype == ROCM_DT_F32;
     if (plan.wide) {
@@ -932,7 +937,7 @@ extern "C" int rocm_acc4_packed_eligible(const RocmMatMulNBitsArgs* a)
     if (!(bs_ok && a->m >= 1 && a->m <= 16 && a->n >= 1)) return 0;
     if ((reinterpret_cast<uintptr_t>(a->b) & 15) != 0 || (reinterpret_cast<uintptr_t>(a->scales) & 3) != 0) return 0;
     const int64_t padded_k = (a->k + a->block_size - 1) / a->block_size * a->block_size;
-    if (a->m * padded_k >= 0x7fffffff) return 0;                          // the codes are addressed with 32-bit offsets
+    if (a->m * padded_k >= 0x7fffffff || a->n > 0x7fffffff) return 0;      // the codes are addressed with 32-bit offsets, sizes are 32-bit arguments
     return static_cast<int64_t>(mnb::packed_groups(a)) * mnb::packed_chunk_bytes(a) < 0x7fffffff;
 }
 
@@ -1002,27 +1007,23 @@ extern "C" int rocm_launch_acc4_packed(const RocmMatMulNBitsArgs* a, const void*
     if (!rocm_acc4_packed_eligible(a)) return -1;
     const int fuse = ws ? 0 : (a->a_dtype == ROCM_DT_BF16 ? 2 : 1);
     if (!ws && !rocm_acc4_packed_fuses_quantizer(a)) return -1;
-    mnb::Acc4PackedParams p;
-    p.qa = ws ? ws->qa : nullptr;
-    p.aq = ws ? ws->aq : nullptr;
-    p.aux16 = ws ? ws->aux : nullptr;
-    p.m = a->m;
-    p.a = a->a;
-    p.k = a->k;
-    p.rounding = rounding;
+    mnb::Acc4PackedParams p{};
+    p.rows = ws ? static_cast<const void*>(ws->qa) : a->a;
+    p.pairs = !ws ? nullptr : a->m > 1 ? ws->aux : ws->aq;
     p.packed = static_cast<const uint8_t*>(packed);
-    p.bias = a->bias;
-    p.y = a->y;
-    p.n = a->n;
-    p.kb = (a->k + a->block_size - 1) / a->block_size;
+    p.m = static_cast<int>(a->m);
+    p.n = static_cast<int>(a->n);
+    p.k = static_cast<int>(a->k);
+    p.kb = static_cast<int>((a->k + a->block_size - 1) / a->block_size);
     p.padded_k = p.kb * a->block_size;
     p.groups = mnb::packed_groups(a);
-    p.chunk_bytes = mnb::packed_chunk_bytes(a);
-    p.cg_stride = static_cast<int64_t>(p.groups) * p.chunk_bytes;
-    p.bias_dtype = a->bias_dtype;
-    p.y_dtype = a->y_dtype;
-    p.scales_bf16 = a->scale_dtype == ROCM_DT_BF16;
-    p.acc_probe = a->acc_probe;
+    p.rest.bias = a->bias;
+    p.rest.y = a->y;
+    p.rest.bias_dtype = a->bias_dtype;
+    p.rest.y_dtype = a->y_dtype;
+    p.rest.rounding = rounding;
+    p.rest.scales_bf16 = a->scale_dtype == ROCM_DT_BF16;
+    p.rest.acc_probe = a->acc_probe;
 
     int w = 0, gpw = 0;
     bool single_set = false;

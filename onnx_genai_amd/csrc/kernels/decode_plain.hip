@@ -11,39 +11,45 @@
 
 namespace mnb {
 
+// Waves per SIMD that the builds are held to: what the compiler reaches when it tries (left alone it takes a few registers more in a third of them).
+constexpr int plain_waves_per_simd(bool bf16, int bs, int rows, bool f32_scales, int bits)
+{
+    // [f16 / bf16][4 bits, 4 bits with f32 scales, 8 bits][rows: 1, 2-4, 5-8, 9-16][block 32, 64, 128]
+    constexpr unsigned char table[2][3][4][3] = {
+        {{{7, 8, 8}, {6, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{7, 7, 8}, {5, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{8, 7, 8}, {6, 7, 7}, {6, 6, 8}, {5, 6, 6}}},
+        {{{7, 8, 8}, {6, 7, 7}, {5, 5, 5}, {4, 4, 4}}, {{6, 7, 8}, {5, 6, 6}, {4, 5, 5}, {4, 4, 4}}, {{7, 8, 8}, {6, 7, 8}, {7, 6, 8}, {5, 6, 6}}},
+    };
+    return table[bf16][bits == 8 ? 2 : f32_scales ? 1 : 0][rows == 1 ? 0 : rows == 4 ? 1 : rows == 8 ? 2 : 3][bs == 32 ? 0 : bs == 64 ? 1 : 2];
+}
+
 // At most 80 scalar registers: with more, which only the rare second summation asks for, seven waves fit a SIMD instead of eight, and one workgroup of
 // fourteen a CU instead of two (8 bits, bf16, one row, 3584 -> 37888: 28.6 -> 32.7 us).
 template <bool BF16, int BS, int MR, typename ST, int BITS>
 __global__ __launch_bounds__((BS == 128 && sizeof(ST) == 2 && (MR != 16 || BF16)) ? 1024 : 512)
-__attribute__((amdgpu_num_sgpr(80)))
-void decode_plain_kernel(PackedParams p)
+__attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(plain_waves_per_simd(BF16, BS, MR, sizeof(ST) == 4, BITS))))
+void decode_plain_kernel(MNB_PACKED_ARGS)
 {
-    decode_packed_body<BF16, BS, MR, ST, 1, false, false, BITS, true>(p);
+    decode_packed_body<BF16, BS, MR, ST, 1, false, false, BITS, true>(MNB_PACKED_PARAMS);
 }
 
 // One block of rows: weights and windows both ahead (8 bits, block 128, 16 rows, 3584 -> 152064: 112 us, windows alone 120, neither 114; act-order
 // 4 bits 83 / 85 / 89); two: neither (registers).
 template <bool BF16, int BS, typename ST, int RB, int WMAX, int BITS>
 __global__ __launch_bounds__(WMAX * 64)
-void decode_plain_wide_kernel(PackedParams p)
+__attribute__((amdgpu_waves_per_eu(BF16 && BS == 128 && RB == 1 && WMAX == kWideWaves && BITS == 8 ? 6 : 1)))
+void decode_plain_wide_kernel(MNB_PACKED_ARGS)
 {
-    decode_wide_body<BF16, BS, ST, RB, false, RB == 1, RB == 1, false, WMAX, BITS, true>(p);
+    decode_wide_body<BF16, BS, ST, RB, false, RB == 1, RB == 1, false, WMAX, BITS, true>(MNB_PACKED_PARAMS);
 }
 
 template <bool BF16, int BS, int MR, typename ST, int BITS>
 static int launch_plain_mr(const PackedParams& p, int waves, hipStream_t stream)
 {
-    const unsigned grid = static_cast<unsigned>((p.n + 15) / 16);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.n) + 15) / 16);
     const size_t stage = static_cast<size_t>(waves) * 2 * (MR == 1 ? 1024 : MR * kRowPitchP);
     const size_t red = static_cast<size_t>(waves) * 1024;
     const size_t lds = stage > red ? stage : red;
-    auto kernel = decode_plain_kernel<BF16, BS, MR, ST, BITS>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return static_cast<int>(e);
-    }
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(waves * 64), lds, stream, p);
-    return static_cast<int>(hipGetLastError());
+    return launch_on(decode_plain_kernel<BF16, BS, MR, ST, BITS>, grid, waves, lds, stream, p);
 }
 
 template <bool BF16, int BS, typename ST, int BITS>
@@ -59,14 +65,8 @@ template <bool BF16, int BS, typename ST, int RB, int WMAX, int BITS>
 static int launch_plain_wide_cfg(const PackedParams& p, int waves, hipStream_t stream)
 {
     constexpr size_t lds = 2 * RB * 16 * (4 / (BITS / 4) * 256 + 16);      // two windows of the activations that four tiles of the stream meet
-    const int64_t col_groups = (p.n + 15) / 16;
-    auto kernel = decode_plain_wide_kernel<BF16, BS, ST, RB, WMAX, BITS>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return static_cast<int>(e);
-    }
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((col_groups + waves - 1) / waves)), dim3(waves * 64), lds, stream, p);
-    return static_cast<int>(hipGetLastError());
+    const int64_t col_groups = (static_cast<int64_t>(p.n) + 15) / 16;
+    return launch_on(decode_plain_wide_kernel<BF16, BS, ST, RB, WMAX, BITS>, static_cast<unsigned>((col_groups + waves - 1) / waves), waves, lds, stream, p);
 }
 
 template <bool BF16, int BS, typename ST, int BITS>
