@@ -22,6 +22,7 @@ HIP_SOURCES = [
     "kernels/gemv_f32.hip",
     "kernels/gemm_f32.hip",
     "kernels/decode_mfma.hip",
+    "kernels/packed_launch.hip",
     "kernels/decode_packed.hip",
     "kernels/decode_plain.hip",
     "kernels/prefill_mfma.hip",

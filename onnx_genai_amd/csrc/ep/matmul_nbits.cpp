@@ -482,7 +482,7 @@ bool decode_in_row_blocks(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& ar
         part.bias = rows_of_bias(args, row0);
         int pack_rc = 0;
         if (use_packed(kn, part, pack_rc)) {
-            rc = pack_rc != 0 ? pack_rc : rocm_launch_decode_packed(&part, kn.packed, kn.ep->decode_waves, kn.ep->stream);
+            rc = pack_rc != 0 ? pack_rc : rocm_launch_decode_packed(&part, kn.packed, kn.ep->decode_waves, kn.ep->stream, nullptr);
         } else {
             all_packed = false;
             rc = rocm_launch_decode_mfma(&part, kn.ep->decode_waves, kn.ep->decode_col_groups, kn.ep->stream);
@@ -898,7 +898,7 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         }
     } else if (M <= 64 && use_packed(kn, args, rc)) {
         if (rc == 0) rc = (kn.pair_member && M <= 16) ? rocm_launch_decode_packed_pair_member(&args, kn.packed, kn.ep->decode_waves, stream)
-                                                      : rocm_launch_decode_packed(&args, kn.packed, kn.ep->decode_waves, stream);
+                                                      : rocm_launch_decode_packed(&args, kn.packed, kn.ep->decode_waves, stream, kn.ep->recorded());
         kn.variant = "decode_mfma_packed";
     } else if (M <= 16 && rocm_decode_mfma_eligible(&args)) {
         rc = rocm_launch_decode_mfma(&args, kn.ep->decode_waves, kn.ep->decode_col_groups, stream);

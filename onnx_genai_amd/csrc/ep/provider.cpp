@@ -22,6 +22,7 @@ NxrtRocmEp::~NxrtRocmEp()
         if (dense) rocm_dense_gemm_destroy(dense);
         if (stream) rocm_ffi_stream_destroy(stream);
     }
+    rocm_step_tail_destroy(tail);
     g_live_providers.fetch_sub(1);
 }
 
@@ -99,6 +100,7 @@ NxrtStatus nxrt_rocm_ep_create(uint32_t device_ordinal, const char* const* keys,
         }
         ep->dense_gemm_min_rows = ep->dense_resident ? kDenseGemmMinRowsResident : 0;
         if ((it = ep->config.find("dense_gemm_min_rows")) != ep->config.end()) ep->dense_gemm_min_rows = parse_int(it->second, ep->dense_gemm_min_rows);
+        ep->tail = rocm_step_tail_create();         // (without one every node of a capture is a launch of its own)
         NxrtStatus st = ep->bind();
         if (st.code == NXRT_OK) st = hip_status(rocm_ffi_stream_create(&ep->stream), "hipStreamCreate");
         if (st.code == NXRT_OK) st = hip_status(rocm_ffi_static_scratch(static_cast<int>(ep->device), &ep->static_scratch, &ep->static_scratch_bytes), "hipGetSymbolAddress(static scratch)");
@@ -290,6 +292,7 @@ NxrtStatus nxrt_rocm_ep_capture_begin(NxrtRocmEp* ep)
         if (ep->capturing) return make_status(NXRT_INVALID_ARGUMENT, "capture_begin: a capture is already open on this provider");
         st = hip_status(rocm_ffi_capture_begin(ep->stream), "hipStreamBeginCapture");
         if (st.code == NXRT_OK) {
+            rocm_step_tail_reset(ep->tail);
             ep->capturing = true;
             ep->captures.fetch_add(1);
         }
@@ -304,6 +307,7 @@ NxrtStatus nxrt_rocm_ep_capture_end(NxrtRocmEp* ep, NxrtRocmGraph** out_graph, u
         *out_graph = nullptr;
         if (!ep->capturing) return make_status(NXRT_INVALID_ARGUMENT, "capture_end: no capture is open on this provider");
         ep->capturing = false;
+        rocm_step_tail_reset(ep->tail);
         rocm_graph_exec_t exec = nullptr;
         size_t nodes = 0;
         const int err = rocm_ffi_capture_end(ep->stream, &exec, &nodes);

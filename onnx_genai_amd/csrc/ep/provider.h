@@ -36,6 +36,7 @@ struct NxrtRocmEp {
     std::atomic<uint64_t> launches{0};
     void* static_scratch = nullptr;               // this GPU's static scratch array (device address), resolved when the provider is created
     size_t static_scratch_bytes = 0;
+    RocmStepTail* tail = nullptr;                 // the last launch of an open capture that further nodes may join
     bool capturing = false;                       // a stream capture is open: nothing may allocate or synchronise
     std::atomic<uint64_t> captures{0};            // stream captures opened on this provider so far: while 0, no HIP graph can name a buffer of its kernels
     // The host may release the provider, its kernels and its allocators in any order (each vtable is released exactly
@@ -47,6 +48,7 @@ struct NxrtRocmEp {
 
     NxrtRocmEp();
     ~NxrtRocmEp();
+    RocmStepTail* recorded() const { return capturing ? tail : nullptr; }
     NxrtStatus bind() const;                      // make this provider's GPU current on the calling thread
 };
 

@@ -164,12 +164,21 @@ int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* args, rocm_stream_t stream);
 int rocm_decode_mfma_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_decode_mfma(const RocmMatMulNBitsArgs* args, int waves, int col_groups, rocm_stream_t stream);
 
+/* The last launch that a provider recorded into the stream capture open on its stream: nodes that follow it, read the same
+ * activations and touch nothing it writes join it instead of waiting for it (kernels/packed_launch.hip). One per provider;
+ * reset when a capture opens and when it closes. create returns NULL when there is no memory for it. */
+typedef struct RocmStepTail RocmStepTail;
+RocmStepTail* rocm_step_tail_create(void);
+void rocm_step_tail_destroy(RocmStepTail* tail);
+void rocm_step_tail_reset(RocmStepTail* tail);
+
 /* Decode over constant weights repacked for streaming (M <= 4). `packed` holds rocm_decode_packed_bytes() bytes and is
- * filled once by rocm_launch_pack_decode from args->b / scales / zp; rocm_launch_decode_packed then reads only it. */
+ * filled once by rocm_launch_pack_decode from args->b / scales / zp; rocm_launch_decode_packed then reads only it.
+ * `tail`: NULL, or what the provider recorded last while a capture is open on `stream`. */
 int rocm_decode_packed_eligible(const RocmMatMulNBitsArgs* args);
 uint64_t rocm_decode_packed_bytes(const RocmMatMulNBitsArgs* args);
 int rocm_launch_pack_decode(const RocmMatMulNBitsArgs* args, void* packed, rocm_stream_t stream);
-int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* args, const void* packed, int waves, rocm_stream_t stream);
+int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* args, const void* packed, int waves, rocm_stream_t stream, RocmStepTail* tail);
 /* What rocm_launch_decode_packed would launch for `args` on a chip of `compute_units` CUs, without launching anything (only the
  * shape, dtypes, block size and gamma of `args` are read). pair_member: 0 = a plain call, 1 = one projection of a gate/up pair
  * launched alone, 2 = the paired launch. -1: the shape does not take this route. */

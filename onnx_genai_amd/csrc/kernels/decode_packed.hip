@@ -826,15 +826,13 @@ static mnb::PackedParams packed_params(const RocmMatMulNBitsArgs* a, const void*
     p.k = static_cast<int>(a->k);
     p.n = static_cast<int>(a->n);
     p.groups = mnb::packed_groups(a);
-    p.rest.bias = a->bias;
-    p.rest.y = a->y;
-    p.rest.bias_dtype = a->bias_dtype;
+    p.rest.nodes[0] = mnb::PackedNode{a->bias, a->y, p.packed, p.n, a->bias_dtype};
     p.rest.y_dtype = a->y_dtype;
     return p;
 }
 
 static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, const void* packed_up, int decomposed, int waves, bool probe_only,
-                                bool pair_member, rocm_stream_t stream)
+                                bool pair_member, rocm_stream_t stream, RocmStepTail* tail)
 {
     if (!rocm_decode_packed_eligible(a)) return probe_only ? 0 : -1;
     const int64_t cus = rocm_ffi_compute_units();
@@ -856,25 +854,24 @@ static int launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed
         // the shared-activation kernel's paired form takes up to 16 rows (one block of rows per wave)
         if (probe_only) return a->m <= 16 ? 1 : 0;
         if (packed_up && a->m > 16) return -1;
-        p.groups_per_wave = p.groups;
         if (bf16) return f32_scales ? mnb::launch_wide_bs<true, float>(p, a->block_size, cus, s) : mnb::launch_wide_bs<true, uint16_t>(p, a->block_size, cus, s);
         return f32_scales ? mnb::launch_wide_bs<false, float>(p, a->block_size, cus, s) : mnb::launch_wide_bs<false, uint16_t>(p, a->block_size, cus, s);
     }
     const int w = plan.waves;
     const int w_max = w_max_of(a, f32_scales);
     const bool single_set = plan.single_set;
-    p.groups_per_wave = plan.groups_per_wave;
+    p.split = static_cast<uint32_t>(plan.groups_per_wave);
     // a paired launch keeps each projection's own split of K (so that it adds up in the same order) and needs twice the waves
     if (probe_only) return a->m <= 4 && 2 * w <= w_max ? 1 : 0;
     if (packed_up && (a->m > 4 || 2 * w > w_max)) return -1;
 
-    if (bf16) return f32_scales ? mnb::launch_packed_bs<true, float>(p, a->block_size, w, single_set, s) : mnb::launch_packed_bs<true, uint16_t>(p, a->block_size, w, single_set, s);
-    return f32_scales ? mnb::launch_packed_bs<false, float>(p, a->block_size, w, single_set, s) : mnb::launch_packed_bs<false, uint16_t>(p, a->block_size, w, single_set, s);
+    if (bf16) return f32_scales ? mnb::launch_packed_bs<true, float>(p, a->block_size, w, single_set, s, tail) : mnb::launch_packed_bs<true, uint16_t>(p, a->block_size, w, single_set, s, tail);
+    return f32_scales ? mnb::launch_packed_bs<false, float>(p, a->block_size, w, single_set, s, tail) : mnb::launch_packed_bs<false, uint16_t>(p, a->block_size, w, single_set, s, tail);
 }
 
-extern "C" int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
+extern "C" int rocm_launch_decode_packed(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream, RocmStepTail* tail)
 {
-    return launch_decode_packed(a, packed, nullptr, 0, waves, false, false, stream);
+    return launch_decode_packed(a, packed, nullptr, 0, waves, false, false, stream, tail);
 }
 
 extern "C" int rocm_decode_plain_eligible(const RocmMatMulNBitsArgs* a)
@@ -898,7 +895,7 @@ static int launch_decode_plain(const RocmMatMulNBitsArgs* a, const RocmMatMulNBi
         const bool in_between = a->m <= 16 && (bits == 8 || a->block_size != 32) && col_groups > cus * mnb::kWideWaves && col_groups <= cus * mnb::kWideWavesMax;
         return mnb::launch_plain_wide(p, bits, bf16, f32_scales, a->block_size, in_between ? static_cast<int>((col_groups + cus - 1) / cus) : mnb::kWideWaves, s);
     }
-    p.groups_per_wave = plan.groups_per_wave;
+    p.split = static_cast<uint32_t>(plan.groups_per_wave);
     return mnb::launch_plain(p, bits, bf16, f32_scales, a->block_size, plan.waves, s);
 }
 
@@ -916,19 +913,19 @@ extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const vo
 
 extern "C" int rocm_launch_decode_packed_pair_member(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
 {
-    return launch_decode_packed(a, packed, nullptr, 0, waves, false, true, stream);
+    return launch_decode_packed(a, packed, nullptr, 0, waves, false, true, stream, nullptr);
 }
 
 extern "C" int rocm_decode_packed_pair_fits(const RocmMatMulNBitsArgs* a, int waves)
 {
-    return launch_decode_packed(a, nullptr, nullptr, 0, waves, true, true, nullptr);
+    return launch_decode_packed(a, nullptr, nullptr, 0, waves, true, true, nullptr, nullptr);
 }
 
 extern "C" int rocm_launch_decode_packed_pair(const RocmMatMulNBitsArgs* a, const void* packed_gate, const void* packed_up, int decomposed, int waves,
                                               rocm_stream_t stream)
 {
     if (!packed_gate || !packed_up || a->y_dtype != a->a_dtype) return -1;
-    return launch_decode_packed(a, packed_gate, packed_up, decomposed, waves, false, true, stream);
+    return launch_decode_packed(a, packed_gate, packed_up, decomposed, waves, false, true, stream, nullptr);
 }
 
 extern "C" int rocm_acc4_packed_eligible(const RocmMatMulNBitsArgs* a)

@@ -1,0 +1,136 @@
+// One launch for the nodes of a recorded step that read the same activations.
+//
+// A stream capture records the calls of one stream as a chain, so each node of a step waits for the one before it, though the step's data
+// asks for less: q, k and v read one input, and so do gate and up of a model that was exported without fused nodes. A launch that depends on another costs
+// about 2 us before it has read a byte, more than half the time of such a node of a 0.5B model.
+// A node that could run beside the one recorded just before it is therefore not recorded as a launch of its own: it becomes a further row of that launch's
+// grid, with its own columns, bias and result. Each keeps its own split of K, so its sums are those of a launch by itself, bit for bit.
+// 24 layers of a 0.5B model at one row, f16, block 32: 169 launches 585 us, 97 launches 393.
+// What may join: the capture's only open end is the launch recorded last (anything recorded in between, by whomever, is another end); the same kernel
+// build, activations, rows, K, split of K and result type; and no result of one that is an input or a result of the other.
+// The recorded node gets new arguments and a larger grid while the capture is open (hipGraphKernelNodeSetParams), so the graph is complete after every call
+// and nothing is left to do when the capture ends.
+#include <mutex>
+#include <new>
+
+#include "packed_launch.hiph"
+
+struct RocmStepTail {
+    std::mutex mu;
+    unsigned long long capture = 0;
+    hipGraphNode_t node = nullptr;          // NULL: nothing to join
+    mnb::PackedLaunch launch;               // as it stands in `node`
+};
+
+namespace mnb {
+namespace {
+
+// The one node that the next operation on `stream` would depend on.
+bool open_end(hipStream_t stream, unsigned long long* capture, hipGraphNode_t* node)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    const hipGraphNode_t* ends = nullptr;
+    size_t count = 0;
+    if (hipStreamGetCaptureInfo_v2(stream, &status, capture, nullptr, &ends, &count) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (status != hipStreamCaptureStatusActive || count != 1) return false;
+    *node = ends[0];
+    return true;
+}
+
+struct Range {
+    uintptr_t begin, end;
+};
+bool meet(const Range& a, const Range& b) { return a.begin < b.end && b.begin < a.end; }
+Range range(const void* p, int64_t elements, int dtype)
+{
+    const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+    return p ? Range{at, at + static_cast<uintptr_t>(elements) * (dtype == ROCM_DT_F32 ? 4 : 2)} : Range{0, 0};
+}
+Range result(const PackedParams& p, const PackedNode& node) { return range(node.y, static_cast<int64_t>(p.m) * node.n, p.rest.y_dtype); }
+Range bias(const PackedParams& p, const PackedNode& node)
+{
+    return range(node.bias, (node.bias_dtype & ROCM_BIAS_PER_ROW) ? static_cast<int64_t>(p.m) * node.n : node.n, node.bias_dtype & 0xff);
+}
+
+// `to` with the node of `add` as a further row, or false: they do not go together.
+bool joined(const PackedLaunch& to, const PackedLaunch& add, PackedLaunch* out)
+{
+    const PackedParams &p = to.p, &q = add.p;
+    if (to.nodes < 1 || to.nodes == kMaxNodes || add.nodes != 1 || to.kernel != add.kernel || to.threads != add.threads || to.lds != add.lds) return false;
+    if (p.a != q.a || p.m != q.m || p.k != q.k || p.groups != q.groups || p.split != q.split || p.rest.y_dtype != q.rest.y_dtype) return false;
+    const PackedNode& node = q.rest.nodes[0];
+    const Range a = range(q.a, static_cast<int64_t>(q.m) * q.k, ROCM_DT_F16), y = result(q, node), b = bias(q, node);
+    if (meet(y, a)) return false;
+    for (int i = 0; i < to.nodes; ++i) {
+        const Range other = result(p, p.rest.nodes[i]);
+        if (meet(y, other) || meet(a, other) || meet(b, other) || meet(y, bias(p, p.rest.nodes[i]))) return false;
+    }
+    *out = to;
+    if (to.nodes == 1) {
+        out->p.packed_up = node.packed;
+        out->p.n_up = node.n;
+    }
+    out->p.rest.nodes[out->nodes++] = node;
+    if (out->grid < add.grid) out->grid = add.grid;
+    // every row of the grid is as long as the widest node's: not where the workgroups without columns would be most of many
+    int64_t busy = 0;
+    for (int i = 0; i < out->nodes; ++i) busy += (static_cast<int64_t>(out->p.rest.nodes[i].n) + 15) / 16;
+    return static_cast<int64_t>(out->grid) * out->nodes <= 2 * busy + 512;
+}
+
+}  // namespace
+
+int start_packed(const PackedLaunch& launch, hipStream_t stream, RocmStepTail* tail)
+{
+    auto arguments = [](PackedParams& p, void* (&to)[11]) {
+        void* const all[11] = {&p.a, &p.packed, &p.packed_up, &p.gamma, &p.m, &p.k, &p.n, &p.n_up, &p.groups, &p.split, &p.rest};
+        for (int i = 0; i < 11; ++i) to[i] = all[i];
+    };
+    void* args[11];
+    auto alone = [&] {
+        PackedParams p = launch.p;
+        arguments(p, args);
+        return static_cast<int>(hipLaunchKernel(launch.kernel, dim3(launch.grid), dim3(launch.threads), args, launch.lds, stream));
+    };
+    if (!tail) return alone();
+    std::lock_guard<std::mutex> lock(tail->mu);
+    unsigned long long capture = 0;
+    hipGraphNode_t node = nullptr;
+    PackedLaunch both;
+    if (tail->node && open_end(stream, &capture, &node) && capture == tail->capture && node == tail->node && joined(tail->launch, launch, &both)) {
+        arguments(both.p, args);
+        hipKernelNodeParams params{};
+        params.func = const_cast<void*>(both.kernel);
+        params.gridDim = dim3(both.grid, static_cast<unsigned>(both.nodes));
+        params.blockDim = dim3(both.threads);
+        params.sharedMemBytes = static_cast<unsigned>(both.lds);
+        params.kernelParams = args;
+        if (hipGraphKernelNodeSetParams(node, &params) == hipSuccess) {
+            tail->launch = both;
+            return 0;
+        }
+        (void)hipGetLastError();               // the node is what it was: a launch of its own
+    }
+    tail->node = nullptr;
+    const int rc = alone();
+    if (rc == 0 && open_end(stream, &capture, &node)) {
+        tail->capture = capture;
+        tail->node = node;
+        tail->launch = launch;
+    }
+    return rc;
+}
+
+}  // namespace mnb
+
+extern "C" RocmStepTail* rocm_step_tail_create(void) { return new (std::nothrow) RocmStepTail(); }
+extern "C" void rocm_step_tail_destroy(RocmStepTail* tail) { delete tail; }
+extern "C" void rocm_step_tail_reset(RocmStepTail* tail)
+{
+    if (!tail) return;
+    std::lock_guard<std::mutex> lock(tail->mu);
+    tail->node = nullptr;
+}
