@@ -254,14 +254,17 @@ bool weights_in_16_bits(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs
     return !kn.no_alloc && static_cast<uint64_t>(args.n) * static_cast<uint64_t>(args.k) * 2 <= kn.ep->dense_gemm_max_bytes && rocm_prefill_dense16_eligible(&args);
 }
 
+bool use_packed(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& rc);
+
 // Constant act-order weights (`args.g_idx` set and checked) as an ordinary node: args.b becomes the copy sorted by group, made on
 // first use, args.a the call's activations in the same order, args.g_idx null. Returns false with `args` untouched where the groups
 // are not whole blocks, where no kernel for contiguous blocks is the better one, or the copy or the gather's buffer cannot be made now (a
 // capture is open, no memory): the kernels that look groups up per element take the call then. `in_16_bits`: weights_in_16_bits of the call as it
-// came. `rc` receives a HIP error.
-bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_16_bits, int& rc)
+// came. `rc` receives a HIP error. `order`: not null where the decode kernel gathers the row itself; args.a is the caller's then.
+bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_16_bits, const uint16_t*& order, int& rc)
 {
     rc = 0;
+    order = nullptr;
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[4]) return false;
     if (args.a_dtype != ROCM_DT_F32) {
         if (args.y_dtype == ROCM_DT_F32 && !in_16_bits) return false;      // (f32 results of 16-bit rows keep the f32 GEMV)
@@ -275,7 +278,8 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
             if (!tiled && !(args.m <= 32 && rocm_decode_plain_eligible(&probe))) return false;
         }
     }
-    const size_t order_bytes = (static_cast<size_t>(args.k) * sizeof(int32_t) + 255) / 256 * 256;
+    const size_t order16_at = (static_cast<size_t>(args.k) * sizeof(int32_t) + 255) / 256 * 256, order16_bytes = args.k <= 65536 ? (static_cast<size_t>(args.k) * sizeof(uint16_t) + 255) / 256 * 256 : 0;
+    const size_t order_bytes = order16_at + order16_bytes;
     if (kn.regrouped_from[0] != args.b || kn.regrouped_from[1] != args.g_idx) {
         if (frozen(kn)) return false;
         if (kn.regrouped) {
@@ -291,10 +295,11 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
                 kn.regrouped = nullptr;
                 return false;
             }
-            int32_t* const order = static_cast<int32_t*>(kn.regrouped);
-            rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, order, &regular, kn.ep->stream);
+            int32_t* const to = static_cast<int32_t*>(kn.regrouped);
+            uint16_t* const to16 = order16_bytes ? reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(kn.regrouped) + order16_at) : nullptr;
+            rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, to, to16, &regular, kn.ep->stream);
             if (rc == 0 && regular)
-                rc = rocm_launch_regroup(args.b, order, args.n, args.k, args.block_size, static_cast<int>(kn.bits), static_cast<uint8_t*>(kn.regrouped) + order_bytes, kn.ep->stream);
+                rc = rocm_launch_regroup(args.b, to, args.n, args.k, args.block_size, static_cast<int>(kn.bits), static_cast<uint8_t*>(kn.regrouped) + order_bytes, kn.ep->stream);
             if (rc != 0 || !regular) {
                 rocm_ffi_free(kn.regrouped);
                 kn.regrouped = nullptr;
@@ -307,9 +312,21 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
     }
     if (kn.regroup_failed) return false;
     const size_t need = static_cast<size_t>(args.m) * static_cast<size_t>(args.k) * (args.a_dtype == ROCM_DT_F32 ? 4 : 2);
-    if (kn.gathered_bytes < need && (frozen(kn) || grow_buffer(kn.gathered, kn.gathered_bytes, need, kn.retired) != 0)) return false;
-    const int32_t* const order = static_cast<const int32_t*>(kn.regrouped);
-    rc = rocm_launch_gather_columns(args.a, args.a_dtype, order, args.m, args.k, kn.gathered, kn.ep->stream);
+    // (also where the kernel gathers: a call recorded later may come with a row that it does not take)
+    const bool room = kn.gathered_bytes >= need || (!frozen(kn) && grow_buffer(kn.gathered, kn.gathered_bytes, need, kn.retired) == 0);
+    if (kn.bits == 4 && args.a_dtype != ROCM_DT_F32 && order16_bytes) {
+        RocmMatMulNBitsArgs inside = args;
+        inside.b = static_cast<const uint8_t*>(kn.regrouped) + order_bytes;
+        inside.g_idx = nullptr;
+        if (rocm_decode_plain_gathers(&inside, kn.ep->decode_waves) && use_packed(kn, inside, rc)) {
+            args = inside;
+            order = reinterpret_cast<const uint16_t*>(static_cast<const uint8_t*>(kn.regrouped) + order16_at);
+            return true;
+        }
+        if (rc != 0) return false;
+    }
+    if (!room) return false;
+    rc = rocm_launch_gather_columns(args.a, args.a_dtype, static_cast<const int32_t*>(kn.regrouped), args.m, args.k, kn.gathered, kn.ep->stream);
     kn.ep->launches.fetch_add(1);
     args.a = kn.gathered;
     args.b = static_cast<const uint8_t*>(kn.regrouped) + order_bytes;
@@ -805,7 +822,8 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
     // Asked before the rows are gathered: what keeps its weights in 32 bits for an A off a 16-byte boundary keeps them behind the gather, too.
     const bool in_16_bits = weights_in_16_bits(kn, args);
     const bool dense_off = args.g_idx && args.a_dtype != ROCM_DT_F32 && (reinterpret_cast<uintptr_t>(args.a) & 15) != 0;
-    const bool sorted = G && sort_by_group(kn, args, in_16_bits, rc);
+    const uint16_t* order = nullptr;
+    const bool sorted = G && sort_by_group(kn, args, in_16_bits, order, rc);
     if (rc != 0) return hip_status(rc, "MatMulNBits: act-order weights");
     if (kn.bits != 4 || args.g_idx) {
         // Up to 32 rows of 8-bit weights stream the repacked copy (above, the tiled kernel: 3584 -> 37888 at 33 / 64 rows 90 us where four
@@ -884,7 +902,10 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
         }
     } else if (sorted && args.a_dtype != ROCM_DT_F32) {
         // (the kernels over the 4-bit stream whose accumulators carry an offset are not for these: see decode_packed.hiph)
-        if (stream_sorted(kn, args, in_16_bits, rc)) {
+        if (order) {
+            rc = rocm_launch_decode_plain_gathered(&args, kn.packed, order, kn.ep->decode_waves, stream);
+            kn.variant = "decode_mfma_packed";
+        } else if (stream_sorted(kn, args, in_16_bits, rc)) {
             // done
         } else if (!dense_off && dense_route(kn, args, rc)) {
             // done: weights expanded to 16 bits, then the library GEMM

@@ -904,6 +904,24 @@ extern "C" int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* a, const void
     return rocm_decode_plain_eligible(a) ? launch_decode_plain(a, a, 4, packed, waves, stream) : -1;
 }
 
+// One row in another order than the weights': gathered by the kernel where a thread has at most four pieces of it to bring to LDS and two workgroups fit a CU's.
+extern "C" int rocm_decode_plain_gathers(const RocmMatMulNBitsArgs* a, int waves)
+{
+    if (a->m != 1 || a->k > 65536 || (reinterpret_cast<uintptr_t>(a->a) & 15) != 0 || !rocm_decode_plain_eligible(a)) return 0;
+    const PackedPlan plan = plan_decode_packed(a, waves, false, false, rocm_ffi_compute_units());
+    return !plan.wide && a->k <= static_cast<int64_t>(plan.waves) * 64 * 8 * mnb::kGatherPieces && mnb::plain_gather_lds(a->k, plan.waves) <= 80 * 1024;
+}
+
+extern "C" int rocm_launch_decode_plain_gathered(const RocmMatMulNBitsArgs* a, const void* packed, const uint16_t* order, int waves, rocm_stream_t stream)
+{
+    if (!rocm_decode_plain_gathers(a, waves)) return -1;
+    const PackedPlan plan = plan_decode_packed(a, waves, false, false, rocm_ffi_compute_units());
+    mnb::PackedParams p = packed_params(a, packed);
+    p.gamma = order;
+    p.split = static_cast<uint32_t>(plan.groups_per_wave);
+    return mnb::launch_plain_gather(p, a->a_dtype == ROCM_DT_BF16, a->scale_dtype == ROCM_DT_F32, a->block_size, plan.waves, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int rocm_launch_decode_packed8(const RocmMatMulNBitsArgs* a, const void* packed, int waves, rocm_stream_t stream)
 {
     if (!rocm_decode_packed8_eligible(a)) return -1;

@@ -32,6 +32,15 @@ void decode_plain_kernel(MNB_PACKED_ARGS)
     decode_packed_body<BF16, BS, MR, ST, 1, false, false, BITS, true>(MNB_PACKED_PARAMS);
 }
 
+// One row of activations that it gathers itself.
+template <bool BF16, int BS, typename ST>
+__global__ __launch_bounds__((BS == 128 && sizeof(ST) == 2) ? 1024 : 512)
+__attribute__((amdgpu_num_sgpr(80), amdgpu_waves_per_eu(plain_waves_per_simd(BF16, BS, 1, sizeof(ST) == 4, 4))))
+void decode_plain_gather_kernel(MNB_PACKED_ARGS)
+{
+    decode_packed_body<BF16, BS, 1, ST, 1, false, false, 4, true, true>(MNB_PACKED_PARAMS);
+}
+
 // One block of rows: weights and windows both ahead (8 bits, block 128, 16 rows, 3584 -> 152064: 112 us, windows alone 120, neither 114; act-order
 // 4 bits 83 / 85 / 89); two: neither (registers).
 template <bool BF16, int BS, typename ST, int RB, int WMAX, int BITS>
@@ -106,6 +115,16 @@ int launch_plain(const PackedParams& p, int bits, bool bf16, bool f32_scales, in
 {
     return by_build(bits, bf16, f32_scales, block_size, [&](auto bf, auto bs, auto st, auto bi) {
         return launch_plain_bs<decltype(bf)::value, decltype(bs)::value, decltype(st), decltype(bi)::value>(p, waves, stream);
+    });
+}
+
+int launch_plain_gather(const PackedParams& p, bool bf16, bool f32_scales, int block_size, int waves, hipStream_t stream)
+{
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(p.n) + 15) / 16);
+    const size_t lds = plain_gather_lds(p.k, waves);
+    return by_build(4, bf16, f32_scales, block_size, [&](auto bf, auto bs, auto st, auto bi) {
+        if constexpr (decltype(bi)::value == 4) return launch_on(decode_plain_gather_kernel<decltype(bf)::value, decltype(bs)::value, decltype(st)>, grid, waves, lds, stream, p);
+        else return -1;
     });
 }
 

@@ -2,7 +2,7 @@
 // block_size elements of K, scattered. Sorting K by group turns such a node into an ordinary one over
 //   B'[n, j] = B[n, order[j]],  A'[m, j] = A[m, order[j]],  order = the elements of K, group by group,
 // with the scales and zero points as they are, so that the kernels for contiguous blocks serve it - of those over the repacked stream the ones with plain
-// sums, which the per-element kernels have too. B' is made once for constant weights and the stream once more from it: two copies of the weights beside the caller's; A' costs one gather per call (7 KB of a 3584-element row: 2 us) where the kernels that look a group up per element
+// sums, which the per-element kernels have too. B' is made once for constant weights and the stream once more from it: two copies of the weights beside the caller's; A' costs one gather per call (7 KB of a 3584-element row: 2 us; one row is gathered inside the decode kernel) where the kernels that look a group up per element
 // paid for it on every weight: 3584 -> 37888, one f16 row, block 128: 501 us, against 18.1 us for gather and repacked-stream kernel together.
 #include <vector>
 
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void gather_columns_kernel(const T* __restrict
 
 }  // namespace mnb
 
-extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, int* regular, rocm_stream_t stream)
+extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, uint16_t* order16, int* regular, rocm_stream_t stream)
 {
     *regular = 0;
     std::vector<int32_t> groups(static_cast<size_t>(k)), sorted(static_cast<size_t>(k));
@@ -67,6 +67,10 @@ extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, 
         sorted[static_cast<size_t>(g * block_size + filled[static_cast<size_t>(g)]++)] = static_cast<int32_t>(i);
     }
     e = rocm_ffi_memcpy_h2d(order, sorted.data(), sorted.size() * sizeof(int32_t), stream);
+    if (e == 0 && order16) {
+        const std::vector<uint16_t> narrow(sorted.begin(), sorted.end());
+        e = rocm_ffi_memcpy_h2d(order16, narrow.data(), narrow.size() * sizeof(uint16_t), stream);
+    }
     if (e == 0) *regular = 1;
     return e;
 }

@@ -133,3 +133,30 @@ def test_a_height_recorded_without_a_repacked_copy(ep, port, bs, m):
         ep.deallocate(ab)
         ep.deallocate(yb)
         ops.free()
+
+
+@pytest.mark.parametrize("first", [0.0, np.inf])
+@pytest.mark.parametrize("a_dt,bs,s_dt,k", [(E.F16, 128, E.F16, 1000), (E.BF16, 128, E.BF16, 3584), (E.BF16, 32, E.F32, 1000), (E.F16, 64, E.F32, 520), (E.F16, 32, E.F16, 8),
+                                            (E.F16, 128, E.F16, 18944), (E.BF16, 128, E.BF16, 26624), (E.BF16, 128, E.BF16, 26632), (E.F16, 32, E.F16, 16384), (E.F16, 32, E.F16, 16392)])
+def test_one_row_gathered_inside_the_kernel(ep, a_dt, bs, s_dt, k, first):
+    """The bits of a row gathered by a launch of its own, which a row off a 16-byte boundary takes: ragged K, the longest rows the kernel takes and the first that it
+    does not, and a row whose first element, which the places beyond K point at, is infinite."""
+    n = 72
+    b, s, zp = synth.make_weights(n, k, bs, k, zero_points=True, scale_lo=0.005, scale_hi=0.02, scale_dtype=s_dt)
+    ops = E.DeviceOperands(ep, b, s, s_dt, zp, n, k, bs, g_idx=shuffled_groups(k, bs, k))
+    a = np.asarray(synth.to_f32(synth.make_activation(1, k, 7, a_dt), a_dt)).copy().reshape(1, k)
+    if first != 0.0:
+        a[0, 0] = first
+    a = np.asarray(synth.to_dtype(a, a_dt)).view(np.uint16).ravel()
+    ab, yb = ep.upload(np.concatenate([a, np.zeros(4, np.uint16), a])), ep.allocate(n * 2)
+    got = []
+    try:
+        for start in (0, k * 2 + 8):                       # (K is a multiple of 8: the second row is off by half of 16 bytes)
+            ops.run(E.DeviceBuffer(ab.ptr + start, k * 2), a_dt, 1, yb)
+            assert ops.kernel.last_variant() == "act_order+decode_mfma_packed"
+            got.append(ep.download(yb, (n,), np.uint16))
+        assert np.array_equal(got[0], got[1])
+    finally:
+        ep.deallocate(ab)
+        ep.deallocate(yb)
+        ops.free()
