@@ -297,7 +297,8 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
             }
             int32_t* const to = static_cast<int32_t*>(kn.regrouped);
             uint16_t* const to16 = order16_bytes ? reinterpret_cast<uint16_t*>(static_cast<uint8_t*>(kn.regrouped) + order16_at) : nullptr;
-            rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, to, to16, &regular, kn.ep->stream);
+            rc = rocm_gidx_order(args.g_idx, args.k, args.block_size, to, &regular, kn.ep->stream);
+            if (rc == 0 && regular && to16) rc = rocm_launch_narrow_order(to, args.k, to16, kn.ep->stream);
             if (rc == 0 && regular)
                 rc = rocm_launch_regroup(args.b, to, args.n, args.k, args.block_size, static_cast<int>(kn.bits), static_cast<uint8_t*>(kn.regrouped) + order_bytes, kn.ep->stream);
             if (rc != 0 || !regular) {

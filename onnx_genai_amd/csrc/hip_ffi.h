@@ -144,7 +144,8 @@ int rocm_g_idx_first_bad(const int32_t* g_idx, int64_t count, int64_t kb, int64_
  * `order` (device, [K]) receives the elements of K group by group and *regular 1; *regular 0 and nothing written when the groups
  * are not of that form. Synchronizes (never inside a graph capture). regroup: B'[n, j] = B[n, order[j]] in B's layout (row dwords
  * of kb * block_size * bits / 32), for any of the widths; gather_columns: A'[m, j] = A[m, order[j]]. */
-int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, uint16_t* order16, int* regular, rocm_stream_t stream);
+int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, int* regular, rocm_stream_t stream);
+int rocm_launch_narrow_order(const int32_t* order, int64_t k, uint16_t* order16, rocm_stream_t stream);
 int rocm_launch_regroup(const uint8_t* b, const int32_t* order, int64_t n, int64_t k, int block_size, int bits, void* out, rocm_stream_t stream);
 int rocm_launch_gather_columns(const void* a, int a_dtype, const int32_t* order, int64_t m, int64_t k, void* out, rocm_stream_t stream);
 
@@ -213,7 +214,7 @@ int rocm_launch_decode_packed_pair(const RocmMatMulNBitsArgs* args, const void* 
 int rocm_decode_plain_eligible(const RocmMatMulNBitsArgs* args);
 int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* args, const void* packed, int waves, rocm_stream_t stream);
 /* One row (args->a as the caller has it) whose elements the kernel takes in the order of the sorted weights itself: `order` as
- * rocm_gidx_order leaves it. rocm_decode_plain_gathers says whether it does. */
+ * rocm_launch_narrow_order leaves it. rocm_decode_plain_gathers says whether it does. */
 int rocm_decode_plain_gathers(const RocmMatMulNBitsArgs* args, int waves);
 int rocm_launch_decode_plain_gathered(const RocmMatMulNBitsArgs* args, const void* packed, const uint16_t* order, int waves, rocm_stream_t stream);
 

@@ -49,9 +49,21 @@ __global__ __launch_bounds__(256) void gather_columns_kernel(const T* __restrict
     }
 }
 
+__global__ __launch_bounds__(256) void narrow_order_kernel(const int32_t* __restrict__ order, int64_t k, uint16_t* __restrict__ order16)
+{
+    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (i < k) order16[i] = static_cast<uint16_t>(order[i]);
+}
+
 }  // namespace mnb
 
-extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, uint16_t* order16, int* regular, rocm_stream_t stream)
+extern "C" int rocm_launch_narrow_order(const int32_t* order, int64_t k, uint16_t* order16, rocm_stream_t stream)
+{
+    hipLaunchKernelGGL(mnb::narrow_order_kernel, dim3(static_cast<unsigned>((k + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), order, k, order16);
+    return static_cast<int>(hipGetLastError());
+}
+
+extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, int32_t* order, int* regular, rocm_stream_t stream)
 {
     *regular = 0;
     std::vector<int32_t> groups(static_cast<size_t>(k)), sorted(static_cast<size_t>(k));
@@ -67,10 +79,6 @@ extern "C" int rocm_gidx_order(const int32_t* g_idx, int64_t k, int block_size, 
         sorted[static_cast<size_t>(g * block_size + filled[static_cast<size_t>(g)]++)] = static_cast<int32_t>(i);
     }
     e = rocm_ffi_memcpy_h2d(order, sorted.data(), sorted.size() * sizeof(int32_t), stream);
-    if (e == 0 && order16) {
-        const std::vector<uint16_t> narrow(sorted.begin(), sorted.end());
-        e = rocm_ffi_memcpy_h2d(order16, narrow.data(), narrow.size() * sizeof(uint16_t), stream);
-    }
     if (e == 0) *regular = 1;
     return e;
 }
