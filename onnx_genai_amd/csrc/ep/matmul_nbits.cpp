@@ -335,6 +335,12 @@ bool sort_by_group(NxrtRocmMatMulNBits& kn, RocmMatMulNBitsArgs& args, bool in_1
     return true;
 }
 
+// The repacked copy was made from these tensors.
+bool packed_is_current(const NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args)
+{
+    return kn.packed && kn.packed_from[0] == args.b && kn.packed_from[1] == args.scales && kn.packed_from[2] == args.zp && kn.packed_scale_dtype == args.scale_dtype;
+}
+
 // True when the call can run on the repacked copy of constant weights; makes that copy on first use (never while a
 // graph capture is open: a capture may neither allocate nor should it record the one-time repack). `rc` receives a
 // HIP error of the repack.
@@ -344,9 +350,7 @@ bool use_packed(NxrtRocmMatMulNBits& kn, const RocmMatMulNBitsArgs& args, int& r
     if (!kn.ep->prepack || !kn.constant_inputs[1] || !kn.constant_inputs[2] || (args.zp && !kn.constant_inputs[3])) return false;
     const bool eight = kn.bits == 8;
     if (!(eight ? rocm_decode_packed8_eligible(&args) : kn.accuracy_level == 4 ? rocm_acc4_packed_eligible(&args) : rocm_decode_packed_eligible(&args))) return false;
-    const bool current = kn.packed && kn.packed_from[0] == args.b && kn.packed_from[1] == args.scales && kn.packed_from[2] == args.zp &&
-                         kn.packed_scale_dtype == args.scale_dtype;
-    if (current) return true;
+    if (packed_is_current(kn, args)) return true;
     if (frozen(kn)) return false;
     if (kn.packed) {
         drop_weight_copy(kn, kn.packed);
@@ -605,7 +609,8 @@ struct NormPrologue {
 };
 
 // a -> round16((a * inv_std) * gamma), [rows, K] of a 16-bit type, into owner.norm; `a` is replaced by the buffer.
-NxrtStatus normalize_rows(const NormPrologue& np, const void*& a, int a_dtype, uint64_t rows, uint64_t k)
+// `ahead`: the weights that the launch behind it streams, or null.
+NxrtStatus normalize_rows(const NormPrologue& np, const void*& a, int a_dtype, uint64_t rows, uint64_t k, const RocmWeightsAhead* ahead = nullptr)
 {
     NxrtRocmMatMulNBits& owner = *np.owner;
     const uint64_t need = rows * k * 2;
@@ -618,7 +623,7 @@ NxrtStatus normalize_rows(const NormPrologue& np, const void*& a, int a_dtype, u
     }
     if ((reinterpret_cast<uintptr_t>(a) & 7) != 0 || (reinterpret_cast<uintptr_t>(np.gamma) & 15) != 0)
         return make_status(NXRT_INVALID_ARGUMENT, err("rmsnorm_prologue fusion needs A at an 8-byte and gamma at a 16-byte boundary (data pointer plus byte offset)"));
-    const int rc = rocm_launch_rmsnorm16(a, np.gamma, np.gamma_dtype, static_cast<int64_t>(rows), static_cast<int64_t>(k), np.epsilon, a_dtype, owner.norm, owner.ep->stream);
+    const int rc = rocm_launch_rmsnorm16(a, np.gamma, np.gamma_dtype, static_cast<int64_t>(rows), static_cast<int64_t>(k), np.epsilon, a_dtype, owner.norm, ahead, owner.ep->stream);
     if (rc != 0) return hip_status(rc, "MatMulNBits: kernel launch");
     owner.ep->launches.fetch_add(1);
     a = owner.norm;
@@ -790,7 +795,9 @@ NxrtStatus execute_impl(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in, u
             args = fused;
             norm->fused = true;
         } else {
-            const NxrtStatus ns = normalize_rows(*norm, args.a, args.a_dtype, M, K);
+            RocmWeightsAhead ahead{};
+            const bool known = kn.bits == 4 && !G && kn.accuracy_level != 4 && packed_is_current(kn, args) && rocm_decode_packed_ahead(&args, kn.packed, nullptr, kn.ep->decode_waves, &ahead);
+            const NxrtStatus ns = normalize_rows(*norm, args.a, args.a_dtype, M, K, known ? &ahead : nullptr);
             if (ns.code != NXRT_OK) return ns;
         }
     }
@@ -1029,7 +1036,9 @@ NxrtStatus execute_swiglu(NxrtRocmMatMulNBits& kn, const NxrtRocmTensorView* in,
                 args.norm_epsilon = norm->epsilon;
             } else if (norm) {
                 normalized = args.a;
-                const NxrtStatus ns = normalize_rows(*norm, normalized, args.a_dtype, M, K);
+                RocmWeightsAhead ahead{};
+                const bool known = rocm_decode_packed_pair_fits(&args, kn.ep->decode_waves) && rocm_decode_packed_ahead(&args, kn.gate->packed, kn.up->packed, kn.ep->decode_waves, &ahead);
+                const NxrtStatus ns = normalize_rows(*norm, normalized, args.a_dtype, M, K, known ? &ahead : nullptr);
                 if (ns.code != NXRT_OK) return ns;
                 args.a = normalized;                     // whatever runs below sees these rows
             }

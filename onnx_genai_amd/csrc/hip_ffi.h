@@ -125,8 +125,16 @@ int rocm_launch_swiglu(const void* gate, const void* up, int64_t count, int dtyp
 
 /* out = round16((a * inv_std) * gamma) per row of K 16-bit elements (K % 128 == 0), inv_std = 1 / sqrt(mean(a^2) + eps),
  * summed in the reference's order (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4125-4205). gamma: f32 or 16-bit. */
+/* The repacked weights that the launch after a normalization streams: workgroup w of it reads `bytes` from first + w * bytes, and as many of `second`
+ * where that is not NULL (device pointers, 16-byte aligned; workgroups * bytes lie within each). */
+typedef struct RocmWeightsAhead {
+  const void* first;
+  const void* second;
+  uint64_t bytes;
+  uint32_t workgroups;
+} RocmWeightsAhead;
 int rocm_launch_rmsnorm16(const void* a, const void* gamma, int gamma_dtype, int64_t rows, int64_t k, float epsilon, int dtype, void* out,
-                          rocm_stream_t stream);
+                          const RocmWeightsAhead* ahead, rocm_stream_t stream);
 
 /* bits = 2 or 8 (element i of a packed row in byte i / (8 / bits) at bit (i % (8 / bits)) * bits; zero points packed alike,
  * default 1 << (bits - 1)): w[n,k] = (q - zp) * scale as f32, f16 or bf16 [N, K] (one f32 multiply, then one rounding), and
@@ -193,6 +201,8 @@ typedef struct RocmDecodePackedPlan {
   int64_t workgroups;
 } RocmDecodePackedPlan;
 int rocm_decode_packed_plan(const RocmMatMulNBitsArgs* args, int waves, int pair_member, int compute_units, RocmDecodePackedPlan* out);
+/* What that launch over `packed` (and `packed_up`, a gate/up pair's) reads, for the normalization ahead of it. 0: the shape does not take this route. */
+int rocm_decode_packed_ahead(const RocmMatMulNBitsArgs* args, const void* packed, const void* packed_up, int waves, RocmWeightsAhead* out);
 /* 1 when the launch above (and the paired one below) applies args->gamma inside the kernel: up to 4 rows, K % 128 == 0, gamma f32 or
  * of the activations' type and 16-byte aligned, and a shape the split-K kernel takes (not the shared-activation one). */
 int rocm_decode_packed_fuses_norm(const RocmMatMulNBitsArgs* args);

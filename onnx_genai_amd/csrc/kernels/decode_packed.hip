@@ -816,6 +816,20 @@ extern "C" int rocm_decode_packed_plan(const RocmMatMulNBitsArgs* a, int waves, 
     return 0;
 }
 
+extern "C" int rocm_decode_packed_ahead(const RocmMatMulNBitsArgs* a, const void* packed, const void* packed_up, int waves, RocmWeightsAhead* out)
+{
+    if (!rocm_decode_packed_eligible(a)) return 0;
+    const bool pair = packed_up != nullptr;
+    const PackedPlan plan = plan_decode_packed(a, waves, pair, pair, rocm_ffi_compute_units());
+    if (plan.wide && !plan.w.ok) return 0;
+    const int64_t col_groups = (a->n + 15) / 16, each = plan.wide ? (pair ? plan.waves / 2 : plan.waves) : 1;
+    out->first = packed;
+    out->second = packed_up;
+    out->bytes = static_cast<uint64_t>(each) * mnb::packed_groups(a) * mnb::packed_chunk_bytes(a);
+    out->workgroups = static_cast<uint32_t>(col_groups / each);            // whole ones
+    return 1;
+}
+
 // Operands and stream geometry of a launch over `a`'s stream.
 static mnb::PackedParams packed_params(const RocmMatMulNBitsArgs* a, const void* packed)
 {
