@@ -24,20 +24,22 @@
 
 namespace mnb {
 
+// Fourteen dwords of plain arguments, which are in scalar registers when a wave starts, and what is needed behind the loads.
+struct GemmF32Rest {
+    const void* bias;
+    void* y;
+    int scale_dtype, bias_dtype, y_dtype;
+};
 struct GemmF32Params {
     const float* a;
     const uint8_t* b;
     const void* scales;
     const uint8_t* zp;
-    const void* bias;
-    void* y;
-    int64_t m, n, k, kb;
-    int64_t row_bytes, zp_row;
+    int m, n, k, kb;
     int bs_log2;
-    int scale_dtype, bias_dtype, y_dtype;
     int units_per_wave;     // runs of 32 k a wave walks
-    uint32_t nibble_mask, magic;    // 0x000F000F, 0x64006400 (see plain_nibbles)
 };
+#define MNB_GEMM_F32_ARGS const float *a, const uint8_t *b, const void *scales, const uint8_t *zp, int m, int n, int k, int kb, int bs_log2, int units_per_wave, GemmF32Rest rest
 
 // 8 * GROUPS f32 values as three bf16 operands each: plane[p][group], in plain_nibbles' order. What a cut leaves of an infinity is NaN; with WIDE it is 0.
 template <int GROUPS, bool WIDE>
@@ -86,8 +88,10 @@ template <> struct TileOps<16> {
 // WHOLE: K is a whole number of blocks, so that no run is cut short: activations go through LDS, and the offsets of a wave's loads do not change from
 // run to run (the run goes into the scalar offset). The other build works out per run and load whether elements lie within K.
 template <int TILE, int CN, int DEPTH, int WAVES, typename ST, bool WHOLE>
-__global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
+__global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(MNB_GEMM_F32_ARGS)
 {
+    const GemmF32Params p{a, b, scales, zp, m, n, k, kb, bs_log2, units_per_wave};
+    const int64_t row_bytes = (static_cast<int64_t>(kb) << bs_log2) / 2, zp_row = (kb + 1) / 2;
     using Ops = TileOps<TILE>;
     using acc_t = typename Ops::acc_t;
     constexpr int G = Ops::kMfmas;                         // groups of 8 k a lane holds of a run
@@ -102,12 +106,12 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
 
     const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.a + m_base * p.k, static_cast<uint64_t>(rows_left * p.k) * 4);
-    const __amdgpu_buffer_rsrc_t srd_b = make_srd(p.b + n_base * p.row_bytes, static_cast<uint64_t>(cols_left * p.row_bytes));
+    const __amdgpu_buffer_rsrc_t srd_b = make_srd(p.b + n_base * row_bytes, static_cast<uint64_t>(cols_left * row_bytes));
     const __amdgpu_buffer_rsrc_t srd_s = make_srd(static_cast<const ST*>(p.scales) + n_base * p.kb, static_cast<uint64_t>(cols_left * p.kb) * sizeof(ST));
-    const __amdgpu_buffer_rsrc_t srd_z = make_srd(p.zp ? p.zp + n_base * p.zp_row : nullptr, p.zp ? static_cast<uint64_t>(cols_left * p.zp_row) : 0);
+    const __amdgpu_buffer_rsrc_t srd_z = make_srd(p.zp ? p.zp + n_base * zp_row : nullptr, p.zp ? static_cast<uint64_t>(cols_left * zp_row) : 0);
     const uint32_t zp_mask = p.zp ? 0xfu : 0u, zp_default = p.zp ? 0u : 8u;
-    const bool scale_bf16 = p.scale_dtype == ROCM_DT_BF16;
-    const uint32_t mask = __builtin_amdgcn_mov_dpp(p.nibble_mask, 0xE4, 0xf, 0xf, false);
+    const bool scale_bf16 = rest.scale_dtype == ROCM_DT_BF16;
+    const uint32_t mask = __builtin_amdgcn_mov_dpp(opaque_scalar(0x000F000Fu), 0xE4, 0xf, 0xf, false), magic = opaque_scalar(0x64006400u);
 
     const uint32_t a_off = static_cast<uint32_t>(r) * static_cast<uint32_t>(p.k) * 4u;
     const bool row_live = r < rows_left;
@@ -125,9 +129,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     uint32_t b_off[CN], s_off[CN], z_off[CN];
 #pragma unroll
     for (int j = 0; j < CN; ++j) {                         // a column beyond N lies out of range by itself
-        b_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.row_bytes) + static_cast<uint32_t>(part * 4 * G);
+        b_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(row_bytes) + static_cast<uint32_t>(part * 4 * G);
         s_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.kb) * static_cast<uint32_t>(sizeof(ST));
-        z_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(p.zp_row);
+        z_off[j] = static_cast<uint32_t>(j * TILE + r) * static_cast<uint32_t>(zp_row);
     }
 
     struct Run {
@@ -227,7 +231,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
             const uint32_t zq = ((x.z[j] >> x.zsh) & zp_mask) | zp_default;
             uint4 w[G];
 #pragma unroll
-            for (int g = 0; g < G; ++g) w[g] = plain_nibbles<true>(x.b[j][g], zq, mask, p.magic);
+            for (int g = 0; g < G; ++g) w[g] = plain_nibbles<true>(x.b[j][g], zq, mask, magic);
             acc_t acc = zero;
 #pragma unroll
             for (int q = 2; q >= 0; --q)                                      // smallest parts first
@@ -242,6 +246,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
     Run x[DEPTH];
 #pragma unroll
     for (int d = 0; d < DEPTH - 1; ++d) request(x[d], u0 + d);
+    asm volatile("" : : "s"(rest.bias), "s"(rest.y), "s"(rest.bias_dtype), "s"(rest.y_dtype));      // there from here on, not read behind the last barrier
     for (int u = u0; u < u1; u += DEPTH) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
@@ -287,23 +292,23 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(GemmF32Params p)
 #pragma unroll
         for (int e = 0; e < Ops::kAcc; ++e) parts[((wave * CN + j) * Ops::kAcc + e) * 64 + lane] = sum[j][e];
     __syncthreads();
-    for (int i = t; i < kOuts; i += static_cast<int>(blockDim.x)) {
+    for (int i = t; i < kOuts; i += waves * 64) {
         float v = 0.f;
         for (int w = 0; w < waves; ++w) v += parts[w * kOuts + i];
         const int l = i & 63;
         const int64_t row = m_base + Ops::row_of((i >> 6) & (Ops::kAcc - 1), l);
         const int64_t col = n_base + (i / (Ops::kAcc * 64)) * TILE + (l & (TILE - 1));
-        if (row < p.m && col < p.n) store_from_f32(p.y, p.y_dtype, row * p.n + col, with_bias(v, p.bias, p.bias_dtype, row, p.n, col, p.y_dtype));
+        if (row < p.m && col < p.n) store_from_f32(rest.y, rest.y_dtype, row * p.n + col, with_bias(v, rest.bias, rest.bias_dtype, row, p.n, col, rest.y_dtype));
     }
 }
 
 template <int TILE, int CN, int DEPTH, int WAVES, typename ST, bool WHOLE>
-static int launch_gemm_f32(const GemmF32Params& p, int waves, hipStream_t stream)
+static int launch_gemm_f32(const GemmF32Params& p, const GemmF32Rest& rest, int waves, hipStream_t stream)
 {
-    const dim3 grid(static_cast<unsigned>((p.n + TILE * CN - 1) / (TILE * CN)), static_cast<unsigned>((p.m + TILE - 1) / TILE));
+    const dim3 grid(static_cast<unsigned>((static_cast<int64_t>(p.n) + TILE * CN - 1) / (TILE * CN)), static_cast<unsigned>((p.m + TILE - 1) / TILE));
     constexpr int kWaveLds = CN * TileOps<TILE>::kAcc * 256, kStageLds = WHOLE ? TILE * 128 : 0;
     const size_t lds = static_cast<size_t>(waves) * (kWaveLds > kStageLds ? kWaveLds : kStageLds);        // at most 64 KiB
-    hipLaunchKernelGGL((gemm_f32_kernel<TILE, CN, DEPTH, WAVES, ST, WHOLE>), grid, dim3(static_cast<unsigned>(waves * 64)), lds, stream, p);
+    hipLaunchKernelGGL((gemm_f32_kernel<TILE, CN, DEPTH, WAVES, ST, WHOLE>), grid, dim3(static_cast<unsigned>(waves * 64)), lds, stream, p.a, p.b, p.scales, p.zp, p.m, p.n, p.k, p.kb, p.bs_log2, p.units_per_wave, rest);
     return static_cast<int>(hipGetLastError());
 }
 
@@ -313,7 +318,7 @@ extern "C" int rocm_gemm_f32_eligible(const RocmMatMulNBitsArgs* a)
 {
     if (a->a_dtype != ROCM_DT_F32 || a->m < 1 || a->n < 1 || a->k < 1 || a->block_size < 32 || a->k % 4 != 0) return 0;
     const int64_t kb = (a->k + a->block_size - 1) / a->block_size;
-    if (kb * a->block_size / 2 * 64 >= 0x7ffffff0 || a->k * 4 * 32 >= 0x7ffffff0 || (a->m + 31) / 32 > 65535) return 0;    // 32-bit offsets inside one tile
+    if (kb * a->block_size / 2 * 64 >= 0x7ffffff0 || a->k * 4 * 32 >= 0x7ffffff0 || (a->m + 31) / 32 > 65535 || a->n > 0x7fffffff) return 0;    // 32-bit offsets inside one tile, 32-bit sizes
     return (reinterpret_cast<uintptr_t>(a->a) & 15) == 0 && (reinterpret_cast<uintptr_t>(a->b) & 7) == 0;
 }
 
@@ -325,8 +330,10 @@ namespace {
 //   * 32 x 32 otherwise, two of them per wave once single ones make more than one workgroup per CU: the cut activations are used
 //     twice (4864 -> 896 at 512 rows 39.5 against 44.3; at 200 rows, 196 workgroups, 35.3 against 23.4).
 //   * eight waves share K up to one workgroup per CU, four beyond (896 -> 9728 at 512 rows 62.5 against 80.5 us), each with two runs or more.
-// The lines were drawn before activations went through LDS and hold at these shapes; between them single tiles of eight waves can be the better ones
-// (896 -> 4864 at 200 rows, 1064 of them, 19.6 against 21.1).
+//   * between two and three single tiles per CU (five where K is at most 1536): single tiles of eight waves, of which a CU holds two workgroups at a time, where
+//     the last of the few rounds of double ones would be half empty (single / double, us: 896 -> 4864 at 100 / 200 / 256 rows, 2.4 / 4.2 / 4.8 a CU, 12.6 / 18.7 / 19.3
+//     against 15.1 / 20.4 / 21.8; 3584 -> 3584 at 150, 2.2, 37.3 against 42.4; 8960 -> 1536 at 400, 2.4, 98.8 against 109.0). Beyond they lose: 3584 -> 3584 at 200 rows,
+//     3.1, 48.9 against 44.5; 1536 -> 8960 at 150, 5.5, 34.2 against 31.5; 896 -> 4864 at 512, 9.5, 34.6 against 33.3.
 struct F32Plan { int tile, cn, waves; };
 F32Plan plan_gemm_f32(const RocmMatMulNBitsArgs* a, int units, int64_t cus)
 {
@@ -334,7 +341,9 @@ F32Plan plan_gemm_f32(const RocmMatMulNBitsArgs* a, int units, int64_t cus)
     F32Plan plan{32, 1, 8};
     if (workgroups(16, 16) <= cus) plan.tile = 16;
     else if (workgroups(32, 32) > cus) plan.cn = 2;
-    if (workgroups(plan.tile, plan.tile * plan.cn) > cus) plan.waves = 4;
+    const int64_t single = workgroups(32, 32);
+    if (single > 2 * cus && single <= (a->k <= 1536 ? 5 : 3) * cus) plan.cn = 1;
+    else if (workgroups(plan.tile, plan.tile * plan.cn) > cus) plan.waves = 4;
     while (plan.waves > 1 && units < 2 * plan.waves) plan.waves >>= 1;
     return plan;
 }
@@ -357,22 +366,14 @@ extern "C" int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* a, rocm_stream_t 
     p.b = a->b;
     p.scales = a->scales;
     p.zp = a->zp;
-    p.bias = a->bias;
-    p.y = a->y;
-    p.m = a->m;
-    p.n = a->n;
-    p.k = a->k;
-    p.kb = (a->k + a->block_size - 1) / a->block_size;
-    p.row_bytes = p.kb * a->block_size / 2;
-    p.zp_row = (p.kb + 1) / 2;
+    p.m = static_cast<int>(a->m);
+    p.n = static_cast<int>(a->n);
+    p.k = static_cast<int>(a->k);
+    p.kb = static_cast<int>((a->k + a->block_size - 1) / a->block_size);
     p.bs_log2 = __builtin_ctz(static_cast<unsigned>(a->block_size));
-    p.scale_dtype = a->scale_dtype;
-    p.nibble_mask = 0x000F000Fu;
-    p.magic = 0x64006400u;
-    p.bias_dtype = a->bias_dtype;
-    p.y_dtype = a->y_dtype;
+    const mnb::GemmF32Rest rest{a->bias, a->y, a->scale_dtype, a->bias_dtype, a->y_dtype};
     const int64_t cus = rocm_ffi_compute_units();
-    const int units = static_cast<int>(p.kb * a->block_size / 32);
+    const int units = static_cast<int>(static_cast<int64_t>(p.kb) * a->block_size / 32);
     const F32Plan plan = plan_gemm_f32(a, units, cus);
     const int tile = plan.tile, cn = plan.cn, waves = plan.waves;
     p.units_per_wave = (units + waves - 1) / waves;
@@ -380,8 +381,8 @@ extern "C" int rocm_launch_gemm_f32(const RocmMatMulNBitsArgs* a, rocm_stream_t 
     auto go = [&](auto st, auto whole) {
         using ST = decltype(st);
         constexpr bool W = decltype(whole)::value;
-        if (tile == 16) return mnb::launch_gemm_f32<16, 1, 4, 8, ST, W>(p, waves, s);
-        return cn == 2 ? mnb::launch_gemm_f32<32, 2, 2, 8, ST, W>(p, waves, s) : mnb::launch_gemm_f32<32, 1, 2, 8, ST, W>(p, waves, s);
+        if (tile == 16) return mnb::launch_gemm_f32<16, 1, 4, 8, ST, W>(p, rest, waves, s);
+        return cn == 2 ? mnb::launch_gemm_f32<32, 2, 2, 8, ST, W>(p, rest, waves, s) : mnb::launch_gemm_f32<32, 1, 2, 8, ST, W>(p, rest, waves, s);
     };
     if (a->k % a->block_size != 0) return a->scale_dtype == ROCM_DT_F32 ? go(float{}, std::false_type{}) : go(uint16_t{}, std::false_type{});
     return a->scale_dtype == ROCM_DT_F32 ? go(float{}, std::true_type{}) : go(uint16_t{}, std::true_type{});
