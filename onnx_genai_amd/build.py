@@ -5,12 +5,14 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "lib", "libnxrt_ep_rocm.so")
+CALLS = os.path.join(HERE, "_calls.so")              # the Python module that ep.py makes its calls through
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 HIP_SOURCES = [
@@ -112,6 +114,7 @@ def build(force: bool = True) -> str:
     if spilled:
         raise RuntimeError("kernels that use scratch memory:\n" + "\n".join(f"  {n}: {u}" for n, u in sorted(spilled.items())))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs, "-ldl", "-Wl,-z,defs", "-Wl,--exclude-libs,ALL"])
+    _run(["gcc", "-O2", "-std=c11", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "py", "calls.c"), "-o", CALLS])
     return LIB
 
 

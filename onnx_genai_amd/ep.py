@@ -17,6 +17,11 @@ import numpy as np
 
 from . import synth
 
+try:
+    from . import _calls
+except ImportError as missing:
+    raise ImportError(f"{os.path.dirname(os.path.abspath(__file__))}/_calls.so is not built; run `python -m onnx_genai_amd.build`") from missing
+
 F32, U8, I8, I32, F16, BF16 = 1, 2, 3, 6, 10, 16
 DEVICE_ROCM = 2
 _ITEM = {F32: 4, U8: 1, I8: 1, I32: 4, F16: 2, BF16: 2}
@@ -162,6 +167,7 @@ def load_library() -> C.CDLL:
     L.nxrt_rocm_ep_kernel_launch_count.argtypes = [v]
     L.nxrt_rocm_live_provider_count.restype = u64
     L.nxrt_rocm_live_provider_count.argtypes = []
+    L.execute_at = C.cast(L.nxrt_rocm_matmul_nbits_execute, v).value
     _lib = L
     return L
 
@@ -467,6 +473,13 @@ class MatMulNBitsKernel:
         return out.bytes, out.alignment
 
     def execute(self, inputs, outputs, workspace: DeviceBuffer | None = None) -> None:
+        if self.handle:
+            failed = _calls.execute(self.lib.execute_at, self.handle.value, inputs, outputs, workspace.ptr if workspace else 0, workspace.nbytes if workspace else 0)
+            if failed is None:
+                return
+            if failed:
+                raise EpError(failed[0], failed[1].decode("utf-8", "replace"))
+        # views with fields that are not plain integers
         buf, at = _packed_views((*inputs, *outputs))
         self.lib.nxrt_rocm_matmul_nbits_execute(self.handle, at, len(inputs), at + _VIEW_BYTES * len(inputs), len(outputs),
                                                 workspace.ptr if workspace else None, workspace.nbytes if workspace else 0).check()
