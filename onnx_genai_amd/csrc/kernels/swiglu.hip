@@ -4,6 +4,7 @@
 // the exponential taken in double and rounded to f32, and the product is rounded once. `decomposed` reproduces a graph
 // that spelled silu as Sigmoid and Mul: the sigmoid and x * sigmoid are each rounded to the 16-bit type.
 #include "swiglu.hiph"
+#include "weights_ahead.hiph"
 
 namespace mnb {
 
@@ -48,38 +49,14 @@ __device__ __forceinline__ float add_rotated(float x)
 }
 
 // STAGED: the row passes through LDS (K * 2 bytes of it); otherwise (rows beyond LDS) the sums read memory.
-// Blocks from `rows` on read weights that the launch behind this one streams, and keep nothing: while a row is normalized the memory is idle, and what they
-// read comes from the near cache later. Each XCD has its own: block b runs on XCD b % 8, as the workgroup of the next launch that reads the same bytes does. A
-// block asks for 32 KB at once (one block for all that a workgroup of the next launch reads, up to 305 KB, made the launch 2 us longer instead).
-struct WeightsAhead {
-    const uint4 *first, *second;    // the streams of one projection or two
-    uint32_t pieces;                // 16-byte pieces of each stream that one workgroup of the next launch reads
-    uint32_t from;                  // first block of these, a multiple of 8
-    uint32_t parts;                 // blocks that share such a workgroup's pieces of one stream
-    uint32_t workgroups;            // of the next launch that are read ahead, a multiple of 8
-};
-constexpr int kAheadInFlight = 8;
-__device__ __forceinline__ void read_ahead(const WeightsAhead& w)
-{
-    if (blockIdx.x < w.from) return;
-    const uint32_t each = w.parts * (w.second ? 2 : 1), j = blockIdx.x - w.from, turn = j / 8;
-    const uint32_t workgroup = turn / each * 8 + j % 8, part = turn % each;
-    const uint4* const from = (part < w.parts ? w.first : w.second) + static_cast<int64_t>(workgroup) * w.pieces;
-    const uint32_t piece = part % w.parts * (kAheadInFlight * 256) + threadIdx.x;
-    uint4 v[kAheadInFlight];
-#pragma unroll
-    for (int i = 0; i < kAheadInFlight; ++i) v[i] = from[min(piece + i * 256, w.pieces - 1)];
-#pragma unroll
-    for (int i = 0; i < kAheadInFlight; ++i) asm volatile("" : : "v"(v[i].x), "v"(v[i].y), "v"(v[i].z), "v"(v[i].w));
-}
-
+// Blocks from `rows` on read weights of the launch behind this one ahead: while a row is normalized the memory is idle.
 template <bool BF16, bool STAGED>
 __global__ __launch_bounds__(256) void rmsnorm16_kernel(const uint16_t* __restrict__ a, const void* __restrict__ gamma, uint16_t* __restrict__ out, int gamma_dtype, int64_t k, float epsilon,
                                                         uint32_t rows, WeightsAhead ahead)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     if (blockIdx.x >= rows) {
-        read_ahead(ahead);
+        read_ahead(ahead, blockIdx.x, 256);
         return;
     }
     const int t = threadIdx.x;
@@ -185,16 +162,7 @@ extern "C" int rocm_launch_rmsnorm16(const void* a, const void* gamma, int gamma
     const size_t lds = staged ? static_cast<size_t>(k) * 2 : 0;
     mnb::WeightsAhead w{};
     unsigned blocks = static_cast<unsigned>(rows);
-    if (ahead && ahead->first && ahead->bytes >= 16 && rows <= 64) {
-        w.first = static_cast<const uint4*>(ahead->first);
-        w.second = static_cast<const uint4*>(ahead->second);
-        w.pieces = static_cast<uint32_t>(ahead->bytes / 16);
-        w.from = (blocks + 7) / 8 * 8;
-        w.parts = (w.pieces + mnb::kAheadInFlight * 256 - 1) / (mnb::kAheadInFlight * 256);
-        const uint64_t streams = w.second ? 2 : 1, fit = static_cast<uint64_t>(mnb::kAheadBytes) / (ahead->bytes * streams);
-        w.workgroups = static_cast<uint32_t>(fit < ahead->workgroups ? fit : ahead->workgroups) / 8 * 8;
-        if (w.workgroups > 0) blocks = w.from + w.workgroups * w.parts * static_cast<uint32_t>(streams);
-    }
+    if (ahead && rows <= 64) blocks = static_cast<unsigned>(mnb::plan_weights_ahead(*ahead, mnb::kAheadBytes, 256, blocks, 0, &w));
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), lds, s, static_cast<const uint16_t*>(a), gamma, static_cast<uint16_t*>(out), gamma_dtype, k, epsilon, static_cast<uint32_t>(rows), w);
         return static_cast<int>(hipGetLastError());

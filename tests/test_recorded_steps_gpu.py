@@ -172,3 +172,15 @@ def test_a_step_of_layers(ep):
             calls.append((Node(ep, k, n, bs, dt, 10 * layer + i), reads[name], out[name].ptr, m))
         x = out["down"].ptr
     check(ep, calls, 8)
+
+
+@pytest.mark.parametrize("m,dt,bs", [(1, E.F16, 32), (3, E.BF16, 128), (9, E.BF16, 64)])
+def test_a_chain_that_reads_weights_ahead(ep, m, dt, bs):
+    """Each launch reads weights of the next: grids that do not end on a multiple of eight workgroups, next ones of fewer than eight, streams longer than a block's share, and pairs
+    of nodes behind a launch."""
+    widths = [896, 304, 72, 1000, 16, 4096, 896]
+    buffers = [rows(ep, m, widths[0], dt, 5)] + [ep.allocate(m * n * 2) for n in widths[1:]]
+    calls = [(Node(ep, k, n, bs, dt, i), buffers[i].ptr, buffers[i + 1].ptr, m) for i, (k, n) in enumerate(zip(widths, widths[1:]))]
+    side = ep.allocate(m * 304 * 2)
+    calls.insert(6, (Node(ep, 4096, 304, bs, dt, 9), buffers[5].ptr, side.ptr, m))
+    check(ep, calls, 6)
