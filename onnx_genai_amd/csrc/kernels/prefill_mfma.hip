@@ -28,14 +28,16 @@ namespace mnb {
 // BITS: 4, or 8 (bytes of B are weights; zero points are bytes, 128 when absent): the bytes are dequantized on their way to LDS like
 // nibbles, instead of by a launch that writes all of B as 16 bits first (bf16, block 128, 500 rows: 3584 -> 37888 391 -> 208 us, 18944 -> 3584
 // 197 -> 103; 65 rows 262 -> 90 and 180 -> 50), and the 256 x 256 tile and slices of K are open to them.
-template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false, int BITS = 4>
-__global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
+// MW: waves along M (the other 8 / MW lie along N). m_base: first row of the tile.
+template <bool BF16, int BM, int BN, bool SF32, bool DENSE, int BITS, int MW>
+__device__ __forceinline__ void prefill_body(const PrefillParams& p, int64_t m_base)
 {
     static_assert(BITS == 4 || (BITS == 8 && !DENSE && !SF32), "packed weights of 4 bits, or of 8 with 16-bit scales");
     static_assert(!DENSE || (BN <= 128 && !SF32), "dense weights: four times the bytes per column, so only the narrower tiles have the registers");
     constexpr bool F32MATH = BF16 || SF32;
-    constexpr int WM = BM / 4;             // wave sub-tile rows
-    constexpr int WN = BN / 2;             // and columns
+    constexpr int NW = 8 / MW;
+    constexpr int WM = BM / MW;            // wave sub-tile rows
+    constexpr int WN = BN / NW;            // and columns
     constexpr int TM = WM / 32;            // 32x32 MFMA tiles per wave along M
     constexpr int TN = WN / 32;            // and along N
     constexpr int A_LOADS = BM / 64;       // 16-byte pieces of A per lane per step
@@ -51,10 +53,9 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
     const int t = threadIdx.x;
     const int lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = wave >> 1, wn = wave & 1;      // 4 x 2 waves
+    const int wm = wave / NW, wn = wave % NW;
     // Column blocks vary fastest: the workgroups running at one time share a few row blocks of A (each XCD's L2 then
     // holds them once) and sweep the small packed B.
-    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * BM;
     const int64_t n_base = static_cast<int64_t>(blockIdx.x) * BN;
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
 
@@ -258,6 +259,27 @@ __global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
     }
 
     store_tile<TM, TN>(p, acc, m_base, n_base, wm * WM, wn * WN, lane, wave, smem);
+}
+
+// A last row block of at most kTailRows rows of the 256 x 256 build is a tile of 64 x 256 with its eight waves side by side: a quarter of the multiplications, A and
+// LDS traffic of a whole tile, and what is left is bringing 256 columns of weights to LDS. It sums in the whole tile's order, so the bits are the same. Whole tile -> this, us (auto plan):
+// f16, block 32, 4096 -> 14336 at 777 / 2057 rows 115.7 -> 109.1, 250.6 -> 244.4, 14336 -> 4096 at 4105 rows 654 -> 606; bf16, block 128, 3584 -> 37888
+// at 777 / 1300 / 1545 / 2057 rows 305 / 424 / 521 / 633 -> 264 / 381 / 435 / 553; calls without such a block are level. (Bodies for four, two and one live
+// waves of the 4 x 2 layout spilled.)
+constexpr int kTailRows = 64;
+__host__ __device__ constexpr bool has_tail_tile(int bm, int bn) { return bm == 256 && bn == 256; }
+
+template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false, int BITS = 4>
+__global__ __launch_bounds__(512) void prefill_mfma_kernel(PrefillParams p)
+{
+    const int64_t m_base = static_cast<int64_t>(blockIdx.y) * BM;
+    if constexpr (has_tail_tile(BM, BN)) {
+        if (p.m - m_base <= kTailRows) {
+            prefill_body<BF16, kTailRows, BN, SF32, DENSE, BITS, 1>(p, m_base);
+            return;
+        }
+    }
+    prefill_body<BF16, BM, BN, SF32, DENSE, BITS, 4>(p, m_base);
 }
 
 // Y = sum over slices of the partial sums, in slice order, plus bias; one thread per element.
