@@ -247,6 +247,8 @@ uint64_t rocm_prefill_mfma_scratch_bytes(const RocmMatMulNBitsArgs* args, int ti
 /* The plan rocm_launch_prefill_mfma would follow with `scratch_bytes` of scratch: the tile and the slices of K (no GPU work;
  * only the shape, dtype and pointer alignment of `args` are read). -1: shape not eligible. */
 int rocm_prefill_mfma_plan(const RocmMatMulNBitsArgs* args, int tile_choice, uint64_t scratch_bytes, int* tile_rows, int* tile_cols, int* slices);
+/* How many of the call's last columns go to smaller tiles in a launch of their own (0: none), and that tile. */
+int64_t rocm_prefill_mfma_rest(const RocmMatMulNBitsArgs* args, int tile_choice, uint64_t scratch_bytes, int* tile_rows, int* tile_cols);
 /* Y = sum over `slices` of partial[slice][M][N] (f32), in slice order, + bias. */
 int rocm_launch_slice_reduce(const float* partial, int slices, int64_t m, int64_t n, const void* bias, int bias_dtype, void* y, int y_dtype,
                              rocm_stream_t stream);

@@ -56,7 +56,7 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& p, int64_t m_b
     const int wm = wave / NW, wn = wave % NW;
     // Column blocks vary fastest: the workgroups running at one time share a few row blocks of A (each XCD's L2 then
     // holds them once) and sweep the small packed B.
-    const int64_t n_base = static_cast<int64_t>(blockIdx.x) * BN;
+    const int64_t n_base = p.first_col + static_cast<int64_t>(blockIdx.x) * BN;
     const int64_t rows_left = p.m - m_base, cols_left = p.n - n_base;
 
     const __amdgpu_buffer_rsrc_t srd_a = make_srd(p.a + m_base * p.k, static_cast<uint64_t>(rows_left * p.k) * 2);
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
 template <bool BF16, int BM, int BN, bool SF32, bool DENSE = false, int BITS = 4>
 static int launch_prefill(const PrefillParams& p, int splits, hipStream_t stream)
 {
-    const dim3 grid(static_cast<unsigned>((p.n + BN - 1) / BN), static_cast<unsigned>((p.m + BM - 1) / BM), static_cast<unsigned>(splits));
+    const dim3 grid(static_cast<unsigned>((p.cols + BN - 1) / BN), static_cast<unsigned>((p.m + BM - 1) / BM), static_cast<unsigned>(splits));
     const size_t lds = 2 * static_cast<size_t>(BM + BN) * kPitch;
     auto kernel = prefill_mfma_kernel<BF16, BM, BN, SF32, DENSE, BITS>;
     if (lds > 65536) {
@@ -327,12 +327,14 @@ struct PrefillPlan {
     int tile;        // 0: 128 x 128, 1: 256 x 128, 2: 256 x 256, 3: 128 x 64
     int splits;      // slices of K (1 = none)
     int steps_per_split;
+    int rest_tile;   // tile of the columns from whole_cols on, by a launch of their own, or -1: none
+    int64_t whole_cols;
 };
 
 // The largest tile that still gives every CU a workgroup: 256 x 256, then 256 x 128, 128 x 128. If 128 x 128 tiles leave
 // CUs idle, K is cut into slices over grid.z (measured at M = 512: 18944 -> 3584 113 us against 134 us with 128 x 64
 // tiles in slices; 14336 -> 4096 106 against 111 us); shapes too short for that take 128 x 64 tiles, sliced if they can be.
-PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t scratch_bytes)
+PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t scratch_bytes, bool dense = false)
 {
     const int steps = static_cast<int>(a->k / 64);
     const int64_t cus = rocm_ffi_compute_units();      // (256 where no device can be asked: the plan of a host without a GPU is the MI355X's)
@@ -352,8 +354,28 @@ PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t
         while (want > 1 && static_cast<uint64_t>(want) * per_split > scratch_bytes) --want;
         return want < 1 ? 1 : want;
     };
+    // 256 x 256 tiles beyond the last whole round of the CUs last as long as a round (one such workgroup holds a CU). Where those columns in smaller tiles fit the chip, one
+    // workgroup to a CU, they are a launch of their own: 128 x 64 before 128 x 128 before 256 x 128. Same sums, same bits. The plan without it -> this, us: bf16, block 128,
+    // 3584 -> 37888 at 300 / 512 / 1024 / 1536 / 4096 rows 158 / 201 / 314 / 424 / 1066 -> 127 / 154 / 279 / 401 / 1028 (8 bits at 500: 202 -> 156), f16, block 32, 4096 -> 14336 at
+    // 1280 / 1536 / 2560 rows 217 / 216 / 343 -> 169 / 194 / 308, 14336 -> 4096 at 4352 / 5000 667 / 684 -> 546 / 634. With two to a CU it loses: 14336 -> 4096 at 6144 rows
+    // 792 -> 928, 3584 -> 37888 at 768 rows 229 -> 250, at 2048 574 -> 592. 256 x 128 tiles are left out beyond six rounds, when workgroups have drifted apart and
+    // a second launch has to wait for the last: 4096 -> 28672 at 4352 rows 975 -> 1015. (Over 232 calls of 257 to 5000 rows: mean 0.965, the others level.)
+    const int64_t whole = workgroups(2) / cus * cus / ((a->m + 255) / 256) * 256;
+    int rest_tile = -1;
+    int64_t rest_workgroups = 0;
+    if (!dense && tile_choice <= 0 && workgroups(2) % cus != 0 && whole > 0 && whole < a->n) {
+        const int small[3][3] = {{3, 128, 64}, {0, 128, 128}, {1, 256, 128}};
+        for (const auto& t : small) {
+            rest_workgroups = ((a->m + t[1] - 1) / t[1]) * ((a->n - whole + t[2] - 1) / t[2]);
+            if (rest_workgroups > cus || (t[0] == 1 && workgroups(2) / cus > 6)) continue;
+            rest_tile = t[0];
+            break;
+        }
+    }
     PrefillPlan plan;
     plan.splits = 1;
+    plan.rest_tile = -1;
+    plan.whole_cols = a->n;
     if (tile_choice >= 1 && tile_choice <= 4) {
         plan.tile = tile_choice == 4 ? 3 : tile_choice - 1;
         plan.splits = slices(plan.tile);
@@ -383,8 +405,8 @@ PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t
     // and 15 % at worst; the rule above alone is 13 % and 41 %.
     if (tile_choice <= 0 && a->m >= 256) {
         const bool bf16 = a->a_dtype == ROCM_DT_BF16;
+        static const double step_us[4] = {0.78, 1.42, 2.52, 0.45};
         auto modelled = [&](int tile, int splits) {
-            static const double step_us[4] = {0.78, 1.42, 2.52, 0.45};
             const int occ = tile == 3 ? 2 : (tile == 0 && !bf16) ? 2 : 1;                 // workgroups per CU
             const int sps = (steps + splits - 1) / splits;
             const int sl = (steps + sps - 1) / sps;
@@ -396,6 +418,9 @@ PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t
             else if (rem > 0) t += work * (0.4 + 0.6 * rem / static_cast<double>(cus)) + 8.0;
             if (sl > 1) t += sl * static_cast<double>(a->m) * static_cast<double>(a->n) * 4.0 / 4e6 + 3.0;
             return t;
+        };
+        auto modelled_with_rest = [&] {
+            return workgroups(2) / cus * (steps * step_us[2] + 8.0) + steps * step_us[rest_tile] * (0.4 + 0.6 * rest_workgroups / static_cast<double>(cus)) + 8.0;
         };
         double best = modelled(plan.tile, plan.splits) * 0.97;
         const PrefillPlan base = plan;
@@ -411,9 +436,17 @@ PrefillPlan plan_prefill(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t
                 }
             }
         }
+        if (rest_tile >= 0 && modelled_with_rest() < best) {
+            plan.tile = 2;
+            plan.splits = 1;
+        }
     }
     plan.steps_per_split = (steps + plan.splits - 1) / plan.splits;
     plan.splits = (steps + plan.steps_per_split - 1) / plan.steps_per_split;
+    if (plan.tile == 2 && plan.splits == 1 && rest_tile >= 0) {
+        plan.rest_tile = rest_tile;
+        plan.whole_cols = whole;
+    }
     return plan;
 }
 
@@ -436,7 +469,18 @@ extern "C" int rocm_prefill_mfma_plan(const RocmMatMulNBitsArgs* a, int tile_cho
     return 0;
 }
 
-// The launch of both entry points below. `dense`: a->b is a [N, K] matrix of the activations' 16-bit type instead of packed weights.
+// How many of the last columns a launch of their own computes (0: none), and its tile.
+extern "C" int64_t rocm_prefill_mfma_rest(const RocmMatMulNBitsArgs* a, int tile_choice, uint64_t scratch_bytes, int* tile_rows, int* tile_cols)
+{
+    if (!rocm_prefill_mfma_eligible(a)) return -1;
+    const PrefillPlan plan = plan_prefill(a, tile_choice, scratch_bytes);
+    if (plan.rest_tile < 0) return 0;
+    if (tile_rows) *tile_rows = plan.rest_tile == 1 ? 256 : 128;
+    if (tile_cols) *tile_cols = plan.rest_tile == 3 ? 64 : 128;
+    return a->n - plan.whole_cols;
+}
+
+// The launches of the entry points below. `dense`: a->b is a [N, K] matrix of the activations' 16-bit type instead of packed weights.
 static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int bits, int tile_choice, void* scratch, uint64_t scratch_bytes, rocm_stream_t stream)
 {
     mnb::PrefillParams p;
@@ -458,9 +502,11 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int bits, int 
     p.y_dtype = a->y_dtype;
     p.nibble_mask = 0x000F000Fu;
     p.magic = a->a_dtype == ROCM_DT_BF16 ? 0x43004300u : 0x64006400u;
-    PrefillPlan plan = plan_prefill(a, tile_choice, scratch ? scratch_bytes : 0);
+    PrefillPlan plan = plan_prefill(a, tile_choice, scratch ? scratch_bytes : 0, dense);
     if (dense && plan.tile == 2) plan.tile = 1;          // dense weights: no 256 x 256 build (four times the bytes per column in registers)
     p.steps_per_split = plan.steps_per_split;
+    p.first_col = 0;
+    p.cols = a->n;
     p.partial = plan.splits > 1 ? static_cast<float*>(scratch) : nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool bf16 = a->a_dtype == ROCM_DT_BF16;
@@ -485,13 +531,22 @@ static int launch_tiled(const RocmMatMulNBitsArgs* a, bool dense, int bits, int 
         if (plan.tile == 3) return mnb::launch_prefill<B, 128, 64, false, false, 8>(p, plan.splits, s);
         return mnb::launch_prefill<B, 128, 128, false, false, 8>(p, plan.splits, s);
     };
-    int rc;
-    if (bits == 8) rc = bf16 ? go8(std::true_type{}) : go8(std::false_type{});
-    else if (dense) rc = bf16 ? go_dense(std::true_type{}) : go_dense(std::false_type{});
-    else if (bf16 && sf32) rc = go(std::true_type{}, std::true_type{});
-    else if (bf16) rc = go(std::true_type{}, std::false_type{});
-    else if (sf32) rc = go(std::false_type{}, std::true_type{});
-    else rc = go(std::false_type{}, std::false_type{});
+    auto start = [&] {
+        if (bits == 8) return bf16 ? go8(std::true_type{}) : go8(std::false_type{});
+        if (dense) return bf16 ? go_dense(std::true_type{}) : go_dense(std::false_type{});
+        if (bf16) return sf32 ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+        return sf32 ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+    };
+    if (plan.rest_tile >= 0) {
+        p.cols = plan.whole_cols;
+        const int rc = start();
+        if (rc != 0) return rc;
+        p.first_col = plan.whole_cols;
+        p.cols = a->n - plan.whole_cols;
+        plan.tile = plan.rest_tile;
+        return start();
+    }
+    const int rc = start();
     if (rc != 0 || plan.splits == 1) return rc;
     return rocm_launch_slice_reduce(static_cast<const float*>(scratch), plan.splits, a->m, a->n, a->bias, a->bias_dtype, a->y, a->y_dtype, stream);
 }
