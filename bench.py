@@ -180,6 +180,7 @@ class Node:
         self.y = ep.allocate(m * n * 2)
         self.bytes = synth.algorithmic_bytes(m, n, k, bs, a_dtype=a_dt, scale_dtype=a_dt, zero_points=zero_points)
         self.flops = synth.matmul_flops(m, n, k)
+        self.own_input, self.inputs = True, {}   # a copy of its input for this node: nodes of a recorded graph that read one buffer would share a launch
         self.workspace = None
         if accuracy_level == 4:
             need, _ = self.ops.kernel.workspace_requirement([((m, k), a_dt)])
@@ -187,10 +188,17 @@ class Node:
 
     def run(self, a_buf):
         out = [E.TensorView(self.y.ptr, self.a_dt, (self.m, self.n), device_index=self.ops.ep.device_index)]
+        if self.own_input and self.m <= 16:
+            if self.m not in self.inputs:            # (by rows: a sweep changes them)
+                self.inputs[self.m] = self.ops.ep.upload(self.ops.ep.download(a_buf, (self.m, self.k), E._NP[self.a_dt]))
+            a_buf = self.inputs[self.m]
+            assert a_buf.nbytes >= self.m * self.k * 2
         self.ops.kernel.execute(self.ops.views(a_buf, self.a_dt, self.m), out, workspace=self.workspace)
 
     def free(self, ep):
         ep.deallocate(self.y)
+        for a in self.inputs.values():
+            ep.deallocate(a)
         if self.workspace:
             ep.deallocate(self.workspace)
         self.ops.free()
@@ -239,7 +247,9 @@ def small_model_step(ep):
     hidden, inter, vocab, layers, kv = 896, 4864, 151936, 24, 128
     shapes = [("q", hidden, hidden), ("k", hidden, kv), ("v", hidden, kv), ("o", hidden, hidden),
               ("gate", hidden, inter), ("up", hidden, inter), ("down", inter, hidden)]
-    a_bufs = {k: ep.upload(synth.make_activation(1, k, 6, E.F16)) for k in (hidden, inter)}
+    # q, k and v read one input, and gate and up one; o, down and lm_head their own
+    read = {"q": "x", "k": "x", "v": "x", "gate": "h", "up": "h"}
+    inputs = {name: ep.upload(synth.make_activation(1, inter if name == "down" else hidden, 6, E.F16)) for name in ("x", "o", "h", "down", "lm_head")}
     nodes, reuse = [], {}
     for layer in range(layers):
         for name, k, n in shapes:
@@ -249,10 +259,13 @@ def small_model_step(ep):
             nodes.append(node)
     nodes.append(Node(ep, "lm_head", hidden, vocab, 32, 98, E.F16, 1))
     nodes[-1].host_b = None
+    of_node = [inputs[read.get(name, name)] for name in [name for name, _, _ in shapes] * layers + ["lm_head"]]
+    for node in nodes:
+        node.own_input = False
 
     def one_step():
-        for node in nodes:
-            node.run(a_bufs[node.k])
+        for node, a in zip(nodes, of_node):
+            node.run(a)
 
     one_step()
     ep.sync()
@@ -267,7 +280,7 @@ def small_model_step(ep):
            "kernel_variants": sorted({n.ops.kernel.last_variant() for n in nodes})}
     for node in nodes:
         node.free(ep)
-    for buf in a_bufs.values():
+    for buf in inputs.values():
         ep.deallocate(buf)
     return out
 
