@@ -180,6 +180,19 @@ typedef struct RocmStepTail RocmStepTail;
 RocmStepTail* rocm_step_tail_create(void);
 void rocm_step_tail_destroy(RocmStepTail* tail);
 void rocm_step_tail_reset(RocmStepTail* tail);
+/* What workgroup (x, y) of the one launch of `nodes` nodes (1 .. 4, in the order of their calls) reads of their repacked copies, `stream` bytes to 16 columns:
+ * `bytes` from `first`, 0 where it has no columns. No GPU work and nothing dereferenced. -1: these do not share a launch. */
+typedef struct RocmStepNodes {
+  int nodes;
+  int columns[4];
+  const void* packed[4];
+  uint32_t stream;
+} RocmStepNodes;
+typedef struct RocmStepReads {
+  uint32_t grid, rows;        /* of the launch */
+  uint64_t first, bytes;
+} RocmStepReads;
+int rocm_step_reads(const RocmStepNodes* launch, uint32_t x, uint32_t y, RocmStepReads* out);
 
 /* Decode over constant weights repacked for streaming (M <= 4). `packed` holds rocm_decode_packed_bytes() bytes and is
  * filled once by rocm_launch_pack_decode from args->b / scales / zp; rocm_launch_decode_packed then reads only it.

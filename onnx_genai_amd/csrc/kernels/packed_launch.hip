@@ -127,6 +127,25 @@ bool reads_ahead(const PackedLaunch& before, const PackedLaunch& next, PackedLau
     return out->p.rest.ahead.workgroups != 0 && grid_rows(*out) <= 65535;
 }
 
+// The launch of `nodes`, as one after the other would be recorded.
+bool launch_of(const RocmStepNodes& nodes, PackedLaunch* out)
+{
+    for (int i = 0; i < nodes.nodes; ++i) {
+        PackedLaunch one{};
+        one.p.packed = static_cast<const uint8_t*>(nodes.packed[i]);
+        one.p.n = nodes.columns[i];
+        one.p.split = 1u << 24;
+        one.p.rest.nodes[0] = PackedNode{nullptr, nullptr, one.p.packed, one.p.n, ROCM_DT_F32};
+        one.grid = (static_cast<unsigned>(one.p.n) + 15u) / 16u;
+        one.nodes = 1;
+        one.stream = nodes.stream;
+        const PackedLaunch before = *out;
+        if (i == 0) *out = one;
+        else if (!joined(before, one, out)) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 int start_packed(const PackedLaunch& launch, hipStream_t stream, RocmStepTail* tail)
@@ -189,4 +208,18 @@ extern "C" void rocm_step_tail_reset(RocmStepTail* tail)
     if (!tail) return;
     std::lock_guard<std::mutex> lock(tail->mu);
     tail->node = tail->before = nullptr;
+}
+extern "C" int rocm_step_reads(const RocmStepNodes* nodes, uint32_t x, uint32_t y, RocmStepReads* out)
+{
+    mnb::PackedLaunch launch{};
+    if (nodes->nodes < 1 || nodes->nodes > mnb::kMaxNodes || !mnb::launch_of(*nodes, &launch)) return -1;
+    const mnb::PackedParams& p = launch.p;
+    *out = RocmStepReads{launch.grid, p.rows(), 0, 0};
+    if (x >= out->grid || y >= out->rows) return -1;
+    const int n = y == 0 ? p.n : y == 1 ? p.n_up : p.rest.nodes[y].n;                          // (as the kernel finds them)
+    const uint8_t* const packed = y == 0 ? p.packed : y == 1 ? p.packed_up : p.rest.nodes[y].packed;
+    if (!mnb::has_columns(x, n)) return 0;
+    out->first = reinterpret_cast<uintptr_t>(packed) + static_cast<uint64_t>(x) * launch.stream;
+    out->bytes = launch.stream;
+    return 0;
 }

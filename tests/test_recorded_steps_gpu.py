@@ -184,3 +184,13 @@ def test_a_chain_that_reads_weights_ahead(ep, m, dt, bs):
     side = ep.allocate(m * 304 * 2)
     calls.insert(6, (Node(ep, 4096, 304, bs, dt, 9), buffers[5].ptr, side.ptr, m))
     check(ep, calls, 6)
+
+
+@pytest.mark.parametrize("m,dt,bs", [(1, E.F16, 32), (3, E.BF16, 128), (16, E.BF16, 64)])
+def test_a_narrow_node_may_come_first(ep, m, dt, bs):
+    """k, v, q: the rows of the first nodes end long before the grid does."""
+    k = 896
+    x = rows(ep, m, k, dt, 7)
+    nodes = [Node(ep, k, n, bs, dt, n, bias=bias) for n, bias in ((16, "row"), (130, None), (1000, "row"))]
+    y = [ep.allocate(m * node.n * 2) for node in nodes]
+    check(ep, [(node, x.ptr, out.ptr, m) for node, out in zip(nodes, y)], 1)
