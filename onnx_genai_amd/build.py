@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import os
 import re
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -12,7 +13,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "lib", "libnxrt_ep_rocm.so")
-CALLS = os.path.join(HERE, "_calls.so")              # the Python module that ep.py makes its calls through
+# The Python module that ep.py makes its calls through, named for the interpreter whose layout it is built for (another one does not find it)
+CALLS = os.path.join(HERE, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 HIP_SOURCES = [
@@ -89,6 +91,18 @@ def _run(cmd):
     return _resource_usage(r.stderr)
 
 
+def _build_calls():
+    """The native call path of ep.py. Without a C compiler or the interpreter's headers it is left out: ep.py's calls go through ctypes then."""
+    for old in {CALLS, os.path.join(HERE, "_calls.so")}:         # (a name without the interpreter's tag fits every one)
+        if os.path.exists(old):
+            os.remove(old)
+    include = sysconfig.get_paths()["include"]
+    if shutil.which("gcc") is None or not os.path.exists(os.path.join(include, "Python.h")):
+        sys.stderr.write(f"{CALLS} is not built: it needs gcc and {include}/Python.h\n")
+        return
+    _run(["gcc", "-O2", "-std=c11", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I", include, os.path.join(CSRC, "py", "calls.c"), "-o", CALLS])
+
+
 def build(force: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
@@ -114,7 +128,7 @@ def build(force: bool = True) -> str:
     if spilled:
         raise RuntimeError("kernels that use scratch memory:\n" + "\n".join(f"  {n}: {u}" for n, u in sorted(spilled.items())))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB, *objs, "-ldl", "-Wl,-z,defs", "-Wl,--exclude-libs,ALL"])
-    _run(["gcc", "-O2", "-std=c11", "-fPIC", "-shared", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "py", "calls.c"), "-o", CALLS])
+    _build_calls()
     return LIB
 
 

@@ -9,6 +9,7 @@ fallback: if the library is missing or no GPU is visible, construction raises.
 from __future__ import annotations
 
 import ctypes as C
+import importlib
 import os
 import struct
 from dataclasses import dataclass
@@ -18,9 +19,9 @@ import numpy as np
 from . import synth
 
 try:
-    from . import _calls
-except ImportError as missing:
-    raise ImportError(f"{os.path.dirname(os.path.abspath(__file__))}/_calls.so is not built; run `python -m onnx_genai_amd.build`") from missing
+    _calls = importlib.import_module("._calls", __package__)
+except ModuleNotFoundError:      # a tree not built for this interpreter: every call is packed here and goes through ctypes
+    _calls = None
 
 F32, U8, I8, I32, F16, BF16 = 1, 2, 3, 6, 10, 16
 DEVICE_ROCM = 2
@@ -473,13 +474,13 @@ class MatMulNBitsKernel:
         return out.bytes, out.alignment
 
     def execute(self, inputs, outputs, workspace: DeviceBuffer | None = None) -> None:
-        if self.handle:
+        if _calls is not None and self.handle:
             failed = _calls.execute(self.lib.execute_at, self.handle.value, inputs, outputs, workspace.ptr if workspace else 0, workspace.nbytes if workspace else 0)
             if failed is None:
                 return
             if failed:
                 raise EpError(failed[0], failed[1].decode("utf-8", "replace"))
-        # views with fields that are not plain integers
+        # views with fields that are not plain integers, or no native path
         buf, at = _packed_views((*inputs, *outputs))
         self.lib.nxrt_rocm_matmul_nbits_execute(self.handle, at, len(inputs), at + _VIEW_BYTES * len(inputs), len(outputs),
                                                 workspace.ptr if workspace else None, workspace.nbytes if workspace else 0).check()

@@ -1,10 +1,15 @@
 """The native call path of ep.py: the records that reach the C ABI are those of the packed views, and what is not plain is left alone."""
 import ctypes as C
+import os
+import shutil
 import subprocess
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
 
+from onnx_genai_amd import build
 from onnx_genai_amd import ep as E
 
 SOURCE = r"""
@@ -79,3 +84,49 @@ def test_what_is_not_plain_is_left_alone(recorder, view):
     assert call(recorder, iter([]), []) is False
     assert call(recorder, [E.TensorView.absent()] * 17, []) is False
     assert C.c_int.in_dll(recorder, "used").value == -1
+
+
+def execute(lib, inputs, outputs, workspace=None):
+    """The public execute of a kernel whose library is the recorder; -> what the recorder saw."""
+    kernel = E.MatMulNBitsKernel.__new__(E.MatMulNBitsKernel)
+    lib.execute_at = C.cast(lib.record, C.c_void_p).value
+    lib.nxrt_rocm_matmul_nbits_execute = lib.record
+    lib.record.restype = E.NxrtStatus
+    lib.record.argtypes = [C.c_void_p, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint64]
+    kernel.lib, kernel.handle = lib, C.c_void_p(0x77)
+    kernel.execute(inputs, outputs, workspace)
+    return list((C.c_int64 * C.c_int.in_dll(lib, "used").value).in_dll(lib, "seen"))
+
+
+def test_calls_without_the_native_path_are_the_same(recorder, monkeypatch):
+    inputs = [E.TensorView(0x1000, E.F32, (2, 3, 896)), E.TensorView.absent(E.U8), E.TensorView(0x2000, E.BF16, (4, 8), strides=(-16, 2), byte_offset=32)]
+    outputs, workspace = [E.TensorView(0x5000, E.F16, (1, 4))], E.DeviceBuffer(0x9000, 512)
+    want = execute(recorder, inputs, outputs, workspace)
+    code = C.c_uint32.in_dll(recorder, "code")
+    messages = []
+    for native in (E._calls, None):
+        monkeypatch.setattr(E, "_calls", native)
+        assert execute(recorder, inputs, outputs, workspace) == want
+        code.value = 3
+        try:
+            with pytest.raises(E.EpError) as failed:
+                execute(recorder, inputs, outputs)
+        finally:
+            code.value = 0
+        messages.append((failed.value.code, failed.value.message))
+    assert messages == [(3, "wrong")] * 2
+
+
+def test_the_package_imports_in_a_tree_that_is_not_built(tmp_path):
+    """Only loading the library asks for a build; a module of another interpreter's name is not taken."""
+    package = tmp_path / "onnx_genai_amd"
+    shutil.copytree(build.HERE, package, ignore=lambda where, names: [n for n in names if n in ("build", "lib", "csrc", "__pycache__") or n.endswith(".so")])
+    (package / "_calls.cpython-399-x86_64-linux-gnu.so").write_bytes(b"of another interpreter")
+    code = "from onnx_genai_amd import ep\nassert ep._calls is None and ep.__file__.startswith({!r}), ep.__file__\ntry:\n    ep.load_library()\nexcept (OSError, RuntimeError) as e:\n    print('refused', e)"
+    env = {k: v for k, v in os.environ.items() if k not in ("NXRT_ROCM_LIBRARY", "PYTHONPATH")}
+    out = subprocess.run([sys.executable, "-c", code.format(str(tmp_path))], cwd=tmp_path, env=env, capture_output=True, text=True)
+    assert out.returncode == 0 and "refused" in out.stdout, out.stdout + out.stderr
+
+
+def test_the_module_carries_its_interpreter():
+    assert E._calls.__file__ == build.CALLS and build.CALLS.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
