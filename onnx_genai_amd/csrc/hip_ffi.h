@@ -123,8 +123,6 @@ int rocm_dense_gemm_run(RocmDenseGemm* g, const void* w_nk, const void* a, void*
  * (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4207-4233, 4375-4386). decomposed = 1: silu spelled as Sigmoid and Mul. */
 int rocm_launch_swiglu(const void* gate, const void* up, int64_t count, int dtype, int decomposed, void* y, rocm_stream_t stream);
 
-/* out = round16((a * inv_std) * gamma) per row of K 16-bit elements (K % 128 == 0), inv_std = 1 / sqrt(mean(a^2) + eps),
- * summed in the reference's order (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4125-4205). gamma: f32 or 16-bit. */
 /* The repacked weights that the launch after a normalization streams: workgroup w of it reads `bytes` from first + w * bytes, and as many of `second`
  * where that is not NULL (device pointers, 16-byte aligned; workgroups * bytes lie within each). */
 typedef struct RocmWeightsAhead {
@@ -133,6 +131,9 @@ typedef struct RocmWeightsAhead {
   uint64_t bytes;
   uint32_t workgroups;
 } RocmWeightsAhead;
+/* out = round16((a * inv_std) * gamma) per row of K 16-bit elements (K % 128 == 0), inv_std = 1 / sqrt(mean(a^2) + eps),
+ * summed in the reference's order (onnx-runtime-ep-cuda/src/kernels/matmul_nbits.rs:4125-4205). gamma: f32 or 16-bit. `ahead`: NULL, or what
+ * further blocks of the launch read meanwhile. */
 int rocm_launch_rmsnorm16(const void* a, const void* gamma, int gamma_dtype, int64_t rows, int64_t k, float epsilon, int dtype, void* out,
                           const RocmWeightsAhead* ahead, rocm_stream_t stream);
 
@@ -180,21 +181,25 @@ typedef struct RocmStepTail RocmStepTail;
 RocmStepTail* rocm_step_tail_create(void);
 void rocm_step_tail_destroy(RocmStepTail* tail);
 void rocm_step_tail_reset(RocmStepTail* tail);
-/* What workgroup (x, y) of the one launch of `nodes` nodes (1 .. 4, in the order of their calls) reads of their repacked copies, `stream` bytes to 16 columns:
- * `bytes` from `first`, 0 where it has no columns. No GPU work and nothing dereferenced. -1: these do not share a launch. */
+/* What workgroup (x, y) of the one launch of `nodes` nodes (1 .. 4, in the order of their calls) reads of repacked copies, `stream` bytes to 16 columns: `bytes` from
+ * `first`, 0: nothing. With `next` (or NULL) that launch is recorded behind it, and rows of the grid behind the nodes' read the first `ahead` workgroups' share of
+ * each of its (up to two) streams ahead. No GPU work, nothing dereferenced. -1: nodes that do not share a launch, or no such workgroup. */
 typedef struct RocmStepNodes {
   int nodes;
   int columns[4];
   const void* packed[4];
-  uint32_t stream;
+  uint32_t stream, threads;
 } RocmStepNodes;
 typedef struct RocmStepReads {
   uint32_t grid, rows;        /* of the launch */
+  uint32_t ahead;
   uint64_t first, bytes;
 } RocmStepReads;
-int rocm_step_reads(const RocmStepNodes* launch, uint32_t x, uint32_t y, RocmStepReads* out);
+int rocm_step_reads(const RocmStepNodes* launch, const RocmStepNodes* next, uint32_t x, uint32_t y, RocmStepReads* out);
+/* The same of block `block` behind the first `blocks` of another launch that reads up to `budget` bytes of `next` ahead. Returns the blocks of that launch. */
+uint64_t rocm_weights_ahead_reads(const RocmWeightsAhead* next, uint64_t budget, uint32_t threads, uint32_t blocks, uint32_t block, RocmStepReads* out);
 
-/* Decode over constant weights repacked for streaming (M <= 4). `packed` holds rocm_decode_packed_bytes() bytes and is
+/* Decode over constant weights repacked for streaming: up to 16 rows, up to 64 where the shared-activation kernel takes the shape. `packed` holds rocm_decode_packed_bytes() bytes and is
  * filled once by rocm_launch_pack_decode from args->b / scales / zp; rocm_launch_decode_packed then reads only it.
  * `tail`: NULL, or what the provider recorded last while a capture is open on `stream`. */
 int rocm_decode_packed_eligible(const RocmMatMulNBitsArgs* args);

@@ -115,7 +115,7 @@ bool reads_ahead(const PackedLaunch& before, const PackedLaunch& next, PackedLau
     if (!before.carries || next.stream == 0 || own > kShortLaunch) return false;
     RocmWeightsAhead ahead{};
     ahead.first = next.p.packed;
-    ahead.second = next.nodes > 1 && next.grid % 8 == 0 ? next.p.packed_up : nullptr;      // (its workgroups lie on the same XCDs then)
+    ahead.second = next.nodes > 1 && next.grid % kXcds == 0 ? next.p.packed_up : nullptr;      // (its workgroups lie on the same XCDs then)
     ahead.bytes = next.stream;
     ahead.workgroups = next.grid;
     for (int i = 0; i < (ahead.second ? 2 : 1); ++i) {
@@ -137,6 +137,8 @@ bool launch_of(const RocmStepNodes& nodes, PackedLaunch* out)
         one.p.split = 1u << 24;
         one.p.rest.nodes[0] = PackedNode{nullptr, nullptr, one.p.packed, one.p.n, ROCM_DT_F32};
         one.grid = (static_cast<unsigned>(one.p.n) + 15u) / 16u;
+        one.threads = nodes.threads;
+        one.carries = true;
         one.nodes = 1;
         one.stream = nodes.stream;
         const PackedLaunch before = *out;
@@ -209,17 +211,32 @@ extern "C" void rocm_step_tail_reset(RocmStepTail* tail)
     std::lock_guard<std::mutex> lock(tail->mu);
     tail->node = tail->before = nullptr;
 }
-extern "C" int rocm_step_reads(const RocmStepNodes* nodes, uint32_t x, uint32_t y, RocmStepReads* out)
+extern "C" int rocm_step_reads(const RocmStepNodes* nodes, const RocmStepNodes* next, uint32_t x, uint32_t y, RocmStepReads* out)
 {
-    mnb::PackedLaunch launch{};
-    if (nodes->nodes < 1 || nodes->nodes > mnb::kMaxNodes || !mnb::launch_of(*nodes, &launch)) return -1;
+    mnb::PackedLaunch launch{}, behind{}, changed{};
+    auto shared = [](const RocmStepNodes* of, mnb::PackedLaunch* to) { return of->nodes >= 1 && of->nodes <= mnb::kMaxNodes && mnb::launch_of(*of, to); };
+    if (!shared(nodes, &launch) || (next && !shared(next, &behind))) return -1;
+    if (next && mnb::reads_ahead(launch, behind, &changed)) launch = changed;
     const mnb::PackedParams& p = launch.p;
-    *out = RocmStepReads{launch.grid, p.rows(), 0, 0};
+    *out = RocmStepReads{launch.grid, mnb::grid_rows(launch), p.rest.ahead.workgroups, 0, 0};
     if (x >= out->grid || y >= out->rows) return -1;
-    const int n = y == 0 ? p.n : y == 1 ? p.n_up : p.rest.nodes[y].n;                          // (as the kernel finds them)
+    if (y >= p.rows()) {                                                                       // (rows as the kernel tells them apart)
+        mnb::ahead_range(p.rest.ahead, y * p.rest.ahead.grid + x, launch.threads, &out->first, &out->bytes);
+        return 0;
+    }
+    const int n = y == 0 ? p.n : y == 1 ? p.n_up : p.rest.nodes[y].n;
     const uint8_t* const packed = y == 0 ? p.packed : y == 1 ? p.packed_up : p.rest.nodes[y].packed;
     if (!mnb::has_columns(x, n)) return 0;
     out->first = reinterpret_cast<uintptr_t>(packed) + static_cast<uint64_t>(x) * launch.stream;
     out->bytes = launch.stream;
     return 0;
+}
+
+extern "C" uint64_t rocm_weights_ahead_reads(const RocmWeightsAhead* next, uint64_t budget, uint32_t threads, uint32_t blocks, uint32_t block, RocmStepReads* out)
+{
+    mnb::WeightsAhead w;
+    const uint64_t all = mnb::plan_weights_ahead(*next, budget, threads, blocks, 0, &w);
+    *out = RocmStepReads{0, 0, w.workgroups, 0, 0};
+    mnb::ahead_range(w, block, threads, &out->first, &out->bytes);
+    return all;
 }
