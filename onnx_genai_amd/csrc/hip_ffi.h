@@ -244,6 +244,8 @@ int rocm_launch_decode_plain(const RocmMatMulNBitsArgs* args, const void* packed
 /* One row (args->a as the caller has it) whose elements the kernel takes in the order of the sorted weights itself: `order` as
  * rocm_launch_narrow_order leaves it. rocm_decode_plain_gathers says whether it does. */
 int rocm_decode_plain_gathers(const RocmMatMulNBitsArgs* args, int waves);
+/* Waves per SIMD that the builds for 1, 2-4, 5-8 and 9-16 rows are held to (`bits` 4 or 8); a test holds it against what the build reported. */
+int rocm_decode_plain_waves_per_simd(int block_size, int m, int f32_scales, int bf16, int bits);
 int rocm_launch_decode_plain_gathered(const RocmMatMulNBitsArgs* args, const void* packed, const uint16_t* order, int waves, rocm_stream_t stream);
 
 /* Plain sums for 8-bit weights (args->b [N, kb, bs], zp [N, kb] or NULL = 128; scales of the activations' type): a copy of the same form with

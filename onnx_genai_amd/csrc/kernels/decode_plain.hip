@@ -16,7 +16,7 @@ constexpr int plain_waves_per_simd(bool bf16, int bs, int rows, bool f32_scales,
 {
     // [f16 / bf16][4 bits, 4 bits with f32 scales, 8 bits][rows: 1, 2-4, 5-8, 9-16][block 32, 64, 128]
     constexpr unsigned char table[2][3][4][3] = {
-        {{{7, 8, 8}, {6, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{7, 7, 8}, {5, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{8, 7, 8}, {6, 7, 7}, {6, 6, 8}, {5, 6, 6}}},
+        {{{7, 8, 8}, {6, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{7, 7, 8}, {5, 6, 7}, {5, 5, 5}, {4, 4, 4}}, {{8, 8, 8}, {6, 7, 7}, {6, 6, 8}, {5, 6, 6}}},
         {{{7, 8, 8}, {6, 7, 7}, {5, 5, 5}, {4, 4, 4}}, {{6, 7, 8}, {5, 6, 6}, {4, 5, 5}, {4, 4, 4}}, {{7, 8, 8}, {6, 7, 8}, {7, 6, 8}, {5, 6, 6}}},
     };
     return table[bf16][bits == 8 ? 2 : f32_scales ? 1 : 0][rows == 1 ? 0 : rows == 4 ? 1 : rows == 8 ? 2 : 3][bs == 32 ? 0 : bs == 64 ? 1 : 2];
@@ -136,3 +136,8 @@ int launch_plain_wide(const PackedParams& p, int bits, bool bf16, bool f32_scale
 }
 
 }  // namespace mnb
+
+extern "C" int rocm_decode_plain_waves_per_simd(int block_size, int m, int f32_scales, int bf16, int bits)
+{
+    return mnb::plain_waves_per_simd(bf16 != 0, block_size, m <= 1 ? 1 : m <= 4 ? 4 : m <= 8 ? 8 : 16, f32_scales != 0, bits);
+}

@@ -283,6 +283,27 @@ def test_launcher_occupancy_table_matches_the_build():
     assert seen == 2 * 3 * 4 * 2
 
 
+def test_plain_occupancy_table_matches_the_build():
+    """The waves per SIMD that the plain-sum builds are held to are what the build reported: a register more and the compiler gives way without a word."""
+    from onnx_genai_amd import build
+    report = os.path.join(build.OBJ, "kernel_resources.txt")
+    if not os.path.exists(report):
+        pytest.skip("no build report in this tree")
+    lib = C.CDLL(build.LIB)
+    # _ZN3mnb..decode_plain_kernelILb<bf16>ELi<block>ELi<rows staged>E<t|f: scale type>Li<bits>EEEv..., decode_plain_gather_kernelILb<bf16>ELi<block>E<t|f>EEv...
+    pats = (re.compile(r"decode_plain_kernelILb([01])ELi(\d+)ELi(\d+)E([tf])Li([48])EEE\S* .*Occupancy \[waves/SIMD\]=(\d+)"),
+            re.compile(r"decode_plain_gather_kernelILb([01])ELi(\d+)E()([tf])()EE\S* .*Occupancy \[waves/SIMD\]=(\d+)"))
+    seen = [0, 0]
+    for line in open(report).read().splitlines():
+        for i, pat in enumerate(pats):
+            m = pat.search(line)
+            if m:
+                bf16, bs, rows, f32, bits, built = int(m.group(1)), int(m.group(2)), int(m.group(3) or 1), m.group(4) == "f", int(m.group(5) or 4), int(m.group(6))
+                assert lib.rocm_decode_plain_waves_per_simd(bs, rows, int(f32), bf16, bits) == built, line
+                seen[i] += 1
+    assert seen == [2 * 3 * 4 * 3, 2 * 3 * 2]
+
+
 class _FfiArgs(C.Structure):
     """RocmMatMulNBitsArgs of csrc/hip_ffi.h (the internal kernel-launch interface), for the calls below that do no GPU work."""
     _fields_ = [("a", C.c_void_p), ("b", C.c_void_p), ("scales", C.c_void_p), ("zp", C.c_void_p), ("bias", C.c_void_p), ("y", C.c_void_p),
