@@ -236,7 +236,9 @@ void nxrt_rocm_ep_event_destroy(NxrtRocmEp* ep, NxrtRocmEvent* event);
  * ep-cuda matmul_nbits.rs:11136-11162) ---------------------------------------------------------
  * Between begin and end, execute calls on this provider are recorded instead of run. Only calls that
  * allocate nothing may be recorded: accuracy_level 0 always, accuracy_level 4 with a caller workspace.
- * A recorded graph replays the same launches on the same device pointers. */
+ * A recorded graph does on the same device pointers what the calls would have done, bit for bit, though not launch for launch: calls
+ * made in a row that read the same activations and do not depend on each other may share a launch (*out_num_nodes is smaller
+ * then), and a launch may read weights of the recorded call behind it into the caches ahead of time. */
 typedef struct NxrtRocmGraph NxrtRocmGraph;
 NxrtStatus nxrt_rocm_ep_capture_begin(NxrtRocmEp* ep);
 NxrtStatus nxrt_rocm_ep_capture_end(NxrtRocmEp* ep, NxrtRocmGraph** out_graph, uint64_t* out_num_nodes);
@@ -245,6 +247,9 @@ void nxrt_rocm_ep_graph_release(NxrtRocmEp* ep, NxrtRocmGraph* graph);
 
 /* Counters a harness reads to prove the provider, not a fallback, did the work
  * (the role of nxrt_ep_compiled_node_count in ep-cuda-plugin/src/lib.rs:345-372). */
+/* Counts the steps of calls that were run or recorded: one for a product, with all that it takes (quantized rows, expanded weights,
+ * blocks of rows, slices of K), and one for each normalization, gather of act-order rows and SwiGLU epilogue beside it. A recorded
+ * call counts the same whether it is a launch of its own or shares one; replays do not count. */
 uint64_t nxrt_rocm_ep_kernel_launch_count(const NxrtRocmEp* ep);
 uint64_t nxrt_rocm_live_provider_count(void);
 /* Device allocations (hipMalloc calls) the library has made in this process so far. */

@@ -193,4 +193,9 @@ def test_a_narrow_node_may_come_first(ep, m, dt, bs):
     x = rows(ep, m, k, dt, 7)
     nodes = [Node(ep, k, n, bs, dt, n, bias=bias) for n, bias in ((16, "row"), (130, None), (1000, "row"))]
     y = [ep.allocate(m * node.n * 2) for node in nodes]
-    check(ep, [(node, x.ptr, out.ptr, m) for node, out in zip(nodes, y)], 1)
+    calls = [(node, x.ptr, out.ptr, m) for node, out in zip(nodes, y)]
+    check(ep, calls, 1)
+    before = ep.kernel_launch_count()
+    graph = recorded(ep, calls)
+    assert ep.kernel_launch_count() - before == 2 * len(calls)                     # (run once and recorded once; a recorded call counts whether or not it shares a launch)
+    graph.release()
