@@ -4,7 +4,7 @@
 // asks for less: q, k and v read one input, and so do gate and up of a model that was exported without fused nodes. A launch that depends on another costs
 // about 2 us before it has read a byte, more than half the time of such a node of a 0.5B model.
 // A node that could run beside the one recorded just before it is therefore not recorded as a launch of its own: it becomes a further row of that launch's
-// grid, with its own columns, bias and result. Each keeps its own split of K, so its sums are those of a launch by itself, bit for bit.
+// grid, with its own columns, bias and result; every row is as long as the widest node's, and workgroups beyond a row's columns read nothing. Each keeps its own split of K, so its sums are those of a launch by itself, bit for bit.
 // 24 layers of a 0.5B model at one row, f16, block 32: 169 launches 585 us, 97 launches 393.
 // What may join: the capture's only open end is the launch recorded last (anything recorded in between, by whomever, is another end); the same kernel
 // build, activations, rows, K, split of K and result type; and no result of one that is an input or a result of the other.
@@ -87,7 +87,8 @@ bool joined(const PackedLaunch& to, const PackedLaunch& add, PackedLaunch* out)
     return static_cast<int64_t>(out->grid) * out->nodes <= 2 * busy + 512;
 }
 
-// Launches that read no more weights than this leave the memory idle for long enough to read the next one's, up to this many together. Steps of a 0.5B model at
+// Launches that read no more weights than this leave the memory idle for long enough to read the next one's, up to this many together (bytes, as in
+// swiglu.hip: the memory's rate and the size of the near caches set them). Steps of a 0.5B model at
 // one row and of a 7B model at one / 16 rows: 392, 1,117 / 1,538 us with nothing read ahead here, 388, 1,115 / 1,527 with launches of at most 1 MB, 387, 1,114 / 1,528 of
 // 5 MB, 383, 1,112 / 1,527 of 10 MB; 14, 18 or 22 MB together are level to 0.5 %.
 constexpr uint64_t kShortLaunch = 10000000, kAheadTogether = 18000000;

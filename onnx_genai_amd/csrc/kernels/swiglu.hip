@@ -36,10 +36,12 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const uint16_t* __restrict_
 // row through LDS, and every wave sums it from there - lanes 0..31 the running sums s0 and s1 of the reference's lanes, lanes 32..63
 // s2 and s3 - so that nothing but one barrier lies between the row's arrival and its results. K = 3584, one / 16 rows, as a node of a
 // recorded step: 6.2 / 8.0 us with one wave summing two rows straight from memory, 4.6 / 4.8 us so (3.0 with everything in a near cache).
-// Weights that a normalization launch brings to the near caches, at most: what fits the time that the launch takes anyway. 7B steps of 142 and 170 launches at
+constexpr int kHeld = 2;                     // 16-byte pieces of the row a thread keeps: 4096 elements a row
+
+// Weights that a normalization launch brings to the near caches, at most: what fits the time that the launch takes anyway. (Bytes and no multiple of the CUs: the memory's rate sets them,
+// and the eight caches of 4 MB that have to hold them.) 7B steps of 142 and 170 launches at
 // one / 16 rows (29 and 57 normalizations), bytes read ahead 0, 2, 4, 8, 16 MB: 1,140 / 1,553, 1,133 / 1,545, 1,125 / 1,536, 1,113 / 1,519, 1,128 / 1,526 us.
 constexpr uint32_t kAheadBytes = 8000000;
-constexpr int kHeld = 2;                     // 16-byte pieces of the row a thread keeps: 4096 elements a row
 
 // x + (x of the lane `N` further on in its row of 16, cyclically)
 template <int N>
